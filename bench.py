@@ -343,7 +343,6 @@ def main():
                           "triples": st.get("triples" + sfx), "triples_gemm": st.get("triples_gemm" + sfx),
                           "triples_w_first": st.get("triples_w_first" + sfx),
                           "triples_w_slices": st.get("triples_w_slices" + sfx),
-                          "triples_w_batched": st.get("triples_w_batched" + sfx),
                           "triples_energy": st.get("triples_energy" + sfx)}), flush=True)
         ctx.close()
         return
@@ -385,35 +384,25 @@ def main():
     # rocprofv3 lists them separately)
     FP32_MFMA_PEAK_TFLOPS = 157.3
     BF16_MFMA_PEAK_TFLOPS = 2500.0
-    # launches per timed span: the (T) W build of a chunk is three launches (FP64, FP32), or in split-BF16x3
-    # the first launch and the other four classes as one launch over the slices of W (or two batched
-    # launches where v does not fit the slice tiles), each with a span of its own
-    launches_per_call = {"ladder": 1, "triples_gemm": 3, "triples_w_first": 1, "triples_w_slices": 1,
-                         "triples_w_batched": 2}
+    # launches per timed span: the (T) W build of a chunk is the first launch and the slice launch, each with
+    # a span of its own
+    launches_per_call = {"ladder": 1, "triples_gemm": 2, "triples_w_first": 1, "triples_w_slices": 1}
     # FP64/FP32 kernel template arguments: BM, BN, BK, TA, TB, waves-per-EU hint, tag, FP32 MFMA,
-    # operand type, output type, lanes along M, two-segment K; bf16x3 kernel: BK, TA, TB, tag,
-    # operand type, output type, vector loads, lanes along M, two-segment K
+    # operand type, output type; bf16x3 kernel: BK, TA, TB, tag, operand type, output type, vector loads, BM;
+    # W build: element type, K segments, 16-wide blocks / K segments, 32-wide blocks of a wavefront
     variants = {
-        "": ({"ladder": "k_gemm<64, 64, 16, false, false, 4, 1, false, double, double, true, false> (PP ladder, "
-                        "FP64 MFMA)",
-              "triples_gemm": "k_gemm<64, 64, 8, false, false, 4, 2, false, double, double, {true|false}, true> ((T) "
-                              "W build, FP64 MFMA)"},
+        "": ({"ladder": "k_gemm<64, 64, 16, false, false, 4, 1, false, double, double> (PP ladder, FP64 MFMA)",
+              "triples_gemm": "k_triples_w<double, {2|4}, NB> ((T) W build, FP64 MFMA)"},
              FP64_MFMA_PEAK_TFLOPS, "FP64 MFMA dense"),
-        "_fp32": ({"ladder": "k_gemm<64, 64, 16, false, false, 4, 1, true, float, double, true, false> (PP ladder, "
-                             "FP32 MFMA)",
-                   "triples_gemm": "k_gemm<64, 64, 8, false, false, 4, 2, true, float, float, {true|false}, true> "
-                                   "((T) W build, FP32 MFMA)"},
+        "_fp32": ({"ladder": "k_gemm<64, 64, 16, false, false, 4, 1, true, float, double> (PP ladder, FP32 MFMA)",
+                   "triples_gemm": "k_triples_w<float, {2|4}, NB> ((T) W build, FP32 MFMA)"},
                   FP32_MFMA_PEAK_TFLOPS, "FP32 MFMA dense"),
         "_bf16x3": ({"ladder": "k_gemm_bf3<16, false, false, 1, float, double, true, 256> (PP ladder, "
                                "split-BF16x3 MFMA, 256 x 128 tiles)",
-                     "triples_w_first": "k_gemm_bf3_sl<2> (k_gemm_bf3_kk<{192|128}, true> where its 32-bit indexing "
-                                        "does not hold) ((T) W build, first launch: classes abc + bac as one GEMM with "
-                                        "two K segments, split-BF16x3 MFMA on k-contiguous operands copied straight "
-                                        "into LDS)",
-                     "triples_w_slices": "k_gemm_bf3_sl<4> ((T) W build: classes cab, acb, cba, bca as one launch "
-                                         "over the fixed-c slices of W, 192 x 192 tiles, split-BF16x3 MFMA)",
-                     "triples_w_batched": "k_gemm_bf3_kk<{192|128}, {true|false}> ((T) W build: classes cab + acb and "
-                                          "cba + bca as two batched launches, split-BF16x3 MFMA)"},
+                     "triples_w_first": "k_triples_w_bf3<2, {2|3}> ((T) W build, first launch: classes abc + bac as "
+                                        "one GEMM per run of k with two K segments, split-BF16x3 MFMA)",
+                     "triples_w_slices": "k_triples_w_bf3<4, {2|3}> ((T) W build: classes cab, acb, cba, bca over "
+                                         "the fixed-c slices of W, split-BF16x3 MFMA)"},
                     BF16_MFMA_PEAK_TFLOPS / 3.0, "BF16 MFMA dense / 3 products (FP32-equivalent)"),
     }
 

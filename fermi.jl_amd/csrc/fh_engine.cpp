@@ -367,11 +367,11 @@ static void contract(Ctx& c, double alpha, const TView& A, const std::string& ia
   auto gemm = [&](bool ta, bool tb, int64_t m, int64_t n, double al, const void* a, int64_t la, const void* b,
                   int64_t lb, double be, const double* cc, double* d, int64_t ld) {
     if (bf3)
-      gemm_bf3<float, double>(c.s, ta, tb, m, n, Ksz, al, static_cast<const float*>(a), la, 0,
-                              static_cast<const float*>(b), lb, 0, be, cc, ld, 0, d, ld, 0, 1, 0, nullptr);
+      gemm_bf3(c.s, ta, tb, m, n, Ksz, al, static_cast<const float*>(a), la, static_cast<const float*>(b), lb, be, cc,
+               ld, d, ld, 0);
     else
       gemm_f64(c.s, ta, tb, m, n, Ksz, al, static_cast<const double*>(a), la, 0, static_cast<const double*>(b), lb, 0,
-               be, cc, ld, 0, d, ld, 0, 1, 0, work.d(), wsz, nullptr, c.lowp != 0);
+               be, cc, ld, 0, d, ld, 0, 1, 0, work.d(), wsz, c.lowp != 0);
   };
   if (cmode == 0) {
     gemm(transA, transB, Msz, Nsz, alpha, pA, lda, pB, ldb, beta, C.p, C.p, Msz);
@@ -572,8 +572,8 @@ static void residual(Ctx& c, const double* t1p, const double* t2p, double* R1, d
       }
       if (c.lowp == 2) {
         Timer tl(c, "ladder_bf16x3", 2.0 * o_ * o_ * v_ * v_ * v_ * v_);
-        gemm_bf3<float, double>(c.s, false, false, o * o, v * v, v * v, 1.0, tau32.f(), o * o, 0, bY.f(), v * v, 0, 1.0,
-                                P.p, o * o, 0, P.p, o * o, 0, 1, 1, nullptr);
+        gemm_bf3(c.s, false, false, o * o, v * v, v * v, 1.0, tau32.f(), o * o, bY.f(), v * v, 1.0, P.p, o * o, P.p,
+                 o * o, 1);
       } else {
         Timer tl(c, "ladder_fp32", 2.0 * o_ * o_ * v_ * v_ * v_ * v_);
         gemm_f32_fd(c.s, o * o, v * v, v * v, 1.0, tau32.f(), o * o, bY.f(), v * v, 1.0, P.p, o * o, P.p, o * o, 1);
@@ -754,7 +754,7 @@ static void mp2_energy_noalloc(Ctx& c, int o, int v, int naux, const double* eo,
     const int n = std::min(nj, o - j0);
     // X[(i,a),(b,j)] = sum_Q Bov[Q,(i,a)] Bvo[Q,(b,j)]
     gemm_f64(c.s, true, false, ov, (int64_t)v * n, Q, 1.0, Bov, Q, 0, Bvo + Q * v * j0, Q, 0, 0.0, nullptr, ov, 0, X,
-             ov, 0, 1, 0, nullptr, 0, nullptr, false, nullptr);
+             ov, 0, 1, 0);
     mp2_pairs(c.s, o, v, j0, n, X, eo, ev, part + np);
     np += mp2_pairs_blocks(v, n);
   }
@@ -1235,58 +1235,6 @@ static void solve(Ctx& c, const fh_cc_opts& op, fh_cc_result& res) {
 }
 
 // ------------------------------------------------------------------ (T), ijk.jl:20-150
-template <typename TO>
-__global__ void k_build_av(int o, int v, int ndp, bool swap_xy, bool kfast, const double* __restrict__ ovvv,
-                           const double* __restrict__ t2, TO* __restrict__ av) {
-  // AV[(x,y), d', n] : d' < v  -> (n y | x d') = OVVV[n, y, x, d']   (ijk2.jl:33 vvvo layout)
-  //                    v <= d' < v+o -> -T2[n, l, y, x], l = d' - v  (T2_n with the GEMM's minus sign)
-  //                    d' >= v+o -> 0 (K padded to ndp, a multiple of 8, for aligned vector loads and
-  //                    8-wide k chunks)
-  // The GEMM operand AV_n is rows (x,y) x k = d' with leading dimension v^2: consecutive k lie v^2
-  // elements apart, so that a k tile of the W-build GEMMs stays within a few pages (with n between
-  // (x,y) and d' they lay v^2 o elements apart, one page per k).  swap_xy stores the rows as (y,x).
-  // kfast stores AV[d', (x,y), n] instead (k contiguous, leading dimension ndp: the operand of the
-  // split-BF16x3 W build, whose 16-byte copies carry 4 consecutive k of one row).
-  const int64_t vv = (int64_t)v * v, nd = (int64_t)v + o;
-  const int64_t total = vv * o * ndp;
-  for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < total; idx += (int64_t)gridDim.x * 256) {
-    int64_t r0, r1, dp, n;
-    if (kfast) {
-      dp = idx % ndp; r0 = (idx / ndp) % v; r1 = (idx / ((int64_t)ndp * v)) % v; n = idx / (vv * ndp);
-    } else {
-      r0 = idx % v; r1 = (idx / v) % v; dp = (idx / vv) % ndp; n = idx / (vv * ndp);
-    }
-    const int64_t x = swap_xy ? r1 : r0, y = swap_xy ? r0 : r1;
-    double val = 0.0;
-    if (dp < v) val = ovvv[n + (int64_t)o * (y + (int64_t)v * (x + (int64_t)v * dp))];
-    else if (dp < nd) {
-      const int64_t l = dp - v;
-      val = -t2[n + (int64_t)o * (l + (int64_t)o * (y + (int64_t)v * x))];
-    }
-    av[idx] = (TO)val;
-  }
-}
-template <typename TO>
-__global__ void k_build_bv(int o, int v, int ndp, bool swap_pq, const double* __restrict__ t2,
-                           const double* __restrict__ ooov, TO* __restrict__ bv) {
-  // Bcat_{p,q}[d', z]: d' < v -> T2p[d', z, p, q] = T2[q, p, z, d'];  v <= d' < v+o -> ovoo[l, z, p, q] =
-  // OOOV[l, p, q, z]; d' >= v+o -> 0 (padding); stored as bv[d', z, p, q] (swap_pq = false) or
-  // bv[d', z, q, p] (swap_pq = true) with leading dimension ndp
-  const int64_t nd = (int64_t)v + o;
-  const int64_t total = (int64_t)ndp * v * o * o;
-  for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < total; idx += (int64_t)gridDim.x * 256) {
-    const int64_t dp = idx % ndp, z = (idx / ndp) % v, r = (idx / ((int64_t)ndp * v)) % o,
-                  s = idx / ((int64_t)ndp * v * o);
-    const int64_t p = swap_pq ? s : r, q = swap_pq ? r : s;
-    double val = 0.0;
-    if (dp < v) val = t2[q + (int64_t)o * (p + (int64_t)o * (z + (int64_t)v * dp))];
-    else if (dp < nd) {
-      const int64_t l = dp - v;
-      val = ooov[l + (int64_t)o * (p + (int64_t)o * (q + (int64_t)o * z))];
-    }
-    bv[idx] = (TO)val;
-  }
-}
 __global__ void k_accumulate(int64_t n, const double* __restrict__ partials, double* __restrict__ acc) {
   // single block; fixed order -> deterministic
   __shared__ double red[256];
@@ -1301,98 +1249,31 @@ __global__ void k_accumulate(int64_t n, const double* __restrict__ partials, dou
   if (threadIdx.x == 0) *acc += red[0];
 }
 
-// one W-build GEMM of the (T) driver (tag 2), FP64 or FP32 data
-static void tgemm(hipStream_t st, int64_t M, int64_t N, int64_t K, const double* A, int64_t lda, int64_t sA,
-                  const double* B, int64_t ldb, int64_t sB, double beta, double* W, int64_t ldd, int64_t sD,
-                  int64_t batch, const OutMap* map, bool, bool ka, const KSeg* seg) {
-  FH_CHECK(!ka, -3, "(T) W build: k-contiguous A is the split-BF16x3 layout");
-  gemm_f64(st, false, false, M, N, K, 1.0, A, lda, sA, B, ldb, sB, beta, beta != 0.0 ? W : nullptr, ldd, sD, W, ldd, sD,
-           batch, 2, nullptr, 0, map, false, seg);
-}
-static void tgemm(hipStream_t st, int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, int64_t sA,
-                  const float* B, int64_t ldb, int64_t sB, double beta, float* W, int64_t ldd, int64_t sD,
-                  int64_t batch, const OutMap* map, bool bf3, bool ka, const KSeg* seg) {
-  FH_CHECK(bf3 || !ka, -3, "(T) W build: k-contiguous A is the split-BF16x3 layout");
-  if (bf3)
-    gemm_bf3<float, float>(st, ka, false, M, N, K, 1.0, A, lda, sA, B, ldb, sB, beta, beta != 0.0 ? W : nullptr, ldd,
-                           sD, W, ldd, sD, batch, 2, map, seg);
-  else
-    gemm_f32_ff(st, M, N, K, 1.0, A, lda, sA, B, ldb, sB, beta, beta != 0.0 ? W : nullptr, ldd, sD, W, ldd, sD, batch,
-                2, map, seg);
-}
-
-// (T) with W-build operands and W stored as T (double: FP64 path; float: FP32 MFMA path, or
-// split-BF16x3 MFMA when bf3)
+// (T) with W stored as T (double: FP64 path; float: FP32 MFMA W build, or split-BF16x3 when bf3).
 // Triples t0 .. t0+nt-1 of the reference's loop order (for i, for j <= i, for k <= j; ijk.jl:49,63,83),
 // t(i,j,k) = i(i+1)(i+2)/6 + j(j+1)/2 + k; nt < 0: all triples.
+//
+// The triples go in chunks of W slots, several (i, j) pairs to a chunk; each chunk is two W-build launches
+// (fh_triples.hip) and one energy launch over device tables that are made and uploaded once.
 template <typename T>
 static double triples_t(Ctx& c, bool bf3, int64_t t0 = 0, int64_t nt = -1) {
   prepare(c);
   FH_CHECK(c.have_amp, -6, "no amplitudes for (T)");
   const bool lowp = std::is_same<T, float>::value;
-  const int64_t o = c.o, v = c.v, vv = v * v;
-  const int64_t nd = ((v + o + 7) / 8) * 8;  // K = v + o padded with zeros to a multiple of 8
+  const int fmt = bf3 ? 2 : (lowp ? 1 : 0);
+  const int64_t o = c.o, v = c.v, vv = v * v, v3 = vv * v;
   const double o_ = (double)o, v_ = (double)v;
   const double ntrip_all = o_ * (o_ + 1) * (o_ + 2) / 6.0;
   const double ntrip = nt < 0 ? ntrip_all : std::max(0.0, std::min((double)nt, ntrip_all - (double)t0));
   const std::string sfx = bf3 ? "_bf16x3" : (lowp ? "_fp32" : "");
   Timer tall(c, "triples" + sfx, ntrip * 12.0 * (v_ * v_ * v_ * v_ + o_ * v_ * v_ * v_));
-  // AV[(x,y),d',n] and the row-swapped copy AVs[(y,x),d',n] share one allocation;
-  // BVq (Bcat_{p,q} stored [d',z,q,p]) and BVp (stored [d',z,p,q]) likewise
-  const int64_t avsz = vv * o * nd, bvsz = nd * v * o * o;
-  // the split-BF16x3 W build takes AV k-contiguous (AV[d', (x,y), n], leading dimension nd)
-  const bool kfast = bf3;
-  const int64_t alda = kfast ? nd : vv;
-  // split-BF16x3 with v close below a multiple of 192: the four batched classes as one launch over the
-  // v x v slices of W (FERMIHIP_TRIPLES_SLICE = 1 / 0 forces it on / off, for tests)
-  const char* slice_env = std::getenv("FERMIHIP_TRIPLES_SLICE");
-  const bool slices = kfast && (slice_env ? std::atoi(slice_env) == 1 : bf3_slices_fit(v));
-  // the first launch on the 192 x 192 two-segment kernel where it fits (FERMIHIP_TRIPLES_PAIR192 = 0 keeps
-  // it on k_gemm_bf3_kk, for tests)
-  const char* pair_env = std::getenv("FERMIHIP_TRIPLES_PAIR192");
-  const bool pair_ok = kfast && !(pair_env && std::atoi(pair_env) == 0);
-  Buf AVall(c.pool.get(), (size_t)(2 * avsz) * sizeof(T)), BVqp(c.pool.get(), (size_t)(2 * bvsz) * sizeof(T));
-  T* AV = static_cast<T*>(AVall.p);
-  T* AVs = AV + avsz;
-  T* BVq = static_cast<T*>(BVqp.p);
-  T* BVp = BVq + bvsz;
-  Buf T1p = dalloc(c, v * o), vvoo = dalloc(c, vv * o * o), vvb;
-  {
-    auto g = [](int64_t n) { int64_t b = (n + 255) / 256; return (unsigned)std::min<int64_t>(b, 65536 * 4); };
-    hipLaunchKernelGGL(k_build_av<T>, dim3(g(avsz)), dim3(256), 0, c.s, (int)o, (int)v, (int)nd, false, kfast,
-                       c.OVVV.d(), c.T2.d(), AV);
-    hipLaunchKernelGGL(k_build_av<T>, dim3(g(avsz)), dim3(256), 0, c.s, (int)o, (int)v, (int)nd, true, kfast,
-                       c.OVVV.d(), c.T2.d(), AVs);
-    hipLaunchKernelGGL(k_build_bv<T>, dim3(g(bvsz)), dim3(256), 0, c.s, (int)o, (int)v, (int)nd, false, c.T2.d(),
-                       c.OOOV.d(), BVp);
-    hipLaunchKernelGGL(k_build_bv<T>, dim3(g(bvsz)), dim3(256), 0, c.s, (int)o, (int)v, (int)nd, true, c.T2.d(),
-                       c.OOOV.d(), BVq);
-    FH_HIP(hipGetLastError());
-    perm(c, tv(c.T1.d(), {o, v}), "ia", tv(T1p.d(), {v, o}), "ai", 1.0, 0.0);
-    perm(c, tv(c.OVOV.d(), {o, v, o, v}), "iajb", tv(vvoo.d(), {v, v, o, o}), "abij", 1.0, 0.0);
-    vvb = dalloc(c, triples_vv_blocked_elems((int)o, (int)v));
-    triples_block_vv(c.s, (int)o, (int)v, vvoo.d(), vvb.d());
-    vvoo.reset();
-  }
-  // k-chunk: W for all k of a chunk, bounded to ~8 GB (a second stream for consecutive pairs was measured
-  // to gain nothing: the launches of one pair already fill the device)
-  const int64_t v3 = vv * v;
-  int64_t KC = std::max<int64_t>(1, std::min<int64_t>(o, (int64_t)(8e9 / ((double)sizeof(T) * (double)v3))));
-  Buf Wbuf(c.pool.get(), (size_t)(v3 * KC) * sizeof(T));
-  std::vector<int> orb;
-  triples_orbits((int)v, orb);
-  const int64_t norb = (int64_t)orb.size() / 3;
-  Buf orbits(c.pool.get(), orb.size() * sizeof(int));
-  FH_HIP(hipMemcpyAsync(orbits.p, orb.data(), orb.size() * sizeof(int), hipMemcpyHostToDevice, c.s));
-  FH_HIP(hipStreamSynchronize(c.s));
-  Buf part = dalloc(c, norb * KC + 16);
-  Buf acc = dalloc(c, 1);
-  fill_f64(c.s, 1, 0.0, acc.d());
-  const int64_t bstride = nd * v;  // one (p,q) column block of BVp/BVq
-  // output maps into W[a + v*b + v^2*c + v^3*kk]
-  OutMap m_acb, m_bca;
-  m_acb.rmod = v; m_acb.rs0 = 1; m_acb.rs1 = vv; m_acb.cmod = 0; m_acb.cs0 = v;                   // rows (a,c), col b
-  m_bca.rmod = v; m_bca.rs0 = v; m_bca.rs1 = vv; m_bca.cmod = 0; m_bca.cs0 = 1;                   // rows (b,c), col a
+
+  // runs of consecutive k of one (i, j)
+  struct Run {
+    int i, j, k0, nk;
+  };
+  std::vector<Run> runs;
+  int64_t ntot = 0;
   const int64_t tend = nt < 0 ? INT64_MAX : t0 + nt;
   for (int64_t i = 0; i < o; ++i)
     for (int64_t j = 0; j <= i; ++j) {
@@ -1400,80 +1281,108 @@ static double triples_t(Ctx& c, bool bf3, int64_t t0 = 0, int64_t nt = -1) {
       const int64_t kbeg = std::max<int64_t>(0, t0 - base);
       int64_t kend = (i == j) ? j : j + 1;  // i=j=k has zero weight (ijk.jl:133)
       if (tend - base < kend) kend = std::max<int64_t>(0, tend - base);
-      for (int64_t k0 = kbeg; k0 < kend; k0 += KC) {
-        const int64_t nk = std::min<int64_t>(KC, kend - k0);
-        hipStream_t sq = c.s;
-        T* W = static_cast<T*>(Wbuf.p);
-        std::unique_ptr<Timer> tg(new Timer(c, "triples_gemm" + sfx,
-                                            12.0 * (double)vv * (double)v * (double)(v + o) * (double)nk, 0.0, sq));
-        // The six permutation classes of ijk2.jl:109-153, G = AV_n (rows (x,y)) * Bcat_{p,q}
-        // (cols z), accumulated into W[a,b,c,kk] (W[a,b,c] += G[class-permuted (a,b,c)]).  The two
-        // classes of each output layout form one GEMM with two K segments:
-        //   abc (n=j, B_{i,k}, rows (a,b), cols (c,kk)) + bac (n=i row-swapped, B_{j,k}): identity map;
-        //   cab (n=i row-swapped, B_{k,j}) + acb (n=k, B_{i,j}): rows (a,c), col b, batched over kk;
-        //   cba (n=j row-swapped, B_{k,i}) + bca (n=k, B_{j,i}): rows (b,c), col a, batched over kk.
-        // With c fixed the last four are all GEMMs with rows a and columns b; the split-BF16x3 path
-        // runs them as one four-segment launch over the slices W[:, :, c, kk] where v fits its tiles.
-        KSeg s_bac, s_acb, s_bca;
-        const int64_t an = vv * nd;  // one occupied index n of AV / AVs
-        // per-launch spans beside the chunk's: the first launch (two classes) and the other four classes
-        const double fcls = 2.0 * (double)vv * (double)v * (double)(v + o) * (double)nk;  // one class
-        std::unique_ptr<Timer> tf(new Timer(c, "triples_w_first" + sfx, 2.0 * fcls, 0.0, sq));
-        s_bac.A = AVs + an * i; s_bac.lda = alda; s_bac.B = BVq + bstride * (k0 + o * j); s_bac.ldb = nd; s_bac.K1 = nd;
-        bool pair192 = false;
-        if constexpr (std::is_same<T, float>::value) {
-          // the first launch on the slice kernel's 192 x 192 tiles (3 x 3 blocks per wavefront: 27 MFMAs per
-          // k step for 48 split values, against 18 for 40 in k_gemm_bf3_kk) wherever its 32-bit indexing
-          // holds (M = v^2 and N = v nk pad little at any v)
-          if (pair_ok && bf3_pair192_fits(vv, v * nk, nd, vv)) {
-            gemm_bf3_pair192(sq, vv, v * nk, nd, AV + an * j, BVq + bstride * (k0 + o * i), AVs + an * i,
-                             BVq + bstride * (k0 + o * j), W, vv);
-            pair192 = true;
-          }
-        }
-        if (!pair192)
-          tgemm(sq, vv, v * nk, 2 * nd, AV + an * j, alda, 0, BVq + bstride * (k0 + o * i), nd, 0, 0.0, W, vv, 0, 1,
-                nullptr, bf3, kfast, &s_bac);
-        tf.reset();
-        std::unique_ptr<Timer> tr(new Timer(c, (slices ? "triples_w_slices" : "triples_w_batched") + sfx, 4.0 * fcls, 0.0, sq));
-        if (slices) {
-          // the four classes as GEMMs over the slices W[:, :, c, kk] (rows a, columns b), batch c + v kk
-          // (slices is set for the split-BF16x3 path only, whose operands and W are FP32)
-          if constexpr (std::is_same<T, float>::value) {
-            SliceSeg sl;
-            // acb and bca read the same block AV_k[(., c)] (as rows, then as columns): adjacent in k, so
-            // that the second read finds it in L2
-            sl.A[0] = AVs + an * i; sl.sAc[0] = nd * v; sl.sAk[0] = 0;                    // cab: AV_i[(c,a)]
-            sl.B[0] = BVp + bstride * (k0 + o * j); sl.sBc[0] = 0; sl.sBk[0] = bstride;  //      Bcat_{k,j}[., b]
-            sl.A[1] = BVp + bstride * (k0 + o * i); sl.sAc[1] = 0; sl.sAk[1] = bstride;  // cba: Bcat_{k,i}[., a]
-            sl.B[1] = AVs + an * j; sl.sBc[1] = nd * v; sl.sBk[1] = 0;                   //      AV_j[(c,b)]
-            sl.A[2] = AV + an * k0; sl.sAc[2] = nd * v; sl.sAk[2] = an;                  // acb: AV_k[(a,c)]
-            sl.B[2] = BVp + bstride * (i + o * j); sl.sBc[2] = 0; sl.sBk[2] = 0;         //      Bcat_{i,j}[., b]
-            sl.A[3] = BVp + bstride * (j + o * i); sl.sAc[3] = 0; sl.sAk[3] = 0;         // bca: Bcat_{j,i}[., a]
-            sl.B[3] = AV + an * k0; sl.sBc[3] = nd * v; sl.sBk[3] = an;                  //      AV_k[(b,c)]
-            gemm_bf3_slices(sq, v, nd, v, nk, sl, 1.0, W, v, vv);
-          }
-        } else {
-          s_acb.A = AV + an * k0; s_acb.lda = alda; s_acb.sA = an; s_acb.B = BVp + bstride * (i + o * j);
-          s_acb.ldb = nd; s_acb.K1 = nd;
-          tgemm(sq, vv, v, 2 * nd, AVs + an * i, alda, 0, BVp + bstride * (k0 + o * j), nd, bstride, 1.0, W, vv, v3,
-                nk, &m_acb, bf3, kfast, &s_acb);
-          s_bca.A = AV + an * k0; s_bca.lda = alda; s_bca.sA = an; s_bca.B = BVp + bstride * (j + o * i);
-          s_bca.ldb = nd; s_bca.K1 = nd;
-          tgemm(sq, vv, v, 2 * nd, AVs + an * j, alda, 0, BVp + bstride * (k0 + o * i), nd, bstride, 1.0, W, vv, v3,
-                nk, &m_bca, bf3, kfast, &s_bca);
-        }
-        tr.reset();
-        tg.reset();
-        // algorithmic bytes: the chunk's W read once
-        Timer te(c, "triples_energy" + sfx, 0.0, (double)sizeof(T) * (double)v3 * (double)nk, sq);
-        int64_t nb = 0;
-        triples_energy(sq, (int)o, (int)v, (int)i, (int)j, (int)k0, (int)nk, W, static_cast<const int*>(orbits.p),
-                       T1p.d(), vvb.d(), c.eo.d(), c.ev.d(), part.d(), &nb);
-        hipLaunchKernelGGL(k_accumulate, dim3(1), dim3(256), 0, sq, nb, part.d(), acc.d());
-        FH_HIP(hipGetLastError());
+      if (kend > kbeg) {
+        runs.push_back({(int)i, (int)j, (int)kbeg, (int)(kend - kbeg)});
+        ntot += kend - kbeg;
       }
     }
+  if (runs.empty()) return c.last_et = 0.0;
+
+  const TriplesTiles tt = triples_tiles(fmt, (int)o, (int)v, (double)ntot / (double)runs.size());
+  const int64_t KC = triples_chunk_slots((int)v, (int)sizeof(T), tt, ntot);
+
+  // tables of every chunk: W slots, column tiles of the first launch, energy runs
+  struct Chunk {
+    int64_t slots, cols, eruns;  // offsets (ints) into the table
+    int nslot, ncol, nerun;
+  };
+  std::vector<int> tab, orb;
+  std::vector<Chunk> chunks;
+  triples_orbits((int)v, orb);
+  const int64_t norb = (int64_t)orb.size() / 3;
+  int max_erun = 0;
+  for (size_t r = 0, done = 0; r < runs.size();) {
+    std::vector<Run> in;
+    int64_t ns = 0;
+    while (r < runs.size() && ns < KC) {
+      const int take = (int)std::min<int64_t>(runs[r].nk - (int64_t)done, KC - ns);
+      in.push_back({runs[r].i, runs[r].j, runs[r].k0 + (int)done, take});
+      ns += take;
+      done += take;
+      if ((int)done == runs[r].nk) { ++r; done = 0; }
+    }
+    Chunk ch;
+    ch.nslot = (int)ns;
+    ch.slots = (int64_t)tab.size();
+    for (const Run& q : in)
+      for (int k = q.k0; k < q.k0 + q.nk; ++k) tab.insert(tab.end(), {q.i, q.j, k, 0});
+    ch.cols = (int64_t)tab.size();
+    int slot = 0;
+    for (const Run& q : in) {
+      triples_col_tiles(tt, (int)v, q.i, q.j, q.k0, q.nk, slot, tab);
+      slot += q.nk;
+    }
+    ch.ncol = (int)(((int64_t)tab.size() - ch.cols) / 8);
+    ch.eruns = (int64_t)tab.size();
+    const int kpw = triples_energy_kpw((int)norb, (int)ns);
+    slot = 0;
+    for (const Run& q : in) {
+      const int np = (q.nk + kpw - 1) / kpw;
+      for (int p = 0; p < np; ++p) {
+        const int b = q.nk * p / np, e = q.nk * (p + 1) / np;
+        tab.insert(tab.end(), {q.i, q.j, q.k0 + b, e - b, slot + b, 0, 0, 0});
+      }
+      slot += q.nk;
+    }
+    ch.nerun = (int)(((int64_t)tab.size() - ch.eruns) / 8);
+    max_erun = std::max(max_erun, ch.nerun);
+    chunks.push_back(ch);
+  }
+  Buf orbits(c.pool.get(), orb.size() * sizeof(int)), table(c.pool.get(), tab.size() * sizeof(int));
+  FH_HIP(hipMemcpyAsync(orbits.p, orb.data(), orb.size() * sizeof(int), hipMemcpyHostToDevice, c.s));
+  FH_HIP(hipMemcpyAsync(table.p, tab.data(), tab.size() * sizeof(int), hipMemcpyHostToDevice, c.s));
+  FH_HIP(hipStreamSynchronize(c.s));
+  const int* dtab = static_cast<const int*>(table.p);
+
+  // operands: AV and its row-swapped copy share one allocation, BVp and BVq likewise
+  const int64_t nd = triples_pitch_elems((int)o, (int)v), avsz = vv * o * nd, bvsz = nd * v * o * o;
+  Buf AVall(c.pool.get(), (size_t)(2 * avsz) * sizeof(T)), BVqp(c.pool.get(), (size_t)(2 * bvsz) * sizeof(T));
+  TriplesOperands op;
+  op.av = AVall.p;
+  op.avs = static_cast<T*>(AVall.p) + avsz;
+  op.bvq = BVqp.p;
+  op.bvp = static_cast<T*>(BVqp.p) + bvsz;
+  triples_operands(c.s, fmt, (int)o, (int)v, c.OVVV.d(), c.T2.d(), c.OOOV.d(), op.av, op.avs, op.bvp, op.bvq);
+  Buf T1p = dalloc(c, v * o), vvb = dalloc(c, triples_vv_blocked_elems((int)o, (int)v));
+  {
+    Buf vvoo = dalloc(c, vv * o * o);
+    perm(c, tv(c.T1.d(), {o, v}), "ia", tv(T1p.d(), {v, o}), "ai", 1.0, 0.0);
+    perm(c, tv(c.OVOV.d(), {o, v, o, v}), "iajb", tv(vvoo.d(), {v, v, o, o}), "abij", 1.0, 0.0);
+    triples_block_vv(c.s, (int)o, (int)v, vvoo.d(), vvb.d());
+  }
+  Buf Wbuf(c.pool.get(), (size_t)(v3 * std::min(KC, ntot)) * sizeof(T));
+  T* W = static_cast<T*>(Wbuf.p);
+  Buf part = dalloc(c, norb * max_erun + 16);
+  Buf acc = dalloc(c, 1);
+  fill_f64(c.s, 1, 0.0, acc.d());
+  for (const Chunk& ch : chunks) {
+    const double fcls = 2.0 * v_ * v_ * v_ * (v_ + o_) * (double)ch.nslot;  // one permutation class
+    {
+      Timer tg(c, "triples_gemm" + sfx, 6.0 * fcls);
+      {
+        Timer tf(c, "triples_w_first" + sfx, 2.0 * fcls);
+        triples_w_first(c.s, fmt, (int)o, (int)v, tt, op, W, dtab + ch.cols, ch.ncol);
+      }
+      Timer tr(c, "triples_w_slices" + sfx, 4.0 * fcls);
+      triples_w_slices(c.s, fmt, (int)o, (int)v, tt, op, W, dtab + ch.slots, ch.nslot);
+    }
+    // algorithmic bytes: the chunk's W read once
+    Timer te(c, "triples_energy" + sfx, 0.0, (double)sizeof(T) * (double)v3 * (double)ch.nslot);
+    triples_energy(c.s, (int)o, (int)v, ch.nerun, dtab + ch.eruns, W, (int)norb, static_cast<const int*>(orbits.p),
+                   T1p.d(), vvb.d(), c.eo.d(), c.ev.d(), part.d());
+    hipLaunchKernelGGL(k_accumulate, dim3(1), dim3(256), 0, c.s, norb * ch.nerun, part.d(), acc.d());
+    FH_HIP(hipGetLastError());
+  }
   const double Et = read_scalar(c, acc.d());
   c.last_et = Et;
   return Et;

@@ -28,12 +28,11 @@ namespace fh {
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-template <int BM, int BN, int BK, bool TA, bool TB, int OCC, int TAG, bool F32, typename TI, typename TO, bool LM,
-          bool SEG>
+template <int BM, int BN, int BK, bool TA, bool TB, int OCC, int TAG, bool F32, typename TI, typename TO>
 __global__ __launch_bounds__(256, OCC) void k_gemm(
     int64_t M, int64_t N, int64_t K, double alpha, const TI* __restrict__ A, int64_t lda, int64_t sA,
     const TI* __restrict__ B, int64_t ldb, int64_t sB, double beta, const TO* C, int64_t ldc, int64_t sC, TO* D,
-    int64_t ldd, int64_t sD, int tilesM, int tilesN, int64_t kchunk, int gn, OutMap om, KSeg sg) {
+    int64_t ldd, int64_t sD, int tilesM, int tilesN, int64_t kchunk, int gn) {
   static_assert(F32 || std::is_same<TI, double>::value, "FP64 MFMA needs FP64 operands");
   using T = typename std::conditional<F32, float, double>::type;
   using Acc = typename std::conditional<F32, f32x4, f64x4>::type;
@@ -77,11 +76,6 @@ __global__ __launch_bounds__(256, OCC) void k_gemm(
   }
   if (C) C += bz * sC;
   D += bz * sD;
-  // second K segment (SEG; split-K is never combined with it)
-  const TI* A2 = SEG ? static_cast<const TI*>(sg.A) + bz * sg.sA : nullptr;
-  const TI* B2 = SEG ? static_cast<const TI*>(sg.B) + bz * sg.sB : nullptr;
-  const int64_t K1 = SEG ? sg.K1 : K;
-
   TI ra[LA], rb[LB];
   auto gload = [&](int64_t k0) {
 #pragma unroll
@@ -91,10 +85,7 @@ __global__ __launch_bounds__(256, OCC) void k_gemm(
       if (!TA) { mm = e % BM; kk = e / BM; } else { kk = e % BK; mm = e / BK; }
       const int64_t gm = m0 + mm, gk = k0 + kk;
       TI val = 0;
-      if (gm < M && gk < K) {
-        if (!SEG || gk < K1) val = TA ? A[gk + lda * gm] : A[gm + lda * gk];
-        else val = TA ? A2[(gk - K1) + sg.lda * gm] : A2[gm + sg.lda * (gk - K1)];
-      }
+      if (gm < M && gk < K) val = TA ? A[gk + lda * gm] : A[gm + lda * gk];
       ra[t] = val;
     }
 #pragma unroll
@@ -104,10 +95,7 @@ __global__ __launch_bounds__(256, OCC) void k_gemm(
       if (!TB) { kk = e % BK; nn = e / BK; } else { nn = e % BN; kk = e / BN; }
       const int64_t gcol = n0 + nn, gk = k0 + kk;
       TI val = 0;
-      if (gcol < N && gk < K) {
-        if (!SEG || gk < K1) val = TB ? B[gcol + ldb * gk] : B[gk + ldb * gcol];
-        else val = TB ? B2[gcol + sg.ldb * (gk - K1)] : B2[(gk - K1) + sg.ldb * gcol];
-      }
+      if (gcol < N && gk < K) val = TB ? B[gcol + ldb * gk] : B[gk + ldb * gcol];
       rb[t] = val;
     }
   };
@@ -152,62 +140,23 @@ __global__ __launch_bounds__(256, OCC) void k_gemm(
       for (int i = 0; i < MB; ++i)
 #pragma unroll
         for (int j = 0; j < NB; ++j) {
-          // LM: B fragment as the first MFMA operand, so the accumulator lanes run along M
-          if constexpr (F32) {
-            if constexpr (LM) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[j], af[i], acc[i][j], 0, 0, 0);
-            else acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i], bf[j], acc[i][j], 0, 0, 0);
-          } else {
-            if constexpr (LM) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bf[j], af[i], acc[i][j], 0, 0, 0);
-            else acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i], bf[j], acc[i][j], 0, 0, 0);
-          }
+          // B fragment as the first MFMA operand, so the accumulator lanes run along M
+          if constexpr (F32) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[j], af[i], acc[i][j], 0, 0, 0);
+          else acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bf[j], af[i], acc[i][j], 0, 0, 0);
         }
     }
     if (s + 1 < nst) sstore(buf ^ 1);
     __syncthreads();
   }
 
-  // epilogue: the accumulator of block (i, j) holds, in lane l and register r, the element at
-  // (lane index = l & 15, register index = (l >> 4) + 4 r for FP64 MFMA or 4 (l >> 4) + r for FP32
-  // MFMA) of the 16x16 block; the lane index runs along M when LM (rows of D), else along N.
-  // Output address: column-major with ldd, or (om.rmod > 0) the two-mode map
-  // row r -> (r % rmod)*rs0 + (r / rmod)*rs1, column c -> (c % cmod)*cs0 + (c / cmod)*cs1
-  // (cmod = 0: c*cs0), which lets a GEMM accumulate into a permuted tensor.  LM is chosen so
-  // that the lanes of one store run along the unit-stride axis of the output.
-  // The map's div/mod is done once per row and per column the thread owns (rows depend on (i,
-  // lane) and columns on (j, register) when LM, the other way round otherwise); with beta != 0
-  // every C value of the thread is loaded (unconditionally, an element outside D reading C[0])
-  // before the first store.
-  const int li = lane & 15;
-  auto rix = [&](int rr) { return F32 ? 4 * (lane >> 4) + rr : (lane >> 4) + 4 * rr; };
-  auto map_row = [&](int64_t row) { return om.rmod > 0 ? (row % om.rmod) * om.rs0 + (row / om.rmod) * om.rs1 : row; };
-  auto map_col = [&](int64_t col, int64_t ld) {
-    return om.rmod > 0 ? (om.cmod > 0 ? (col % om.cmod) * om.cs0 + (col / om.cmod) * om.cs1 : col * om.cs0) : ld * col;
-  };
-  constexpr int RR = LM ? 1 : 4, CR = LM ? 4 : 1;
-  int64_t roff[MB][RR], coff[NB][CR], ccoff[NB][CR];
-  bool rok[MB][RR], cok[NB][CR];
-#pragma unroll
-  for (int i = 0; i < MB; ++i)
-#pragma unroll
-    for (int q = 0; q < RR; ++q) {
-      const int64_t row = m0 + wm * WM + i * 16 + (LM ? li : rix(q));
-      rok[i][q] = row < M;
-      roff[i][q] = map_row(rok[i][q] ? row : 0);
-    }
-#pragma unroll
-  for (int j = 0; j < NB; ++j)
-#pragma unroll
-    for (int q = 0; q < CR; ++q) {
-      const int64_t col = n0 + wn * WN + j * 16 + (LM ? rix(q) : li);
-      cok[j][q] = col < N;
-      coff[j][q] = map_col(cok[j][q] ? col : 0, ldd);
-      ccoff[j][q] = map_col(cok[j][q] ? col : 0, ldc);
-    }
-  auto at = [&](int i, int j, int rr, int64_t& off, int64_t& offc) {
-    const int qr = LM ? 0 : rr, qc = LM ? rr : 0;
-    off = roff[i][qr] + coff[j][qc];
-    offc = om.rmod > 0 ? off : roff[i][qr] + ccoff[j][qc];
-    return rok[i][qr] && cok[j][qc];
+  // epilogue: the accumulator of block (i, j) holds, in lane l and register r, the element at row l & 15 and
+  // column (l >> 4) + 4 r (FP64 MFMA) or 4 (l >> 4) + r (FP32 MFMA) of the 16x16 block.  With beta != 0 every C
+  // value of the thread is loaded (unconditionally, an element outside D reading C[0]) before the first
+  // store.
+  auto at = [&](int i, int j, int rr, int64_t& row, int64_t& col) {
+    row = m0 + wm * WM + i * 16 + (lane & 15);
+    col = n0 + wn * WN + j * 16 + (F32 ? 4 * (lane >> 4) + rr : (lane >> 4) + 4 * rr);
+    return row < M && col < N;
   };
   if (beta != 0.0) {
     TO cv[MB][NB][4];
@@ -217,9 +166,9 @@ __global__ __launch_bounds__(256, OCC) void k_gemm(
       for (int j = 0; j < NB; ++j)
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) {
-          int64_t off, offc;
-          const bool in = at(i, j, rr, off, offc);
-          cv[i][j][rr] = C[in ? offc : 0];
+          int64_t row, col;
+          const bool in = at(i, j, rr, row, col);
+          cv[i][j][rr] = C[in ? row + ldc * col : 0];
         }
 #pragma unroll
     for (int i = 0; i < MB; ++i)
@@ -227,8 +176,9 @@ __global__ __launch_bounds__(256, OCC) void k_gemm(
       for (int j = 0; j < NB; ++j)
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) {
-          int64_t off, offc;
-          if (at(i, j, rr, off, offc)) D[off] = (TO)(alpha * (double)acc[i][j][rr] + beta * (double)cv[i][j][rr]);
+          int64_t row, col;
+          if (at(i, j, rr, row, col))
+            D[row + ldd * col] = (TO)(alpha * (double)acc[i][j][rr] + beta * (double)cv[i][j][rr]);
         }
   } else {
 #pragma unroll
@@ -237,17 +187,10 @@ __global__ __launch_bounds__(256, OCC) void k_gemm(
       for (int j = 0; j < NB; ++j)
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) {
-          int64_t off, offc;
-          if (at(i, j, rr, off, offc)) D[off] = (TO)(alpha * (double)acc[i][j][rr]);
+          int64_t row, col;
+          if (at(i, j, rr, row, col)) D[row + ldd * col] = (TO)(alpha * (double)acc[i][j][rr]);
         }
   }
-}
-
-// lanes along M unless only the output's column axis has unit stride
-static bool lanes_along_m(const OutMap& om) {
-  if (om.rmod <= 0) return true;
-  if (om.rs0 == 1) return true;
-  return om.cs0 != 1;
 }
 
 // L2 budget of the B blocks of one raster group (bytes)
@@ -256,7 +199,7 @@ static constexpr int64_t kGroupBytes = 1 << 20;
 template <int BM, int BN, int BK, bool TA, bool TB, int TAG, bool F32, typename TI, typename TO>
 static void launch(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const TI* A, int64_t lda, int64_t sA,
                    const TI* B, int64_t ldb, int64_t sB, double beta, const TO* C, int64_t ldc, int64_t sC, TO* D,
-                   int64_t ldd, int64_t sD, int64_t batch, int64_t kchunk, const OutMap& om, const KSeg& sg) {
+                   int64_t ldd, int64_t sD, int64_t batch, int64_t kchunk) {
   const int64_t tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
   FH_CHECK(tm * tn < (int64_t)1 << 31 && batch < 65536, -3, "gemm grid too large");
   dim3 grid((unsigned)(tm * tn), (unsigned)batch);
@@ -268,23 +211,8 @@ static void launch(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha,
     gn = (int)std::max<int64_t>(1, std::min<int64_t>(tn, kGroupBytes / per));
   }
   constexpr int OCC = BM * BN > 8192 ? 1 : 4;
-#define FH_GO(LM_, SEG_)                                                                                           \
-  hipLaunchKernelGGL((k_gemm<BM, BN, BK, TA, TB, OCC, TAG, F32, TI, TO, LM_, SEG_>), grid, dim3(256), 0, s, M, N, K, \
-                     alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, D, ldd, sD, (int)tm, (int)tn, kchunk, gn, om, sg)
-  if constexpr (TAG == 2) {
-    // the (T) W build: output maps (lane orientation along N when only the columns are unit-stride)
-    // and two-segment K
-    const bool lm = lanes_along_m(om);
-    if (sg.A) {
-      if (lm) FH_GO(true, true); else FH_GO(false, true);
-    } else {
-      if (lm) FH_GO(true, false); else FH_GO(false, false);
-    }
-  } else {
-    FH_CHECK(!sg.A, -3, "gemm: two-segment K is only instantiated for the (T) W build");
-    FH_GO(true, false);
-  }
-#undef FH_GO
+  hipLaunchKernelGGL((k_gemm<BM, BN, BK, TA, TB, OCC, TAG, F32, TI, TO>), grid, dim3(256), 0, s, M, N, K, alpha, A, lda,
+                     sA, B, ldb, sB, beta, C, ldc, sC, D, ldd, sD, (int)tm, (int)tn, kchunk, gn);
   FH_HIP(hipGetLastError());
 }
 
@@ -294,14 +222,14 @@ static void launch(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha,
 template <bool TA, bool TB, int TAG, bool F32, typename TI, typename TO>
 static void pick(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const TI* A, int64_t lda, int64_t sA,
                  const TI* B, int64_t ldb, int64_t sB, double beta, const TO* C, int64_t ldc, int64_t sC, TO* D,
-                 int64_t ldd, int64_t sD, int64_t batch, int64_t kchunk, const OutMap& om, const KSeg& sg) {
+                 int64_t ldd, int64_t sD, int64_t batch, int64_t kchunk) {
   const int64_t kl = kchunk > 0 ? kchunk : K;
   if (kl <= 512)
     launch<64, 64, 8, TA, TB, TAG, F32, TI, TO>(s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, D, ldd, sD,
-                                                batch, kchunk, om, sg);
+                                                batch, kchunk);
   else
     launch<64, 64, 16, TA, TB, TAG, F32, TI, TO>(s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, D, ldd,
-                                                 sD, batch, kchunk, om, sg);
+                                                 sD, batch, kchunk);
 }
 
 // split-K sizing: few output tiles and a long K leave most CUs idle; cut K into slices
@@ -333,33 +261,20 @@ __global__ void k_splitk_reduce(int64_t M, int64_t N, int64_t S, const double* _
 }
 
 static void check_args(int64_t M, int64_t K, int64_t N, bool ta, bool tb, int64_t lda, int64_t ldb, int64_t ldd,
-                       double beta, const void* C, const void* D, int64_t ldc, const OutMap* map) {
+                       double beta, const void* C, int64_t ldc) {
   FH_CHECK(K >= 0, -3, "gemm: negative K");
-  FH_CHECK(lda >= (ta ? (K > 0 ? K : 1) : M) && ldb >= (tb ? N : (K > 0 ? K : 1)) && (map || ldd >= M), -3,
+  FH_CHECK(lda >= (ta ? (K > 0 ? K : 1) : M) && ldb >= (tb ? N : (K > 0 ? K : 1)) && ldd >= M, -3,
            "gemm: leading dimension too small");
-  FH_CHECK(beta == 0.0 || (C != nullptr && (map || ldc >= M)), -3, "gemm: C missing");
-  FH_CHECK(!map || (map->rmod > 0 && (beta == 0.0 || C == D)), -3, "gemm: mapped output needs rmod > 0 and C == D");
-}
-
-// the second K segment covers k in [K1, K): its operands must hold K - K1 values along k
-void check_seg(int64_t M, int64_t N, int64_t K, bool ta, bool tb, const KSeg& sg) {
-  if (!sg.A) return;
-  FH_CHECK(sg.B != nullptr && sg.K1 > 0 && sg.K1 < K && sg.K1 % 4 == 0, -3,
-           "gemm: second K segment must start at a positive multiple of 4 below K");
-  const int64_t K2 = K - sg.K1;
-  FH_CHECK(sg.lda >= (ta ? K2 : M) && sg.ldb >= (tb ? N : K2), -3, "gemm: second K segment leading dimension too small");
+  FH_CHECK(beta == 0.0 || (C != nullptr && ldc >= M), -3, "gemm: C missing");
 }
 
 void gemm_f64(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, double alpha, const double* A,
               int64_t lda, int64_t sA, const double* B, int64_t ldb, int64_t sB, double beta, const double* C,
               int64_t ldc, int64_t sC, double* D, int64_t ldd, int64_t sD, int64_t batch, int tag, double* work,
-              int64_t work_elems, const OutMap* map, bool f32, const KSeg* seg) {
+              int64_t work_elems, bool f32) {
   if (M <= 0 || N <= 0 || batch <= 0) return;
-  check_args(M, seg ? seg->K1 : K, N, ta, tb, lda, ldb, ldd, beta, C, D, ldc, map);
-  const OutMap om = map ? *map : OutMap{};
-  const KSeg sg = seg ? *seg : KSeg{};
-  check_seg(M, N, K, ta, tb, sg);
-  const int64_t sl = (map || sg.A) ? 1 : splitk_slices(M, N, K, batch);
+  check_args(M, K, N, ta, tb, lda, ldb, ldd, beta, C, ldc);
+  const int64_t sl = splitk_slices(M, N, K, batch);
   const bool split = sl > 1 && work != nullptr && work_elems >= sl * M * N;
   const int64_t kchunk = split ? (K + sl - 1) / sl : 0;
   const int64_t nb = split ? (K + kchunk - 1) / kchunk : batch;
@@ -371,13 +286,10 @@ void gemm_f64(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, 
   do {                                                                                                              \
     if (tag == 1)                                                                                                   \
       pick<TA_, TB_, 1, F_, double, double>(s, M, N, K, al, A, lda, sA, B, ldb, sB, be, Cc, ldc, sC, Dd, lddd, sDD, nb, \
-                                            kchunk, om, sg);                                                        \
-    else if (tag == 2)                                                                                              \
-      pick<TA_, TB_, 2, F_, double, double>(s, M, N, K, al, A, lda, sA, B, ldb, sB, be, Cc, ldc, sC, Dd, lddd, sDD, nb, \
-                                            kchunk, om, sg);                                                        \
+                                            kchunk);                                                        \
     else                                                                                                            \
       pick<TA_, TB_, 0, F_, double, double>(s, M, N, K, al, A, lda, sA, B, ldb, sB, be, Cc, ldc, sC, Dd, lddd, sDD, nb, \
-                                            kchunk, om, sg);                                                        \
+                                            kchunk);                                                        \
   } while (0)
 #define FH_PICK(TA_, TB_)              \
   do {                                 \
@@ -399,48 +311,33 @@ void gemm_f64(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, 
   }
 }
 
-// FP32-MFMA GEMMs with FP32 operands and/or outputs in HBM (NN, no split-K)
+// FP32-MFMA GEMMs with FP32 operands or output in HBM (NN, no split-K)
 template <int TAG, typename TI, typename TO>
 static void gemm_nn_f32(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const TI* A, int64_t lda,
-                        int64_t sA, const TI* B, int64_t ldb, int64_t sB, double beta, const TO* C, int64_t ldc,
-                        int64_t sC, TO* D, int64_t ldd, int64_t sD, int64_t batch, const OutMap* map,
-                        const KSeg* seg = nullptr) {
-  if (M <= 0 || N <= 0 || batch <= 0) return;
-  check_args(M, seg ? seg->K1 : K, N, false, false, lda, ldb, ldd, beta, C, D, ldc, map);
-  const OutMap om = map ? *map : OutMap{};
-  const KSeg sg = seg ? *seg : KSeg{};
-  check_seg(M, N, K, false, false, sg);
-  pick<false, false, TAG, true, TI, TO>(s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, D, ldd, sD, batch,
-                                        0, om, sg);
+                        const TI* B, int64_t ldb, double beta, const TO* C, int64_t ldc, TO* D, int64_t ldd) {
+  if (M <= 0 || N <= 0) return;
+  check_args(M, K, N, false, false, lda, ldb, ldd, beta, C, ldc);
+  pick<false, false, TAG, true, TI, TO>(s, M, N, K, alpha, A, lda, 0, B, ldb, 0, beta, C, ldc, 0, D, ldd, 0, 1, 0);
 }
 
 void gemm_f32_fd(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const float* A, int64_t lda,
                  const float* B, int64_t ldb, double beta, const double* C, int64_t ldc, double* D, int64_t ldd, int tag) {
-  if (tag == 1) gemm_nn_f32<1>(s, M, N, K, alpha, A, lda, 0, B, ldb, 0, beta, C, ldc, 0, D, ldd, 0, 1, nullptr);
-  else gemm_nn_f32<0>(s, M, N, K, alpha, A, lda, 0, B, ldb, 0, beta, C, ldc, 0, D, ldd, 0, 1, nullptr);
+  if (tag == 1) gemm_nn_f32<1>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, D, ldd);
+  else gemm_nn_f32<0>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, D, ldd);
 }
 
 void gemm_f32_df(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const double* A, int64_t lda,
                  const double* B, int64_t ldb, double beta, const float* C, int64_t ldc, float* D, int64_t ldd) {
-  gemm_nn_f32<0>(s, M, N, K, alpha, A, lda, 0, B, ldb, 0, beta, C, ldc, 0, D, ldd, 0, 1, nullptr);
-}
-
-void gemm_f32_ff(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const float* A, int64_t lda, int64_t sA,
-                 const float* B, int64_t ldb, int64_t sB, double beta, const float* C, int64_t ldc, int64_t sC, float* D,
-                 int64_t ldd, int64_t sD, int64_t batch, int tag, const OutMap* map, const KSeg* seg) {
-  if (tag == 2) gemm_nn_f32<2>(s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, D, ldd, sD, batch, map, seg);
-  else gemm_nn_f32<0>(s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, D, ldd, sD, batch, map, seg);
+  gemm_nn_f32<0>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, D, ldd);
 }
 
 // FP32 operands and output, any transposition (the T2-guess network's layers; tag 3)
 void gemm_f32(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, double alpha, const float* A,
               int64_t lda, const float* B, int64_t ldb, double beta, float* C, int64_t ldc) {
   if (M <= 0 || N <= 0) return;
-  check_args(M, K, N, ta, tb, lda, ldb, ldc, beta, C, C, ldc, nullptr);
-  const OutMap om{};
+  check_args(M, K, N, ta, tb, lda, ldb, ldc, beta, C, ldc);
 #define FH_F32(TA_, TB_) \
-  pick<TA_, TB_, 3, true, float, float>(s, M, N, K, alpha, A, lda, 0, B, ldb, 0, beta, C, ldc, 0, C, ldc, 0, 1, 0, om, \
-                                        KSeg{})
+  pick<TA_, TB_, 3, true, float, float>(s, M, N, K, alpha, A, lda, 0, B, ldb, 0, beta, C, ldc, 0, C, ldc, 0, 1, 0)
   if (ta) {
     if (tb) FH_F32(true, true); else FH_F32(true, false);
   } else {

@@ -14,7 +14,7 @@
 // for BM = 256) at a time through double-buffered LDS (hi and lo planes of both operands).
 // Each wavefront owns BM/2 x 64 as 32x32 accumulator blocks.  The MFMA is issued with the B tile
 // as its first operand, so the accumulator's lane index runs along the rows of D (the output's
-// unit-stride axis).  The (T) W build has a kernel of its own (k_gemm_bf3_kk, below).
+// unit-stride axis).  The (T) W build has kernels of its own (fh_triples.hip).
 //
 // Global loads: k-contiguous operands load four consecutive k per thread (dwordx4 for FP32) when
 // the leading dimensions, batch strides and base addresses allow it (VEC), scalar loads
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(256, (BK == 16 && BM == 128) ? 3 : 2) void k_gemm_b
                                                      const TI* __restrict__ A, int64_t lda, int64_t sA,
                                                      const TI* __restrict__ B, int64_t ldb, int64_t sB, double beta,
                                                      const TO* C, int64_t ldc, int64_t sC, TO* D, int64_t ldd,
-                                                     int64_t sD, int tilesM, int tilesN, int gn, OutMap om) {
+                                                     int64_t sD, int tilesM, int tilesN, int gn) {
   constexpr int BN = 128;        // tile width
   constexpr int kRow = BK + 8;   // LDS row (bf16)
   constexpr int KG = BK / 8;      // k per thread (row-contiguous) = loads per thread (both patterns)
@@ -358,40 +358,10 @@ __global__ __launch_bounds__(256, (BK == 16 && BM == 128) ? 3 : 2) void k_gemm_b
     else put_k(Bs[buf][0], Bs[buf][1], rb, LB);
   };
 
-  auto axis_off = [](int64_t x, int64_t mod, int64_t s0, int64_t s1) {
-    return mod > 0 ? (x % mod) * s0 + (x / mod) * s1 : x * s0;
-  };
-  // offset of base + d (0 <= d < 32) along an axis with map (mod, s0, s1), from base's (q, r)
-  auto axis_step = [](int64_t q, int64_t r, int d, int64_t mod, int64_t s0, int64_t s1) {
-    int64_t rr = r + d, qq = q;
-    while (rr >= mod) { rr -= mod; ++qq; }
-    return rr * s0 + qq * s1;
-  };
-  const bool mapped = om.rmod > 0;
-  // per 32x32 block: the lane axis offset and the register axis' (q, r) start
-  // lanes along the rows of the block, register elements along its columns
-  struct Blk {
-    int64_t lane_off, q, r, amod, as0, as1, abase, lrow;
-  };
-  auto block = [&](int i, int j) {
-    Blk b;
-    b.lrow = m0 + wm * (BM / 2) + i * 32 + (lane & 31);
-    b.abase = n0 + wn * (BN / 2) + j * 32;
-    b.q = b.r = 0;
-    if (!mapped) {
-      b.lane_off = b.lrow;
-      b.amod = 0; b.as0 = ldd; b.as1 = 0;
-    } else {
-      b.lane_off = axis_off(b.lrow, om.rmod, om.rs0, om.rs1);
-      b.amod = om.cmod; b.as0 = om.cs0; b.as1 = om.cs1;
-    }
-    if (b.amod > 0) { b.q = b.abase / b.amod; b.r = b.abase - b.q * b.amod; }
-    return b;
-  };
-  auto elem = [&](const Blk& b, int e, int64_t& off) {
-    const int ri = 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-    const int64_t row = b.lrow, col = b.abase + ri;
-    off = b.lane_off + (b.amod > 0 ? axis_step(b.q, b.r, ri, b.amod, b.as0, b.as1) : (b.abase + ri) * b.as0);
+  // element e of the lane in block (i, j): row (l & 31), column 8 (e >> 2) + 4 (l >> 5) + (e & 3) of the block
+  auto elem = [&](int i, int j, int e, int64_t& row, int64_t& col) {
+    row = m0 + wm * (BM / 2) + i * 32 + (lane & 31);
+    col = n0 + wn * (BN / 2) + j * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
     return row < M && col < N;
   };
   f32x16 acc[MI][NJ];
@@ -443,359 +413,33 @@ __global__ __launch_bounds__(256, (BK == 16 && BM == 128) ? 3 : 2) void k_gemm_b
     __syncthreads();
   }
 
-  // epilogue (FP64 output): element e of lane l of accumulator (i, j) sits at row (l & 31) and
-  // column 8 (e >> 2) + 4 (l >> 5) + (e & 3) of the 32x32 block.  Output addresses as in the FP64
-  // kernel (column-major with ldd, or the two-mode OutMap); the map's div/mod is done once per
-  // 32-wide block and advanced incrementally.  With beta != 0 (C may alias D: in-place
-  // accumulation), per half block the thread's 8 values of C are loaded (unconditionally, an element
-  // outside D reading C[0]) before the 8 stores, so the loads overlap instead of each waiting behind
-  // the previous store.
+  // epilogue (FP64 output).  With beta != 0 (C may alias D: in-place accumulation), per half block the
+  // thread's 8 values of C are loaded (unconditionally, an element outside D reading C[0]) before the 8
+  // stores, so the loads overlap instead of each waiting behind the previous store.
   for_blocks<0, 0, MI, NJ>([&](auto ii, auto jj) {
     constexpr int i = decltype(ii)::value, j = decltype(jj)::value;
-    const Blk b = block(i, j);
     if (beta != 0.0) {
 #pragma unroll
       for (int h = 0; h < 16; h += 8) {
-        int64_t off[8], coff[8];
+        int64_t row[8], col[8];
         bool in[8];
         TO cv[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          in[e] = elem(b, h + e, off[e]);
-          const int ri = 8 * ((h + e) >> 2) + 4 * (lane >> 5) + ((h + e) & 3);
-          const int64_t row = b.lrow, col = b.abase + ri;
-          coff[e] = in[e] ? (mapped ? off[e] : row + ldc * col) : 0;
-        }
+        for (int e = 0; e < 8; ++e) in[e] = elem(i, j, h + e, row[e], col[e]);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) cv[e] = C[coff[e]];
+        for (int e = 0; e < 8; ++e) cv[e] = C[in[e] ? row[e] + ldc * col[e] : 0];
 #pragma unroll
         for (int e = 0; e < 8; ++e)
-          if (in[e]) D[off[e]] = (TO)(alpha * (double)acc[i][j][h + e] + beta * (double)cv[e]);
+          if (in[e]) D[row[e] + ldd * col[e]] = (TO)(alpha * (double)acc[i][j][h + e] + beta * (double)cv[e]);
       }
     } else {
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        int64_t off;
-        if (elem(b, e, off)) D[off] = (TO)(alpha * (double)acc[i][j][e]);
+        int64_t row, col;
+        if (elem(i, j, e, row, col)) D[row + ldd * col] = (TO)(alpha * (double)acc[i][j][e]);
       }
     }
   });
-}
-
-// ---------------------------------------------------------------------------------------------
-// (T) W build on k-contiguous operands, A(m, k) = A[k + lda m] and B(k, n) = B[k + ldb n] (the
-// split-BF16x3 (T) stores AV with d' fastest), copied straight into LDS: gfx950
-// global_load_lds_dwordx4 moves 16 bytes per lane, lane l writing 16 l bytes past the wave-uniform
-// LDS address in M0, and costs no registers, so a ring of NS slots keeps NS - 1 k steps in flight.  A copy instruction carries 16 rows (columns of B) x 16 k: lane l the 4 k starting at
-// 4 (l / 16) of row 16 p + l % 16, so that slot holds [row / 16][k / 4][row % 16][4 k].  A wave reads
-// its MFMA fragment (8 consecutive k of one row) as two 16-byte LDS reads and splits it into the bf16
-// hi/lo pair in registers right before the MFMAs: one barrier per k step, no staging registers and
-// no second pass through LDS.  Rows of A beyond M and columns of B beyond N are copied from row M - 1
-// (column N - 1): they only reach outputs that are not stored.  The launcher requires K % 16 == 0,
-// K1 % 4 == 0 and 16-byte aligned operands, leading dimensions and batch strides.
-typedef __attribute__((address_space(3))) void* lds_vptr;
-typedef __attribute__((address_space(1))) void* glb_vptr;
-typedef float f32v4 __attribute__((ext_vector_type(4)));
-
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 16, "vmcnt immediate");
-  __builtin_amdgcn_s_waitcnt(N | (0x7 << 4) | (0xF << 8));
-}
-
-// workgroup barrier after this wave's LDS accesses have completed (gfx950 barriers do not wait for
-// them, and the compiler adds no wait before a bare s_barrier); the operand copies keep flying
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_s_waitcnt(0xF | (0x7 << 4) | (0x0 << 8) | (0x3 << 14));
-  __builtin_amdgcn_s_barrier();
-}
-
-__device__ __forceinline__ unsigned lds_addr(const void* p) { return (unsigned)(uintptr_t)(lds_vptr)(p); }
-
-// 8 consecutive FP32 k values -> bf16x8 hi and lo (value = hi + lo to about 2^-16 relative)
-__device__ __forceinline__ void split8(const f32v4& p, const f32v4& q, bf16x8& hi, bf16x8& lo) {
-  uint32_t h[4], l[4];
-  split2(p.x, p.y, h[0], l[0]);
-  split2(p.z, p.w, h[1], l[1]);
-  split2(q.x, q.y, h[2], l[2]);
-  split2(q.z, q.w, h[3], l[3]);
-  __builtin_memcpy(&hi, h, 16);
-  __builtin_memcpy(&lo, l, 16);
-}
-
-// The fragments of one k step: two 16-byte reads per 32-row block, at block offsets of 2048 bytes.
-// The compiler tracks the operand copies with the vector-memory counter and, unable to tell the slots
-// apart, would wait for every copy in flight before an ordinary LDS read of them; these reads carry
-// their own LDS wait (the caller orders them after the copies of their slot with an explicit
-// vector-memory wait and a barrier), and their outputs are early-clobber so that no destination
-// shares an address register while a read is in flight.
-template <int NJ>
-__device__ __forceinline__ void read_frags(unsigned a, unsigned b, f32v4 (&fa)[2][2], f32v4 (&fb)[NJ][2]);
-template <>
-__device__ __forceinline__ void read_frags<2>(unsigned a, unsigned b, f32v4 (&fa)[2][2], f32v4 (&fb)[2][2]) {
-  asm volatile(
-      "ds_read_b128 %0, %8\n\tds_read_b128 %1, %8 offset:256\n\t"
-      "ds_read_b128 %2, %8 offset:2048\n\tds_read_b128 %3, %8 offset:2304\n\t"
-      "ds_read_b128 %4, %9\n\tds_read_b128 %5, %9 offset:256\n\t"
-      "ds_read_b128 %6, %9 offset:2048\n\tds_read_b128 %7, %9 offset:2304\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(fa[0][0]), "=&v"(fa[0][1]), "=&v"(fa[1][0]), "=&v"(fa[1][1]), "=&v"(fb[0][0]), "=&v"(fb[0][1]),
-        "=&v"(fb[1][0]), "=&v"(fb[1][1])
-      : "v"(a), "v"(b)
-      : "memory");
-}
-template <>
-__device__ __forceinline__ void read_frags<3>(unsigned a, unsigned b, f32v4 (&fa)[2][2], f32v4 (&fb)[3][2]) {
-  asm volatile(
-      "ds_read_b128 %0, %10\n\tds_read_b128 %1, %10 offset:256\n\t"
-      "ds_read_b128 %2, %10 offset:2048\n\tds_read_b128 %3, %10 offset:2304\n\t"
-      "ds_read_b128 %4, %11\n\tds_read_b128 %5, %11 offset:256\n\t"
-      "ds_read_b128 %6, %11 offset:2048\n\tds_read_b128 %7, %11 offset:2304\n\t"
-      "ds_read_b128 %8, %11 offset:4096\n\tds_read_b128 %9, %11 offset:4352\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(fa[0][0]), "=&v"(fa[0][1]), "=&v"(fa[1][0]), "=&v"(fa[1][1]), "=&v"(fb[0][0]), "=&v"(fb[0][1]),
-        "=&v"(fb[1][0]), "=&v"(fb[1][1]), "=&v"(fb[2][0]), "=&v"(fb[2][1])
-      : "v"(a), "v"(b)
-      : "memory");
-}
-
-// tile width BN (128 or 192) and ring depth NS; 192-wide tiles hold two workgroups per CU (4 slots of
-// 20 KB), 128-wide ones three (3 slots of 16 KB)
-template <int BN> constexpr int kk_stages() { return BN == 128 ? 3 : 4; }
-template <int BN> constexpr int kk_occupancy() { return BN == 192 ? 2 : 3; }
-
-template <int BN, bool LM>
-__global__ __launch_bounds__(256, kk_occupancy<BN>()) void k_gemm_bf3_kk(int64_t M, int64_t N, int64_t K, double alpha,
-                                                        const float* __restrict__ A, int64_t lda, int64_t sA,
-                                                        const float* __restrict__ B, int64_t ldb, int64_t sB,
-                                                        double beta, const float* C, float* D, int64_t ldd,
-                                                        int64_t sD, int tilesM, int tilesN, int bfold, OutMap om,
-                                                        KSeg sg) {
-  constexpr int BM = 128, BK = 16, NJ = BN / 64, NS = kk_stages<BN>();
-  constexpr int NA = BM / 16 / 4, NB = BN / 16 / 4;             // copy instructions per wave and stage
-  constexpr int CPS = NA + NB;
-  constexpr int ABYTES = BM * BK * 4, SLOT = (BM + BN) * BK * 4;  // bytes
-  __shared__ __attribute__((aligned(16))) float ring[NS * SLOT / 4];
-
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int wm = wid & 1, wn = wid >> 1;
-  const int64_t nb = bfold > 0 ? bfold : 1;
-  const int64_t nwg = (int64_t)tilesM * tilesN * nb;
-  const int64_t w = blockIdx.x;
-  // XCD-aware raster: workgroup w runs on XCD w % 8; each XCD takes a contiguous range of tiles
-  const int64_t q8 = nwg >> 3, r8 = nwg & 7, x8 = w & 7;
-  const int64_t L0 = x8 * q8 + (x8 < r8 ? x8 : r8) + (w >> 3);
-  const int64_t L = bfold > 0 ? L0 / nb : L0;
-  const int64_t bz = bfold > 0 ? L0 - L * nb : (int64_t)blockIdx.y;
-  const int64_t mt = L % tilesM, nt = L / tilesM;
-  const int64_t m0 = mt * BM, n0 = nt * BN;
-  A += bz * sA;
-  B += bz * sB;
-  if (C) C += bz * sD;
-  D += bz * sD;
-  const float* A2 = static_cast<const float*>(sg.A) + bz * sg.sA;
-  const float* B2 = static_cast<const float*>(sg.B) + bz * sg.sB;
-  const int64_t K1 = sg.K1, lda2 = sg.lda, ldb2 = sg.ldb;
-  const int64_t nst = K / BK;
-
-  // this lane's copies: rows of A (clamped into M) and columns of B (clamped into N), k quad l / 16, as
-  // 32-bit byte offsets from the start of a segment, the same in both K segments (the launcher checks equal
-  // leading dimensions and that every byte offset fits in 31 bits); a step adds its uniform k offset
-  // as the copies' scalar offset
-  const int kq = 4 * (lane >> 4);
-  const int K1i = (int)K1;
-  const int widu = __builtin_amdgcn_readfirstlane(wid);
-  int lofa[NA], lofb[NB];
-#pragma unroll
-  for (int t = 0; t < NA; ++t) {
-    const int64_t r = m0 + 16 * (wid * NA + t) + (lane & 15);
-    lofa[t] = 4 * (kq + (int)(lda * (r < M ? r : M - 1)));
-  }
-#pragma unroll
-  for (int t = 0; t < NB; ++t) {
-    const int64_t c = n0 + 16 * (wid * NB + t) + (lane & 15);
-    lofb[t] = 4 * (kq + (int)(ldb * (c < N ? c : N - 1)));
-  }
-  char* const ring_b = reinterpret_cast<char*>(ring);
-  // the copies go through buffer resources, one per operand and K segment; their bases are the
-  // workgroup's (uniform) operand pointers, taken from the first lane so that the compiler keeps them in
-  // scalar registers
-  auto rsrc = [](const float* p) {
-    const uint64_t u = reinterpret_cast<uint64_t>(p);
-    const uint64_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u);
-    const uint64_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32));
-    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(lo | (hi << 32)), (short)0, 0x7fffffff, 0x00020000);
-  };
-  const __amdgpu_buffer_rsrc_t ra1 = rsrc(A), ra2 = rsrc(A2), rb1 = rsrc(B), rb2 = rsrc(B2);
-  // byte offset of a copy: lane offset + va (per lane, 0 outside the step that crosses K1) + so (scalar)
-  auto copies = [&](__amdgpu_buffer_rsrc_t rsa, __amdgpu_buffer_rsrc_t rsb, int va, int so, int slot) {
-#pragma unroll
-    for (int t = 0; t < NA; ++t)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_vptr)(ring_b + slot * SLOT + (widu * NA + t) * 1024), 16,
-                                               (unsigned)(lofa[t] + va), so, 0, 0);
-#pragma unroll
-    for (int t = 0; t < NB; ++t)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsb, (lds_vptr)(ring_b + slot * SLOT + ABYTES + (widu * NB + t) * 1024),
-                                               16, (unsigned)(lofb[t] + va), so, 0, 0);
-  };
-  // lanes whose 4-wide k group lies in the second segment copy in a second, masked pass of the step that
-  // crosses K1 (its k offset in that segment is negative, so it goes into the lane offsets, which stay
-  // non-negative for those lanes).  The passes end in different (empty) asm markers: merged into one copy
-  // with a per-lane choice of resource, they would run as a loop over the distinct resources of the wave.
-  auto dma = [&](int64_t st, int slot) {
-    const int k0 = (int)st * BK;
-    const int k = k0 + kq;
-    if (k < K1i) {
-      copies(ra1, rb1, 0, 4 * k0, slot);
-      asm volatile("; first K segment");
-    }
-    if (k >= K1i) {
-      if (k0 >= K1i) {
-        copies(ra2, rb2, 0, 4 * (k0 - K1i), slot);
-        asm volatile("; second K segment");
-      } else {
-        copies(ra2, rb2, 4 * (k0 - K1i), 0, slot);
-        asm volatile("; second K segment, crossing step");
-      }
-    }
-  };
-  // fragment addresses within a slot: row (column) r of a block at (r / 16) 1024 + (l / 32) 512 + (r % 16) 16
-  const unsigned frag_lane = (unsigned)(((lane >> 4) & 1) * 1024 + (lane >> 5) * 512 + (lane & 15) * 16);
-  const unsigned a_off = (unsigned)(wm * 4 * 1024) + frag_lane;
-  const unsigned b_off = (unsigned)(ABYTES + wn * (BN / 32) * 1024) + frag_lane;
-  const unsigned ring_base = lds_addr(ring);
-
-  f32x16 acc[2][NJ];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-  auto compute = [&](int slot) {
-    f32v4 fa[2][2], fb[NJ][2];
-    read_frags<NJ>(ring_base + slot * SLOT + a_off, ring_base + slot * SLOT + b_off, fa, fb);
-    bf16x8 ah[2], al[2], bh[NJ], bl[NJ];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) split8(fa[i][0], fa[i][1], ah[i], al[i]);
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) split8(fb[j][0], fb[j][1], bh[j], bl[j]);
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        if constexpr (LM) {
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bl[j], ah[i], acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bh[j], al[i], acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bh[j], ah[i], acc[i][j], 0, 0, 0);
-        } else {
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bl[j], acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[i], bh[j], acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bh[j], acc[i][j], 0, 0, 0);
-        }
-      }
-  };
-  // stages 0 .. NS - 2 in flight; at step s the copies issued after stage s are those of
-  // min(NS - 2, nst - 1 - s) stages, and stage s + NS - 1 goes into the slot that stage s - 1 left
-  static_assert(NS == 3 || NS == 4, "the vector-memory waits below count at most two later stages");
-#pragma unroll
-  for (int p = 0; p < NS - 1; ++p)
-    if (p < nst) dma(p, p);
-  for (int64_t s = 0; s < nst; ++s) {
-    const int64_t later = std::min<int64_t>(NS - 2, nst - 1 - s);
-    if (NS == 4 && later >= 2) wait_vmcnt<(NS == 4 ? 2 : 1) * CPS>();
-    else if (later >= 1) wait_vmcnt<CPS>();
-    else wait_vmcnt<0>();
-    lds_barrier();                        // stage s landed for every wave; slot of stage s - 1 read by all
-    if (s + NS - 1 < nst) dma(s + NS - 1, (int)((s + NS - 1) % NS));
-    compute((int)(s % NS));
-  }
-
-  // epilogue: mapped outputs and in-place accumulation with beta != 0 as in k_gemm_bf3's (T) epilogue,
-  // in 32-bit index arithmetic (the launcher checks that every output offset of a batch element fits)
-  const int Mi = (int)M, Ni = (int)N;
-  const bool mapped = om.rmod > 0;
-  const int rmod = (int)om.rmod, rs0 = (int)om.rs0, rs1 = (int)om.rs1;
-  const int cmod = (int)om.cmod, cs0 = (int)om.cs0, cs1 = (int)om.cs1, lddi = (int)ldd;
-  auto axis_off = [](int x, int mod, int s0, int s1) { return mod > 0 ? (x % mod) * s0 + (x / mod) * s1 : x * s0; };
-  struct Blk {
-    int lane_off, q, r, amod, as0, as1, abase, lrow, lcol, rbase, cbase;
-  };
-  auto block = [&](int i, int j) {
-    Blk b;
-    const int li = lane & 31;
-    b.rbase = (int)m0 + wm * 64 + i * 32;
-    b.cbase = (int)n0 + wn * (BN / 2) + j * 32;
-    b.lrow = b.rbase + (LM ? li : 0);
-    b.lcol = b.cbase + (LM ? 0 : li);
-    b.q = b.r = 0;
-    if (!mapped) {
-      b.lane_off = LM ? b.lrow : lddi * b.lcol;
-      b.amod = 0; b.as0 = LM ? lddi : 1; b.as1 = 0;
-    } else if (LM) {
-      b.lane_off = axis_off(b.lrow, rmod, rs0, rs1);
-      b.amod = cmod; b.as0 = cs0; b.as1 = cs1;
-    } else {
-      b.lane_off = axis_off(b.lcol, cmod, cs0, cs1);
-      b.amod = rmod; b.as0 = rs0; b.as1 = rs1;
-    }
-    b.abase = LM ? b.cbase : b.rbase;
-    if (b.amod > 0) { b.q = b.abase / b.amod; b.r = b.abase - b.q * b.amod; }
-    return b;
-  };
-  // offset of register element e of the lane in block b; false outside D
-  auto elem = [&](const Blk& b, int e, int& off) {
-    const int ri = 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-    const int row = LM ? b.lrow : b.rbase + ri, col = LM ? b.cbase + ri : b.lcol;
-    if (b.amod > 0) {
-      int rr = b.r + ri, qq = b.q;
-      while (rr >= b.amod) { rr -= b.amod; ++qq; }
-      off = b.lane_off + rr * b.as0 + qq * b.as1;
-    } else {
-      off = b.lane_off + (b.abase + ri) * b.as0;
-    }
-    return row < Mi && col < Ni;
-  };
-  if (beta != 0.0) {
-    // per 32-row block of the wave, the C values of all NJ column blocks (3 x 16) are loaded before
-    // the first of their stores: two memory round trips per tile instead of one per 32 x 32 block
-    // (an element outside D reads C[0])
-    auto rmw_row = [&](auto ii) {
-      constexpr int i = decltype(ii)::value;
-      float cv[NJ][16];
-      for_blocks<0, 0, 1, NJ>([&](auto, auto jj) {
-        constexpr int j = decltype(jj)::value;
-        const Blk b = block(i, j);
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          int off;
-          const bool in = elem(b, e, off);
-          cv[j][e] = C[in ? off : 0];
-        }
-      });
-      for_blocks<0, 0, 1, NJ>([&](auto, auto jj) {
-        constexpr int j = decltype(jj)::value;
-        const Blk b = block(i, j);
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          int off;
-          if (elem(b, e, off)) D[off] = (float)(alpha * (double)acc[i][j][e] + beta * (double)cv[j][e]);
-        }
-      });
-    };
-    rmw_row(std::integral_constant<int, 0>{});
-    rmw_row(std::integral_constant<int, 1>{});
-  } else {
-    for_blocks<0, 0, 2, NJ>([&](auto ii, auto jj) {
-      constexpr int i = decltype(ii)::value, j = decltype(jj)::value;
-      const Blk b = block(i, j);
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        int off;
-        if (elem(b, e, off)) D[off] = (float)(alpha * (double)acc[i][j][e]);
-      }
-    });
-  }
 }
 
 // L2 budget of the B blocks of one raster group (bytes; 1, 4 and 16 MB measured alike)
@@ -809,7 +453,7 @@ static bool aligned4(const TI* p, int64_t ld, int64_t stride) {
 template <bool TA, bool TB, int TAG, typename TI, typename TO>
 static void launch_bf3(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const TI* A, int64_t lda,
                        int64_t sA, const TI* B, int64_t ldb, int64_t sB, double beta, const TO* C, int64_t ldc,
-                       int64_t sC, TO* D, int64_t ldd, int64_t sD, int64_t batch, const OutMap& om) {
+                       int64_t sC, TO* D, int64_t ldd, int64_t sD, int64_t batch) {
   // tile height: 128, or 256 (each wavefront 128 rows: fewer LDS fragment reads and operand bytes per
   // MFMA) for the PP ladder (272 vs 241 TFLOP/s at o = 40, v = 190) and for tag 0 NN GEMMs with
   // M >= 1024 (the o^3 v^3 ring contractions of the residual, K = o v: 188 against 174 TFLOP/s at
@@ -831,7 +475,7 @@ static void launch_bf3(hipStream_t s, int64_t M, int64_t N, int64_t K, double al
   const bool vec = aligned4(A, lda, batch > 1 ? sA : 0) && aligned4(B, ldb, batch > 1 ? sB : 0);
 #define FH_BF3_GO(BK_, V_, BM_)                                                                                     \
   hipLaunchKernelGGL((k_gemm_bf3<BK_, TA, TB, TAG, TI, TO, V_, BM_>), grid, dim3(256), 0, s, M, N, K, alpha, A, lda, \
-                     sA, B, ldb, sB, beta, C, ldc, sC, D, ldd, sD, (int)tm, (int)tn, gn, om)
+                     sA, B, ldb, sB, beta, C, ldc, sC, D, ldd, sD, (int)tm, (int)tn, gn)
   // BK = 16 (three workgroups per CU) for the contractions (tag 0; the o^3 v^3 ring GEMMs, K = o v,
   // measured 3% faster than BK = 32) and short K; BK = 32 for the long-K PP ladder (tag 1, 5% faster);
   // 256-row tiles stage BK = 16 (two workgroups per CU)
@@ -851,367 +495,25 @@ static void launch_bf3(hipStream_t s, int64_t M, int64_t N, int64_t K, double al
   FH_HIP(hipGetLastError());
 }
 
-// the fragments of a k step of the slice kernel: three 32-row blocks of each operand
-__device__ __forceinline__ void read_frags33(unsigned a, unsigned b, f32v4 (&fa)[3][2], f32v4 (&fb)[3][2]) {
-  asm volatile(
-      "ds_read_b128 %0, %12\n\tds_read_b128 %1, %12 offset:256\n\t"
-      "ds_read_b128 %2, %12 offset:2048\n\tds_read_b128 %3, %12 offset:2304\n\t"
-      "ds_read_b128 %4, %12 offset:4096\n\tds_read_b128 %5, %12 offset:4352\n\t"
-      "ds_read_b128 %6, %13\n\tds_read_b128 %7, %13 offset:256\n\t"
-      "ds_read_b128 %8, %13 offset:2048\n\tds_read_b128 %9, %13 offset:2304\n\t"
-      "ds_read_b128 %10, %13 offset:4096\n\tds_read_b128 %11, %13 offset:4352\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(fa[0][0]), "=&v"(fa[0][1]), "=&v"(fa[1][0]), "=&v"(fa[1][1]), "=&v"(fa[2][0]), "=&v"(fa[2][1]),
-        "=&v"(fb[0][0]), "=&v"(fb[0][1]), "=&v"(fb[1][0]), "=&v"(fb[1][1]), "=&v"(fb[2][0]), "=&v"(fb[2][1])
-      : "v"(a), "v"(b)
-      : "memory");
-}
-
-// ---------------------------------------------------------------------------------------------
-// The four batched (T) permutation classes in one launch (cab, acb, cba, bca: with c fixed, each is a
-// GEMM with rows a and columns b): batch z = c + nc kk, K = NSEG nd in NSEG = 4 segments, 192 x 192 tiles
-// (an n x n slice of W with n = v <= 192 is one tile), each wavefront 96 x 96 (3 x 3 blocks of 32 x 32).
-// Operands are copied into a ring of 3 LDS slots of 24 KB as in k_gemm_bf3_kk; a k step carries 27
-// MFMAs per wavefront for 48 split values.  The output accumulates in place (beta) into a plain M x N
-// column-major slice.  With NSEG = 2 and one batch element the same kernel runs the first launch
-// (abc + bac, an M = v^2 by N = v nk GEMM with two segments, beta = 0).
-template <int NSEG>
-__global__ __launch_bounds__(256, 2) void k_gemm_bf3_sl(int64_t M, int64_t N, int64_t nd, int64_t nc, int tilesM,
-                                                        int tilesN, double beta, float* D, int64_t ldd, int64_t sD,
-                                                        SliceSeg sg) {
-  constexpr int BM = 192, BN = 192, BK = 16, MI = 3, NJ = 3, NS = 3;
-  constexpr int NA = BM / 16 / 4, NB = BN / 16 / 4;             // copy instructions per wave and stage
-  constexpr int CPS = NA + NB;
-  constexpr int ABYTES = BM * BK * 4, SLOT = (BM + BN) * BK * 4;  // bytes
-  __shared__ __attribute__((aligned(16))) float ring[NS * SLOT / 4];
-
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int wm = wid & 1, wn = wid >> 1;
-  const int64_t nwg = (int64_t)gridDim.x;
-  const int64_t w = blockIdx.x;
-  // XCD-aware raster, the batch index fastest: consecutive c of one kk share the B blocks of the first
-  // segment and the A blocks of the third
-  const int64_t q8 = nwg >> 3, r8 = nwg & 7, x8 = w & 7;
-  const int64_t L0 = x8 * q8 + (x8 < r8 ? x8 : r8) + (w >> 3);
-  const int64_t nbat = nwg / ((int64_t)tilesM * tilesN);
-  const int64_t L = L0 / nbat, z = L0 - L * nbat;
-  const int64_t c = z % nc, kk = z / nc;
-  const int64_t m0 = (L % tilesM) * BM, n0 = (L / tilesM) * BN;
-  D += z * sD;
-  const float *A0 = sg.A[0] + c * sg.sAc[0] + kk * sg.sAk[0], *A1 = sg.A[1] + c * sg.sAc[1] + kk * sg.sAk[1];
-  const float *A2 = sg.A[2] + c * sg.sAc[2] + kk * sg.sAk[2], *A3 = sg.A[3] + c * sg.sAc[3] + kk * sg.sAk[3];
-  const float *B0 = sg.B[0] + c * sg.sBc[0] + kk * sg.sBk[0], *B1 = sg.B[1] + c * sg.sBc[1] + kk * sg.sBk[1];
-  const float *B2 = sg.B[2] + c * sg.sBc[2] + kk * sg.sBk[2], *B3 = sg.B[3] + c * sg.sBc[3] + kk * sg.sBk[3];
-  const int64_t nst = NSEG * nd / BK;
-
-  // this lane's copies: rows of A (clamped into M) / columns of B (clamped into N), k quad l / 16, as 32-bit
-  // byte offsets 4 (k quad + nd row) from the start of a segment (the launcher checks 4 nd (M + 192) and
-  // 4 nd (N + 192) < 2^31); a step
-  // adds its uniform k offset within the segment as the copies' scalar offset
-  const int kq = 4 * (lane >> 4);
-  const int ndi = (int)nd;
-  const int widu = __builtin_amdgcn_readfirstlane(wid);
-  int lofa[NA], lofb[NB];
-#pragma unroll
-  for (int t = 0; t < NA; ++t) {
-    const int r = (int)m0 + 16 * (wid * NA + t) + (lane & 15);
-    lofa[t] = 4 * (kq + ndi * (r < (int)M ? r : (int)M - 1));
-  }
-#pragma unroll
-  for (int t = 0; t < NB; ++t) {
-    const int r = (int)n0 + 16 * (wid * NB + t) + (lane & 15);
-    lofb[t] = 4 * (kq + ndi * (r < (int)N ? r : (int)N - 1));
-  }
-  char* const ring_b = reinterpret_cast<char*>(ring);
-  // the copies go through buffer resources (a uniform base and a 32-bit byte offset per lane); every
-  // offset lies inside its operand block (rows clamped into M or N, k inside the segment)
-  const __amdgpu_buffer_rsrc_t ra0 = __builtin_amdgcn_make_buffer_rsrc((void*)A0, (short)0, 0x7fffffff, 0x00020000);
-  const __amdgpu_buffer_rsrc_t ra1 = __builtin_amdgcn_make_buffer_rsrc((void*)A1, (short)0, 0x7fffffff, 0x00020000);
-  const __amdgpu_buffer_rsrc_t ra2 = __builtin_amdgcn_make_buffer_rsrc((void*)A2, (short)0, 0x7fffffff, 0x00020000);
-  const __amdgpu_buffer_rsrc_t ra3 = __builtin_amdgcn_make_buffer_rsrc((void*)A3, (short)0, 0x7fffffff, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rb0 = __builtin_amdgcn_make_buffer_rsrc((void*)B0, (short)0, 0x7fffffff, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rb1 = __builtin_amdgcn_make_buffer_rsrc((void*)B1, (short)0, 0x7fffffff, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rb2 = __builtin_amdgcn_make_buffer_rsrc((void*)B2, (short)0, 0x7fffffff, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rb3 = __builtin_amdgcn_make_buffer_rsrc((void*)B3, (short)0, 0x7fffffff, 0x00020000);
-  // byte offset of a copy: lane offset + va (per lane, 0 outside a step that crosses a segment) + so (scalar)
-  auto copy_seg = [&](__amdgpu_buffer_rsrc_t rsa, __amdgpu_buffer_rsrc_t rsb, int va, int so, int slot) {
-#pragma unroll
-    for (int t = 0; t < NA; ++t)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_vptr)(ring_b + slot * SLOT + (widu * NA + t) * 1024), 16,
-                                               (unsigned)(lofa[t] + va), so, 0, 0);
-#pragma unroll
-    for (int t = 0; t < NB; ++t)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsb, (lds_vptr)(ring_b + slot * SLOT + ABYTES + (widu * NB + t) * 1024),
-                                               16, (unsigned)(lofb[t] + va), so, 0, 0);
-  };
-  auto dma = [&](int64_t st, int slot) {
-    // the segment of the step's first k (uniform); lanes whose 4-wide k group lies in the next segment
-    // (nd % 4 == 0: a group never straddles; a 16-wide step spans at most two segments) copy through
-    // that segment's resources in a second, masked pass.  A step with both passes issues more copies
-    // than CPS, which only makes the copy-count waits below more conservative.
-    const int k0 = (int)st * BK;
-    const int s0 = (k0 >= ndi) + (k0 >= 2 * ndi) + (k0 >= 3 * ndi);
-    // (the two passes end in different, empty asm markers: merged into one copy with a per-lane choice of
-    // resource, they would run as a loop over the distinct resources of the wave)
-    // The first pass's k offset in its segment, k0 - s0 nd >= 0, is the scalar offset; the second pass's,
-    // k0 - (s0 + 1) nd < 0, goes into the lane offsets, which stay non-negative for its lanes.
-    const int k = k0 + kq;
-    const bool nxt = k >= (s0 + 1) * ndi;
-    if (!nxt) {
-      const int so = 4 * (k0 - s0 * ndi);
-      if (s0 == 0) copy_seg(ra0, rb0, 0, so, slot);
-      else if (s0 == 1) copy_seg(ra1, rb1, 0, so, slot);
-      else if (s0 == 2) copy_seg(ra2, rb2, 0, so, slot);
-      else copy_seg(ra3, rb3, 0, so, slot);
-      asm volatile("; this segment");
-    }
-    if (nxt) {
-      const int va = 4 * (k0 - (s0 + 1) * ndi);
-      if (s0 == 0) copy_seg(ra1, rb1, va, 0, slot);
-      else if (s0 == 1) copy_seg(ra2, rb2, va, 0, slot);
-      else copy_seg(ra3, rb3, va, 0, slot);
-      asm volatile("; next segment");
-    }
-  };
-  const unsigned frag_lane = (unsigned)(((lane >> 4) & 1) * 1024 + (lane >> 5) * 512 + (lane & 15) * 16);
-  const unsigned a_off = (unsigned)(wm * (BM / 32) * 1024) + frag_lane;
-  const unsigned b_off = (unsigned)(ABYTES + wn * (BN / 32) * 1024) + frag_lane;
-  const unsigned ring_base = lds_addr(ring);
-
-  f32x16 acc[MI][NJ];
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-  auto compute = [&](int slot) {
-    f32v4 fa[3][2], fb[3][2];
-    read_frags33(ring_base + slot * SLOT + a_off, ring_base + slot * SLOT + b_off, fa, fb);
-    bf16x8 ah[MI], al[MI];
-#pragma unroll
-    for (int i = 0; i < MI; ++i) split8(fa[i][0], fa[i][1], ah[i], al[i]);
-    // the MFMA burst at raised wave priority: the other wave of the SIMD issues its LDS reads and
-    // copies under it (measured 1-3% on the slice launch; none on k_gemm_bf3_kk)
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      bf16x8 bh, bl;
-      split8(fb[j][0], fb[j][1], bh, bl);
-#pragma unroll
-      for (int i = 0; i < MI; ++i) {
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bl, ah[i], acc[i][j], 0, 0, 0);
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bh, al[i], acc[i][j], 0, 0, 0);
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bh, ah[i], acc[i][j], 0, 0, 0);
-      }
-    }
-    __builtin_amdgcn_s_setprio(0);
-  };
-  // stages 0 .. NS - 2 in flight; at step s the copies issued after stage s are those of
-  // min(NS - 2, nst - 1 - s) = min(1, nst - 1 - s) stages
-#pragma unroll
-  for (int p = 0; p < NS - 1; ++p)
-    if (p < nst) dma(p, p);
-  for (int64_t s = 0; s < nst; ++s) {
-    if (s + 1 < nst) wait_vmcnt<CPS>();
-    else wait_vmcnt<0>();
-    lds_barrier();                        // stage s landed for every wave; slot of stage s - 1 read by all
-    if (s + NS - 1 < nst) dma(s + NS - 1, (int)((s + NS - 1) % NS));
-    compute((int)(s % NS));
-  }
-
-  // epilogue: element e of lane l of block (i, j) at row l % 32 and column 8 (e / 4) + 4 (l / 32) + e % 4
-  // of the block; offsets row + ldd col in 32 bits (the launcher checks M + ldd N < 2^31).  Per 32-row
-  // block row of the wave, the 3 x 16 values of D are loaded before any of them is stored.
-  const int mi = (int)M, ni = (int)N, lddi = (int)ldd;
-  auto rmw_row = [&](auto ii) {
-    constexpr int i = decltype(ii)::value;
-    const int row = (int)m0 + wm * 96 + i * 32 + (lane & 31);
-    float dv[NJ][16];
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int cb = (int)n0 + wn * 96 + j * 32 + 4 * (lane >> 5);
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int col = cb + 8 * (e >> 2) + (e & 3);
-        const bool in = row < mi && col < ni;
-        dv[j][e] = beta != 0.0 ? D[in ? row + lddi * col : 0] : 0.0f;
-      }
-    }
-    // the sums replace the loaded values, all of them before the first store: a store's data register
-    // is then not reused (which would make the next instruction wait for that store to complete)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e)
-        dv[j][e] = beta == 1.0 ? acc[i][j][e] + dv[j][e] : (float)((double)acc[i][j][e] + beta * (double)dv[j][e]);
-      asm volatile("" : "+v"(dv[j][0]), "+v"(dv[j][1]), "+v"(dv[j][2]), "+v"(dv[j][3]), "+v"(dv[j][4]), "+v"(dv[j][5]),
-                   "+v"(dv[j][6]), "+v"(dv[j][7]), "+v"(dv[j][8]), "+v"(dv[j][9]), "+v"(dv[j][10]), "+v"(dv[j][11]),
-                   "+v"(dv[j][12]), "+v"(dv[j][13]), "+v"(dv[j][14]), "+v"(dv[j][15]));
-    }
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int cb = (int)n0 + wn * 96 + j * 32 + 4 * (lane >> 5);
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int col = cb + 8 * (e >> 2) + (e & 3);
-        if (row < mi && col < ni) D[row + lddi * col] = dv[j][e];
-      }
-    }
-  };
-  rmw_row(std::integral_constant<int, 0>{});
-  rmw_row(std::integral_constant<int, 1>{});
-  rmw_row(std::integral_constant<int, 2>{});
-}
-
-// the (T) W build on k-contiguous operands (k_gemm_bf3_kk): 128-row tiles, the batch index fastest in
-// the tile index of the batched launches (as in launch_bf3)
-static void launch_bf3_kk(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const float* A, int64_t lda,
-                          int64_t sA, const float* B, int64_t ldb, int64_t sB, double beta, const float* C, float* D,
-                          int64_t ldd, int64_t sD, int64_t batch, const OutMap& om, const KSeg& sg) {
-  FH_CHECK(sg.A != nullptr && sg.B != nullptr, -3, "gemm_bf3: the k-contiguous (T) W build takes two K segments");
-  FH_CHECK(K % 16 == 0 && sg.K1 % 4 == 0, -3, "gemm_bf3: the k-contiguous (T) W build needs K % 16 == 0 and K1 % 4 == 0");
-  // the operand copies address a batch element's operand in 32-bit byte offsets, the same in both K segments
-  FH_CHECK(sg.lda == lda && sg.ldb == ldb, -3, "gemm_bf3: the k-contiguous (T) W build takes equal leading dimensions in both K segments");
-  const int64_t lim = (int64_t)1 << 31;
-  FH_CHECK(4 * (std::max(sg.K1, K - sg.K1) + lda * (M - 1)) < lim && 4 * (std::max(sg.K1, K - sg.K1) + ldb * (N - 1)) < lim,
-           -3, "gemm_bf3: the k-contiguous (T) W build addresses an operand in 32-bit byte offsets");
-  const int64_t bs = batch > 1 ? 1 : 0;
-  auto al16 = [](const void* p, int64_t ld, int64_t stride) {
-    return (uintptr_t)p % 16 == 0 && ld % 4 == 0 && stride % 4 == 0;
-  };
-  FH_CHECK(al16(A, lda, bs * sA) && al16(B, ldb, bs * sB) && al16(sg.A, sg.lda, bs * sg.sA) &&
-               al16(sg.B, sg.ldb, bs * sg.sB),
-           -3, "gemm_bf3: the k-contiguous (T) W build needs 16-byte aligned operands, leading dimensions and strides");
-  // tile width: 192, or 128 where that pads N less (N = v = 190: one 192-wide tile).  No 64-wide tile:
-  // each wave splits its own fragments, and 64 columns give it 6 MFMAs per k step for 24 split values,
-  // which measured 20% slower at v = 320 than two 192-wide tiles padded to 384 columns
-  const int bn = (N + 127) / 128 * 128 < (N + 191) / 192 * 192 ? 128 : 192;
-  const int64_t tm = (M + 127) / 128, tn = (N + bn - 1) / bn;
-  FH_CHECK(M < ((int64_t)1 << 31) && N < ((int64_t)1 << 31) && tm * tn * batch < ((int64_t)1 << 31) && batch < 65536,
-           -3, "gemm grid too large");
-  // the epilogue indexes one batch element of the output in 32 bits: largest row + column offset
-  auto axis_max = [](int64_t n, int64_t mod, int64_t s0, int64_t s1) {
-    return mod > 0 ? (std::min(n, mod) - 1) * s0 + ((n - 1) / mod) * s1 : (n - 1) * s0;
-  };
-  const int64_t max_off = om.rmod > 0 ? axis_max(M, om.rmod, om.rs0, om.rs1) + axis_max(N, om.cmod, om.cs0, om.cs1)
-                                      : (M - 1) + ldd * (N - 1);
-  FH_CHECK(max_off < ((int64_t)1 << 31) && om.rs0 >= 0 && om.rs1 >= 0 && om.cs0 >= 0 && om.cs1 >= 0 && ldd >= 0, -3,
-           "gemm_bf3: the k-contiguous (T) W build indexes an output batch element in 32 bits");
-  const int bfold = batch > 1 ? (int)batch : 0;
-  dim3 grid((unsigned)(tm * tn * batch), 1);
-  const bool lm = om.rmod <= 0 || om.rs0 == 1 || om.cs0 != 1;
-  auto go = [&](auto bnc) {
-    constexpr int BNc = decltype(bnc)::value;
-    if (lm)
-      hipLaunchKernelGGL((k_gemm_bf3_kk<BNc, true>), grid, dim3(256), 0, s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta,
-                         C, D, ldd, sD, (int)tm, (int)tn, bfold, om, sg);
-    else
-      hipLaunchKernelGGL((k_gemm_bf3_kk<BNc, false>), grid, dim3(256), 0, s, M, N, K, alpha, A, lda, sA, B, ldb, sB,
-                         beta, C, D, ldd, sD, (int)tm, (int)tn, bfold, om, sg);
-  };
-  if (bn == 192) go(std::integral_constant<int, 192>{});
-  else go(std::integral_constant<int, 128>{});
-  FH_HIP(hipGetLastError());
-}
-
-bool bf3_slices_fit(int64_t n) {
-  const int64_t t = (n + 191) / 192;
-  return n > 0 && (double)n * n >= 0.85 * (double)(192 * t) * (double)(192 * t);
-}
-
-void gemm_bf3_slices(hipStream_t s, int64_t n, int64_t nd, int64_t nc, int64_t nkk, const SliceSeg& sg, double beta,
-                     float* D, int64_t ldd, int64_t sD) {
-  if (n <= 0 || nc <= 0 || nkk <= 0) return;
-  FH_CHECK(nd > 0 && nd % 4 == 0, -3, "gemm_bf3_slices: the segment length must be a positive multiple of 4");
-  FH_CHECK(ldd >= n && (n - 1) + ldd * (n - 1) < ((int64_t)1 << 31) && 4 * nd * (n + 192) < ((int64_t)1 << 31), -3,
-           "gemm_bf3_slices: a slice and an operand block are indexed in 32 bits with ldd >= n");
-  for (int q = 0; q < 4; ++q)
-    FH_CHECK((uintptr_t)sg.A[q] % 16 == 0 && (uintptr_t)sg.B[q] % 16 == 0 && sg.sAc[q] % 4 == 0 && sg.sAk[q] % 4 == 0 &&
-                 sg.sBc[q] % 4 == 0 && sg.sBk[q] % 4 == 0,
-             -3, "gemm_bf3_slices: operands and batch strides must be 16-byte aligned");
-  const int64_t tiles = (n + 191) / 192, nwg = tiles * tiles * nc * nkk;
-  FH_CHECK(nwg < ((int64_t)1 << 31), -3, "gemm grid too large");
-  hipLaunchKernelGGL(k_gemm_bf3_sl<4>, dim3((unsigned)nwg), dim3(256), 0, s, n, n, nd, nc, (int)tiles, (int)tiles, beta, D,
-                     ldd, sD, sg);
-  FH_HIP(hipGetLastError());
-}
-
-bool bf3_pair192_fits(int64_t M, int64_t N, int64_t nd, int64_t ldd) {
-  return M > 0 && N > 0 && nd > 0 && nd % 8 == 0 && ldd >= M && (M - 1) + ldd * (N - 1) < ((int64_t)1 << 31) &&
-         4 * nd * (M + 192) < ((int64_t)1 << 31) && 4 * nd * (N + 192) < ((int64_t)1 << 31);
-}
-
-void gemm_bf3_pair192(hipStream_t s, int64_t M, int64_t N, int64_t nd, const float* A1, const float* B1,
-                      const float* A2, const float* B2, float* D, int64_t ldd) {
+void gemm_bf3(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, double alpha, const float* A,
+              int64_t lda, const float* B, int64_t ldb, double beta, const double* C, int64_t ldc, double* D, int64_t ldd,
+              int tag) {
   if (M <= 0 || N <= 0) return;
-  FH_CHECK(bf3_pair192_fits(M, N, nd, ldd), -3,
-           "gemm_bf3_pair192: needs nd % 8 == 0, ldd >= M and the output and operands indexed in 32 bits");
-  FH_CHECK((uintptr_t)A1 % 16 == 0 && (uintptr_t)B1 % 16 == 0 && (uintptr_t)A2 % 16 == 0 && (uintptr_t)B2 % 16 == 0, -3,
-           "gemm_bf3_pair192: operands must be 16-byte aligned");
-  SliceSeg sg;
-  for (int q = 0; q < 4; ++q) {
-    sg.A[q] = q == 0 ? A1 : A2;   // segments 2 and 3 are never read (two segments); valid pointers all the same
-    sg.B[q] = q == 0 ? B1 : B2;
-    sg.sAc[q] = sg.sAk[q] = sg.sBc[q] = sg.sBk[q] = 0;
-  }
-  const int64_t tm = (M + 191) / 192, tn = (N + 191) / 192, nwg = tm * tn;
-  FH_CHECK(nwg < ((int64_t)1 << 31), -3, "gemm grid too large");
-  hipLaunchKernelGGL(k_gemm_bf3_sl<2>, dim3((unsigned)nwg), dim3(256), 0, s, M, N, nd, (int64_t)1, (int)tm, (int)tn, 0.0,
-                     D, ldd, (int64_t)0, sg);
-  FH_HIP(hipGetLastError());
-}
-
-template <typename TI, typename TO>
-void gemm_bf3(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, double alpha, const TI* A, int64_t lda,
-              int64_t sA, const TI* B, int64_t ldb, int64_t sB, double beta, const TO* C, int64_t ldc, int64_t sC,
-              TO* D, int64_t ldd, int64_t sD, int64_t batch, int tag, const OutMap* map, const KSeg* seg) {
-  if (M <= 0 || N <= 0 || batch <= 0) return;
   FH_CHECK(K >= 0, -3, "gemm: negative K");
-  const int64_t K1 = seg && seg->A ? seg->K1 : K;   // extent of the first K segment
-  FH_CHECK(lda >= (ta ? (K1 > 0 ? K1 : 1) : M) && ldb >= (tb ? N : (K1 > 0 ? K1 : 1)) && (map || ldd >= M), -3,
+  FH_CHECK(lda >= (ta ? (K > 0 ? K : 1) : M) && ldb >= (tb ? N : (K > 0 ? K : 1)) && ldd >= M, -3,
            "gemm: leading dimension too small");
-  FH_CHECK(beta == 0.0 || (C != nullptr && (map || ldc >= M)), -3, "gemm: C missing");
-  FH_CHECK(!map || (map->rmod > 0 && (beta == 0.0 || C == D)), -3, "gemm: mapped output needs rmod > 0 and C == D");
-  const OutMap om = map ? *map : OutMap{};
-  const KSeg sg = seg ? *seg : KSeg{};
-  check_seg(M, N, K, ta, tb, sg);
-  // instantiated variants: FP32 operands with FP64 output, any transposition, tag 0 (the
-  // contraction engine); FP32 operands, no transposition, for the PP ladder (tag 1, FP64 output);
-  // the (T) W build (tag 2, FP32 output, A^T B on k-contiguous operands in two K segments)
-  constexpr bool kOutF64 = std::is_same<TO, double>::value;
-  FH_CHECK(tag == 2 || !sg.A, -3, "gemm_bf3: two-segment K is the (T) W build's (tag 2)");
-  if (tag == 0) {
-    FH_CHECK(kOutF64, -3, "gemm_bf3: tag 0 has FP64 output");
-    if constexpr (kOutF64) {
-      if (ta) {
-        if (tb) launch_bf3<true, true, 0, TI, TO>(s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, D, ldd, sD, batch, om);
-        else launch_bf3<true, false, 0, TI, TO>(s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, D, ldd, sD, batch, om);
-      } else {
-        if (tb) launch_bf3<false, true, 0, TI, TO>(s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, D, ldd, sD, batch, om);
-        else launch_bf3<false, false, 0, TI, TO>(s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, D, ldd, sD, batch, om);
-      }
-    }
-    return;
-  }
-  if constexpr (std::is_same<TI, float>::value) {
-    if constexpr (kOutF64) {
-      FH_CHECK(tag == 1 && !ta && !tb, -3, "gemm_bf3: FP64 output takes tag 0, or tag 1 with untransposed operands");
-      launch_bf3<false, false, 1, TI, TO>(s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, D, ldd, sD, batch, om);
-    } else {
-      FH_CHECK(tag == 2 && ta && !tb, -3, "gemm_bf3: FP32 output is the (T) W build (tag 2, A^T B)");
-      launch_bf3_kk(s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, D, ldd, sD, batch, om, sg);
-    }
+  FH_CHECK(beta == 0.0 || (C != nullptr && ldc >= M), -3, "gemm: C missing");
+#define FH_BF3(TA_, TB_, TAG_) \
+  launch_bf3<TA_, TB_, TAG_, float, double>(s, M, N, K, alpha, A, lda, 0, B, ldb, 0, beta, C, ldc, 0, D, ldd, 0, 1)
+  if (tag == 1) {
+    FH_CHECK(!ta && !tb, -3, "gemm_bf3: the PP ladder (tag 1) takes untransposed operands");
+    FH_BF3(false, false, 1);
+  } else if (ta) {
+    if (tb) FH_BF3(true, true, 0); else FH_BF3(true, false, 0);
   } else {
-    FH_CHECK(false, -3, "gemm_bf3: FP64 operands take tag 0");
+    if (tb) FH_BF3(false, true, 0); else FH_BF3(false, false, 0);
   }
+#undef FH_BF3
 }
-
-template void gemm_bf3<float, float>(hipStream_t, bool, bool, int64_t, int64_t, int64_t, double, const float*, int64_t,
-                                     int64_t, const float*, int64_t, int64_t, double, const float*, int64_t, int64_t,
-                                     float*, int64_t, int64_t, int64_t, int, const OutMap*, const KSeg*);
-template void gemm_bf3<float, double>(hipStream_t, bool, bool, int64_t, int64_t, int64_t, double, const float*,
-                                      int64_t, int64_t, const float*, int64_t, int64_t, double, const double*, int64_t,
-                                      int64_t, double*, int64_t, int64_t, int64_t, int, const OutMap*, const KSeg*);
 
 }  // namespace fh

@@ -87,72 +87,53 @@ inline TView tv(const Buf& b, std::initializer_list<int64_t> dims) {
 }
 
 // ---------------------------------------------------------------- kernel launchers
-// Output address map of a GEMM that accumulates into a permuted tensor (see k_gemm_f64):
-// row r -> (r % rmod)*rs0 + (r / rmod)*rs1, column c -> (c % cmod)*cs0 + (c / cmod)*cs1 (cmod = 0: c*cs0).
-struct OutMap {
-  int64_t rmod = 0, rs0 = 0, rs1 = 0, cmod = 0, cs0 = 0, cs1 = 0;
-};
-
-// Second K segment of a two-segment GEMM, D = alpha (A B + A2 B2) + beta C: for k >= K1 the
-// operands are A2 / B2 at k - K1 (same transposition, their own leading dimensions and batch
-// strides).  K1 must be a multiple of 4 (of 8 for the split-BF16x3 kernel).  A == nullptr: one
-// segment.
-struct KSeg {
-  const void* A = nullptr;
-  int64_t lda = 0, sA = 0;
-  const void* B = nullptr;
-  int64_t ldb = 0, sB = 0;
-  int64_t K1 = 0;
-};
-void check_seg(int64_t M, int64_t N, int64_t K, bool ta, bool tb, const KSeg& sg);
-
 // D = alpha * op(A) * op(B) + beta * C  (column-major, FP64 MFMA); C may alias D.
 // Strided batches: A_i = A + i*sA etc.
 void gemm_f64(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, double alpha,
               const double* A, int64_t lda, int64_t sA, const double* B, int64_t ldb, int64_t sB,
               double beta, const double* C, int64_t ldc, int64_t sC, double* D, int64_t ldd, int64_t sD,
               int64_t batch = 1, int tag = 0, double* work = nullptr, int64_t work_elems = 0,
-              const OutMap* map = nullptr, bool f32 = false, const KSeg* seg = nullptr);
+              bool f32 = false);
 // f32 = true: operands rounded to FP32 in LDS, FP32 MFMA with FP32 accumulation (mixed precision)
 
-// FP32-MFMA GEMMs (NN) with FP32 data in HBM: _fd float operands -> double output,
-// _df double operands -> float output, _ff float operands -> float output (strided batch, map)
+// FP32-MFMA GEMMs (NN) with FP32 data in HBM: _fd float operands -> double output, _df double operands ->
+// float output
 void gemm_f32_fd(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const float* A, int64_t lda,
                  const float* B, int64_t ldb, double beta, const double* C, int64_t ldc, double* D, int64_t ldd, int tag);
 void gemm_f32_df(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const double* A, int64_t lda,
                  const double* B, int64_t ldb, double beta, const float* C, int64_t ldc, float* D, int64_t ldd);
-void gemm_f32_ff(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const float* A, int64_t lda, int64_t sA,
-                 const float* B, int64_t ldb, int64_t sB, double beta, const float* C, int64_t ldc, int64_t sC, float* D,
-                 int64_t ldd, int64_t sD, int64_t batch, int tag, const OutMap* map, const KSeg* seg = nullptr);
 // FP32 operands and output, any transposition, C = alpha op(A) op(B) + beta C (tag 3)
 void gemm_f32(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, double alpha, const float* A,
               int64_t lda, const float* B, int64_t ldb, double beta, float* C, int64_t ldc);
-// split-BF16x3 MFMA GEMM (three bf16 products per FP32 product, FP32 accumulation) on FP32
-// operands: tag 0 any transposition with FP64 output, tag 1 (FP64 output) and tag 2 (FP32 output)
-// untransposed; the tags give distinct kernel symbols as above
-template <typename TI, typename TO>
-void gemm_bf3(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, double alpha, const TI* A, int64_t lda,
-              int64_t sA, const TI* B, int64_t ldb, int64_t sB, double beta, const TO* C, int64_t ldc, int64_t sC,
-              TO* D, int64_t ldd, int64_t sD, int64_t batch, int tag, const OutMap* map, const KSeg* seg = nullptr);
-// The (T) W build's four batched permutation classes as one split-BF16x3 launch over fixed-c slices:
-// for batch index z = c + nc kk, D_z[a, b] += sum_{s < 4} sum_{d < nd} A_s(z)[d + nd a] B_s(z)[d + nd b],
-// an n x n output of leading dimension ldd at D + z sD, with A_s(z) = A[s] + c sAc[s] + kk sAk[s] and
-// B_s(z) likewise (every operand k-contiguous with leading dimension nd).
-struct SliceSeg {
-  const float* A[4];
-  const float* B[4];
-  int64_t sAc[4], sAk[4], sBc[4], sBk[4];
+// split-BF16x3 MFMA GEMM (three bf16 products per FP32 product, FP32 accumulation) on FP32 operands with FP64
+// output: tag 0 any transposition, tag 1 (the PP ladder) untransposed; the tags give distinct kernel symbols
+void gemm_bf3(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, double alpha, const float* A,
+              int64_t lda, const float* B, int64_t ldb, double beta, const double* C, int64_t ldc, double* D, int64_t ldd,
+              int tag);
+
+// ---------------------------------------------------------------- (T) W build (fh_triples.hip)
+// fmt: 0 FP64, 1 FP32, 2 split-BF16x3 (W in FP32).  Operands hold triples_pitch_elems(o, v) values of k per
+// row (8 bytes each for fmt 0, else 4): av, avs v^2 o rows each, bvp, bvq v o^2 rows each.
+struct TriplesOperands {
+  void *av, *avs, *bvp, *bvq;
 };
-void gemm_bf3_slices(hipStream_t s, int64_t n, int64_t nd, int64_t nc, int64_t nkk, const SliceSeg& sg, double beta,
-                     float* D, int64_t ldd, int64_t sD);
-// whether the slice launch tiles n x n with little padding (192 x 192 tiles)
-bool bf3_slices_fit(int64_t n);
-// D[M x N] = A1^T B1 + A2^T B2 on k-contiguous FP32 operands (leading dimension nd for A rows and B
-// columns, two segments of length nd), split-BF16x3 MFMA with the slice launch's 192 x 192 tiles
-void gemm_bf3_pair192(hipStream_t s, int64_t M, int64_t N, int64_t nd, const float* A1, const float* B1,
-                      const float* A2, const float* B2, float* D, int64_t ldd);
-// whether gemm_bf3_pair192 takes these sizes (32-bit indexing, nd % 8 == 0)
-bool bf3_pair192_fits(int64_t M, int64_t N, int64_t nd, int64_t ldd);
+struct TriplesTiles {
+  int grain, nb, per, nt;            // slices: blocks of `grain`, at most `per` of them per tile, nt tiles along v
+  int nb_first, per_first, nt_first; // first launch: the same, nt_first tiles along v^2
+};
+int64_t triples_pitch_elems(int o, int v);
+void triples_operands(hipStream_t s, int fmt, int o, int v, const double* ovvv, const double* t2, const double* ooov,
+                      void* av, void* avs, void* bvp, void* bvq);
+TriplesTiles triples_tiles(int fmt, int o, int v, double nk);  // nk: mean k per run
+// W slots (triples) of a chunk, out of ntot
+int64_t triples_chunk_slots(int v, int elem, const TriplesTiles& tt, int64_t ntot);
+// appends the column tiles of the run k0 .. k0 + nk - 1 of (i, j), its W slots from `slot`: 8 ints each
+void triples_col_tiles(const TriplesTiles& t, int v, int i, int j, int k0, int nk, int slot, std::vector<int>& out);
+// W[a + v b + v^2 c + v^3 slot] = classes abc + bac; then += the other four (slots: 4 ints (i, j, k, 0) each)
+void triples_w_first(hipStream_t s, int fmt, int o, int v, const TriplesTiles& tt, const TriplesOperands& op, void* W,
+                     const int* cols, int ncol);
+void triples_w_slices(hipStream_t s, int fmt, int o, int v, const TriplesTiles& tt, const TriplesOperands& op, void* W,
+                      const int* slots, int nslot);
 // ---------------------------------------------------------------- T2-guess network (fh_mlp.hip)
 struct MlpOffsets {
   size_t W1, b1, W2, b2, W3, b3, w4, b4;
@@ -183,7 +164,7 @@ void t2_mlp_fused(hipStream_t s, int o, int v, const double* t2, const double* e
 
 // workspace (doubles) that gemm_f64 would use to split K for this shape (0: no split)
 int64_t gemm_splitk_elems(int64_t M, int64_t N, int64_t K, int64_t batch);
-// tag selects a distinct kernel symbol for profiling: 0 generic, 1 PP ladder, 2 (T) W build
+// tag selects a distinct kernel symbol for profiling: 0 generic, 1 PP ladder
 
 // out[perm] = alpha * in + beta * out: out dim d has size odim[d] and reads input with stride istr[d].
 void permute_f64(hipStream_t s, int nd, const int64_t* odim, const int64_t* istr, double alpha,
@@ -220,8 +201,8 @@ void mp2_pairs(hipStream_t s, int o, int v, int j0, int nj, const double* X, con
 void scale_cols_rsqrt(hipStream_t s, int n, const double* U, const double* w, double* out);
 void gwh_fock(hipStream_t s, int n, const double* S, const double* H, double* F);
 
-// (T) energy for one (i,j) pair and k in [k0, k0+nk): W[a + v*b + v^2*c + v^3*(k-k0)] holds the
-// W intermediate of ijk.jl:108-115; one FP64 partial per workgroup.
+// (T) energy of nrun runs of k (8 ints each: i, j, k0, nk, W slot of k0): W[a + v*b + v^2*c + v^3*slot]
+// holds the W intermediate of ijk.jl:108-115; one FP64 partial per orbit and run.
 // orbits: device list of cube-block triples (A>=B>=C), 3 ints each (triples_orbits)
 int triples_orbit_count(int v);
 void triples_orbits(int v, std::vector<int>& out);
@@ -229,10 +210,11 @@ void triples_orbits(int v, std::vector<int>& out);
 // (triples_vv_blocked_elems doubles)
 int64_t triples_vv_blocked_elems(int o, int v);
 void triples_block_vv(hipStream_t s, int o, int v, const double* vvoo, double* vvb);
+// k values per run: long enough to amortise the k-independent staging, short enough to fill the chip
+int triples_energy_kpw(int norb, int nslot);
 template <typename TW>  // W stored as double (FP64 path) or float (FP32 W build)
-void triples_energy(hipStream_t s, int o, int v, int i, int j, int k0, int nk, const TW* W, const int* orbits,
-                    const double* t1p, const double* vvb, const double* eo, const double* ev, double* partials,
-                    int64_t* nblocks);
+void triples_energy(hipStream_t s, int o, int v, int nrun, const int* runs, const TW* W, int norb, const int* orbits,
+                    const double* t1p, const double* vvb, const double* eo, const double* ev, double* partials);
 
 // ---------------------------------------------------------------- Gaussian integrals (fh_integrals.hip)
 // shells: packed records (integrals_pack_shell, integrals_shell_bytes each); tab: packed spherical

@@ -507,8 +507,8 @@ __device__ __forceinline__ double rcp_nr(double d) {
 }
 
 template <typename TW>
-__global__ __launch_bounds__(256) void k_triples_energy(int o, int v, int i, int j, int k0, int nk, int kpw,
-                                                        const TW* __restrict__ W, const int* __restrict__ orbits,
+__global__ __launch_bounds__(256) void k_triples_energy(int o, int v, const int4* __restrict__ runs,
+                                                        const TW* __restrict__ Wc, const int* __restrict__ orbits,
                                                         const double* __restrict__ t1p, const double* __restrict__ vvb,
                                                         const double* __restrict__ eo, const double* __restrict__ ev,
                                                         double* __restrict__ partials) {
@@ -522,7 +522,10 @@ __global__ __launch_bounds__(256) void k_triples_energy(int o, int v, int i, int
   // the neighbouring cubes of concurrently resident orbits share the W lines in its L2
   const int nwg = gridDim.x, w = blockIdx.x;
   const int ob = (w & 7) * (nwg >> 3) + min(w & 7, nwg & 7) + (w >> 3);
-  const int kb = blockIdx.y * kpw, ke = min(nk, kb + kpw);
+  const int4 run = runs[2 * blockIdx.y];
+  const int i = run.x, j = run.y, k0 = run.z, kb = 0, ke = run.w;
+  const int64_t vv = (int64_t)v * v;
+  const TW* __restrict__ W = Wc + vv * v * runs[2 * blockIdx.y + 1].x;
   const int blk[3] = {orbits[3 * ob], orbits[3 * ob + 1], orbits[3 * ob + 2]};
   // the six orderings of the orbit's blocks as indices into blk: (abc) (acb) (bac) (bca) (cab) (cba)
   constexpr int pb[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
@@ -536,7 +539,6 @@ __global__ __launch_bounds__(256) void k_triples_energy(int o, int v, int i, int
     for (int q = p - 1; q >= 0; --q)
       if (blk[pb[q][0]] == blk[pb[p][0]] && blk[pb[q][1]] == blk[pb[p][1]] && blk[pb[q][2]] == blk[pb[p][2]]) slot[p] = q;
   }
-  const int64_t vv = (int64_t)v * v;
   // (ia|jb) of occupied pair (p, q) in 8x8 blocks: vvb + PS (p + o q) + 64 (A + nb B) + x + 8 y
   const int nb = (v + CT - 1) / CT;
   const int64_t PS = (int64_t)nb * nb * CT * CT;
@@ -714,27 +716,28 @@ void triples_block_vv(hipStream_t s, int o, int v, const double* vvoo, double* v
   FH_HIP(hipGetLastError());
 }
 
-template <typename TW>
-void triples_energy(hipStream_t s, int o, int v, int i, int j, int k0, int nk, const TW* W, const int* orbits,
-                    const double* t1p, const double* vvb, const double* eo, const double* ev, double* partials,
-                    int64_t* nblocks) {
-  const int norb = triples_orbit_count(v);
-  // k values per workgroup: enough workgroups to fill the chip several times over, and a run of
-  // k long enough to amortise the k-independent staging and overlap W loads with the energy sum
-  // (FERMIHIP_TRIPLES_KPW=n fixes it, for tuning and for the tests that compare runs of k)
+// k values per workgroup: enough workgroups to fill the chip several times over, and a run of k long enough
+// to amortise the k-independent staging and overlap W loads with the energy sum (FERMIHIP_TRIPLES_KPW = n
+// fixes it, for tuning and for the tests that compare runs of k)
+int triples_energy_kpw(int norb, int nslot) {
   int kpw = 1;
-  while (kpw < 8 && (int64_t)norb * ((nk + 2 * kpw - 1) / (2 * kpw)) >= 4096) kpw *= 2;
+  while (kpw < 8 && (int64_t)norb * ((nslot + 2 * kpw - 1) / (2 * kpw)) >= 4096) kpw *= 2;
   if (const char* env = std::getenv("FERMIHIP_TRIPLES_KPW")) kpw = std::max(1, std::min(64, std::atoi(env)));
-  const int nky = (nk + kpw - 1) / kpw;
-  *nblocks = (int64_t)norb * nky;
-  hipLaunchKernelGGL(k_triples_energy<TW>, dim3((unsigned)norb, (unsigned)nky), dim3(256), 0, s, o, v, i, j, k0, nk,
-                     kpw, W, orbits, t1p, vvb, eo, ev, partials);
+  return kpw;
+}
+
+template <typename TW>
+void triples_energy(hipStream_t s, int o, int v, int nrun, const int* runs, const TW* W, int norb, const int* orbits,
+                    const double* t1p, const double* vvb, const double* eo, const double* ev, double* partials) {
+  FH_CHECK(nrun > 0 && nrun < 65536, -3, "(T) energy: too many runs in a launch");
+  hipLaunchKernelGGL(k_triples_energy<TW>, dim3((unsigned)norb, (unsigned)nrun), dim3(256), 0, s, o, v,
+                     reinterpret_cast<const int4*>(runs), W, orbits, t1p, vvb, eo, ev, partials);
   FH_HIP(hipGetLastError());
 }
-template void triples_energy<double>(hipStream_t, int, int, int, int, int, int, const double*, const int*, const double*,
-                                     const double*, const double*, const double*, double*, int64_t*);
-template void triples_energy<float>(hipStream_t, int, int, int, int, int, int, const float*, const int*, const double*,
-                                    const double*, const double*, const double*, double*, int64_t*);
+template void triples_energy<double>(hipStream_t, int, int, int, const int*, const double*, int, const int*,
+                                     const double*, const double*, const double*, const double*, double*);
+template void triples_energy<float>(hipStream_t, int, int, int, const int*, const float*, int, const int*, const double*,
+                                    const double*, const double*, const double*, double*);
 
 // ------------------------------------------------------------------ SCF helpers (RHFHelper.jl:7-59)
 // out[i + n k] = U[i + n k] / sqrt(w[k])  (U diag(w)^-1/2, for S^-1/2 = U diag(w)^-1/2 U^T)

@@ -1,0 +1,838 @@
+// The (T) W build (ijk.jl:108-115 / ijk2.jl:109-153) on CDNA4 matrix cores.
+//
+// For an occupied triple (i, j, k) the six permutation classes are products of AV_n, rows (x, y), with
+// Bcat_{p,q}, columns z, over k = d' (v virtuals, then o occupieds, padded with zeros to nd, a multiple of
+// 8), all accumulating into one W[a, b, c]:
+//   first launch   abc: AV_j[(a,b)] Bcat_{i,k}[c]  + bac: AVs_i[(a,b)] Bcat_{j,k}[c]
+//                  one GEMM per run of k with M = v^2 rows (a, b) and N = v nk columns (c, k);
+//   slice launch   with c fixed the other four are GEMMs with rows a and columns b (K = 4 nd):
+//                  cab: AVs_i[(a,c)] Bcat_{k,j}[b] + cba: Bcat_{k,i}[a] AVs_j[(b,c)]
+//                  acb: AV_k[(a,c)] Bcat_{i,j}[b]  + bca: Bcat_{j,i}[a] AV_k[(b,c)].
+// So W is written once and read and written once more per chunk of triples.  Bcat is kept as BVp (blocks
+// (p, q) with p fastest) and BVq (q fastest), AV as rows (x, y) and AVs as rows (y, x).
+//
+// Operand layout: the k of a row are cut into groups of 8 (32 bytes, 64 for FP64), stored group-major, [group]
+// [row]: a k step of 64 bytes of 16 rows is one or two contiguous runs, whole cache lines.  Row-major
+// operands (64 bytes of a 128-byte line per step) had the L1 wait for lines still in flight in 68% of its
+// cycles (TCP_PENDING_STALL_CYCLES) and moved every line twice.
+//
+// A chunk holds many (i, j) pairs: the W slots of its triples, the column tiles of its runs of k and the
+// energy kernel's runs come from device tables, so one launch carries the whole chunk.  A launch per pair
+// leaves a partial last round of workgroups on every pair (630 tiles on 512 places at o = 27, v = 131).
+//
+// Operand tiles are copied straight into a ring of LDS slots (buffer_load ... lds, 16 bytes per lane, lane l
+// writing 16 l bytes past the wave-uniform LDS address), which costs no registers; a copy instruction carries
+// a piece of 16 rows x 64 bytes.  The ring keeps two k steps in flight behind an explicit vector-memory wait
+// and one barrier per step.
+#include "fh_internal.h"
+
+#include <algorithm>
+#include <cstdlib>
+#include <type_traits>
+
+namespace fh {
+
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void* lds_vptr;
+
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+  static_assert(N >= 0 && N < 16, "vmcnt immediate");
+  __builtin_amdgcn_s_waitcnt(N | (0x7 << 4) | (0xF << 8));
+}
+__device__ __forceinline__ void wait_vmcnt_n(int n) {  // n uniform, 0 .. 6
+  if (n == 6) {  // whole 192 x 192 tiles
+    wait_vmcnt<6>();
+    return;
+  }
+  switch (n) {
+    case 0: wait_vmcnt<0>(); break;
+    case 1: wait_vmcnt<1>(); break;
+    case 2: wait_vmcnt<2>(); break;
+    case 3: wait_vmcnt<3>(); break;
+    case 4: wait_vmcnt<4>(); break;
+    case 5: wait_vmcnt<5>(); break;
+    default: wait_vmcnt<6>(); break;
+  }
+}
+
+// workgroup barrier after this wave's LDS accesses have completed (gfx950 barriers do not wait for
+// them, and the compiler adds no wait before a bare s_barrier); the operand copies keep flying
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_s_waitcnt(0xF | (0x7 << 4) | (0x0 << 8) | (0x3 << 14));
+  __builtin_amdgcn_s_barrier();
+}
+
+__device__ __forceinline__ unsigned lds_addr(const void* p) { return (unsigned)(uintptr_t)(lds_vptr)(p); }
+
+// a buffer resource over a uniform base (taken from the first lane, so that it stays in scalar registers)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t uniform_rsrc(const char* p, int bytes = 0x7fffffff) {
+  const uint64_t u = reinterpret_cast<uint64_t>(p);
+  const uint64_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u);
+  const uint64_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32));
+  return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(lo | (hi << 32)), (short)0, bytes, 0x00020000);
+}
+
+// Fragment reads of a k step: MI + NJ blocks of 32 rows (2048 bytes apart), two 16-byte reads each: hi at pa / pb,
+// lo at qa = pa ^ 16 / qb = pb ^ 16.  The compiler counts the operand copies as vector-memory operations and, unable to tell the ring
+// slots apart, would wait for every copy in flight before an ordinary LDS read; these reads carry their own
+// LDS wait, and their outputs are early-clobber so that no destination shares an address register while a
+// read is in flight.
+#define FH_RD(n, base, off) "ds_read_b128 %[" #n "], %[" #base "] offset:" #off "\n\t"
+#define FH_A1 FH_RD(a0, pa, 0) FH_RD(a1, qa, 0)
+#define FH_A2 FH_A1 FH_RD(a2, pa, 2048) FH_RD(a3, qa, 2048)
+#define FH_A3 FH_A2 FH_RD(a4, pa, 4096) FH_RD(a5, qa, 4096)
+#define FH_B1 FH_RD(b0, pb, 0) FH_RD(b1, qb, 0)
+#define FH_B2 FH_B1 FH_RD(b2, pb, 2048) FH_RD(b3, qb, 2048)
+#define FH_B3 FH_B2 FH_RD(b4, pb, 4096) FH_RD(b5, qb, 4096)
+#define FH_OA1 [a0] "=&v"(fa[0][0]), [a1] "=&v"(fa[0][1])
+#define FH_OA2 FH_OA1, [a2] "=&v"(fa[1][0]), [a3] "=&v"(fa[1][1])
+#define FH_OA3 FH_OA2, [a4] "=&v"(fa[2][0]), [a5] "=&v"(fa[2][1])
+#define FH_OB1 [b0] "=&v"(fb[0][0]), [b1] "=&v"(fb[0][1])
+#define FH_OB2 FH_OB1, [b2] "=&v"(fb[1][0]), [b3] "=&v"(fb[1][1])
+#define FH_OB3 FH_OB2, [b4] "=&v"(fb[2][0]), [b5] "=&v"(fb[2][1])
+#define FH_READ(mi, nj)                                                                                        \
+  if constexpr (MI == mi && NJ == nj)                                                                          \
+    asm volatile(FH_A##mi FH_B##nj "s_waitcnt lgkmcnt(0)" : FH_OA##mi, FH_OB##nj : [pa] "v"(a), [qa] "v"(a ^ 16u), [pb] "v"(b), [qb] "v"(b ^ 16u) : "memory")
+template <int MI, int NJ>
+__device__ __forceinline__ void read_frags(unsigned a, unsigned b, f32x4 (&fa)[MI][2], f32x4 (&fb)[NJ][2]) {
+  FH_READ(1, 1); FH_READ(1, 2); FH_READ(1, 3);
+  FH_READ(2, 1); FH_READ(2, 2); FH_READ(2, 3);
+  FH_READ(3, 1); FH_READ(3, 2); FH_READ(3, 3);
+}
+#undef FH_READ
+
+// one 16-byte read of the wave's A block and one per B block, block stride 1024
+#define FH_Q(j, off) FH_RD(b##j, pb, off)
+#define FH_QO(j) [b##j] "=&v"(fb[j])
+template <int NB>
+__device__ __forceinline__ void read_rows(unsigned a, unsigned b, f32x4& fa, f32x4 (&fb)[NB]) {
+  if constexpr (NB == 2)
+    asm volatile(FH_RD(a0, pa, 0) FH_Q(0, 0) FH_Q(1, 1024) "s_waitcnt lgkmcnt(0)"
+                 : [a0] "=&v"(fa), FH_QO(0), FH_QO(1) : [pa] "v"(a), [pb] "v"(b) : "memory");
+  if constexpr (NB == 3)
+    asm volatile(FH_RD(a0, pa, 0) FH_Q(0, 0) FH_Q(1, 1024) FH_Q(2, 2048) "s_waitcnt lgkmcnt(0)"
+                 : [a0] "=&v"(fa), FH_QO(0), FH_QO(1), FH_QO(2) : [pa] "v"(a), [pb] "v"(b) : "memory");
+  if constexpr (NB == 4)
+    asm volatile(FH_RD(a0, pa, 0) FH_Q(0, 0) FH_Q(1, 1024) FH_Q(2, 2048) FH_Q(3, 3072) "s_waitcnt lgkmcnt(0)"
+                 : [a0] "=&v"(fa), FH_QO(0), FH_QO(1), FH_QO(2), FH_QO(3) : [pa] "v"(a), [pb] "v"(b) : "memory");
+  if constexpr (NB == 5)
+    asm volatile(FH_RD(a0, pa, 0) FH_Q(0, 0) FH_Q(1, 1024) FH_Q(2, 2048) FH_Q(3, 3072) FH_Q(4, 4096)
+                 "s_waitcnt lgkmcnt(0)"
+                 : [a0] "=&v"(fa), FH_QO(0), FH_QO(1), FH_QO(2), FH_QO(3), FH_QO(4) : [pa] "v"(a), [pb] "v"(b) : "memory");
+  if constexpr (NB == 6)
+    asm volatile(FH_RD(a0, pa, 0) FH_Q(0, 0) FH_Q(1, 1024) FH_Q(2, 2048) FH_Q(3, 3072) FH_Q(4, 4096) FH_Q(5, 5120)
+                 "s_waitcnt lgkmcnt(0)"
+                 : [a0] "=&v"(fa), FH_QO(0), FH_QO(1), FH_QO(2), FH_QO(3), FH_QO(4), FH_QO(5)
+                 : [pa] "v"(a), [pb] "v"(b) : "memory");
+}
+
+// two FP32 values -> packed (hi, lo) bf16 pairs, hi = bf16(x), lo = bf16(x - hi)
+__device__ inline void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
+  const f32x2 v = {a, b};
+  const bf16x2 h = __builtin_convertvector(v, bf16x2);
+  __builtin_memcpy(&hi, &h, 4);
+  const f32x2 r = {a - __uint_as_float(hi << 16), b - __uint_as_float(hi & 0xffff0000u)};
+  const bf16x2 l = __builtin_convertvector(r, bf16x2);
+  __builtin_memcpy(&lo, &l, 4);
+}
+
+// Pieces of 16 rows x 64 bytes in LDS, and what lane l copies of one (its destination is 16 l bytes on).
+// GB = 32: two k groups, [group][row][2 units of 16 bytes], the units of rows 8 .. 15 swapped; GB = 64: one group,
+// [row][4 units], unit u of row r at u ^ (r / 4).  Either way the lanes of a copy read contiguous memory and a
+// fragment read (one unit of 16 rows) falls on distinct banks.
+template <int GB>
+__device__ __forceinline__ int copy_row(int lane) { return GB == 32 ? (lane & 31) >> 1 : lane >> 2; }
+template <int GB>
+__device__ __forceinline__ int copy_group(int lane) { return GB == 32 ? lane >> 5 : 0; }
+template <int GB>
+__device__ __forceinline__ int copy_unit(int lane) {
+  return GB == 32 ? (lane & 1) ^ ((lane >> 4) & 1) : (lane & 3) ^ ((lane >> 4) & 3);
+}
+// unit u of k group g of row r
+template <int GB>
+__device__ __forceinline__ unsigned unit_at(int r, int g, int u) {
+  return GB == 32 ? (unsigned)((r >> 4) * 1024 + g * 512 + (r & 15) * 32 + (u ^ ((r >> 3) & 1)) * 16)
+                  : (unsigned)((r >> 4) * 1024 + (r & 15) * 64 + (u ^ ((r >> 2) & 3)) * 16);
+}
+
+// n elements in blocks of g, dealt to nt tiles of nearly equal block counts: first element of tile t
+__host__ __device__ inline int tile_begin(int n, int g, int nt, int t) {
+  const int nb = (n + g - 1) / g;
+  return (int)((int64_t)nb * t / nt) * g;
+}
+
+}  // namespace
+
+// ------------------------------------------------------------------ operands
+// One k group of a row from 8 values at s, s + pitch, ...  FMT: 0 double, 1 float, 2 split-BF16x3 (8 bf16 hi,
+// then 8 bf16 lo).
+template <int FMT>
+__device__ inline void put_k8(char* d, const double* s, int pitch) {
+  if constexpr (FMT == 0) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) reinterpret_cast<double2*>(d)[q] = make_double2(s[2 * q * pitch], s[(2 * q + 1) * pitch]);
+  } else if constexpr (FMT == 1) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      reinterpret_cast<float4*>(d)[q] = make_float4((float)s[4 * q * pitch], (float)s[(4 * q + 1) * pitch],
+                                                    (float)s[(4 * q + 2) * pitch], (float)s[(4 * q + 3) * pitch]);
+  } else {
+    uint32_t h[4], l[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) split2((float)s[2 * q * pitch], (float)s[(2 * q + 1) * pitch], h[q], l[q]);
+    reinterpret_cast<uint4*>(d)[0] = make_uint4(h[0], h[1], h[2], h[3]);
+    reinterpret_cast<uint4*>(d)[1] = make_uint4(l[0], l[1], l[2], l[3]);
+  }
+}
+// AV[d', (x,y), n] and AVs[d', (y,x), n]: d' < v -> (n y|x d') = OVVV[n, y, x, d']; v <= d' < v + o ->
+// -T2[n, l, y, x], l = d' - v; zero up to nd.  One workgroup per 4 x 4 block of (x, y) and k group: n is the
+// sources' unit-stride index and (d', row) the result's, so 32 n at a time turn in LDS, and both copies are
+// written from one read in runs of 4 rows (a cache line).
+template <int FMT>
+__global__ __launch_bounds__(256) void k_triples_av(int o, int v, int nd, const double* __restrict__ ovvv,
+                                                    const double* __restrict__ t2, char* __restrict__ av,
+                                                    char* __restrict__ avs) {
+  constexpr int GB = FMT == 0 ? 64 : 32;
+  __shared__ double tile[8][16][33];  // [d'][x + 4 y][n]
+  const int nb = (v + 3) / 4;
+  const int y0 = 4 * (blockIdx.x % nb), x0 = 4 * (blockIdx.x / nb % nb), g = blockIdx.x / (nb * nb);
+  const int64_t vv = (int64_t)v * v, an = vv * (nd / 8) * GB;
+  for (int n0 = 0; n0 < o; n0 += 32) {
+    __syncthreads();
+    for (int e = threadIdx.x; e < 8 * 16 * 32; e += 256) {
+      const int n = n0 + (e & 31), y = y0 + (e >> 5 & 3), x = x0 + (e >> 7 & 3), d = 8 * g + (e >> 9);
+      double val = 0.0;
+      if (n < o && x < v && y < v) {
+        if (d < v) val = ovvv[n + (int64_t)o * (y + (int64_t)v * (x + (int64_t)v * d))];
+        else if (d < v + o) val = -t2[n + (int64_t)o * (d - v + (int64_t)o * (y + (int64_t)v * x))];
+      }
+      tile[e >> 9][(e >> 7 & 3) + 4 * (e >> 5 & 3)][e & 31] = val;
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < 16 * 32; e += 256) {
+      const int lo = e & 3, hi = e >> 2 & 3, n = e >> 4;
+      if (n0 + n >= o) continue;
+      if (x0 + lo < v && y0 + hi < v)
+        put_k8<FMT>(av + (n0 + n) * an + (vv * g + x0 + lo + (int64_t)v * (y0 + hi)) * GB, &tile[0][lo + 4 * hi][n], 16 * 33);
+      if (y0 + lo < v && x0 + hi < v)
+        put_k8<FMT>(avs + (n0 + n) * an + (vv * g + y0 + lo + (int64_t)v * (x0 + hi)) * GB, &tile[0][hi + 4 * lo][n], 16 * 33);
+    }
+  }
+}
+// Bcat_{p,q}[d', z]: d' < v -> T2[q, p, z, d']; v <= d' < v + o -> OOOV[l, p, q, z]; zero up to nd; stored as
+// BVp (block p + o q) and BVq (block q + o p).  One workgroup per 4 z, k group and 32 pairs q + o p, the
+// unit-stride index of T2.
+template <int FMT>
+__global__ __launch_bounds__(256) void k_triples_bv(int o, int v, int nd, const double* __restrict__ t2,
+                                                    const double* __restrict__ ooov, char* __restrict__ bvp,
+                                                    char* __restrict__ bvq) {
+  constexpr int GB = FMT == 0 ? 64 : 32;
+  __shared__ double tile[8][4][33];  // [d'][z][pair]
+  const int64_t bs = (int64_t)v * (nd / 8) * GB;
+  const int nz = (v + 3) / 4, ng = nd / 8, oo = o * o;
+  const int z0 = 4 * (blockIdx.x % nz), g = blockIdx.x / nz % ng, s0 = 32 * (int)(blockIdx.x / ((int64_t)nz * ng));
+  for (int e = threadIdx.x; e < 8 * 4 * 32; e += 256) {
+    const int s = s0 + (e & 31), z = z0 + (e >> 5 & 3), d = 8 * g + (e >> 7);
+    double val = 0.0;
+    if (s < oo && z < v) {
+      if (d < v) val = t2[s + (int64_t)oo * (z + (int64_t)v * d)];
+      else if (d < v + o) val = ooov[d - v + (int64_t)o * (s / o + (int64_t)o * (s % o + (int64_t)o * z))];
+    }
+    tile[e >> 7][e >> 5 & 3][e & 31] = val;
+  }
+  __syncthreads();
+  const int z = threadIdx.x & 3, s = threadIdx.x >> 2 & 31, q = (s0 + s) % o, p = (s0 + s) / o;
+  if (s0 + s < oo && z0 + z < v) {
+    char* d = threadIdx.x < 128 ? bvq + (s0 + s) * bs : bvp + (p + (int64_t)o * q) * bs;
+    put_k8<FMT>(d + ((int64_t)v * g + z0 + z) * GB, &tile[0][z][s], 4 * 33);
+  }
+}
+
+// ------------------------------------------------------------------ W build
+// slices: W slots that share a c before the next c (1, 4, 8 and 16 measured alike: 430 ms of slice launches at
+// o = 40, v = 190)
+constexpr int kSlotGroup = 8;
+
+// What both W kernels share: the tile of a workgroup, its operands (bases at the tile's first row, per K
+// segment) and its output.
+struct TripW {
+  const char *av, *avs, *bvp, *bvq;
+  void* w;
+  const int4* slots;  // (i, j, k, 0) of each W slot of the chunk
+  const int4* cols;   // first launch: two int4 per column tile: (i, j, k0, slot of k0), (n0, columns, 0, 0)
+  int o, v, nd;
+  int nt;     // tiles along the rows (first launch: of v^2; slices: of v, the same along the columns)
+  int ncol;   // first launch: column tiles; slices: W slots
+  int group;  // slices: W slots of a raster group
+};
+template <int NSEG, int GB>
+struct TripTile {
+  const char *A[NSEG], *B[NSEG];  // per K segment: the operands' first group at the tile's first row / column
+  int rows, cols;
+  int64_t ldw, woff;  // leading dimension of the output tile and its first element's offset in W
+  int bcol, v;        // first launch: the tile's first column within its k
+  int64_t bs;
+
+  // whether segment s takes its A operand from AV / AVs (group stride v^2 rows) and B from Bcat (v rows), or
+  // the other way round
+  static __device__ __forceinline__ constexpr bool a_is_av(int s) { return NSEG == 2 || (s & 1) == 0; }
+
+  __device__ __forceinline__ TripTile(const TripW& t, int grain) {
+    // workgroup w runs on XCD w % 8: each XCD takes a contiguous range of the raster, so that
+    // neighbouring tiles share their operand blocks in its L2
+    const int64_t nwg = gridDim.x, w = blockIdx.x;
+    const int64_t q8 = nwg >> 3, r8 = nwg & 7, x8 = w & 7;
+    const int64_t L = x8 * q8 + (x8 < r8 ? x8 : r8) + (w >> 3);
+    v = t.v;
+    const int o = t.o;
+    const int64_t vv = (int64_t)v * v, an = vv * (t.nd / 8) * GB;
+    bs = (int64_t)v * (t.nd / 8) * GB;
+    bcol = 0;
+    if constexpr (NSEG == 2) {
+      const int ct = (int)(L % t.ncol), mt = (int)(L / t.ncol);
+      const int4 p = t.cols[2 * ct], q = t.cols[2 * ct + 1];
+      const int m0 = tile_begin((int)vv, grain, t.nt, mt);
+      rows = min(tile_begin((int)vv, grain, t.nt, mt + 1), (int)vv) - m0;
+      cols = q.y;
+      const int kk = q.x / v;
+      bcol = q.x - kk * v;
+      A[0] = t.av + an * p.y + (int64_t)GB * m0;
+      A[1] = t.avs + an * p.x + (int64_t)GB * m0;
+      B[0] = t.bvq + bs * (p.z + kk + (int64_t)o * p.x);
+      B[1] = t.bvq + bs * (p.z + kk + (int64_t)o * p.y);
+      ldw = vv;
+      woff = vv * v * p.w + m0 + vv * q.x;
+    } else {
+      // groups of kSlotGroup slots, then c, then the slots of the group, then the tiles of a slice: the 64
+      // workgroups of an XCD in flight share AV_i, AV_j (same c) and the Bcat blocks (same slots)
+      const int tt = t.nt * t.nt;
+      const int64_t per = (int64_t)v * t.group * tt;
+      const int gr = (int)(L / per), s0 = gr * t.group, ns = min(t.group, t.ncol - s0);
+      const int rem = (int)(L - gr * per), c = rem / (ns * tt), r2 = rem - c * ns * tt, s = s0 + r2 / tt, tl = r2 % tt;
+      const int4 p = t.slots[s];
+      const int m0 = tile_begin(v, grain, t.nt, tl % t.nt), n0 = tile_begin(v, grain, t.nt, tl / t.nt);
+      rows = min(tile_begin(v, grain, t.nt, tl % t.nt + 1), v) - m0;
+      cols = min(tile_begin(v, grain, t.nt, tl / t.nt + 1), v) - n0;
+      const int64_t co = (int64_t)GB * v * c, ao = (int64_t)GB * m0, bo = (int64_t)GB * n0;
+      A[0] = t.avs + an * p.x + co + ao;                       // cab: AV_i[(c,a)]
+      B[0] = t.bvp + bs * (p.z + (int64_t)o * p.y) + bo;       //      Bcat_{k,j}[., b]
+      A[1] = t.bvp + bs * (p.z + (int64_t)o * p.x) + ao;       // cba: Bcat_{k,i}[., a]
+      B[1] = t.avs + an * p.y + co + bo;                       //      AV_j[(c,b)]
+      A[2] = t.av + an * p.z + co + ao;                        // acb: AV_k[(a,c)]
+      B[2] = t.bvp + bs * (p.x + (int64_t)o * p.y) + bo;       //      Bcat_{i,j}[., b]
+      A[3] = t.bvp + bs * (p.y + (int64_t)o * p.x) + ao;       // bca: Bcat_{j,i}[., a]
+      B[3] = t.av + an * p.z + co + bo;                        //      AV_k[(b,c)], in L2 from the previous segment
+      ldw = v;
+      woff = vv * v * s + vv * c + m0 + (int64_t)v * n0;
+    }
+  }
+  // byte offset of column n of the tile within a k group of B
+  __device__ __forceinline__ int col_off(int n) const {
+    if constexpr (NSEG == 2) {
+      const int q = bcol + n, kk = q / v;
+      return (int)(bs * kk) + GB * (q - kk * v);
+    } else {
+      return GB * n;
+    }
+  }
+};
+
+// The k steps of a tile in order: step() calls copy(A, B, dga, dgb) with resources at the step's first group
+// and the lane's byte offset from there to its own group.  With 32-byte groups a step is two groups, which may
+// lie in two segments (an odd number of groups per segment): the lanes of the second group then copy in a
+// second, masked pass, which only makes the waits that count copies stricter.  The passes end in different
+// (empty) asm markers: merged into one copy with a choice of resource, they would run as a loop over the
+// wave's distinct resources.
+template <int NSEG, int GB>
+struct Feed {
+  using Tile = TripTile<NSEG, GB>;
+  const char *A[NSEG - 1], *B[NSEG - 1];  // of the segments to come
+  const char *pa, *pb;
+  int64_t sav, sbv;  // group strides of AV and Bcat
+  int ng, seg, g, second;
+  __device__ __forceinline__ Feed(const TripW& t, const Tile& tl, int lane) {
+#pragma unroll
+    for (int s = 0; s + 1 < NSEG; ++s) {
+      A[s] = tl.A[s + 1];
+      B[s] = tl.B[s + 1];
+    }
+    sbv = (int64_t)GB * t.v;
+    sav = sbv * t.v;
+    ng = t.nd / 8;
+    seg = g = 0;
+    pa = tl.A[0];
+    pb = tl.B[0];
+    second = copy_group<GB>(lane);
+  }
+  __device__ __forceinline__ int64_t sa() const { return NSEG == 2 || (seg & 1) == 0 ? sav : sbv; }
+  __device__ __forceinline__ int64_t sb() const { return NSEG == 2 || (seg & 1) == 0 ? sbv : sav; }
+  __device__ __forceinline__ void next_segment() {
+    ++seg;
+    pa = A[0];
+    pb = B[0];
+#pragma unroll
+    for (int s = 0; s + 2 < NSEG; ++s) {
+      A[s] = A[s + 1];
+      B[s] = B[s + 1];
+    }
+  }
+  template <typename Copy>
+  __device__ __forceinline__ void step(Copy&& copy) {
+    constexpr int G = 64 / GB;
+    if (G == 1 || g + 1 < ng) {
+      copy(uniform_rsrc(pa), uniform_rsrc(pb), second ? (int)sa() : 0, second ? (int)sb() : 0);
+      asm volatile("; step");
+      g += G;
+      pa += G * sa();
+      pb += G * sb();
+    } else {
+      if (!second) {
+        copy(uniform_rsrc(pa), uniform_rsrc(pb), 0, 0);
+        asm volatile("; step, last group of a segment");
+      }
+      next_segment();
+      if (second) {
+        copy(uniform_rsrc(pa), uniform_rsrc(pb), 0, 0);
+        asm volatile("; step, first group of a segment");
+      }
+      g = 1;
+      pa += sa();
+      pb += sb();
+    }
+    if (g == ng && seg + 1 < NSEG) {
+      next_segment();
+      g = 0;
+    }
+  }
+};
+
+// Epilogue of a wave's MI x NJ blocks at (r0, c0) of its tile: element e of lane l of block (i, j) at row l % 32
+// and column 8 (e / 4) + 4 (l / 32) + e % 4 of the block.  W goes through a buffer resource that ends with the
+// tile's last column, at one running lane offset: an element outside the tile (a row beyond it starts out of
+// range) reads 0 and is not written, with no masks and no 48 addresses.  Per 32-row block row of the wave the
+// values of W are loaded before any is stored, and the sums replace them before the first store: a store's
+// data register is then not reused, which would make the next instruction wait for that store to complete.
+template <bool ADD, int MI, int NJ>
+__device__ __forceinline__ void store_blocks(const f32x16 (&acc)[MI][NJ], __amdgpu_buffer_rsrc_t rw, int r0, int c0,
+                                             int rows, int ldw4) {
+  const int lane = threadIdx.x & 63, cl = c0 + 4 * (lane >> 5);
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    const int row = r0 + i * 32 + (lane & 31);
+    const unsigned vo = row < rows ? (unsigned)(4 * row + ldw4 * cl) : 0x80000000u;
+    auto step = [&](unsigned& o, int e) {
+      o += (e & 3) == 3 ? 5 * ldw4 : ldw4;
+      asm volatile("" : "+v"(o));  // a running sum: not folded into 48 live offsets
+    };
+    float dv[NJ][16];
+    unsigned o = vo;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        if constexpr (ADD) {
+          dv[j][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rw, o, 0, 0));
+          step(o, e);
+        } else {
+          dv[j][e] = acc[i][j][e];
+        }
+      }
+    }
+    if constexpr (ADD) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) dv[j][e] += acc[i][j][e];
+        asm volatile("" : "+v"(dv[j][0]), "+v"(dv[j][1]), "+v"(dv[j][2]), "+v"(dv[j][3]), "+v"(dv[j][4]),
+                     "+v"(dv[j][5]), "+v"(dv[j][6]), "+v"(dv[j][7]), "+v"(dv[j][8]), "+v"(dv[j][9]), "+v"(dv[j][10]),
+                     "+v"(dv[j][11]), "+v"(dv[j][12]), "+v"(dv[j][13]), "+v"(dv[j][14]), "+v"(dv[j][15]));
+      }
+    }
+    o = vo;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dv[j][e]), rw, o, 0, 0);
+        step(o, e);
+      }
+    }
+  }
+}
+
+// Split-BF16x3: A B ~ Ahi Bhi + Ahi Blo + Alo Bhi with FP32 accumulation (Henry, Tang and Heinecke,
+// ARITH 2019), operands split once when AV and Bcat are built (32 bytes per 8 k: hi, then lo), so that a
+// fragment (8 consecutive k of a row, hi and lo) is two 16-byte LDS reads and no arithmetic.  Tiles of up to
+// 64 MB x 64 MB (MB = 3: two workgroups per CU; MB = 2 for v <= 128: three), 2 x 2 wavefronts of up to
+// MB x MB 32 x 32 blocks.  An axis is cut into tiles of nearly equal numbers of 32-blocks and a tile's
+// blocks are dealt to the two wave rows, so v = 131 costs 5 x 5 blocks, not 6 x 6; blocks, copies and
+// fragment reads beyond the edge are not issued.
+// Bound by the matrix cores at the rate the card sustains (a plain bf16 product of 8192^3 reaches 1122 TFLOP/s,
+// 374 for three products): o = 40, v = 190: first launch 345 TFLOP/s (per-pair launches with row-major operands
+// split in the kernel: 224), slices 336 (224); o = 27, v = 131: slices 202 (two batched launches of 128 x 192
+// tiles: 98).
+template <int NSEG, int MB>
+struct Bf3Tile {
+  static constexpr int NS = 3, ABYTES = 64 * MB * 64, SLOT = 2 * ABYTES;
+  __amdgpu_buffer_rsrc_t rw;
+  char* ring;
+  int lane, wid, rows, cols, nst, npa, npb, cps, ldw4;
+  int rb0, mi, cb0, nj;  // the wave's first row / column block of the tile and its block counts
+  int lofa[MB], lofb[MB];
+
+  __device__ __forceinline__ Bf3Tile(const TripW& t, const TripTile<NSEG, 32>& tl, char* lds) : ring(lds) {
+    lane = threadIdx.x & 63;
+    wid = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    rows = __builtin_amdgcn_readfirstlane(tl.rows);
+    cols = __builtin_amdgcn_readfirstlane(tl.cols);
+    // the two workgroups of a CU start half a grid of CUs apart: swapping the wave roles of every other 256
+    // workgroups puts the larger and the smaller share of an odd block count on different SIMDs
+    const int flip = (blockIdx.x >> 8) & 1;
+    const int wm = (wid & 1) ^ flip, wn = (wid >> 1) ^ flip;
+    const int nrb = (rows + 31) / 32, ncb = (cols + 31) / 32;
+    rb0 = wm ? (nrb + 1) / 2 : 0;
+    mi = wm ? nrb - rb0 : (nrb + 1) / 2;
+    cb0 = wn ? (ncb + 1) / 2 : 0;
+    nj = wn ? ncb - cb0 : (ncb + 1) / 2;
+    ldw4 = 4 * (int)tl.ldw;
+    rw = uniform_rsrc(reinterpret_cast<const char*>(static_cast<float*>(t.w) + tl.woff), ldw4 * cols);
+    nst = NSEG * t.nd / 16;
+    npa = (rows + 15) / 16;
+    npb = (cols + 15) / 16;
+    cps = 0;
+#pragma unroll
+    for (int q = 0; q < MB; ++q) {
+      const int r = 16 * (wid + 4 * q) + copy_row<32>(lane);
+      lofa[q] = 16 * copy_unit<32>(lane) + 32 * min(r, rows - 1);
+      lofb[q] = 16 * copy_unit<32>(lane) + tl.col_off(min(r, cols - 1));
+      cps += (wid + 4 * q < npa) + (wid + 4 * q < npb);
+    }
+  }
+  __device__ __forceinline__ void dma(Feed<NSEG, 32>& feed, int slot) const {
+    feed.step([&](__amdgpu_buffer_rsrc_t rsa, __amdgpu_buffer_rsrc_t rsb, int dga, int dgb) {
+#pragma unroll
+      for (int q = 0; q < MB; ++q)
+        if (wid + 4 * q < npa)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_vptr)(ring + slot * SLOT + (wid + 4 * q) * 1024), 16,
+                                                   (unsigned)(lofa[q] + dga), 0, 0, 0);
+#pragma unroll
+      for (int q = 0; q < MB; ++q)
+        if (wid + 4 * q < npb)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rsb, (lds_vptr)(ring + slot * SLOT + ABYTES + (wid + 4 * q) * 1024), 16,
+                                                   (unsigned)(lofb[q] + dgb), 0, 0, 0);
+    });
+  }
+  // MI x NJ blocks of this wave (0 x 0: a wave without a block, which still copies and meets the barriers).
+  // Steps 0 .. NS - 2 start in flight; at step s the copies issued after step s are those of one step (none
+  // at the end), and step s + 2 goes into the slot that step s - 1 left.
+  template <int MI, int NJ>
+  __device__ __forceinline__ void run(Feed<NSEG, 32> feed) const {
+    // row l % 32 of a block, k group l / 32: units 0 (hi) and 1 (lo)
+    const unsigned frag = lds_addr(ring) + unit_at<32>(lane & 31, lane >> 5, 0);
+    const unsigned a_off = frag + rb0 * 2048, b_off = frag + ABYTES + cb0 * 2048;
+    f32x16 acc[MI > 0 ? MI : 1][NJ > 0 ? NJ : 1];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+    dma(feed, 0);
+    if (nst > 1) dma(feed, 1);
+    int cur = 0, nxt = 2;
+    for (int s = 0; s < nst; ++s) {
+      wait_vmcnt_n(s + 1 < nst ? cps : 0);
+      lds_barrier();  // step s landed for every wave; the slot of step s - 1 read by all
+      if (s + 2 < nst) dma(feed, nxt);
+      if constexpr (MI > 0 && NJ > 0) {
+        f32x4 fa[MI][2], fb[NJ][2];
+        read_frags<MI, NJ>(a_off + cur * SLOT, b_off + cur * SLOT, fa, fb);
+        // the MFMA burst at raised wave priority: the other wave of the SIMD issues its LDS reads and
+        // copies under it
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          const bf16x8 bh = __builtin_bit_cast(bf16x8, fb[j][0]), bl = __builtin_bit_cast(bf16x8, fb[j][1]);
+          // B as the first operand, so that the accumulator's lanes run along the rows of W
+#pragma unroll
+          for (int i = 0; i < MI; ++i)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bl, __builtin_bit_cast(bf16x8, fa[i][0]), acc[i][j], 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < MI; ++i)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bh, __builtin_bit_cast(bf16x8, fa[i][1]), acc[i][j], 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < MI; ++i)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bh, __builtin_bit_cast(bf16x8, fa[i][0]), acc[i][j], 0, 0, 0);
+        }
+        __builtin_amdgcn_s_setprio(0);
+      }
+      cur = cur == NS - 1 ? 0 : cur + 1;
+      nxt = nxt == NS - 1 ? 0 : nxt + 1;
+    }
+    if constexpr (MI > 0 && NJ > 0) store_blocks<NSEG == 4, MI, NJ>(acc, rw, rb0 * 32, cb0 * 32, rows, ldw4);
+  }
+  template <int MI>
+  __device__ __forceinline__ void run_n(const Feed<NSEG, 32>& feed) const {
+    if constexpr (MB == 3) {
+      if (nj == 3) {
+        run<MI, 3>(feed);
+        return;
+      }
+    }
+    if (nj == 2) run<MI, 2>(feed);
+    else run<MI, 1>(feed);
+  }
+};
+template <int NSEG, int MB>
+__global__ __launch_bounds__(256, MB == 3 ? 2 : 3) void k_triples_w_bf3(TripW t) {
+  __shared__ __attribute__((aligned(16))) char ring[Bf3Tile<NSEG, MB>::NS * Bf3Tile<NSEG, MB>::SLOT];
+  const TripTile<NSEG, 32> tl(t, 32);
+  const Feed<NSEG, 32> feed(t, tl, threadIdx.x & 63);
+  const Bf3Tile<NSEG, MB> tile(t, tl, ring);
+  if (tile.mi == 0 || tile.nj == 0) {
+    tile.template run<0, 0>(feed);
+    return;
+  }
+  if constexpr (MB == 3) {
+    if (tile.mi == 3) {
+      tile.template run_n<3>(feed);
+      return;
+    }
+  }
+  if (tile.mi == 2) tile.template run_n<2>(feed);
+  else tile.template run_n<1>(feed);
+}
+
+// FP64 and FP32: tiles of 16 NB x 16 NB, NB wavefronts of one 16-row block each (NB column blocks).  An MFMA
+// takes 64 (FP64) or 32 (FP32) cycles, so the fragment reads (one per block and k step: a lane's 16 bytes
+// are 2 (4) k, fed to 2 (4) MFMAs in turn -- the k order inside a step is free as long as A and B agree) hide
+// behind them with four or more wavefronts per SIMD, and small tiles cost little: the tile follows v in
+// steps of 16 instead of padding N = v = 76 to 128.
+template <typename T, int NSEG, int NB>
+__global__ __launch_bounds__(64 * NB) void k_triples_w(TripW t) {
+  constexpr bool F32 = std::is_same<T, float>::value;
+  constexpr int NS = 3, ABYTES = NB * 1024, SLOT = 2 * ABYTES, KL = F32 ? 4 : 2;
+  using Acc = typename std::conditional<F32, f32x4, f64x4>::type;
+  __shared__ __attribute__((aligned(16))) char ring[NS * SLOT];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  constexpr int GB = F32 ? 32 : 64;
+  const TripTile<NSEG, GB> tl(t, 16);
+  const int rows = tl.rows, cols = tl.cols;
+  Feed<NSEG, GB> feed(t, tl, lane);
+  const int nst = NSEG * (t.nd / 8) * GB / 64;
+  const int r = 16 * wid + copy_row<GB>(lane);
+  const int lofa = 16 * copy_unit<GB>(lane) + GB * min(r, rows - 1);
+  const int lofb = 16 * copy_unit<GB>(lane) + tl.col_off(min(r, cols - 1));
+  auto dma = [&](int slot) {
+    feed.step([&](__amdgpu_buffer_rsrc_t rsa, __amdgpu_buffer_rsrc_t rsb, int dga, int dgb) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_vptr)(ring + slot * SLOT + wid * 1024), 16,
+                                               (unsigned)(lofa + dga), 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsb, (lds_vptr)(ring + slot * SLOT + ABYTES + wid * 1024), 16,
+                                               (unsigned)(lofb + dgb), 0, 0, 0);
+    });
+  };
+  // unit l / 16 of the step of row l % 16 (FP32: units of two groups)
+  const int fu = lane >> 4;
+  const unsigned frag = lds_addr(ring) + unit_at<GB>(lane & 15, F32 ? fu >> 1 : 0, F32 ? fu & 1 : fu);
+  const unsigned a_off = frag + wid * 1024, b_off = frag + ABYTES;
+  Acc acc[NB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) acc[j] = Acc{0, 0, 0, 0};
+  dma(0);
+  if (nst > 1) dma(1);
+  int cur = 0, nxt = 2;
+  for (int s = 0; s < nst; ++s) {
+    if (s + 1 < nst) wait_vmcnt<2>();
+    else wait_vmcnt<0>();
+    lds_barrier();
+    if (s + 2 < nst) dma(nxt);
+    f32x4 fa, fb[NB];
+    read_rows<NB>(a_off + cur * SLOT, b_off + cur * SLOT, fa, fb);
+    T af[KL], bf[NB][KL];
+    __builtin_memcpy(af, &fa, 16);
+#pragma unroll
+    for (int j = 0; j < NB; ++j) __builtin_memcpy(bf[j], &fb[j], 16);
+#pragma unroll
+    for (int q = 0; q < KL; ++q)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        // B as the first operand, so that the accumulator's lanes run along the rows of W
+        if constexpr (F32) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[j][q], af[q], acc[j], 0, 0, 0);
+        else acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bf[j][q], af[q], acc[j], 0, 0, 0);
+      }
+    cur = cur == NS - 1 ? 0 : cur + 1;
+    nxt = nxt == NS - 1 ? 0 : nxt + 1;
+  }
+  // register e of lane l of block j: row l % 16, column (l / 16) + 4 e (FP64) or 4 (l / 16) + e (FP32)
+  T* const W = static_cast<T*>(t.w) + tl.woff;
+  const int ldw = (int)tl.ldw, row = 16 * wid + (lane & 15);
+  auto col = [&](int j, int e) { return 16 * j + (F32 ? 4 * (lane >> 4) + e : (lane >> 4) + 4 * e); };
+  if constexpr (NSEG == 4) {
+    T dv[NB][4];
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dv[j][e] = W[row < rows && col(j, e) < cols ? row + ldw * col(j, e) : 0];
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[j][e] += dv[j][e];
+  }
+#pragma unroll
+  for (int j = 0; j < NB; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (row < rows && col(j, e) < cols) W[row + ldw * col(j, e)] = acc[j][e];
+}
+
+// ------------------------------------------------------------------ host side
+// k values per row, zero-padded to whole groups of 8, so that two segments are whole 64-byte steps
+int64_t triples_pitch_elems(int o, int v) { return ((int64_t)(v + o) + 7) / 8 * 8; }
+
+void triples_operands(hipStream_t s, int fmt, int o, int v, const double* ovvv, const double* t2, const double* ooov,
+                      void* av, void* avs, void* bvp, void* bvq) {
+  const int nd = (int)triples_pitch_elems(o, v);
+  const int64_t n4 = (v + 3) / 4, na = n4 * n4 * (nd / 8), nb = n4 * (nd / 8) * (((int64_t)o * o + 31) / 32);
+  FH_CHECK(na < ((int64_t)1 << 31) && nb < ((int64_t)1 << 31), -3, "(T) operand grid too large");
+  const dim3 ga((unsigned)na), gb((unsigned)nb);
+#define FH_OPS(F)                                                                                                     \
+  do {                                                                                                                \
+    hipLaunchKernelGGL(k_triples_av<F>, ga, dim3(256), 0, s, o, v, nd, ovvv, t2, (char*)av, (char*)avs);              \
+    hipLaunchKernelGGL(k_triples_bv<F>, gb, dim3(256), 0, s, o, v, nd, t2, ooov, (char*)bvp, (char*)bvq);             \
+  } while (0)
+  if (fmt == 0) FH_OPS(0);
+  else if (fmt == 1) FH_OPS(1);
+  else FH_OPS(2);
+#undef FH_OPS
+  FH_HIP(hipGetLastError());
+}
+
+// Tile of an axis of n elements: fmt 2: blocks of 32, at most 2 MB of them; else blocks of 16, at most NB
+TriplesTiles triples_tiles(int fmt, int o, int v, double nk) {
+  TriplesTiles t;
+  const int64_t vv = (int64_t)v * v;
+  FH_CHECK(vv < ((int64_t)1 << 31), -3, "(T): v^2 exceeds 32 bits");
+  auto tiles = [](int64_t n, int g, int per) { return (int)(((n + g - 1) / g + per - 1) / per); };
+  if (fmt == 2) {
+    // 128 x 128 tiles (three workgroups per CU) where v fits one, else up to 192 x 192
+    t.nb = v <= 128 ? 2 : 3;
+    t.grain = 32;
+    t.per = 2 * t.nb;
+    t.nb_first = t.nb;
+  } else {
+    // slices: the block count with the least padded area, wider tiles preferred (operand reuse: a tile reads
+    // 2 / NB of a block per block product)
+    auto best = [&](int64_t m, int64_t n) {
+      int nb = 2;
+      double c0 = 1e300;
+      for (int b = 2; b <= 6; ++b) {
+        const double pm = 16.0 * b * tiles(m, 16, b), pn = 16.0 * b * tiles(n, 16, b);
+        const double cost = pm * pn * (1.0 + 0.6 / b);
+        if (cost < c0) { c0 = cost; nb = b; }
+      }
+      return nb;
+    };
+    t.nb = best(v, v);
+    t.nb_first = best(vv, std::max<int64_t>(1, (int64_t)(v * nk)));
+    t.grain = 16;
+    t.per = t.nb;
+  }
+  t.per_first = fmt == 2 ? 2 * t.nb_first : t.nb_first;
+  t.nt = tiles(v, t.grain, t.per);
+  t.nt_first = tiles(vv, t.grain, t.per_first);
+  (void)o;
+  return t;
+}
+void triples_col_tiles(const TriplesTiles& t, int v, int i, int j, int k0, int nk, int slot, std::vector<int>& out) {
+  const int n = v * nk, nt = ((n + t.grain - 1) / t.grain + t.per_first - 1) / t.per_first;
+  for (int q = 0; q < nt; ++q) {
+    const int n0 = tile_begin(n, t.grain, nt, q), n1 = std::min(tile_begin(n, t.grain, nt, q + 1), n);
+    out.insert(out.end(), {i, j, k0, slot, n0, n1 - n0, 0, 0});
+  }
+}
+
+// 1 GiB of W a chunk (and 2048 slice tiles, four rounds of 512): the (T) of o = 40, v = 190 takes 1147, 1134,
+// 1100, 1061 and 1045 ms at 128, 256, 512, 1024 and 4096 MiB (fewer partial rounds), o = 27, v = 131 takes 126,
+// 114, 108, 106 and 108 ms (at 4096 the W written by the first launch no longer meets the second in the
+// memory-side cache).  FERMIHIP_TRIPLES_CHUNK_MB fixes it, for tests.
+int64_t triples_chunk_slots(int v, int elem, const TriplesTiles& tt, int64_t ntot) {
+  const int64_t slot = (int64_t)v * v * v * elem, tiles = (int64_t)tt.nt * tt.nt * v;
+  int64_t n = std::max(((int64_t)1 << 30) / slot, (2048 + tiles - 1) / tiles);
+  if (const char* env = std::getenv("FERMIHIP_TRIPLES_CHUNK_MB")) n = (std::max<int64_t>(1, std::atoll(env)) << 20) / slot;
+  n = std::min(n, std::min<int64_t>((int64_t)8e9 / slot, 60000));  // 60000: the energy launch's grid
+  return std::max<int64_t>(1, std::min(n, ntot));
+}
+
+template <int NSEG>
+static void launch_w(hipStream_t s, int fmt, int nb, unsigned grid, const TripW& t) {
+#define FH_W(T, NB) hipLaunchKernelGGL((k_triples_w<T, NSEG, NB>), dim3(grid), dim3(64 * NB), 0, s, t)
+#define FH_WT(T)               \
+  switch (nb) {                \
+    case 2: FH_W(T, 2); break; \
+    case 3: FH_W(T, 3); break; \
+    case 4: FH_W(T, 4); break; \
+    case 5: FH_W(T, 5); break; \
+    default: FH_W(T, 6); break; \
+  }
+  if (fmt == 2) {
+    if (nb == 2) hipLaunchKernelGGL((k_triples_w_bf3<NSEG, 2>), dim3(grid), dim3(256), 0, s, t);
+    else hipLaunchKernelGGL((k_triples_w_bf3<NSEG, 3>), dim3(grid), dim3(256), 0, s, t);
+  } else if (fmt == 1) {
+    FH_WT(float)
+  } else {
+    FH_WT(double)
+  }
+#undef FH_WT
+#undef FH_W
+  FH_HIP(hipGetLastError());
+}
+
+static TripW trip_args(int fmt, int o, int v, const TriplesOperands& op, void* W, const int* slots, const int* cols) {
+  TripW t;
+  t.av = static_cast<const char*>(op.av);
+  t.avs = static_cast<const char*>(op.avs);
+  t.bvp = static_cast<const char*>(op.bvp);
+  t.bvq = static_cast<const char*>(op.bvq);
+  t.w = W;
+  t.slots = reinterpret_cast<const int4*>(slots);
+  t.cols = reinterpret_cast<const int4*>(cols);
+  t.o = o;
+  t.v = v;
+  t.nd = (int)triples_pitch_elems(o, v);
+  // offsets inside a k step of an operand tile and inside an output tile are 32-bit byte offsets
+  FH_CHECK((int64_t)v * v * 192 * (fmt == 2 ? 4 : 1) < ((int64_t)1 << 31) &&
+               (192 + 2 * (int64_t)v) * t.nd * 8 < ((int64_t)1 << 31),
+           -3, "(T) W build: a tile exceeds 32-bit offsets");
+  return t;
+}
+void triples_w_first(hipStream_t s, int fmt, int o, int v, const TriplesTiles& tt, const TriplesOperands& op, void* W,
+                     const int* cols, int ncol) {
+  TripW t = trip_args(fmt, o, v, op, W, nullptr, cols);
+  t.nt = tt.nt_first;
+  t.ncol = ncol;
+  t.group = 1;
+  const int64_t g = (int64_t)tt.nt_first * ncol;
+  FH_CHECK(g > 0 && g < ((int64_t)1 << 31), -3, "gemm grid too large");
+  launch_w<2>(s, fmt, tt.nb_first, (unsigned)g, t);
+}
+void triples_w_slices(hipStream_t s, int fmt, int o, int v, const TriplesTiles& tt, const TriplesOperands& op, void* W,
+                      const int* slots, int nslot) {
+  TripW t = trip_args(fmt, o, v, op, W, slots, nullptr);
+  t.nt = tt.nt;
+  t.ncol = nslot;
+  t.group = kSlotGroup;
+  const int64_t g = (int64_t)tt.nt * tt.nt * v * nslot;
+  FH_CHECK(g > 0 && g < ((int64_t)1 << 31), -3, "gemm grid too large");
+  launch_w<4>(s, fmt, tt.nb, (unsigned)g, t);
+}
+
+}  // namespace fh
