@@ -694,7 +694,284 @@ __global__ __launch_bounds__(64 * NB) void k_triples_w(TripW t) {
       if (row < rows && col(j, e) < cols) W[row + ldw * col(j, e)] = acc[j][e];
 }
 
-// ------------------------------------------------------------------ host side
+// ------------------------------------------------------------------ (T) energy epilogue (ijk.jl:116-136)
+// For one occupied triple the reference's restricted sum over a>=b>=c with weights 1/(1+d_ab+d_bc) is, with
+// V = W + T1p[a,i] (jb|kc) + (ia|kc) T1p[b,j] + (ia|jb) T1p[c,k] (ijk.jl:116) and the sums S+ of V and W+ of W
+// over the even orderings (abc, bca, cab) and S-, W- over the odd ones (acb, bac, cba),
+//     Ef = 3 sum_p W_p V_p + W+ (S+ - 2 S-) + W- (S- - 2 S+)                    (ijk.jl:129-132)
+// over D_abc, times (2 - d_ij - d_jk); a=b=c terms vanish.  W[a,b,c] of a W slot has a fastest
+// (W + a + v*b + v^2*c + v^3*slot).  The virtual space is cut into 8x8x8 cubes; one workgroup takes an orbit
+// {A,B,C} (A>=B>=C) of cube blocks for a run of consecutive k: the six permuted cubes and the (jb|kc) and (ia|kc)
+// blocks are copied straight into LDS, and a thread owns two elements (a,b,c) with all six orderings, so the
+// denominator, its reciprocal and the sums are formed once per six elements of W and V never leaves the
+// registers.  What does not depend on k ((ia|jb) and T1 of i and j) stays in registers.  Per k a thread reads all it
+// needs from LDS, and the copies of the next k run while it computes (an LDS read behind a copy in flight
+// would be made to wait for it).
+// o = 40, v = 190, FP32 W: 169 ms per (T) against 260 with one ordering per thread, V cubes in LDS and a
+// reciprocal per element (o = 27, v = 131 17.7 against 27.8; FP64 o = 16, v = 76 1.0 against 1.5).  Bound by the
+// fetch: 314 GB of W and as much again of (ia|jb) blocks that miss the L2, about 4 TB/s together.
+static constexpr int CT = 8, CT3 = CT * CT * CT;
+
+// LDS position of element (x, y, z) of a W cube: a Latin-square swizzle under which every x-, y- and z-plane of
+// the cube covers 64 distinct positions modulo 64, so that the six permuted reads (each a plane with one
+// index fixed) have no bank conflicts.
+__device__ __forceinline__ int cube_off(int x, int y, int z) { return 64 * z + ((x + z) & 7) + 8 * ((y + z) & 7); }
+
+// 1/d by the hardware reciprocal and two Newton steps (relative error ~1 ulp; d is a negative
+// orbital-energy denominator, never zero, denormal or infinite)
+__device__ __forceinline__ double rcp_nr(double d) {
+  double r = __builtin_amdgcn_rcp(d);
+  double e = fma(-d, r, 1.0);
+  r = fma(r, e, r);
+  e = fma(-d, r, 1.0);
+  return fma(r, e, r);
+}
+
+template <typename TW>
+__global__ __launch_bounds__(256, 3) void k_triples_energy(int o, int v, const int4* __restrict__ runs,
+                                                           const TW* __restrict__ Wc, const int* __restrict__ orbits,
+                                                           const double* __restrict__ t1p, const double* __restrict__ vvb,
+                                                           const double* __restrict__ eo, const double* __restrict__ ev,
+                                                           double* __restrict__ partials) {
+  constexpr int ED = (int)sizeof(TW) / 4;  // dwords of a W element
+  __shared__ __attribute__((aligned(16))) TW Wl[6 * CT3];
+  __shared__ __attribute__((aligned(16))) double s_vv[2][10][CT * CT];  // [(jk) (ik)][3 x + y (9: unused)][x + 8 y]
+  __shared__ double red[4];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // consecutive workgroups go to different XCDs: give each XCD a contiguous range of orbits, so
+  // the neighbouring cubes of concurrently resident orbits share the W lines in its L2
+  const int nwg = gridDim.x, w = blockIdx.x;
+  const int ob = (w & 7) * (nwg >> 3) + min(w & 7, nwg & 7) + (w >> 3);
+  const int4 run = runs[2 * blockIdx.y];
+  const int i = run.x, j = run.y, k0 = run.z, nk = run.w;
+  const int64_t vv = (int64_t)v * v;
+  const TW* W = Wc + vv * v * runs[2 * blockIdx.y + 1].x;
+  const int blk[3] = {orbits[3 * ob], orbits[3 * ob + 1], orbits[3 * ob + 2]};
+  // the six orderings of the orbit's blocks: (abc) (acb) (bac) (bca) (cab) (cba)
+  constexpr int pb[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
+  // (ia|jb) of occupied pair (p, q) in 8x8 blocks: vvb + PS (p + o q) + 64 (A + nb B) + x + 8 y
+  const int nb = (v + CT - 1) / CT;
+  const int64_t PS = (int64_t)nb * nb * CT * CT;
+  const double* vv_jk = vvb + PS * (j + (int64_t)o * k0);   // (jk) block of k0; + PS*o per k
+  const double* vv_ik = vvb + PS * (i + (int64_t)o * k0);
+  const double* vv_ij = vvb + PS * (i + (int64_t)o * j);
+
+  // Copies of a k.  W: planes z = wid, wid + 4 of the six cubes, a dword per lane and instruction (ED per plane and
+  // element), lane -> LDS position -> (x, y).  vv: two 512-byte blocks per instruction.
+  // Rows and columns beyond v are copied as they lie (the caller pads the end of W): the elements that would
+  // use them are dropped.
+  int clo[2][ED];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int q = 0; q < ED; ++q) {
+      const int z = wid + 4 * h, pos = (lane + 64 * q) / ED;
+      clo[h][q] = (((pos - z) & 7) + v * (((pos >> 3) - z) & 7)) * (int)sizeof(TW) + 4 * ((lane + 64 * q) % ED);
+    }
+  int vlo[3];
+#pragma unroll
+  for (int l = 0; l < 3; ++l) {
+    const int q = (wid + 4 * l) % 5, e = min(2 * q + (lane >> 5), 8);
+    vlo[l] = (blk[e / 3] + nb * blk[e % 3]) * 512 + (lane & 31) * 16;
+  }
+  auto copy = [&](int kk) {
+    const TW* Wk = W + vv * v * kk;
+#pragma unroll
+    for (int p = 0; p < 6; ++p) {
+      const int X0 = blk[pb[p][0]] * CT, Y0 = blk[pb[p][1]] * CT, Z0 = blk[pb[p][2]] * CT;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int z = wid + 4 * h;
+        if (Z0 + z >= v) continue;
+        const __amdgpu_buffer_rsrc_t r = uniform_rsrc(reinterpret_cast<const char*>(Wk + X0 + (int64_t)v * Y0 + vv * (Z0 + z)));
+#pragma unroll
+        for (int q = 0; q < ED; ++q)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(
+              r, (lds_vptr)(reinterpret_cast<char*>(Wl) + ((p * CT + z) * ED + q) * 256), 4, (unsigned)clo[h][q], 0, 0, 0);
+      }
+    }
+    const __amdgpu_buffer_rsrc_t rj = uniform_rsrc(reinterpret_cast<const char*>(vv_jk + PS * o * kk));
+    const __amdgpu_buffer_rsrc_t ri = uniform_rsrc(reinterpret_cast<const char*>(vv_ik + PS * o * kk));
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+      const int q = wid + 4 * l;
+      if (q < 5) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rj, (lds_vptr)(&s_vv[0][2 * q][0]), 16, (unsigned)vlo[l], 0, 0, 0);
+        asm volatile("; (jk)");
+      } else if (q < 10) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(ri, (lds_vptr)(&s_vv[1][2 * (q - 5)][0]), 16, (unsigned)vlo[l], 0, 0, 0);
+        asm volatile("; (ik)");
+      }
+    }
+  };
+  // the thread's two elements: a and b from the lane, c from the wave and h
+  const int x = lane & 7, y = lane >> 3;
+  const int a = blk[0] * CT + x, b = blk[1] * CT + y;
+  copy(0);
+  auto t1 = [&](int e, int q) { return e < v ? t1p[e + (int64_t)v * q] : 0.0; };
+  auto ij = [&](int P, int Q, int r, int q) { return vv_ij[((int64_t)(blk[P] + nb * blk[Q]) << 6) + r + 8 * q]; };
+  const double ia = t1(a, i), ib = t1(b, i), ja = t1(a, j), jb = t1(b, j);
+  const double ij_ab = ij(0, 1, x, y), ij_ba = ij(1, 0, y, x);
+  double ic[2], jc[2], ij_ac[2], ij_ca[2], ij_bc[2], ij_cb[2], es[2], kc[2];
+  float wt[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int z = wid + 4 * h, c = blk[2] * CT + z;
+    ic[h] = t1(c, i);
+    jc[h] = t1(c, j);
+    ij_ac[h] = ij(0, 2, x, z);
+    ij_ca[h] = ij(2, 0, z, x);
+    ij_bc[h] = ij(1, 2, y, z);
+    ij_cb[h] = ij(2, 1, z, y);
+    const bool in = a < v && b < v && c < v && a >= b && b >= c && a > c;
+    wt[h] = in ? (a == b || b == c ? 0.5f : 1.0f) : 0.0f;
+    es[h] = in ? ev[a] + ev[b] + ev[c] : 0.0;
+  }
+  double ka = t1(a, k0), kb = t1(b, k0), acc = 0.0;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) kc[h] = t1(blk[2] * CT + wid + 4 * h, k0);
+  const double eij = eo[i] + eo[j];
+  for (int kk = 0; kk < nk; ++kk) {
+    const int k = k0 + kk;
+    wait_vmcnt<0>();
+    __syncthreads();
+    TW wv[2][6];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int z = wid + 4 * h;
+      wv[h][0] = Wl[0 * CT3 + cube_off(x, y, z)];
+      wv[h][1] = Wl[1 * CT3 + cube_off(x, z, y)];
+      wv[h][2] = Wl[2 * CT3 + cube_off(y, x, z)];
+      wv[h][3] = Wl[3 * CT3 + cube_off(y, z, x)];
+      wv[h][4] = Wl[4 * CT3 + cube_off(z, x, y)];
+      wv[h][5] = Wl[5 * CT3 + cube_off(z, y, x)];
+    }
+    // u = V - W of the six orderings
+    const double jk_ab = s_vv[0][1][x + 8 * y], jk_ba = s_vv[0][3][y + 8 * x];
+    const double ik_ab = s_vv[1][1][x + 8 * y], ik_ba = s_vv[1][3][y + 8 * x];
+    double u[2][6];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int z = wid + 4 * h;
+      const double jk_ac = s_vv[0][2][x + 8 * z], jk_ca = s_vv[0][6][z + 8 * x];
+      const double jk_bc = s_vv[0][5][y + 8 * z], jk_cb = s_vv[0][7][z + 8 * y];
+      const double ik_ac = s_vv[1][2][x + 8 * z], ik_ca = s_vv[1][6][z + 8 * x];
+      const double ik_bc = s_vv[1][5][y + 8 * z], ik_cb = s_vv[1][7][z + 8 * y];
+      u[h][0] = fma(ia, jk_bc, fma(ik_ac, jb, ij_ab * kc[h]));
+      u[h][1] = fma(ia, jk_cb, fma(ik_ab, jc[h], ij_ac[h] * kb));
+      u[h][2] = fma(ib, jk_ac, fma(ik_bc, ja, ij_ba * kc[h]));
+      u[h][3] = fma(ib, jk_ca, fma(ik_ba, jc[h], ij_bc[h] * ka));
+      u[h][4] = fma(ic[h], jk_ab, fma(ik_cb, ja, ij_ca[h] * kb));
+      u[h][5] = fma(ic[h], jk_ba, fma(ik_ca, jb, ij_cb[h] * ka));
+    }
+    lds_barrier();  // every wave has read this k
+    const double D0 = eij + eo[k];
+    if (kk + 1 < nk) {
+      copy(kk + 1);
+      ka = t1(a, k + 1);
+      kb = t1(b, k + 1);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) kc[h] = t1(blk[2] * CT + wid + 4 * h, k + 1);
+    }
+    double ak = 0.0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const double w0 = (double)wv[h][0], w1 = (double)wv[h][1], w2 = (double)wv[h][2], w3 = (double)wv[h][3],
+                   w4 = (double)wv[h][4], w5 = (double)wv[h][5];
+      const double v0 = w0 + u[h][0], v1 = w1 + u[h][1], v2 = w2 + u[h][2], v3 = w3 + u[h][3], v4 = w4 + u[h][4],
+                   v5 = w5 + u[h][5];
+      const double sp = v0 + v3 + v4, sm = v1 + v2 + v5, wp = w0 + w3 + w4, wm = w1 + w2 + w5;
+      const double xx = fma(w0, v0, fma(w1, v1, fma(w2, v2, fma(w3, v3, fma(w4, v4, w5 * v5)))));
+      const double ef = fma(3.0, xx, fma(wp, fma(-2.0, sm, sp), wm * fma(-2.0, sp, sm)));
+      ak += wt[h] != 0.0f ? (double)wt[h] * ef * rcp_nr(D0 - es[h]) : 0.0;
+    }
+    acc += (2.0 - (i == j ? 1.0 : 0.0) - (j == k ? 1.0 : 0.0)) * ak;
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+  if (lane == 0) red[wid] = acc;
+  __syncthreads();
+  if (tid == 0) partials[blockIdx.x + (int64_t)gridDim.x * blockIdx.y] = red[0] + red[1] + red[2] + red[3];
+}
+
+int triples_orbit_count(int v) {
+  const int nb = (v + CT - 1) / CT;
+  return nb * (nb + 1) * (nb + 2) / 6;
+}
+
+// The orbits a >= b >= c of 8-wide cubes, in blocks of 4 x 4 x 4 cube indices: a 128-byte line of W holds
+// the rows of four x-adjacent cubes, so a line read for one cube of an orbit is read again by the orbits
+// whose corresponding cube differs in x within the same group of four; with the (at most 64) orbits of
+// a block consecutive, and consecutive orbits on one XCD (k_triples_energy), those reads meet in its L2.
+void triples_orbits(int v, std::vector<int>& out) {
+  const int nb = (v + CT - 1) / CT;
+  const int ng = (nb + 3) / 4;
+  out.clear();
+  for (int ga = 0; ga < ng; ++ga)
+    for (int gb = 0; gb <= ga; ++gb)
+      for (int gc = 0; gc <= gb; ++gc)
+        for (int a = 4 * ga; a < std::min(nb, 4 * ga + 4); ++a)
+          for (int b = 4 * gb; b < std::min(a + 1, 4 * gb + 4); ++b)
+            for (int c = 4 * gc; c < std::min(b + 1, 4 * gc + 4); ++c) {
+              out.push_back(a);
+              out.push_back(b);
+              out.push_back(c);
+            }
+}
+
+// (ia|jb) = vvoo[a + v b + v^2 (i + o j)] -> vvb in 8x8 blocks (zero-padded), so that a staged
+// block is one contiguous 512-byte run
+__global__ void k_block_vv(int o, int v, int nb, const double* __restrict__ vvoo, double* __restrict__ vvb) {
+  const int64_t PS = (int64_t)nb * nb * CT * CT, n = PS * o * o;
+  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
+    const int64_t pq = e / PS;
+    const int64_t r = e - pq * PS;
+    const int xy = (int)(r & 63);
+    const int64_t blkid = r >> 6;
+    const int A = (int)(blkid % nb), B = (int)(blkid / nb);
+    const int a = A * CT + (xy & 7), b = B * CT + (xy >> 3);
+    vvb[e] = (a < v && b < v) ? vvoo[a + (int64_t)v * b + (int64_t)v * v * pq] : 0.0;
+  }
+}
+
+int64_t triples_vv_blocked_elems(int o, int v) {
+  const int64_t nb = (v + CT - 1) / CT;
+  return nb * nb * CT * CT * o * o;
+}
+
+void triples_block_vv(hipStream_t s, int o, int v, const double* vvoo, double* vvb) {
+  const int nb = (v + CT - 1) / CT;
+  const int64_t n = triples_vv_blocked_elems(o, v);
+  const int64_t g = std::min<int64_t>((n + 255) / 256, 65536 * 4);
+  hipLaunchKernelGGL(k_block_vv, dim3((unsigned)g), dim3(256), 0, s, o, v, nb, vvoo, vvb);
+  FH_HIP(hipGetLastError());
+}
+
+// k values per workgroup: enough workgroups to fill the chip several times over, and a run of k long enough
+// to amortise the k-independent loads (runs of 1, 2, 4, 8, 16 at o = 40, v = 190: 298, 221, 184, 173, 169 ms;
+// FERMIHIP_TRIPLES_KPW = n fixes it, for tuning and for the tests that compare runs of k)
+int triples_energy_kpw(int norb, int nslot) {
+  int kpw = 1;
+  while (kpw < 16 && (int64_t)norb * ((nslot + 2 * kpw - 1) / (2 * kpw)) >= 4096) kpw *= 2;
+  if (const char* env = std::getenv("FERMIHIP_TRIPLES_KPW")) kpw = std::max(1, std::min(64, std::atoi(env)));
+  return kpw;
+}
+
+template <typename TW>
+void triples_energy(hipStream_t s, int o, int v, int nrun, const int* runs, const TW* W, int norb, const int* orbits,
+                    const double* t1p, const double* vvb, const double* eo, const double* ev, double* partials) {
+  FH_CHECK(nrun > 0 && nrun < 65536, -3, "(T) energy: too many runs in a launch");
+  hipLaunchKernelGGL(k_triples_energy<TW>, dim3((unsigned)norb, (unsigned)nrun), dim3(256), 0, s, o, v,
+                     reinterpret_cast<const int4*>(runs), W, orbits, t1p, vvb, eo, ev, partials);
+  FH_HIP(hipGetLastError());
+}
+template void triples_energy<double>(hipStream_t, int, int, int, const int*, const double*, int, const int*,
+                                     const double*, const double*, const double*, const double*, double*);
+template void triples_energy<float>(hipStream_t, int, int, int, const int*, const float*, int, const int*, const double*,
+                                    const double*, const double*, const double*, double*);
+
+// ------------------------------------------------------------------ host side of the W build
 // k values per row, zero-padded to whole groups of 8, so that two segments are whole 64-byte steps
 int64_t triples_pitch_elems(int o, int v) { return ((int64_t)(v + o) + 7) / 8 * 8; }
 
