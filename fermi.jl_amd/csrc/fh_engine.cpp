@@ -117,8 +117,11 @@ struct Ctx {
   int lowp = 0;  // residual contractions: 0 FP64 MFMA, 1 FP32 MFMA, 2 split-BF16x3 MFMA (large GEMMs)
   Buf eo, ev, Boo, Bov, Bvv;
   // 4-index blocks (Julia index order, column-major)
-  Buf OOOO, OOOV, OOVV, OVOV, OVVV, Lovov, Vperm, Pt;
-  Buf Vperm32;  // FP32 copy of Vperm for the mixed-precision ladder (made on first use)
+  Buf OOOO, OOOV, OOVV, OVOV, OVVV;
+  // constants of the residual: LX[k,c,l,d] = 2 (kc|ld) - (kd|lc) and, n2 further, (kd|lc); the ladder's operand
+  // Vs[cd, ab] over pairs (prepare_ladder) and Pt[c,d,a,k] = (kd|ac); FP32 copies of LX and Vs for the
+  // reduced-precision residual (made on first use)
+  Buf LX, Vs, Pt, LX32, Vs32;
   // GEMM operands made from the integral blocks above (a permuted FP64 copy, or an FP32 copy for
   // split-BF16x3): the same for every CC iteration, so made once and kept, up to opcache_cap
   // bytes; key "<block>|<index order>|<d or f>"
@@ -313,8 +316,8 @@ static void contract(Ctx& c, double alpha, const TView& A, const std::string& ia
                      Buf& tmpf) -> const void* {
     if (ready && !bf3) return X.p;
     const char* blk = X.p == c.OVOV.d() ? "ovov" : X.p == c.OVVV.d() ? "ovvv" : X.p == c.OOOV.d() ? "ooov"
-                      : X.p == c.OOVV.d() ? "oovv" : X.p == c.OOOO.d() ? "oooo" : X.p == c.Lovov.d() ? "Lovov"
-                      : nullptr;
+                      : X.p == c.OOVV.d() ? "oovv" : X.p == c.OOOO.d() ? "oooo" : X.p == c.LX.d() ? "Lovov"
+                      : X.p == c.Pt.d() ? "Pt" : nullptr;
     std::string key;
     if (blk) {
       // the source index string is part of the key: two contractions that bind the letters to the
@@ -367,8 +370,8 @@ static void contract(Ctx& c, double alpha, const TView& A, const std::string& ia
   auto gemm = [&](bool ta, bool tb, int64_t m, int64_t n, double al, const void* a, int64_t la, const void* b,
                   int64_t lb, double be, const double* cc, double* d, int64_t ld) {
     if (bf3)
-      gemm_bf3(c.s, ta, tb, m, n, Ksz, al, static_cast<const float*>(a), la, static_cast<const float*>(b), lb, be, cc,
-               ld, d, ld, 0);
+      gemm_bf3(c.s, ta, tb, m, n, Ksz, al, static_cast<const float*>(a), la, 0, static_cast<const float*>(b), lb, 0, be,
+               cc, ld, d, ld, 0, 1, 0);
     else
       gemm_f64(c.s, ta, tb, m, n, Ksz, al, static_cast<const double*>(a), la, 0, static_cast<const double*>(b), lb, 0,
                be, cc, ld, 0, d, ld, 0, 1, 0, work.d(), wsz, c.lowp != 0);
@@ -404,20 +407,22 @@ static void require_df(Ctx& c, bool full = true) {
   FH_CHECK(!full || !c.ov_only, -6, "only Bov was given to fh_set_df: this entry point needs Boo and Bvv too");
 }
 
-// L[k,c,l,d] = 2 (kc|ld) - (kd|lc), the constant of the factorised residual
-static void build_lovov(Ctx& c) {
+// L[k,c,l,d] = 2 (kc|ld) - (kd|lc) and the exchange block (kd|lc), the ring products' constants
+static void build_lx(Ctx& c) {
   const int64_t o = c.o, v = c.v;
-  c.Lovov = dalloc(c, o * v * o * v);
+  c.LX = dalloc(c, 2 * c.n2());
   TView ovov = tv(c.OVOV.d(), {o, v, o, v});
-  perm(c, ovov, "kcld", tv(c.Lovov.d(), {o, v, o, v}), "kcld", 2.0, 0.0);
-  perm(c, ovov, "kdlc", tv(c.Lovov.d(), {o, v, o, v}), "kcld", -1.0, 1.0);
+  perm(c, ovov, "kdlc", tv(c.LX.d() + c.n2(), {o, v, o, v}), "kcld", 1.0, 0.0);
+  d2d(c, c.LX.d(), c.LX.d() + c.n2(), c.n2());
+  axpby_f64(c.s, c.n2(), 2.0, c.OVOV.d(), -1.0, c.LX.d());
+  c.LX32.reset();
 }
 
 static void prepare(Ctx& c) {
   require_df(c);
   if (c.prepared) return;
   if (c.conventional) {  // the blocks came with fh_set_mo
-    build_lovov(c);
+    build_lx(c);
     c.prepared = true;
     return;
   }
@@ -438,9 +443,9 @@ static void prepare(Ctx& c) {
   contract(c, 1.0, Boo, "Qij", Bvv, "Qab", 0.0, tv(c.OOVV.d(), {o, o, v, v}), "ijab");
   contract(c, 1.0, Bov, "Qia", Bov, "Qjb", 0.0, tv(c.OVOV.d(), {o, v, o, v}), "iajb");
   contract(c, 1.0, Bov, "Qia", Bvv, "Qbc", 0.0, tv(c.OVVV.d(), {o, v, v, v}), "iabc");
-  build_lovov(c);
-  c.Vperm.reset();   // the ladder operands follow on first use (prepare_ladder)
-  c.Vperm32.reset();
+  build_lx(c);
+  c.Vs.reset();   // the ladder operands follow on first use (prepare_ladder)
+  c.Vs32.reset();
   c.Pt.reset();
   c.opcache.clear();  // copies of the previous blocks
   c.opcache_bytes = 0;
@@ -448,19 +453,28 @@ static void prepare(Ctx& c) {
   c.lowp = keep;
 }
 
-// The PP ladder's operands (built on the first residual; (T) does not need them):
-// Vperm[c,d,a,b] = (ca|db) = Bvv[Q,c,a] Bvv[Q,d,b] (DFERI.jl:194 permuted), Pt[c,d,a,k] = (kd|ac)
+// The PP ladder's operands (built on the first residual; (T) does not need them): Vs[cd, ab] = (ca|db) +- (da|cb)
+// over c >= d, a >= b (symmetric, then antisymmetric combinations; k_vv_pairs) and Pt[c,d,a,k] = (kd|ac).
+// S = tau V needs only the symmetric and antisymmetric parts of tau in (c, d) against those of V, a quarter of
+// the flops of the full v^2 x v^2 product; the T1 dressing of V is applied to the o^2 v o product with Pt instead.
 static void prepare_ladder(Ctx& c) {
   prepare(c);
-  if (c.Vperm.p && c.Pt.p) return;
+  if (c.Vs.p && c.Pt.p) return;
   const int keep = c.lowp;
   c.lowp = 0;
-  const int64_t o = c.o, v = c.v, Q = c.naux;
-  if (!c.Vperm.p) {  // DF: from Bvv (the conventional VVVV block is permuted into Vperm by fh_set_mo)
-    Timer t(c, "integrals_vvvv", 2.0 * Q * (double)(v * v * v * v));
-    TView Bvv = tv(c.Bvv.d(), {Q, v, v});
-    c.Vperm = dalloc(c, v * v * v * v);
-    contract(c, 1.0, Bvv, "Qca", Bvv, "Qdb", 0.0, tv(c.Vperm.d(), {v, v, v, v}), "cdab");
+  const int64_t o = c.o, v = c.v, Q = c.naux, np = v * (v + 1) / 2, ldv = vv_pairs_ld(v);
+  if (!c.Vs.p) {  // DF: from Bvv (fh_set_mo makes Vs from the conventional VVVV block)
+    // (ca|db) for a block of a and every b up to its last, at most 1 GiB at a time
+    const int64_t na = std::max<int64_t>(1, std::min<int64_t>(((int64_t)1 << 27) / (v * v * v), std::max<int64_t>(8, v / 8)));
+    Timer t(c, "integrals_vvvv", 1.0 * Q * (double)(v * v * v * v));
+    c.Vs = dalloc(c, 2 * ldv * np);
+    Buf T = dalloc(c, std::min(na, v) * v * v * v);
+    for (int64_t a0 = 0; a0 < v; a0 += na) {
+      const int64_t m = std::min(na, v - a0);
+      gemm_f64(c.s, true, false, v * m, v * (a0 + m), Q, 1.0, c.Bvv.d() + Q * v * a0, Q, 0, c.Bvv.d(), Q, 0, 0.0, nullptr, 0,
+               0, T.d(), v * m, 0);
+      vv_pairs(c.s, (int)v, (int)a0, (int)m, T.d(), v, v * m, v * v * m, false, c.Vs.d());
+    }
   }
   c.Pt = dalloc(c, v * v * v * o);
   perm(c, tv(c.OVVV.d(), {o, v, v, v}), "kdac", tv(c.Pt.d(), {v, v, v, o}), "cdak", 1.0, 0.0);
@@ -478,22 +492,36 @@ static void residual(Ctx& c, const double* t1p, const double* t2p, double* R1, d
   Timer tm(c, "residual", 0.0);
   TView t1 = tv(const_cast<double*>(t1p), {o, v}), t2 = tv(const_cast<double*>(t2p), {o, o, v, v});
   TView ovov = tv(c.OVOV.d(), {o, v, o, v}), oooo = tv(c.OOOO.d(), {o, o, o, o}), oovv = tv(c.OOVV.d(), {o, o, v, v});
-  TView ovvv = tv(c.OVVV.d(), {o, v, v, v}), ooov = tv(c.OOOV.d(), {o, o, o, v}), Lovov = tv(c.Lovov.d(), {o, v, o, v});
+  TView ovvv = tv(c.OVVV.d(), {o, v, v, v}), ooov = tv(c.OOOV.d(), {o, o, o, v}), Lovov = tv(c.LX.d(), {o, v, o, v});
   TView r1 = tv(R1, {o, v});
+  const int64_t n2 = c.n2(), ov = o * v, np = v * (v + 1) / 2, mp = o * (o + 1) / 2, ldv = vv_pairs_ld(v);
 
   Buf bFov = dalloc(c, o * v), bFoo = dalloc(c, o * o), bFvv = dalloc(c, v * v), bX = dalloc(c, o * o);
   TView Fov = tv(bFov, {o, v}), Foo = tv(bFoo, {o, o}), Fvv = tv(bFvv, {v, v}), X = tv(bX, {o, o});
-  Buf bu = dalloc(c, c.n2()), btau = dalloc(c, c.n2());
-  TView u = tv(bu, {o, o, v, v}), tau = tv(btau, {o, o, v, v});
-  // u[i,j,a,b] = 2 t2[i,j,a,b] - t2[i,j,b,a];  tau = t2 + t1 (x) t1
-  perm(c, t2, "ijab", u, "ijab", 2.0, 0.0);
-  perm(c, t2, "ijba", u, "ijab", -1.0, 1.0);
-  tau_f64(c.s, (int)o, (int)v, t1p, t2p, 1.0, tau.p);
+  // forms of the amplitudes (k_amp_forms).  Split-BF16x3 takes the ring operands in FP32 where its GEMM is used
+  // (the o^3 v^3 products of at least 1e9 elements, as in contract); the ladder's pairs are FP32 in both
+  // reduced precisions
+  const bool ring32 = c.lowp == 2 && (double)ov * (double)ov * (double)ov >= 1e9;
+  Buf bu = dalloc(c, n2), btau, bring, bpair;
+  if (t1_only) {
+    amp_forms<double, double>(c.s, (int)o, (int)v, t1p, t2p, bu.d(), nullptr, nullptr, nullptr);
+  } else {
+    btau = dalloc(c, n2);
+    bring = Buf(c.pool.get(), (size_t)(2 * n2) * (ring32 ? sizeof(float) : sizeof(double)));
+    bpair = Buf(c.pool.get(), (size_t)(2 * mp * np) * (c.lowp ? sizeof(float) : sizeof(double)));
+    if (ring32) amp_forms<float, float>(c.s, (int)o, (int)v, t1p, t2p, bu.d(), btau.d(), bring.f(), bpair.f());
+    else if (c.lowp) amp_forms<double, float>(c.s, (int)o, (int)v, t1p, t2p, bu.d(), btau.d(), bring.d(), bpair.f());
+    else amp_forms<double, double>(c.s, (int)o, (int)v, t1p, t2p, bu.d(), btau.d(), bring.d(), bpair.d());
+  }
+  TView u = tv(bu, {o, o, v, v});
 
-  // Fov[k,c] = L[k,c,l,d] t1[l,d];  Foo[k,i] = L[k,c,l,d] t2[i,l,c,d] + Fov[k,c] t1[i,c];
+  // Fov[k,c] = L[k,c,l,d] t1[l,d];  Foo[k,i] = L[k,c,l,d] t2[i,l,c,d] + Fov[k,c] t1[i,c] with L t2 = (kc|ld) u[i,l,c,d];
   // Fvv[a,c] = -L[k,c,l,d] t2[k,l,a,d] - t1[k,a] Fov[k,c]
   contract(c, 1.0, Lovov, "kcld", t1, "ld", 0.0, Fov, "kc");
-  contract(c, 1.0, Lovov, "kcld", t2, "ilcd", 0.0, Foo, "ki");
+  if (!t1_only && !ring32)
+    contract(c, 1.0, ovov, "kcld", tv(bring.d(), {o, v, o, v}), "icld", 0.0, Foo, "ki");
+  else
+    contract(c, 1.0, ovov, "kcld", u, "ilcd", 0.0, Foo, "ki");
   contract(c, 1.0, Fov, "kc", t1, "ic", 1.0, Foo, "ki");
   contract(c, -1.0, Lovov, "kcld", t2, "klad", 0.0, Fvv, "ac");
   contract(c, -1.0, t1, "ka", Fov, "kc", 1.0, Fvv, "ac");
@@ -518,9 +546,11 @@ static void residual(Ctx& c, const double* t1p, const double* t2p, double* R1, d
   contract(c, 1.0, ovvv, "kdac", u, "ikcd", 1.0, r1, "ia");
   contract(c, -1.0, ooov, "kilc", u, "klac", 1.0, r1, "ia");
   if (t1_only) return;
+  bu.reset();
 
-  // ---- T2 numerator: P, then R2 = P + P[j,i,b,a]
-  Buf bP = dalloc(c, c.n2());
+  // ---- T2 numerator: P, the ring products and the ladder, then R2 = P + P[j,i,b,a] + ... (k_t2_numerator)
+  TView tau = tv(btau, {o, o, v, v});
+  Buf bP = dalloc(c, n2);
   TView P = tv(bP, {o, o, v, v});
   perm(c, ovov, "iajb", P, "ijab", 0.5, 0.0);                       // (ia|jb)  (:134)
   contract(c, 1.0, ovvv, "iacb", t1, "jc", 1.0, P, "ijab");          // T1 x (ia|cb)
@@ -545,72 +575,77 @@ static void residual(Ctx& c, const double* t1p, const double* t2p, double* R1, d
     contract(c, 1.0, ovov, "kcld", tau, "ijcd", 1.0, W, "klij");
     contract(c, 0.5, W, "klij", tau, "klab", 1.0, P, "ijab");
   }
+  // particle-particle ladder sum_cd tau[i,j,c,d] ((ca|db) - (kd|ac) t1[k,b] - (kc|bd) t1[k,a]): the first part over
+  // packed pairs (prepare_ladder), the others as P -= (tau[i,j,c,d] (kd|ac)) t1[k,b]
+  Buf bS = dalloc(c, 2 * mp * np);
   {
-    // particle-particle ladder: P += tau[i,j,c,d] * Y[c,d,a,b],
-    // Y = 0.5*(ca|db) - sum_k (kd|ac) t1[k,b]   (Wvvvv with the symmetric half folded into P)
-    const int64_t v3 = v * v * v, v4 = v3 * v;
-    if (!c.lowp) {
-      Buf bY = dalloc(c, v4);
-      {
-        Timer tl(c, "ladder_build", 2.0 * o_ * v_ * v_ * v_ * v_);
-        gemm_f64(c.s, false, false, v3, v, o, -1.0, c.Pt.d(), v3, 0, t1p, o, 0, 0.5, c.Vperm.d(), v3, 0, bY.d(), v3, 0);
-      }
-      Timer tl(c, "ladder", 2.0 * o_ * o_ * v_ * v_ * v_ * v_);
-      gemm_f64(c.s, false, false, o * o, v * v, v * v, 1.0, tau.p, o * o, 0, bY.d(), v * v, 0, 1.0, P.p, o * o, 0, P.p,
-               o * o, 0, 1, /*tag: PP ladder*/ 1);
-    } else {
-      // mixed precision: Y and tau in FP32 in HBM, FP32 MFMA, FP64 accumulation into P
-      if (!c.Vperm32.p) {
-        c.Vperm32 = Buf(c.pool.get(), (size_t)v4 * sizeof(float));
-        cast_f64_to_f32(c.s, v4, c.Vperm.d(), c.Vperm32.f());
-      }
-      Buf bY(c.pool.get(), (size_t)v4 * sizeof(float)), tau32(c.pool.get(), (size_t)c.n2() * sizeof(float));
-      cast_f64_to_f32(c.s, c.n2(), tau.p, tau32.f());
-      {
-        Timer tl(c, "ladder_build_fp32", 2.0 * o_ * v_ * v_ * v_ * v_);
-        gemm_f32_df(c.s, v3, v, o, -1.0, c.Pt.d(), v3, t1p, o, 0.5, c.Vperm32.f(), v3, bY.f(), v3);
-      }
-      if (c.lowp == 2) {
-        Timer tl(c, "ladder_bf16x3", 2.0 * o_ * o_ * v_ * v_ * v_ * v_);
-        gemm_bf3(c.s, false, false, o * o, v * v, v * v, 1.0, tau32.f(), o * o, bY.f(), v * v, 1.0, P.p, o * o, P.p,
-                 o * o, 1);
-      } else {
-        Timer tl(c, "ladder_fp32", 2.0 * o_ * o_ * v_ * v_ * v_ * v_);
-        gemm_f32_fd(c.s, o * o, v * v, v * v, 1.0, tau32.f(), o * o, bY.f(), v * v, 1.0, P.p, o * o, P.p, o * o, 1);
-      }
+    const double fl = 4.0 * (double)mp * (double)np * (double)np;
+    if (c.lowp && !c.Vs32.p) {
+      c.Vs32 = Buf(c.pool.get(), (size_t)(2 * ldv * np) * sizeof(float));
+      cast_f64_to_f32(c.s, 2 * ldv * np, c.Vs.d(), c.Vs32.f());
     }
+    Timer tl(c, c.lowp == 2 ? "ladder_bf16x3" : (c.lowp ? "ladder_fp32" : "ladder"), fl);
+    if (!c.lowp)
+      gemm_f64(c.s, false, false, mp, np, np, 1.0, bpair.d(), mp, mp * np, c.Vs.d(), ldv, ldv * np, 0.0, nullptr, 0, 0,
+               bS.d(), mp, mp * np, 2, /*tag: PP ladder*/ 1);
+    else if (c.lowp == 2)
+      gemm_bf3(c.s, false, false, mp, np, np, 1.0, bpair.f(), mp, mp * np, c.Vs32.f(), ldv, ldv * np, 0.0, nullptr, 0,
+               bS.d(), mp, mp * np, 2, 1);
+    else
+      gemm_f32_fd(c.s, mp, np, np, 1.0, bpair.f(), mp, mp * np, c.Vs32.f(), ldv, ldv * np, 0.0, nullptr, 0, bS.d(), mp,
+                  mp * np, 2, 1);
+  }
+  bpair.reset();
+  {
+    Timer tl(c, "ladder_t1", 2.0 * (double)n2 * (double)ov + 2.0 * (double)n2 * o_);
+    Buf bk = dalloc(c, o * o * v * o);
+    contract(c, 1.0, tau, "ijcd", tv(c.Pt.d(), {v, v, v, o}), "cdak", 0.0, tv(bk, {o, o, v, o}), "ijak");
+    contract(c, -1.0, tv(bk, {o, o, v, o}), "ijak", t1, "kb", 1.0, P, "ijab");
   }
   contract(c, 1.0, Lvv, "ac", t2, "ijcb", 1.0, P, "ijab");
   contract(c, -1.0, Loo, "ki", t2, "kjab", 1.0, P, "ijab");
+  // Rings.  With A = Wvoov[i,a,k,c] and B = Wvovo[i,a,k,c] (operators of the ring and crossed ring) the three
+  // applications A u - B t2 - (crossed) B t2 are
+  //   C u / 2 - Z / 2 - Z[ibja],  C = 2 A - B,  Z[iajb] = B[iakc] t2[kjbc],
+  // and the (kc|ld) t2 parts of C and B are L u / 2 and -(kd|lc) t2[ilda] / 2: four o^3 v^3 products over (o v)
+  // square matrices in [i,a,j,b] order, in two batches of two.
+  Buf bD = dalloc(c, 2 * n2);
   {
-    Timer tr(c, c.lowp == 2 ? "ring_bf16x3" : (c.lowp ? "ring_fp32" : "ring"), 6.0 * 2.0 * o_ * o_ * o_ * v_ * v_ * v_);
-    Buf bWa = dalloc(c, c.n2()), bWb = dalloc(c, c.n2()), bXX = dalloc(c, o * o * o * v);  // XX[l,k,c,i] and XY[l,c,k,i]: o^3 v
-    TView Wvoov = tv(bWa, {v, o, o, v}), Wvovo = tv(bWb, {v, o, v, o});
-    // Wvoov[a,k,i,c]
-    perm(c, ovov, "kcia", Wvoov, "akic", 1.0, 0.0);
-    contract(c, 1.0, ovvv, "kcad", t1, "id", 1.0, Wvoov, "akic");
-    contract(c, -1.0, ooov, "likc", t1, "la", 1.0, Wvoov, "akic");
-    TView XX = tv(bXX, {o, o, v, o});
-    contract(c, 1.0, ovov, "ldkc", t1, "id", 0.0, XX, "lkci");
-    contract(c, -1.0, XX, "lkci", t1, "la", 1.0, Wvoov, "akic");
-    contract(c, 0.5, ovov, "ldkc", u, "ilad", 1.0, Wvoov, "akic");
-    contract(c, -0.5, ovov, "lckd", t2, "ilad", 1.0, Wvoov, "akic");
-    // Wvovo[a,k,c,i]
-    perm(c, oovv, "kiac", Wvovo, "akci", 1.0, 0.0);
-    contract(c, 1.0, ovvv, "kdac", t1, "id", 1.0, Wvovo, "akci");
-    contract(c, -1.0, ooov, "kilc", t1, "la", 1.0, Wvovo, "akci");
-    TView XY = tv(bXX, {o, v, o, o});
-    contract(c, 1.0, ovov, "lckd", t1, "id", 0.0, XY, "lcki");
-    contract(c, -1.0, XY, "lcki", t1, "la", 1.0, Wvovo, "akci");
-    contract(c, -0.5, ovov, "lckd", t2, "ilda", 1.0, Wvovo, "akci");
-    // ring / crossed-ring application
-    contract(c, 1.0, Wvoov, "akic", u, "kjcb", 1.0, P, "ijab");
-    contract(c, -1.0, Wvovo, "akci", t2, "kjcb", 1.0, P, "ijab");
-    contract(c, -1.0, Wvovo, "bkci", t2, "kjac", 1.0, P, "ijab");
+    Timer tr(c, c.lowp == 2 ? "ring_bf16x3" : (c.lowp ? "ring_fp32" : "ring"), 4.0 * 2.0 * o_ * o_ * o_ * v_ * v_ * v_);
+    Buf bW = dalloc(c, 2 * n2), bXX = dalloc(c, o * o * o * v);
+    TView Cw = tv(bW.d(), {o, v, o, v}), Bw = tv(bW.d() + n2, {o, v, o, v});
+    perm(c, oovv, "kiac", Bw, "iakc", 1.0, 0.0);
+    contract(c, 1.0, t1, "id", ovvv, "kdac", 1.0, Bw, "iakc");
+    TView Y = tv(bXX, {o, o, o, v});
+    // Y[k,i,l,c] = (ki|lc) + (lc|kd) t1[i,d]
+    perm(c, ooov, "kilc", Y, "kilc", 1.0, 0.0);
+    contract(c, 1.0, ovov, "lckd", t1, "id", 1.0, Y, "kilc");
+    contract(c, -1.0, Y, "kilc", t1, "la", 1.0, Bw, "iakc");
+    // C = 2 A - B: 2 (ia|kc) + 2 (kc|ad) t1[i,d] - 2 ((li|kc) + (ld|kc) t1[i,d]) t1[l,a] - B
+    d2d(c, Cw.p, Bw.p, n2);
+    axpby_f64(c.s, n2, 2.0, c.OVOV.d(), -1.0, Cw.p);
+    contract(c, 2.0, t1, "id", ovvv, "kcad", 1.0, Cw, "iakc");
+    perm(c, ooov, "likc", Y, "likc", 1.0, 0.0);
+    contract(c, 1.0, ovov, "ldkc", t1, "id", 1.0, Y, "likc");
+    contract(c, -2.0, Y, "likc", t1, "la", 1.0, Cw, "iakc");
+    // [C | B] += 1/2 [u | -t2[ilda]] [L | (lc|kd)], then [D | F] = [C | B] [u | -t2[kjbc]]
+    if (ring32) {
+      if (!c.LX32.p) {
+        c.LX32 = Buf(c.pool.get(), (size_t)(2 * n2) * sizeof(float));
+        cast_f64_to_f32(c.s, 2 * n2, c.LX.d(), c.LX32.f());
+      }
+      gemm_bf3(c.s, false, false, ov, ov, ov, 0.5, bring.f(), ov, n2, c.LX32.f(), ov, n2, 1.0, bW.d(), ov, bW.d(), ov, n2, 2, 0);
+      Buf bW32(c.pool.get(), (size_t)(2 * n2) * sizeof(float));
+      cast_f64_to_f32(c.s, 2 * n2, bW.d(), bW32.f());
+      gemm_bf3(c.s, false, false, ov, ov, ov, 1.0, bW32.f(), ov, n2, bring.f(), ov, n2, 0.0, nullptr, 0, bD.d(), ov, n2, 2, 0);
+    } else {
+      gemm_f64(c.s, false, false, ov, ov, ov, 0.5, bring.d(), ov, n2, c.LX.d(), ov, n2, 1.0, bW.d(), ov, n2, bW.d(), ov, n2,
+               2, 0, nullptr, 0, c.lowp != 0);
+      gemm_f64(c.s, false, false, ov, ov, ov, 1.0, bW.d(), ov, n2, bring.d(), ov, n2, 0.0, nullptr, 0, 0, bD.d(), ov, n2, 2,
+               0, nullptr, 0, c.lowp != 0);
+    }
   }
-  TView r2 = tv(R2, {o, o, v, v});
-  perm(c, P, "ijab", r2, "ijab", 1.0, 0.0);
-  perm(c, P, "jiba", r2, "ijab", 1.0, 1.0);                          // (:190)
+  t2_numerator(c.s, (int)o, (int)v, P.p, bD.d(), bD.d() + n2, bS.d(), R2);   // (:190)
 }
 
 static double energy(Ctx& c, const double* t1, const double* t2) {
@@ -1498,8 +1533,8 @@ static void new_molecule(Ctx& c, int o, int v, int naux, const double* eps_o, co
   c.have_df = false;
   c.prepared = false;
   c.have_amp = false;
-  c.OOOO.reset(); c.OOOV.reset(); c.OOVV.reset(); c.OVOV.reset(); c.OVVV.reset(); c.Lovov.reset();
-  c.Vperm.reset(); c.Vperm32.reset(); c.Pt.reset(); c.T1.reset(); c.T2.reset();
+  c.OOOO.reset(); c.OOOV.reset(); c.OOVV.reset(); c.OVOV.reset(); c.OVVV.reset();
+  c.LX.reset(); c.LX32.reset(); c.Vs.reset(); c.Vs32.reset(); c.Pt.reset(); c.T1.reset(); c.T2.reset();
   c.Boo.reset(); c.Bov.reset(); c.Bvv.reset();
   c.opcache.clear(); c.opcache_bytes = 0;
   c.have_model = false; c.pair_d.reset();
@@ -1536,8 +1571,8 @@ int fh_set_df(fh_ctx* x, int o, int v, int naux, const double* eps_o, const doub
 
 // The conventional (Chonky) integral path of RCCSD(moints, aoints, ::RCCSDa), RCCSDa.jl:25-35: the six
 // 4-index MO blocks are handed over as computed by compute_OOOO! ... compute_VVVV! (Chonky.jl) and
-// Fd / Fia of compute_F! (Fock.jl:1-36).  VVVV goes straight into the ladder's operand layout
-// Vperm[c,d,a,b] = VVVV[c,a,d,b] (the conventional ladder tau[i,j,c,d] VVVV[c,a,d,b],
+// Fd / Fia of compute_F! (Fock.jl:1-36).  VVVV goes straight into the ladder's operand layout, the pairs
+// Vs[cd, ab] of VVVV[c,a,d,b] (the conventional ladder tau[i,j,c,d] VVVV[c,a,d,b],
 // RCCSDHelper.jl:194-202); the other blocks are kept in the reference's index order.
 int fh_set_mo(fh_ctx* x, int o, int v, const double* eps_o, const double* eps_v, const double* Fia,
               const double* OOOO, const double* OOOV, const double* OOVV, const double* OVOV, const double* OVVV,
@@ -1560,8 +1595,8 @@ int fh_set_mo(fh_ctx* x, int o, int v, const double* eps_o, const double* eps_v,
     {
       Buf tmp;
       up(tmp, VVVV, V * V * V * V);
-      c.Vperm = dalloc(c, V * V * V * V);
-      perm(c, tv(tmp.d(), {V, V, V, V}), "cadb", tv(c.Vperm.d(), {V, V, V, V}), "cdab", 1.0, 0.0);
+      c.Vs = dalloc(c, V * (V + 1) * vv_pairs_ld(v));
+      vv_pairs(c.s, v, 0, v, tmp.d(), V, V * V, V * V * V, true, c.Vs.d());
       FH_HIP(hipStreamSynchronize(c.s));
     }
     if (Fia) {

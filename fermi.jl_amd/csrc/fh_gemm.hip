@@ -311,24 +311,18 @@ void gemm_f64(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, 
   }
 }
 
-// FP32-MFMA GEMMs with FP32 operands or output in HBM (NN, no split-K)
-template <int TAG, typename TI, typename TO>
-static void gemm_nn_f32(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const TI* A, int64_t lda,
-                        const TI* B, int64_t ldb, double beta, const TO* C, int64_t ldc, TO* D, int64_t ldd) {
-  if (M <= 0 || N <= 0) return;
+// FP32-MFMA GEMM with FP32 operands in HBM and FP64 output (NN, no split-K)
+void gemm_f32_fd(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const float* A, int64_t lda, int64_t sA,
+                 const float* B, int64_t ldb, int64_t sB, double beta, const double* C, int64_t ldc, double* D, int64_t ldd,
+                 int64_t sD, int64_t batch, int tag) {
+  if (M <= 0 || N <= 0 || batch <= 0) return;
   check_args(M, K, N, false, false, lda, ldb, ldd, beta, C, ldc);
-  pick<false, false, TAG, true, TI, TO>(s, M, N, K, alpha, A, lda, 0, B, ldb, 0, beta, C, ldc, 0, D, ldd, 0, 1, 0);
-}
-
-void gemm_f32_fd(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const float* A, int64_t lda,
-                 const float* B, int64_t ldb, double beta, const double* C, int64_t ldc, double* D, int64_t ldd, int tag) {
-  if (tag == 1) gemm_nn_f32<1>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, D, ldd);
-  else gemm_nn_f32<0>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, D, ldd);
-}
-
-void gemm_f32_df(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const double* A, int64_t lda,
-                 const double* B, int64_t ldb, double beta, const float* C, int64_t ldc, float* D, int64_t ldd) {
-  gemm_nn_f32<0>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, D, ldd);
+  if (tag == 1)
+    pick<false, false, 1, true, float, double>(s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sD, D, ldd, sD,
+                                               batch, 0);
+  else
+    pick<false, false, 0, true, float, double>(s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sD, D, ldd, sD,
+                                               batch, 0);
 }
 
 // FP32 operands and output, any transposition (the T2-guess network's layers; tag 3)

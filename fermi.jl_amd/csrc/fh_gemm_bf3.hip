@@ -496,15 +496,15 @@ static void launch_bf3(hipStream_t s, int64_t M, int64_t N, int64_t K, double al
 }
 
 void gemm_bf3(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, double alpha, const float* A,
-              int64_t lda, const float* B, int64_t ldb, double beta, const double* C, int64_t ldc, double* D, int64_t ldd,
-              int tag) {
-  if (M <= 0 || N <= 0) return;
+              int64_t lda, int64_t sA, const float* B, int64_t ldb, int64_t sB, double beta, const double* C, int64_t ldc,
+              double* D, int64_t ldd, int64_t sD, int64_t batch, int tag) {
+  if (M <= 0 || N <= 0 || batch <= 0) return;
   FH_CHECK(K >= 0, -3, "gemm: negative K");
   FH_CHECK(lda >= (ta ? (K > 0 ? K : 1) : M) && ldb >= (tb ? N : (K > 0 ? K : 1)) && ldd >= M, -3,
            "gemm: leading dimension too small");
   FH_CHECK(beta == 0.0 || (C != nullptr && ldc >= M), -3, "gemm: C missing");
 #define FH_BF3(TA_, TB_, TAG_) \
-  launch_bf3<TA_, TB_, TAG_, float, double>(s, M, N, K, alpha, A, lda, 0, B, ldb, 0, beta, C, ldc, 0, D, ldd, 0, 1)
+  launch_bf3<TA_, TB_, TAG_, float, double>(s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sD, D, ldd, sD, batch)
   if (tag == 1) {
     FH_CHECK(!ta && !tb, -3, "gemm_bf3: the PP ladder (tag 1) takes untransposed operands");
     FH_BF3(false, false, 1);

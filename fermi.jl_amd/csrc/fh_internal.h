@@ -96,20 +96,18 @@ void gemm_f64(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, 
               bool f32 = false);
 // f32 = true: operands rounded to FP32 in LDS, FP32 MFMA with FP32 accumulation (mixed precision)
 
-// FP32-MFMA GEMMs (NN) with FP32 data in HBM: _fd float operands -> double output, _df double operands ->
-// float output
-void gemm_f32_fd(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const float* A, int64_t lda,
-                 const float* B, int64_t ldb, double beta, const double* C, int64_t ldc, double* D, int64_t ldd, int tag);
-void gemm_f32_df(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const double* A, int64_t lda,
-                 const double* B, int64_t ldb, double beta, const float* C, int64_t ldc, float* D, int64_t ldd);
+// FP32-MFMA GEMM (NN) with FP32 operands in HBM and FP64 output
+void gemm_f32_fd(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const float* A, int64_t lda, int64_t sA,
+                 const float* B, int64_t ldb, int64_t sB, double beta, const double* C, int64_t ldc, double* D, int64_t ldd,
+                 int64_t sD, int64_t batch, int tag);
 // FP32 operands and output, any transposition, C = alpha op(A) op(B) + beta C (tag 3)
 void gemm_f32(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, double alpha, const float* A,
               int64_t lda, const float* B, int64_t ldb, double beta, float* C, int64_t ldc);
 // split-BF16x3 MFMA GEMM (three bf16 products per FP32 product, FP32 accumulation) on FP32 operands with FP64
 // output: tag 0 any transposition, tag 1 (the PP ladder) untransposed; the tags give distinct kernel symbols
 void gemm_bf3(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, double alpha, const float* A,
-              int64_t lda, const float* B, int64_t ldb, double beta, const double* C, int64_t ldc, double* D, int64_t ldd,
-              int tag);
+              int64_t lda, int64_t sA, const float* B, int64_t ldb, int64_t sB, double beta, const double* C, int64_t ldc,
+              double* D, int64_t ldd, int64_t sD, int64_t batch, int tag);  // (C strided as D)
 
 // ---------------------------------------------------------------- (T) W build (fh_triples.hip)
 // fmt: 0 FP64, 1 FP32, 2 split-BF16x3 (W in FP32).  Operands hold triples_pitch_elems(o, v) values of k per
@@ -172,8 +170,16 @@ void permute_f64(hipStream_t s, int nd, const int64_t* odim, const int64_t* istr
 
 void axpby_f64(hipStream_t s, int64_t n, double a, const double* x, double b, double* y);  // y = a x + b y
 void fill_f64(hipStream_t s, int64_t n, double v, double* y);
-// out[i,j,a,b] = t2 + t1[i,a] t1[j,b]
-void tau_f64(hipStream_t s, int o, int v, const double* t1, const double* t2, double c, double* out);
+// amplitude forms of the CCSD residual's GEMMs, any output null: u, tau [ijab]; ring [iajb] x 2 (u, -t2[ijba]);
+// pair [ij, ab] over i >= j, a >= b, x 2 (symmetric, antisymmetric)
+template <typename TR, typename TP>
+void amp_forms(hipStream_t s, int o, int v, const double* t1, const double* t2, double* u, double* tau, TR* ring, TP* pair);
+// the PP ladder's operand V[cd,ab] +- V[dc,ab] over c >= d, a >= b for a0 <= a < a0 + na (see k_vv_pairs), columns
+// vv_pairs_ld(v) apart
+int64_t vv_pairs_ld(int64_t v);
+void vv_pairs(hipStream_t s, int v, int a0, int na, const double* T, int64_t sa, int64_t sd, int64_t sb, bool sym, double* out);
+// T2 numerator from P[ijab], the ring products D, F [iajb] and the packed ladder Sp [ij, ab] x 2
+void t2_numerator(hipStream_t s, int o, int v, const double* P, const double* D, const double* F, const double* Sp, double* R2);
 // T1/T2 Jacobi update: new = R / D (D from eps on the fly); writes new into R, err = new - old
 // (as FP64 or FP32) and per-block partial sums of err^2.
 void jacobi_update(hipStream_t s, int o, int v, bool is_t2, const double* eo, const double* ev, double* R,

@@ -226,18 +226,174 @@ void fill_f64(hipStream_t s, int64_t n, double v, double* y) {
   FH_HIP(hipGetLastError());
 }
 
-// tau[i,j,a,b] = t2[i,j,a,b] + c * t1[i,a] t1[j,b]
-__global__ void k_tau(int o, int v, const double* __restrict__ t1, const double* __restrict__ t2, double c,
-                      double* __restrict__ out) {
-  const int64_t n = (int64_t)o * o * v * v;
-  for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < n; idx += (int64_t)gridDim.x * 256) {
-    const int64_t i = idx % o, j = (idx / o) % o, a = (idx / ((int64_t)o * o)) % v, b = idx / ((int64_t)o * o * v);
-    out[idx] = t2[idx] + c * t1[i + o * a] * t1[j + o * b];
+// ------------------------------------------------------------------ CCSD residual: operand forms and assembly
+// Every form of the amplitudes that the residual's GEMMs read, from one read of T2 (each T2[:,:,a,b] tile with its
+// partner [:,:,b,a]; any output may be null):
+//   u[i,j,a,b] = 2 t2[ijab] - t2[ijba],  tau[i,j,a,b] = t2 + t1[ia] t1[jb],
+//   ring[i,a,j,b] = u[ijab] and, n2 further, -t2[ijba],
+//   pair[ij, ab] (i >= j, a >= b) = ts[ijab] + ts[ijba] (a > b; ts[ijaa] for a = b) and, Mp Kp further,
+//   ts[ijab] - ts[ijba], with ts = (tau[ijab] + tau[jiba]) / 2.
+template <typename TR, typename TP>
+__global__ __launch_bounds__(256) void k_amp_forms(int o, int v, const double* __restrict__ t1, const double* __restrict__ t2,
+                                                   double* __restrict__ u, double* __restrict__ tau, TR* __restrict__ ring,
+                                                   TP* __restrict__ pair) {
+  const int64_t oo = (int64_t)o * o, n2 = oo * v * v, ov = (int64_t)o * v;
+  const int64_t np = (int64_t)v * (v + 1) / 2, mp = oo / 2 + (o + 1) / 2;
+  const int64_t nblk = (oo + 255) / 256;
+  for (int64_t w = blockIdx.x; w < np * nblk; w += gridDim.x) {
+    const int64_t p = w / nblk;
+    const int e = (int)(w - p * nblk) * 256 + threadIdx.x;
+    int a = (int)((sqrt(8.0 * (double)p + 1.0) - 1.0) * 0.5);
+    while ((int64_t)a * (a + 1) / 2 > p) --a;
+    while ((int64_t)(a + 1) * (a + 2) / 2 <= p) ++a;
+    const int b = (int)(p - (int64_t)a * (a + 1) / 2);
+    if (e >= oo) continue;
+    const int i = e % o, j = e / o, et = j + o * i;
+    const int64_t ab = oo * (a + (int64_t)v * b), ba = oo * (b + (int64_t)v * a);
+    const double x = t2[ab + e], y = t2[ba + e];
+    const double xt = pair ? t2[ba + et] : 0.0, yt = pair ? t2[ab + et] : 0.0;
+    const double s = t1[i + (int64_t)o * a] * t1[j + (int64_t)o * b], r = t1[i + (int64_t)o * b] * t1[j + (int64_t)o * a];
+    if (u) {
+      u[ab + e] = 2.0 * x - y;
+      u[ba + e] = 2.0 * y - x;
+    }
+    if (tau) {
+      tau[ab + e] = x + s;
+      tau[ba + e] = y + r;
+    }
+    if (ring) {
+      const int64_t f = i + (int64_t)o * a + ov * j + ov * o * b, g = i + (int64_t)o * b + ov * j + ov * o * a;
+      ring[f] = (TR)(2.0 * x - y);
+      ring[g] = (TR)(2.0 * y - x);
+      ring[n2 + f] = (TR)(-y);
+      ring[n2 + g] = (TR)(-x);
+    }
+    if (pair && i >= j) {
+      const double ta = 0.5 * (x + xt) + s, tb = 0.5 * (y + yt) + r;
+      const int64_t m = (int64_t)i * (i + 1) / 2 + j + mp * p;
+      pair[m] = (TP)(a == b ? ta : ta + tb);
+      pair[m + mp * np] = (TP)(a == b ? 0.0 : ta - tb);
+    }
   }
 }
-void tau_f64(hipStream_t s, int o, int v, const double* t1, const double* t2, double c, double* out) {
-  const int64_t n = (int64_t)o * o * v * v;
-  hipLaunchKernelGGL(k_tau, dim3(grid_for(n)), dim3(256), 0, s, o, v, t1, t2, c, out);
+template <typename TR, typename TP>
+void amp_forms(hipStream_t s, int o, int v, const double* t1, const double* t2, double* u, double* tau, TR* ring, TP* pair) {
+  const int64_t w = (int64_t)v * (v + 1) / 2 * (((int64_t)o * o + 255) / 256);
+  hipLaunchKernelGGL((k_amp_forms<TR, TP>), dim3((unsigned)std::min<int64_t>(w, 65536)), dim3(256), 0, s, o, v, t1, t2, u,
+                     tau, ring, pair);
+  FH_HIP(hipGetLastError());
+}
+template void amp_forms<double, double>(hipStream_t, int, int, const double*, const double*, double*, double*, double*, double*);
+template void amp_forms<double, float>(hipStream_t, int, int, const double*, const double*, double*, double*, double*, float*);
+template void amp_forms<float, float>(hipStream_t, int, int, const double*, const double*, double*, double*, float*, float*);
+
+// The PP ladder's operand over pairs c >= d, a >= b: with V[cd,ab] = (ca|db) = T(c, a, d, b) (element c + v-strides,
+// T at sa a + sd d + sb b from its first a),
+//   out[cd, ab] = V[cd,ab] + V[dc,ab]  and, behind all of them,  V[cd,ab] - V[dc,ab];
+// sym: V is replaced by (V[cd,ab] + V[dc,ba]) / 2, its part that reaches the symmetrised residual (T must then
+// hold every a and b).  32 x 32 tiles over (c, d): both reads run along the first index, the writes along d.
+__global__ __launch_bounds__(256) void k_vv_pairs(int v, int a0, int na, const double* __restrict__ T, int64_t sa, int64_t sd,
+                                                  int64_t sb, bool sym, int64_t ldv, double* __restrict__ out) {
+  __shared__ double x[32][33], y[32][33];  // V[cd,ab] as [d][c], V[dc,ab] as [c][d]
+  int ct = 0, q = blockIdx.x;
+  while (q > ct) { q -= ct + 1; ++ct; }
+  const int c0 = 32 * ct, d0 = 32 * q, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  const int a = a0 + blockIdx.y, b = blockIdx.z;
+  if (b > a || a >= a0 + na) return;
+  const double* t = T + sa * (a - a0) + sb * b;
+  const double* r = T + sa * b + sb * a;  // sym only
+  for (int k = ty; k < 32; k += 8) {
+    double p = 0.0, m = 0.0;
+    if (c0 + tx < v && d0 + k < v) p = sym ? 0.5 * t[c0 + tx + sd * (d0 + k)] : t[c0 + tx + sd * (d0 + k)];
+    if (d0 + tx < v && c0 + k < v) m = sym ? 0.5 * t[d0 + tx + sd * (c0 + k)] : t[d0 + tx + sd * (c0 + k)];
+    x[k][tx] = p;
+    y[k][tx] = m;
+  }
+  if (sym) {
+    __syncthreads();
+    for (int k = ty; k < 32; k += 8) {
+      // + V[dc,ba] = T(d, b, c, a) to V[cd,ab], + V[cd,ba] = T(c, b, d, a) to V[dc,ab]
+      if (d0 + tx < v && c0 + k < v) x[tx][k] += 0.5 * r[d0 + tx + sd * (c0 + k)];
+      if (c0 + tx < v && d0 + k < v) y[tx][k] += 0.5 * r[c0 + tx + sd * (d0 + k)];
+    }
+  }
+  __syncthreads();
+  const int64_t col = ldv * ((int64_t)a * (a + 1) / 2 + b), anti = ldv * ((int64_t)v * (v + 1) / 2);
+  for (int k = ty; k < 32; k += 8) {
+    const int c = c0 + k, d = d0 + tx;
+    if (c >= v || d > c) continue;
+    const int64_t at = col + (int64_t)c * (c + 1) / 2 + d;
+    out[at] = x[tx][k] + y[k][tx];
+    out[at + anti] = x[tx][k] - y[k][tx];
+  }
+  if (c0 + 32 >= v && d0 == 0 && threadIdx.x < 4) {  // the padding of the column
+    const int64_t np = (int64_t)v * (v + 1) / 2 + threadIdx.x;
+    if (np < ldv) out[col + np] = out[col + anti + np] = 0.0;
+  }
+}
+// whole 16-byte loads of FP32 columns
+int64_t vv_pairs_ld(int64_t v) { return (v * (v + 1) / 2 + 3) / 4 * 4; }
+void vv_pairs(hipStream_t s, int v, int a0, int na, const double* T, int64_t sa, int64_t sd, int64_t sb, bool sym, double* out) {
+  const int nt = (v + 31) / 32;
+  FH_CHECK(v < 65536, -3, "vv_pairs: grid too large");
+  hipLaunchKernelGGL(k_vv_pairs, dim3((unsigned)(nt * (nt + 1) / 2), (unsigned)na, (unsigned)(a0 + na)), dim3(256), 0, s, v, a0,
+                     na, T, sa, sd, sb, sym, vv_pairs_ld(v), out);
+  FH_HIP(hipGetLastError());
+}
+
+// T2 numerator from its parts:
+//   R2[ijab] = G[ijab] + G[jiba] + S[ijab],  G[ijab] = P[ijab] + (D[iajb] + F[iajb]) / 2 + F[ibja],
+// D, F the two ring products in [i,a,j,b] order and S the ladder, S[ijab] = (Sp +- Sm)[ij, ab] / 2 over the packed
+// pairs (+ where i >= j and a >= b agree).  One 32 x 32 (i, j) tile of an (a >= b) pair per workgroup step gives
+// R2[ijab] and its mirror R2[jiba].
+__global__ __launch_bounds__(256) void k_t2_numerator(int o, int v, const double* __restrict__ P, const double* __restrict__ D,
+                                                      const double* __restrict__ F, const double* __restrict__ Sp,
+                                                      double* __restrict__ R2) {
+  __shared__ double gt[32][33];  // G[jiba] as [i][j]
+  const int64_t oo = (int64_t)o * o, ov = (int64_t)o * v, np = (int64_t)v * (v + 1) / 2, mp = oo / 2 + (o + 1) / 2;
+  const int nt = (o + 31) / 32, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  for (int64_t w = blockIdx.x; w < np * nt * nt; w += gridDim.x) {
+    const int64_t p = w / (nt * nt);
+    const int tl = (int)(w - p * nt * nt), i0 = 32 * (tl % nt), j0 = 32 * (tl / nt);
+    int a = (int)((sqrt(8.0 * (double)p + 1.0) - 1.0) * 0.5);
+    while ((int64_t)a * (a + 1) / 2 > p) --a;
+    while ((int64_t)(a + 1) * (a + 2) / 2 <= p) ++a;
+    const int b = (int)(p - (int64_t)a * (a + 1) / 2);
+    const int64_t ab = oo * (a + (int64_t)v * b), ba = oo * (b + (int64_t)v * a);
+    const int64_t rab = (int64_t)o * a + ov * o * b, rba = (int64_t)o * b + ov * o * a;  // ring offsets of (a, b), (b, a)
+    __syncthreads();
+    for (int k = ty; k < 32; k += 8) {
+      const int j = j0 + tx, i = i0 + k;  // G[j,i,b,a]: j the unit-stride index
+      if (j < o && i < o) {
+        const int64_t q = j + ov * i;
+        gt[k][tx] = P[ba + j + (int64_t)o * i] + 0.5 * (D[rba + q] + F[rba + q]) + F[rab + q];
+      }
+    }
+    __syncthreads();
+    for (int k = ty; k < 32; k += 8) {
+      const int i = i0 + tx, j = j0 + k;
+      if (i < o && j < o) {
+        const int64_t q = i + ov * j;
+        const int64_t m = (i >= j ? (int64_t)i * (i + 1) / 2 + j : (int64_t)j * (j + 1) / 2 + i) + mp * p;
+        const double sp = Sp[m], sm = Sp[m + mp * np];
+        const double r = P[ab + i + (int64_t)o * j] + 0.5 * (D[rab + q] + F[rab + q]) + F[rba + q] + gt[tx][k] +
+                         0.5 * (i >= j ? sp + sm : sp - sm);
+        R2[ab + i + (int64_t)o * j] = r;
+        gt[tx][k] = r;
+      }
+    }
+    if (a != b) {
+      __syncthreads();
+      for (int k = ty; k < 32; k += 8) {
+        const int j = j0 + tx, i = i0 + k;
+        if (j < o && i < o) R2[ba + j + (int64_t)o * i] = gt[k][tx];
+      }
+    }
+  }
+}
+void t2_numerator(hipStream_t s, int o, int v, const double* P, const double* D, const double* F, const double* Sp, double* R2) {
+  const int64_t nt = (o + 31) / 32, w = (int64_t)v * (v + 1) / 2 * nt * nt;
+  hipLaunchKernelGGL(k_t2_numerator, dim3((unsigned)std::min<int64_t>(w, 65536)), dim3(256), 0, s, o, v, P, D, F, Sp, R2);
   FH_HIP(hipGetLastError());
 }
 
