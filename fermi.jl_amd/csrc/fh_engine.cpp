@@ -584,16 +584,19 @@ static void residual(Ctx& c, const double* t1p, const double* t2p, double* R1, d
       c.Vs32 = Buf(c.pool.get(), (size_t)(2 * ldv * np) * sizeof(float));
       cast_f64_to_f32(c.s, 2 * ldv * np, c.Vs.d(), c.Vs32.f());
     }
+    const int64_t wl = c.lowp == 2 ? 0 : gemm_splitk_elems(mp, np, np, 2);
+    Buf work;
+    if (wl) work = dalloc(c, wl);
     Timer tl(c, c.lowp == 2 ? "ladder_bf16x3" : (c.lowp ? "ladder_fp32" : "ladder"), fl);
     if (!c.lowp)
       gemm_f64(c.s, false, false, mp, np, np, 1.0, bpair.d(), mp, mp * np, c.Vs.d(), ldv, ldv * np, 0.0, nullptr, 0, 0,
-               bS.d(), mp, mp * np, 2, /*tag: PP ladder*/ 1);
+               bS.d(), mp, mp * np, 2, /*tag: PP ladder*/ 1, work.d(), wl);
     else if (c.lowp == 2)
       gemm_bf3(c.s, false, false, mp, np, np, 1.0, bpair.f(), mp, mp * np, c.Vs32.f(), ldv, ldv * np, 0.0, nullptr, 0,
                bS.d(), mp, mp * np, 2, 1);
     else
       gemm_f32_fd(c.s, mp, np, np, 1.0, bpair.f(), mp, mp * np, c.Vs32.f(), ldv, ldv * np, 0.0, nullptr, 0, bS.d(), mp,
-                  mp * np, 2, 1);
+                  mp * np, 2, 1, work.d(), wl);
   }
   bpair.reset();
   {
@@ -639,10 +642,13 @@ static void residual(Ctx& c, const double* t1p, const double* t2p, double* R1, d
       cast_f64_to_f32(c.s, 2 * n2, bW.d(), bW32.f());
       gemm_bf3(c.s, false, false, ov, ov, ov, 1.0, bW32.f(), ov, n2, bring.f(), ov, n2, 0.0, nullptr, 0, bD.d(), ov, n2, 2, 0);
     } else {
+      const int64_t wl = gemm_splitk_elems(ov, ov, ov, 2);
+      Buf work;
+      if (wl) work = dalloc(c, wl);
       gemm_f64(c.s, false, false, ov, ov, ov, 0.5, bring.d(), ov, n2, c.LX.d(), ov, n2, 1.0, bW.d(), ov, n2, bW.d(), ov, n2,
-               2, 0, nullptr, 0, c.lowp != 0);
+               2, 0, work.d(), wl, c.lowp != 0);
       gemm_f64(c.s, false, false, ov, ov, ov, 1.0, bW.d(), ov, n2, bring.d(), ov, n2, 0.0, nullptr, 0, 0, bD.d(), ov, n2, 2,
-               0, nullptr, 0, c.lowp != 0);
+               0, work.d(), wl, c.lowp != 0);
     }
   }
   t2_numerator(c.s, (int)o, (int)v, P.p, bD.d(), bD.d() + n2, bS.d(), R2);   // (:190)

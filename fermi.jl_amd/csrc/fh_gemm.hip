@@ -3,8 +3,12 @@
 // Workgroup: 256 threads = 4 wavefronts in a 2x2 arrangement; each wavefront owns a
 // (BM/2)x(BN/2) block of the output as 16x16 MFMA accumulators.  Operand tiles are staged
 // through LDS with double buffering (global loads for stage s+1 are in flight while stage s
-// is multiplied).  LDS row paddings put the fragment reads of a half (FP64) or full (FP32)
-// wavefront on distinct bank pairs.
+// is multiplied).  Both tiles lie k-contiguous in LDS, whatever the source's order: a lane's
+// fragments are 16-byte reads of two (FP64) or four (FP32) of k, and the padded rows put 16 of
+// them on distinct banks, as they do the stores.  A full step has no bounds check.  (An m-major
+// tile of A with 8-byte reads, checked loads and scattered stores for a k-contiguous source left
+// the matrix pipes busy 52 % of the time, bank conflicts as many cycles as the MFMAs: TN
+// 7600 x 7600 x 840 in FP64 2.74 ms (35 TFLOP/s), so 2.03 ms (48 TFLOP/s, pipes busy 80 %).)
 //
 // Precision variants (template F32 and the global element types TI / TO):
 //   F32 = false: FP64 operands, v_mfma_f64_16x16x4f64, FP64 accumulation (TI = TO = double);
@@ -36,11 +40,16 @@ __global__ __launch_bounds__(256, OCC) void k_gemm(
   static_assert(F32 || std::is_same<TI, double>::value, "FP64 MFMA needs FP64 operands");
   using T = typename std::conditional<F32, float, double>::type;
   using Acc = typename std::conditional<F32, f32x4, f64x4>::type;
-  constexpr int PADA = 16, PADB = F32 ? 4 : 2;
   constexpr int WM = BM / 2, WN = BN / 2, MB = WM / 16, NB = WN / 16;
-  constexpr int LA = BM * BK / 256, LB = BN * BK / 256;
-  __shared__ T As[2][BK][BM + PADA];
-  __shared__ T Bs[2][BN][BK + PADB];
+  // an LDS read holds KV of k of a row, k group g = lane / 16 of a wavefront KV g .. KV g + KV - 1 of 4 KV (the order
+  // of k is the same for both operands, so any will do); KS is the row stride that spreads 16 rows over all banks
+  constexpr int KV = F32 && BK > 8 ? 4 : 2, KS = BK + (F32 ? 4 : 2);
+  constexpr int LA = BM * BK / 512, LB = BN * BK / 512;   // pairs of k that a thread copies
+  typedef T TV __attribute__((ext_vector_type(KV)));
+  typedef T T2 __attribute__((ext_vector_type(2)));
+  typedef TI TI2 __attribute__((ext_vector_type(2), aligned(sizeof(TI))));
+  __shared__ __attribute__((aligned(16))) T As[2][BM][KS];
+  __shared__ __attribute__((aligned(16))) T Bs[2][BN][KS];
 
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int wm = wid & 1, wn = wid >> 1;
@@ -63,57 +72,71 @@ __global__ __launch_bounds__(256, OCC) void k_gemm(
   }
   const int64_t m0 = mt * BM, n0 = nt * BN;
 
-  const int64_t bz = blockIdx.y;
+  const int64_t bz = blockIdx.y, kz = blockIdx.z;
+  A += bz * sA;
+  B += bz * sB;
   if (kchunk > 0) {
-    // split-K: slice bz covers k in [bz*kchunk, min(K, (bz+1)*kchunk)) and writes its own D slice
-    const int64_t kb = bz * kchunk;
+    // split-K: slice kz covers k in [kz*kchunk, min(K, (kz+1)*kchunk)) and writes its own D slice
+    const int64_t kb = kz * kchunk;
     K = (K - kb < kchunk) ? K - kb : kchunk;
     A += TA ? kb : lda * kb;
     B += TB ? ldb * kb : kb;
-  } else {
-    A += bz * sA;
-    B += bz * sB;
   }
   if (C) C += bz * sC;
-  D += bz * sD;
-  TI ra[LA], rb[LB];
-  auto gload = [&](int64_t k0) {
+  D += (kz * gridDim.y + bz) * sD;
+  // The thread's pairs of consecutive k: row (or column) index r and pair index kp; lanes run along the contiguous
+  // axis of the source.  Source pointers advance by BK of k a step.  Rows and columns outside the output read its
+  // last ones (their products go to elements that are not stored), so a full step has no bounds check.
+  auto rowA = [&](int t) { const int e = tid + 256 * t; return TA ? e / (BK / 2) : e % BM; };
+  auto kpA = [&](int t) { const int e = tid + 256 * t; return TA ? e % (BK / 2) : e / BM; };
+  auto rowB = [&](int t) { const int e = tid + 256 * t; return TB ? e % BN : e / (BK / 2); };
+  auto kpB = [&](int t) { const int e = tid + 256 * t; return TB ? e / BN : e % (BK / 2); };
+  TI2 ra[LA], rb[LB];
+  const TI *pa[LA], *pb[LB];
+  const int64_t skA = TA ? 1 : lda, skB = TB ? ldb : 1;   // stride of k
+#pragma unroll
+  for (int t = 0; t < LA; ++t) {
+    const int64_t gm = m0 + rowA(t) < M ? m0 + rowA(t) : M - 1;
+    pa[t] = A + gm * (TA ? lda : 1) + 2 * kpA(t) * skA;
+  }
+#pragma unroll
+  for (int t = 0; t < LB; ++t) {
+    const int64_t gc = n0 + rowB(t) < N ? n0 + rowB(t) : N - 1;
+    pb[t] = B + gc * (TB ? 1 : ldb) + 2 * kpB(t) * skB;
+  }
+  auto gload = [&]() {
 #pragma unroll
     for (int t = 0; t < LA; ++t) {
-      const int e = tid + 256 * t;
-      int mm, kk;
-      if (!TA) { mm = e % BM; kk = e / BM; } else { kk = e % BK; mm = e / BK; }
-      const int64_t gm = m0 + mm, gk = k0 + kk;
-      TI val = 0;
-      if (gm < M && gk < K) val = TA ? A[gk + lda * gm] : A[gm + lda * gk];
-      ra[t] = val;
+      if constexpr (TA) ra[t] = *reinterpret_cast<const TI2*>(pa[t]);
+      else ra[t] = TI2{pa[t][0], pa[t][lda]};
+      pa[t] += BK * skA;
     }
 #pragma unroll
     for (int t = 0; t < LB; ++t) {
-      const int e = tid + 256 * t;
-      int nn, kk;
-      if (!TB) { kk = e % BK; nn = e / BK; } else { nn = e % BN; kk = e / BN; }
-      const int64_t gcol = n0 + nn, gk = k0 + kk;
-      TI val = 0;
-      if (gcol < N && gk < K) val = TB ? B[gcol + ldb * gk] : B[gk + ldb * gcol];
-      rb[t] = val;
+      if constexpr (!TB) rb[t] = *reinterpret_cast<const TI2*>(pb[t]);
+      else rb[t] = TI2{pb[t][0], pb[t][ldb]};
+      pb[t] += BK * skB;
     }
+  };
+  // the last step when BK does not divide K: kr (1 .. BK - 1) of k are left; the others read the first and count
+  // as zero
+  auto gload_tail = [&](int kr) {
+    auto get = [&](const TI* p, int64_t sk, int k) {
+      const TI v = p[k < kr ? 0 : -(int64_t)k * sk];
+      return k < kr ? v : TI(0);
+    };
+#pragma unroll
+    for (int t = 0; t < LA; ++t) ra[t] = TI2{get(pa[t], skA, 2 * kpA(t)), get(pa[t] + skA, skA, 2 * kpA(t) + 1)};
+#pragma unroll
+    for (int t = 0; t < LB; ++t) rb[t] = TI2{get(pb[t], skB, 2 * kpB(t)), get(pb[t] + skB, skB, 2 * kpB(t) + 1)};
   };
   auto sstore = [&](int buf) {
 #pragma unroll
-    for (int t = 0; t < LA; ++t) {
-      const int e = tid + 256 * t;
-      int mm, kk;
-      if (!TA) { mm = e % BM; kk = e / BM; } else { kk = e % BK; mm = e / BK; }
-      As[buf][kk][mm] = (T)ra[t];
-    }
+    for (int t = 0; t < LA; ++t)
+      *reinterpret_cast<T2*>(&As[buf][rowA(t)][2 * kpA(t)]) = T2{(T)ra[t][0], (T)ra[t][1]};
 #pragma unroll
-    for (int t = 0; t < LB; ++t) {
-      const int e = tid + 256 * t;
-      int nn, kk;
-      if (!TB) { kk = e % BK; nn = e / BK; } else { nn = e % BN; kk = e / BN; }
-      Bs[buf][nn][kk] = (T)rb[t];
-    }
+    for (int t = 0; t < LB; ++t)
+      *reinterpret_cast<T2*>(&Bs[buf][rowB(t)][2 * kpB(t)]) = T2{(T)rb[t][0], (T)rb[t][1]};
   };
 
   Acc acc[MB][NB];
@@ -123,27 +146,37 @@ __global__ __launch_bounds__(256, OCC) void k_gemm(
     for (int j = 0; j < NB; ++j) acc[i][j] = Acc{0, 0, 0, 0};
 
   const int64_t nst = (K + BK - 1) / BK;
-  gload(0);
-  sstore(0);
+  const int kr = (int)(K % BK);
+  auto fetch = [&](int64_t st) {
+    if (st + 1 == nst && kr) gload_tail(kr); else gload();
+  };
+  if (nst) {
+    fetch(0);
+    sstore(0);
+  }
   __syncthreads();
   for (int64_t s = 0; s < nst; ++s) {
     const int buf = s & 1;
-    if (s + 1 < nst) gload((s + 1) * BK);
+    if (s + 1 < nst) fetch(s + 1);
 #pragma unroll
-    for (int kk = 0; kk < BK / 4; ++kk) {
-      T af[MB], bf[NB];
-#pragma unroll
-      for (int i = 0; i < MB; ++i) af[i] = As[buf][kk * 4 + (lane >> 4)][wm * WM + i * 16 + (lane & 15)];
-#pragma unroll
-      for (int j = 0; j < NB; ++j) bf[j] = Bs[buf][wn * WN + j * 16 + (lane & 15)][kk * 4 + (lane >> 4)];
+    for (int ks = 0; ks < BK; ks += 4 * KV) {
+      TV af[MB], bf[NB];
 #pragma unroll
       for (int i = 0; i < MB; ++i)
+        af[i] = *reinterpret_cast<const TV*>(&As[buf][wm * WM + i * 16 + (lane & 15)][ks + KV * (lane >> 4)]);
 #pragma unroll
-        for (int j = 0; j < NB; ++j) {
-          // B fragment as the first MFMA operand, so the accumulator lanes run along M
-          if constexpr (F32) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[j], af[i], acc[i][j], 0, 0, 0);
-          else acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bf[j], af[i], acc[i][j], 0, 0, 0);
-        }
+      for (int j = 0; j < NB; ++j)
+        bf[j] = *reinterpret_cast<const TV*>(&Bs[buf][wn * WN + j * 16 + (lane & 15)][ks + KV * (lane >> 4)]);
+#pragma unroll
+      for (int q = 0; q < KV; ++q)
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+          for (int j = 0; j < NB; ++j) {
+            // B fragment as the first MFMA operand, so the accumulator lanes run along M
+            if constexpr (F32) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[j][q], af[i][q], acc[i][j], 0, 0, 0);
+            else acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bf[j][q], af[i][q], acc[i][j], 0, 0, 0);
+          }
     }
     if (s + 1 < nst) sstore(buf ^ 1);
     __syncthreads();
@@ -202,7 +235,7 @@ static void launch(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha,
                    int64_t ldd, int64_t sD, int64_t batch, int64_t kchunk) {
   const int64_t tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
   FH_CHECK(tm * tn < (int64_t)1 << 31 && batch < 65536, -3, "gemm grid too large");
-  dim3 grid((unsigned)(tm * tn), (unsigned)batch);
+  dim3 grid((unsigned)(tm * tn), (unsigned)batch, (unsigned)(kchunk > 0 ? (K + kchunk - 1) / kchunk : 1));
   // A larger than B: group N-tiles so that a group's B blocks stay in L2
   int gn = 0;
   if (M > N) {
@@ -210,21 +243,43 @@ static void launch(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha,
     const int64_t per = std::max<int64_t>(1, kl * BN * (int64_t)sizeof(TI));
     gn = (int)std::max<int64_t>(1, std::min<int64_t>(tn, kGroupBytes / per));
   }
-  constexpr int OCC = BM * BN > 8192 ? 1 : 4;
+  constexpr int OCC = BM == 32 && !F32 ? 3 : 4;   // workgroups per CU that the LDS holds
   hipLaunchKernelGGL((k_gemm<BM, BN, BK, TA, TB, OCC, TAG, F32, TI, TO>), grid, dim3(256), 0, s, M, N, K, alpha, A, lda,
                      sA, B, ldb, sB, beta, C, ldc, sC, D, ldd, sD, (int)tm, (int)tn, kchunk, gn);
   FH_HIP(hipGetLastError());
 }
 
-// 64x64 tiles at up to four workgroups per CU measured fastest on every shape of this engine
-// (the latency of the next operand tile is hidden by the other workgroups); BK = 8 when the
-// per-tile K loop is short.
+// How a shape is cut.  64x64 tiles at up to four workgroups per CU measured fastest wherever there are enough of
+// them (the latency of the next operand tile is hidden by the other workgroups); BK = 8 when the per-tile K loop
+// is short.  Below 1.5 tiles per CU the K loop of a tile is exposed, so K is cut into slices of at least 128
+// towards four workgroups per CU; a K under 384 is not, as the reduction (about 4 us) costs what it saves.
+// Measured in FP64: (136, 2926, 2926) in a batch of two, 276 tiles, 286 us uncut, 160 us in three slices and 9 us to
+// add them; one tile with K = 1805 110 us uncut, 6 + 4 us cut.
+// A shape that leaves the chip under 256 workgroups even so is bound by the latency of a K step, about 1 us
+// whatever its depth: 32x32 tiles in K steps of 32 spread it over more CUs in a quarter of the steps (the products
+// of the residual at o = 5, v = 19: 10 us each with 64x64 tiles in steps of 8, 5 us so).
+struct GemmPlan {
+  bool small;
+  int64_t slices;
+};
+static GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t batch) {
+  const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64) * batch;
+  if (tiles >= 384) return {false, 1};
+  const int64_t most = K < 384 ? 1 : K / 128;
+  if (tiles * most >= 256) return {false, std::min<int64_t>(std::max<int64_t>(1, 1024 / tiles), most)};
+  const int64_t tiles32 = ((M + 31) / 32) * ((N + 31) / 32) * batch;
+  return {true, std::min<int64_t>(std::max<int64_t>(1, 512 / tiles32), most)};
+}
+
 template <bool TA, bool TB, int TAG, bool F32, typename TI, typename TO>
-static void pick(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const TI* A, int64_t lda, int64_t sA,
-                 const TI* B, int64_t ldb, int64_t sB, double beta, const TO* C, int64_t ldc, int64_t sC, TO* D,
-                 int64_t ldd, int64_t sD, int64_t batch, int64_t kchunk) {
+static void pick(hipStream_t s, bool small, int64_t M, int64_t N, int64_t K, double alpha, const TI* A, int64_t lda,
+                 int64_t sA, const TI* B, int64_t ldb, int64_t sB, double beta, const TO* C, int64_t ldc, int64_t sC,
+                 TO* D, int64_t ldd, int64_t sD, int64_t batch, int64_t kchunk) {
   const int64_t kl = kchunk > 0 ? kchunk : K;
-  if (kl <= 512)
+  if (small)
+    launch<32, 32, 32, TA, TB, TAG, F32, TI, TO>(s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, D, ldd,
+                                                 sD, batch, kchunk);
+  else if (kl <= 512)
     launch<64, 64, 8, TA, TB, TAG, F32, TI, TO>(s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, D, ldd, sD,
                                                 batch, kchunk);
   else
@@ -232,32 +287,39 @@ static void pick(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, c
                                                  sD, batch, kchunk);
 }
 
-// split-K sizing: few output tiles and a long K leave most CUs idle; cut K into slices
-static int64_t splitk_slices(int64_t M, int64_t N, int64_t K, int64_t batch) {
-  if (batch != 1 || K < 4096) return 1;
-  const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
-  if (tiles >= 256) return 1;
-  int64_t sl = (1024 + tiles - 1) / tiles;
-  sl = std::min<int64_t>(sl, K / 512);
-  return std::max<int64_t>(sl, 1);
-}
-
 int64_t gemm_splitk_elems(int64_t M, int64_t N, int64_t K, int64_t batch) {
-  const int64_t sl = splitk_slices(M, N, K, batch);
-  return sl > 1 ? sl * M * N : 0;
+  if (M <= 0 || N <= 0 || batch <= 0) return 0;
+  const int64_t sl = gemm_plan(M, N, K, batch).slices;
+  return sl > 1 ? sl * M * N * batch : 0;
 }
 
-__global__ void k_splitk_reduce(int64_t M, int64_t N, int64_t S, const double* __restrict__ W, double alpha, double beta,
-                                const double* C, int64_t ldc, double* D, int64_t ldd) {
-  const int64_t n = M * N;
+// D = alpha sum over the S slices of W [M N][batch][S] + beta C, summed in FP64
+template <typename T>
+__global__ __launch_bounds__(256) void k_splitk_reduce(int64_t M, int64_t N, int64_t S, const T* __restrict__ W,
+                                                       double alpha, double beta, const T* C, int64_t ldc, int64_t sC,
+                                                       T* D, int64_t ldd, int64_t sD) {
+  const int64_t n = M * N, st = n * gridDim.y;
+  W += n * blockIdx.y;
+  C += sC * blockIdx.y;
+  D += sD * blockIdx.y;
   for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < n; idx += (int64_t)gridDim.x * 256) {
     const int64_t m = idx % M, c = idx / M;
     double acc = 0.0;
-    for (int64_t q = 0; q < S; ++q) acc += W[idx + q * n];
+#pragma unroll 8
+    for (int64_t q = 0; q < S; ++q) acc += (double)W[idx + q * st];
     double val = alpha * acc;
-    if (beta != 0.0) val += beta * C[m + ldc * c];
-    D[m + ldd * c] = val;
+    if (beta != 0.0) val += beta * (double)C[m + ldc * c];
+    D[m + ldd * c] = (T)val;
   }
+}
+
+template <typename T>
+static void splitk_reduce(hipStream_t s, int64_t M, int64_t N, int64_t S, const T* W, double alpha, double beta,
+                          const T* C, int64_t ldc, int64_t sC, T* D, int64_t ldd, int64_t sD, int64_t batch) {
+  const int64_t g = std::min<int64_t>((M * N + 255) / 256, 65536);
+  hipLaunchKernelGGL((k_splitk_reduce<T>), dim3((unsigned)g, (unsigned)batch), dim3(256), 0, s, M, N, S, W, alpha,
+                     beta, C, ldc, sC, D, ldd, sD);
+  FH_HIP(hipGetLastError());
 }
 
 static void check_args(int64_t M, int64_t K, int64_t N, bool ta, bool tb, int64_t lda, int64_t ldb, int64_t ldd,
@@ -274,10 +336,9 @@ void gemm_f64(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, 
               int64_t work_elems, bool f32) {
   if (M <= 0 || N <= 0 || batch <= 0) return;
   check_args(M, K, N, ta, tb, lda, ldb, ldd, beta, C, ldc);
-  const int64_t sl = splitk_slices(M, N, K, batch);
-  const bool split = sl > 1 && work != nullptr && work_elems >= sl * M * N;
-  const int64_t kchunk = split ? (K + sl - 1) / sl : 0;
-  const int64_t nb = split ? (K + kchunk - 1) / kchunk : batch;
+  const GemmPlan plan = gemm_plan(M, N, K, batch);
+  const bool split = plan.slices > 1 && work != nullptr && work_elems >= plan.slices * M * N * batch;
+  const int64_t kchunk = split ? (K + plan.slices - 1) / plan.slices : 0;
   const double al = split ? 1.0 : alpha, be = split ? 0.0 : beta;
   const double* Cc = split ? nullptr : C;
   double* Dd = split ? work : D;
@@ -285,11 +346,11 @@ void gemm_f64(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, 
 #define FH_PICK2(TA_, TB_, F_)                                                                                      \
   do {                                                                                                              \
     if (tag == 1)                                                                                                   \
-      pick<TA_, TB_, 1, F_, double, double>(s, M, N, K, al, A, lda, sA, B, ldb, sB, be, Cc, ldc, sC, Dd, lddd, sDD, nb, \
-                                            kchunk);                                                        \
+      pick<TA_, TB_, 1, F_, double, double>(s, plan.small, M, N, K, al, A, lda, sA, B, ldb, sB, be, Cc, ldc, sC, Dd,  \
+                                            lddd, sDD, batch, kchunk);                                              \
     else                                                                                                            \
-      pick<TA_, TB_, 0, F_, double, double>(s, M, N, K, al, A, lda, sA, B, ldb, sB, be, Cc, ldc, sC, Dd, lddd, sDD, nb, \
-                                            kchunk);                                                        \
+      pick<TA_, TB_, 0, F_, double, double>(s, plan.small, M, N, K, al, A, lda, sA, B, ldb, sB, be, Cc, ldc, sC, Dd,  \
+                                            lddd, sDD, batch, kchunk);                                              \
   } while (0)
 #define FH_PICK(TA_, TB_)              \
   do {                                 \
@@ -303,41 +364,52 @@ void gemm_f64(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, 
   }
 #undef FH_PICK
 #undef FH_PICK2
-  if (split) {
-    int64_t g = (M * N + 255) / 256;
-    if (g > 65536) g = 65536;
-    hipLaunchKernelGGL(k_splitk_reduce, dim3((unsigned)g), dim3(256), 0, s, M, N, nb, work, alpha, beta, C, ldc, D, ldd);
-    FH_HIP(hipGetLastError());
-  }
+  if (split)
+    splitk_reduce<double>(s, M, N, (K + kchunk - 1) / kchunk, work, alpha, beta, C, ldc, sC, D, ldd, sD, batch);
 }
 
-// FP32-MFMA GEMM with FP32 operands in HBM and FP64 output (NN, no split-K)
+// FP32-MFMA GEMM with FP32 operands in HBM and FP64 output (NN)
 void gemm_f32_fd(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const float* A, int64_t lda, int64_t sA,
                  const float* B, int64_t ldb, int64_t sB, double beta, const double* C, int64_t ldc, double* D, int64_t ldd,
-                 int64_t sD, int64_t batch, int tag) {
+                 int64_t sD, int64_t batch, int tag, double* work, int64_t work_elems) {
   if (M <= 0 || N <= 0 || batch <= 0) return;
   check_args(M, K, N, false, false, lda, ldb, ldd, beta, C, ldc);
-  if (tag == 1)
-    pick<false, false, 1, true, float, double>(s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sD, D, ldd, sD,
-                                               batch, 0);
-  else
-    pick<false, false, 0, true, float, double>(s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sD, D, ldd, sD,
-                                               batch, 0);
+  const GemmPlan plan = gemm_plan(M, N, K, batch);
+  const bool split = plan.slices > 1 && work != nullptr && work_elems >= plan.slices * M * N * batch;
+  const int64_t kchunk = split ? (K + plan.slices - 1) / plan.slices : 0;
+  auto run = [&](auto tagc) {
+    if (split)
+      pick<false, false, decltype(tagc)::value, true, float, double>(s, plan.small, M, N, K, 1.0, A, lda, sA, B, ldb, sB,
+                                                                     0.0, nullptr, 0, 0, work, M, M * N, batch, kchunk);
+    else
+      pick<false, false, decltype(tagc)::value, true, float, double>(s, plan.small, M, N, K, alpha, A, lda, sA, B, ldb,
+                                                                     sB, beta, C, ldc, sD, D, ldd, sD, batch, 0);
+  };
+  if (tag == 1) run(std::integral_constant<int, 1>()); else run(std::integral_constant<int, 0>());
+  if (split)
+    splitk_reduce<double>(s, M, N, (K + kchunk - 1) / kchunk, work, alpha, beta, C, ldc, sD, D, ldd, sD, batch);
 }
 
 // FP32 operands and output, any transposition (the T2-guess network's layers; tag 3)
 void gemm_f32(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, double alpha, const float* A,
-              int64_t lda, const float* B, int64_t ldb, double beta, float* C, int64_t ldc) {
+              int64_t lda, const float* B, int64_t ldb, double beta, float* C, int64_t ldc, float* work,
+              int64_t work_elems) {
   if (M <= 0 || N <= 0) return;
   check_args(M, K, N, ta, tb, lda, ldb, ldc, beta, C, ldc);
-#define FH_F32(TA_, TB_) \
-  pick<TA_, TB_, 3, true, float, float>(s, M, N, K, alpha, A, lda, 0, B, ldb, 0, beta, C, ldc, 0, C, ldc, 0, 1, 0)
+  const GemmPlan plan = gemm_plan(M, N, K, 1);
+  const bool split = plan.slices > 1 && work != nullptr && work_elems >= plan.slices * M * N;
+  const int64_t kchunk = split ? (K + plan.slices - 1) / plan.slices : 0;
+#define FH_F32(TA_, TB_)                                                                                             \
+  pick<TA_, TB_, 3, true, float, float>(s, plan.small, M, N, K, split ? 1.0 : alpha, A, lda, 0, B, ldb, 0,           \
+                                        split ? 0.0 : beta, split ? nullptr : C, ldc, 0, split ? work : C,           \
+                                        split ? M : ldc, split ? M * N : 0, 1, kchunk)
   if (ta) {
     if (tb) FH_F32(true, true); else FH_F32(true, false);
   } else {
     if (tb) FH_F32(false, true); else FH_F32(false, false);
   }
 #undef FH_F32
+  if (split) splitk_reduce<float>(s, M, N, (K + kchunk - 1) / kchunk, work, alpha, beta, C, ldc, 0, C, ldc, 0, 1);
 }
 
 }  // namespace fh

@@ -99,10 +99,11 @@ void gemm_f64(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, 
 // FP32-MFMA GEMM (NN) with FP32 operands in HBM and FP64 output
 void gemm_f32_fd(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const float* A, int64_t lda, int64_t sA,
                  const float* B, int64_t ldb, int64_t sB, double beta, const double* C, int64_t ldc, double* D, int64_t ldd,
-                 int64_t sD, int64_t batch, int tag);
+                 int64_t sD, int64_t batch, int tag, double* work = nullptr, int64_t work_elems = 0);
 // FP32 operands and output, any transposition, C = alpha op(A) op(B) + beta C (tag 3)
 void gemm_f32(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, double alpha, const float* A,
-              int64_t lda, const float* B, int64_t ldb, double beta, float* C, int64_t ldc);
+              int64_t lda, const float* B, int64_t ldb, double beta, float* C, int64_t ldc, float* work = nullptr,
+              int64_t work_elems = 0);
 // split-BF16x3 MFMA GEMM (three bf16 products per FP32 product, FP32 accumulation) on FP32 operands with FP64
 // output: tag 0 any transposition, tag 1 (the PP ladder) untransposed; the tags give distinct kernel symbols
 void gemm_bf3(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, double alpha, const float* A,
@@ -160,7 +161,7 @@ size_t t2_mlp_fused_scratch_bytes();
 void t2_mlp_fused(hipStream_t s, int o, int v, const double* t2, const double* eo, const double* ev, const double* dij,
                   const float* xm, const float* xs, const float* P, void* wsplit, float* Y);
 
-// workspace (doubles) that gemm_f64 would use to split K for this shape (0: no split)
+// workspace (elements of the partial sums' type) that the GEMMs would use to split K for this shape (0: no split)
 int64_t gemm_splitk_elems(int64_t M, int64_t N, int64_t K, int64_t batch);
 // tag selects a distinct kernel symbol for profiling: 0 generic, 1 PP ladder
 
