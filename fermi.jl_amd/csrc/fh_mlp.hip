@@ -15,6 +15,7 @@
 // (T2_CCSD - T2_MP2) / y_scale, and the guess is symmetrised in (ij)(ab).
 #include "fh_internal.h"
 
+#include <algorithm>
 #include <cmath>
 
 namespace fh {
@@ -99,25 +100,46 @@ __global__ void k_rowsum_part(int h, int64_t B, int64_t cols, const float* __res
     part[(int64_t)blockIdx.x * h + threadIdx.x] = u;
   }
 }
-// out[r] = sum_b part[b, r]
-__global__ void k_rowsum_final(int h, int nb, const float* __restrict__ part, float* __restrict__ out) {
-  for (int r = blockIdx.x * 256 + threadIdx.x; r < h; r += gridDim.x * 256) {
-    float u = 0.0f;
-    for (int b = 0; b < nb; ++b) u += part[(int64_t)b * h + r];
-    out[r] = u;
+// out[r] = sum_b part[b, r]: one workgroup a row
+__global__ __launch_bounds__(256) void k_rowsum_final(int h, int nb, const float* __restrict__ part,
+                                                      float* __restrict__ out) {
+  __shared__ float red[256];
+  const int r = blockIdx.x;
+  float u = 0.0f;
+  for (int b = threadIdx.x; b < nb; b += 256) u += part[(int64_t)b * h + r];
+  red[threadIdx.x] = u;
+  __syncthreads();
+  for (int st = 128; st > 0; st >>= 1) {
+    if ((int)threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
+    __syncthreads();
   }
+  if (threadIdx.x == 0) out[r] = red[0];
 }
 
-static constexpr int64_t kRowsumCols = 4096;
+// Columns of one k_rowsum_part workgroup: 64 keep its chain of dependent adds at 32 for h = 128, and with up to 1024
+// workgroups the chip is full from B = 16 k on (h = 128, B = 8192: 345 us with 4096 columns a workgroup, 9 us so).
+static int64_t rowsum_cols(int64_t B) { return std::max<int64_t>(64, (B + 1023) / 1024); }
+static int64_t rowsum_blocks(int64_t B) { return (B + rowsum_cols(B) - 1) / rowsum_cols(B); }
 
 static void rowsum(hipStream_t s, int h, int64_t B, const float* Mx, float* part, float* out) {
-  const int nb = (int)((B + kRowsumCols - 1) / kRowsumCols);
-  hipLaunchKernelGGL(k_rowsum_part, dim3(nb), dim3(256), 0, s, h, B, kRowsumCols, Mx, part);
-  hipLaunchKernelGGL(k_rowsum_final, dim3(grid1(h)), dim3(256), 0, s, h, nb, part, out);
+  const int nb = (int)rowsum_blocks(B);
+  hipLaunchKernelGGL(k_rowsum_part, dim3(nb), dim3(256), 0, s, h, B, rowsum_cols(B), Mx, part);
+  hipLaunchKernelGGL(k_rowsum_final, dim3(h), dim3(256), 0, s, h, nb, part, out);
   FH_HIP(hipGetLastError());
 }
 
-int64_t mlp_partial_elems(int h, int64_t B) { return ((B + kRowsumCols - 1) / kRowsumCols) * std::max(h, 1) + 1024; }
+// Scratch of the weight gradients' GEMMs ([h, h], [h, 6] and [h, 1], K = B, cut into slices of at least 128 of K,
+// at most 1024 workgroups of 64 x 64): a bound that grows with B, as a shorter last batch uses the buffer of a full
+// one.
+static int64_t wgrad_elems(int h, int64_t B) {
+  const int64_t t = (h + 63) / 64, most = B / 128;
+  return std::max(std::min(most, 1024 / (t * t)) * h * h, std::min(most, 1024 / t) * h * 6);
+}
+
+int64_t mlp_partial_elems(int h, int64_t B) {
+  const int64_t blocks = std::min<int64_t>((B + 63) / 64, 1024);   // >= rowsum_blocks of every batch up to B
+  return std::max(blocks * std::max(h, 1) + 1024, wgrad_elems(h, B));
+}
 
 void mlp_forward(hipStream_t s, int h, const float* P, int64_t B, const float* X, float* A1, float* A2, float* A3,
                  float* y) {
@@ -139,24 +161,25 @@ void mlp_backward(hipStream_t s, int h, const float* P, int64_t B, const float* 
                   float* part, double* lpart, int64_t* nlpart) {
   const MlpOffsets o = mlp_offsets(h);
   const unsigned gb = grid1(B);
+  const int64_t wl = wgrad_elems(h, B);
   hipLaunchKernelGGL(k_out_back, dim3(gb), dim3(256), 0, s, B, y, T, dy, lpart);
   *nlpart = gb;
   hipLaunchKernelGGL(k_out_dz, dim3(grid1(h * B)), dim3(256), 0, s, h, (int64_t)h * B, P + o.w4, A3, dy, dZ);
   // output layer: g w4 = A3 dy, g b4 = sum dy
-  gemm_f32(s, false, false, h, 1, B, 1.0, A3, h, dy, B, 0.0, G + o.w4, h);
+  gemm_f32(s, false, false, h, 1, B, 1.0, A3, h, dy, B, 0.0, G + o.w4, h, part, wl);
   rowsum(s, 1, B, dy, part, G + o.b4);
   // layer 3
-  gemm_f32(s, false, true, h, h, B, 1.0, dZ, h, A2, h, 0.0, G + o.W3, h);
+  gemm_f32(s, false, true, h, h, B, 1.0, dZ, h, A2, h, 0.0, G + o.W3, h, part, wl);
   rowsum(s, h, B, dZ, part, G + o.b3);
   gemm_f32(s, true, false, h, B, h, 1.0, P + o.W3, h, dZ, h, 0.0, dA, h);
   hipLaunchKernelGGL(k_tanh_back, dim3(grid1(h * B)), dim3(256), 0, s, (int64_t)h * B, A2, dA);
   // layer 2 (dA now holds dZ2)
-  gemm_f32(s, false, true, h, h, B, 1.0, dA, h, A1, h, 0.0, G + o.W2, h);
+  gemm_f32(s, false, true, h, h, B, 1.0, dA, h, A1, h, 0.0, G + o.W2, h, part, wl);
   rowsum(s, h, B, dA, part, G + o.b2);
   gemm_f32(s, true, false, h, B, h, 1.0, P + o.W2, h, dA, h, 0.0, dZ, h);
   hipLaunchKernelGGL(k_tanh_back, dim3(grid1(h * B)), dim3(256), 0, s, (int64_t)h * B, A1, dZ);
   // layer 1 (dZ holds dZ1)
-  gemm_f32(s, false, true, h, 6, B, 1.0, dZ, h, X, 6, 0.0, G + o.W1, h);
+  gemm_f32(s, false, true, h, 6, B, 1.0, dZ, h, X, 6, 0.0, G + o.W1, h, part, wl);
   rowsum(s, h, B, dZ, part, G + o.b1);
   FH_HIP(hipGetLastError());
 }
