@@ -2138,11 +2138,9 @@ static std::vector<char> sph_tab(int spherical) {
   integrals_pack_table(out.data(), t, spherical);
   return out;
 }
-// a basis set with its primitives offset by `poff0` (two sets uploaded as one primitive array)
-static Buf upload_ints(Ctx& c, const std::vector<int>& v) {
-  Buf b(c.pool.get(), std::max<size_t>(v.size(), 1) * sizeof(int));
-  FH_HIP(hipMemcpyAsync(b.p, v.data(), v.size() * sizeof(int), hipMemcpyHostToDevice, c.s));
-  return b;
+static IntBasis int_basis(const fh_basis& b) {
+  return {(int)b.l.size(), b.nbf, b.spherical, (int)b.exps.size(), b.l.data(), b.nprim.data(), b.poff.data(), b.foff.data(),
+          b.center.data(), b.exps.data(), b.coefs.data()};
 }
 }  // namespace fh
 
@@ -2254,21 +2252,12 @@ int fh_eri_2e4c(fh_ctx* x, const fh_basis* b, double* eri) {
     FH_CHECK((double)n * n * n * n < 4.0e9, -1, "fh_eri_2e4c: 4-index tensor too large (nbf^4 >= 4e9)");
     DeviceGuard g(x->c.device);
     Ctx& c = x->c;
-    DevBasis d = upload_basis(c, *b);
     const auto tab = sph_tab(b->spherical);
-    std::vector<int> pairs, fpairs;
-    const int ns = (int)b->l.size();
-    for (int i = 0; i < ns; ++i)
-      for (int j = 0; j <= i; ++j) { pairs.push_back(i); pairs.push_back(j); }
-    for (int r = 0; r < n; ++r)
-      for (int s2 = 0; s2 <= r; ++s2) { fpairs.push_back(r); fpairs.push_back(s2); }
-    Buf dp = upload_ints(c, pairs), dfp = upload_ints(c, fpairs), dfun = upload_ints(c, b->fun);
+    IntScratch sc;
     Buf out = dalloc(c, n * n * n * n);
     {
       Timer t(c, "ao_eri_4c");
-      integrals_eri4c(c.s, (int)(pairs.size() / 2), static_cast<const int*>(dp.p), (int)(fpairs.size() / 2),
-                      static_cast<const int*>(dfp.p), d.shells.p, static_cast<const int*>(dfun.p), (int)n, d.ex.d(),
-                      d.cf.d(), tab.data(), out.d());
+      integrals_eri4c(c.s, c.pool.get(), sc, int_basis(*b), tab.data(), out.d());
     }
     d2h(c, eri, out.d(), n * n * n * n);
     flush_timers(c);
@@ -2284,26 +2273,12 @@ int fh_eri_2e3c(fh_ctx* x, const fh_basis* b, const fh_basis* aux, double* Pqp) 
     const int64_t n = b->nbf, Q = aux->nbf;
     DeviceGuard g(x->c.device);
     Ctx& c = x->c;
-    // one primitive array for both sets: the auxiliary shells' offsets move behind the orbital ones
-    fh_basis both = *b;
-    const int p0 = (int)b->exps.size();
-    both.exps.insert(both.exps.end(), aux->exps.begin(), aux->exps.end());
-    both.coefs.insert(both.coefs.end(), aux->coefs.begin(), aux->coefs.end());
-    fh_basis ash = *aux;
-    for (int& q : ash.poff) q += p0;
-    DevBasis d = upload_basis(c, both);
-    DevBasis da = upload_basis(c, ash);
     const auto tab = sph_tab(b->spherical);
-    std::vector<int> pairs;
-    const int ns = (int)b->l.size();
-    for (int i = 0; i < ns; ++i)
-      for (int j = 0; j <= i; ++j) { pairs.push_back(i); pairs.push_back(j); }
-    Buf dp = upload_ints(c, pairs), dafun = upload_ints(c, aux->fun);
+    IntScratch sc;
     Buf out = dalloc(c, n * n * Q);
     {
       Timer t(c, "ao_eri_3c");
-      integrals_eri3c(c.s, (int)(pairs.size() / 2), static_cast<const int*>(dp.p), d.shells.p, da.shells.p,
-                      static_cast<const int*>(dafun.p), (int)Q, (int)n, d.ex.d(), d.cf.d(), tab.data(), out.d());
+      integrals_eri3c(c.s, c.pool.get(), sc, int_basis(*b), int_basis(*aux), tab.data(), out.d());
     }
     d2h(c, Pqp, out.d(), n * n * Q);
     flush_timers(c);
@@ -2317,14 +2292,12 @@ int fh_eri_2e2c(fh_ctx* x, const fh_basis* aux, double* J) {
     const int64_t Q = aux->nbf;
     DeviceGuard g(x->c.device);
     Ctx& c = x->c;
-    DevBasis d = upload_basis(c, *aux);
     const auto tab = sph_tab(aux->spherical);
-    Buf dafun = upload_ints(c, aux->fun);
+    IntScratch sc;
     Buf out = dalloc(c, Q * Q);
     {
       Timer t(c, "ao_eri_2c");
-      integrals_eri2c(c.s, (int)Q, (int)aux->l.size(), d.shells.p, static_cast<const int*>(dafun.p), d.ex.d(),
-                      d.cf.d(), tab.data(), out.d());
+      integrals_eri2c(c.s, c.pool.get(), sc, int_basis(*aux), tab.data(), out.d());
     }
     d2h(c, J, out.d(), Q * Q);
     flush_timers(c);

@@ -225,8 +225,7 @@ void triples_energy(hipStream_t s, int o, int v, int nrun, const int* runs, cons
 
 // ---------------------------------------------------------------- Gaussian integrals (fh_integrals.hip)
 // shells: packed records (integrals_pack_shell, integrals_shell_bytes each); tab: packed spherical
-// table (integrals_pack_table); pairs / fpairs / fun / afun: int pairs (shell i >= j; function r >= s;
-// function -> (shell, component))
+// table (integrals_pack_table)
 size_t integrals_shell_bytes();
 size_t integrals_table_bytes();
 int integrals_max_l_orbital();
@@ -238,12 +237,21 @@ void integrals_one_electron(hipStream_t s, int nshell, const void* shells, const
                             double* T, double* V);
 void integrals_dipole(hipStream_t s, int nshell, const void* shells, const double* ex, const double* cf,
                       const double* origin, const void* tab, int nbf, double* Dx, double* Dy, double* Dz);
-void integrals_eri3c(hipStream_t s, int npair, const int* pairs, const void* shells, const void* ashells,
-                     const int* afun, int naux, int nbf, const double* ex, const double* cf, const void* tab,
+// a basis set as the host holds it: nexp primitives, shell i's from poff[i] on, its functions from foff[i] on
+struct IntBasis {
+  int nshell, nbf, spherical, nexp;
+  const int *l, *nprim, *poff, *foff;
+  const double *center, *exps, *coefs;
+};
+// lists and tables of a Coulomb integral call: kept until the stream has been synchronised
+struct IntScratch {
+  std::vector<char> host;
+  Buf lists, tables;
+};
+// (mu nu|P), (P|Q) and (mu nu|la si) into out (orbital shells up to d, fitting shells up to f)
+void integrals_eri3c(hipStream_t s, Pool* pool, IntScratch& sc, const IntBasis& b, const IntBasis& aux, const void* tab,
                      double* out);
-void integrals_eri2c(hipStream_t s, int naux, int nshell, const void* ashells, const int* afun, const double* ex,
-                     const double* cf, const void* tab, double* out);
-void integrals_eri4c(hipStream_t s, int npair, const int* pairs, int nfp, const int* fpairs, const void* shells,
-                     const int* fun, int nbf, const double* ex, const double* cf, const void* tab, double* out);
+void integrals_eri2c(hipStream_t s, Pool* pool, IntScratch& sc, const IntBasis& aux, const void* tab, double* out);
+void integrals_eri4c(hipStream_t s, Pool* pool, IntScratch& sc, const IntBasis& b, const void* tab, double* out);
 
 }  // namespace fh
