@@ -696,44 +696,25 @@ static void update_amp(Ctx& c, const double* t1, const double* t2, double* n1, d
   *r2 = std::sqrt(h[1] / (double)c.n2());
 }
 
-// DF-MP2 correlation energy RMP2_energy (RMP2a.jl:91-144) from Bov and the orbital energies
-// alone.  Instead of the reference's loop over pairs i <= j with one v x v GEMM each, the
-// integrals X = (ia|jb) of a block of j come from one FP64 MFMA GEMM (K = naux) against a
-// [Q, b, j] copy of Bov, then k_mp2_pairs reduces them.  The blocks of j keep X under
-// FERMIHIP_MP2_BLOCK_MB MiB (default 4096; one block up to o v = 23 000).
+// DF-MP2 correlation energy RMP2_energy (RMP2a.jl:91-144) from Bov and the orbital energies alone:
+// the reference's pairs i <= j, every pair and tile of (ia|jb) reduced to energy where it is made
+// (fh_mp2.hip), so nothing but the partial sums is stored.
 static double mp2_energy(Ctx& c) {
   require_df(c, false);
   FH_CHECK(!c.conventional, -6, "fh_mp2_energy: the DF-MP2 energy needs BOV; this context holds conventional blocks");
-  const int keep = c.lowp;
-  c.lowp = 0;
-  const int64_t o = c.o, v = c.v, Q = c.naux, ov = c.nov();
-  Timer t(c, "df_mp2", 2.0 * (double)Q * (double)ov * (double)ov);
-  Buf Bvo = dalloc(c, Q * ov);
-  perm(c, tv(c.Bov.d(), {Q, o, v}), "Qjb", tv(Bvo.d(), {Q, v, o}), "Qbj", 1.0, 0.0);
-  int64_t cap_mb = 4096;
-  if (const char* env = std::getenv("FERMIHIP_MP2_BLOCK_MB")) cap_mb = std::max<int64_t>(1, std::atoll(env));
-  const int64_t per_j = ov * v * (int64_t)sizeof(double);
-  const int nj = (int)std::max<int64_t>(1, std::min<int64_t>(o, (cap_mb << 20) / per_j));
-  const int nblk = (int)((o + nj - 1) / nj);
-  Buf X = dalloc(c, ov * v * nj);
-  Buf part = dalloc(c, mp2_pairs_blocks((int)v, nj) * nblk);
-  int64_t np = 0;
-  for (int j0 = 0; j0 < o; j0 += nj) {
-    const int n = (int)std::min<int64_t>(nj, o - j0);
-    contract(c, 1.0, tv(c.Bov.d(), {Q, o, v}), "Qia", tv(Bvo.d() + Q * v * j0, {Q, v, (int64_t)n}), "Qbj", 0.0,
-             tv(X.d(), {o, v, v, (int64_t)n}), "iabj");
-    mp2_pairs(c.s, (int)o, (int)v, j0, n, X.d(), c.eo.d(), c.ev.d(), part.d() + np);
-    np += mp2_pairs_blocks((int)v, n);
-  }
+  const int o = c.o, v = c.v;
+  Timer t(c, "df_mp2", (double)c.naux * (double)o * (o + 1.0) * (double)v * (double)v);
+  const int64_t np = mp2_partials(o, v);
+  Buf part = dalloc(c, np);
+  mp2_pair_energy(c.s, o, v, c.naux, c.Bov.d(), c.eo.d(), c.ev.d(), part.d());
   if (!c.scal.p) c.scal = dalloc(c, 64);
   sum_partials(c.s, np, part.d(), c.scal.d() + 2);
-  c.lowp = keep;
   return read_scalar(c, c.scal.d() + 2);
 }
 
 // ------------------------------------------------------------------ allocation-free DF-MP2 energy
-// fh_mp2_energy_noalloc keeps its intermediates (the [Q, b, j] copy of Bov, the (ia|jb) blocks and
-// the partial sums) in this file-scope device array instead of allocating them.  Each GPU holds its
+// fh_mp2_energy_noalloc keeps its intermediates (the partial sums) in this file-scope device array
+// instead of allocating them.  Each GPU holds its
 // own copy (128 MiB) from the library's load to the end of the process.  In host code `scratch` is
 // only a host-side stand-in for the symbol: its device address on each device comes from
 // hipGetSymbolAddress at fh_create (with that device current) and is kept in g_scratch[device].
@@ -757,49 +738,27 @@ static double* noalloc_scratch(int device) {
   return (device >= 0 && device < kNoAllocMaxDevices) ? g_scratch[device] : nullptr;
 }
 
-// Scratch layout for (o, v, naux): Bvo [Q, v, o] | X [(i, a), (b, j)] for nj values of j | partial
-// sums of every block.  Returns the largest nj <= o that fits kNoAllocDoubles, 0 if none does.
-static int noalloc_mp2_block(int64_t o, int64_t v, int64_t Q, int64_t* x_off, int64_t* part_off) {
+// The sizes that the entry point takes: those whose [Q, b, j] copy of Bov, (ia|jb) blocks of some nj values of j and up
+// to 2048 partial sums a block would fit the scratch array.  The pair kernel needs its partial sums only (at most 16384),
+// but callers size their problems by this limit, and a size that was refused is refused.
+static bool noalloc_mp2_fits(int64_t o, int64_t v, int64_t Q) {
   const int64_t ov = o * v;
-  for (int64_t nj = std::min<int64_t>(o, std::max<int64_t>(1, (kNoAllocDoubles - Q * ov) / (ov * v))); nj >= 1; --nj) {
-    const int64_t nblk = (o + nj - 1) / nj;
-    const int64_t need = Q * ov + ov * v * nj + nblk * mp2_pairs_blocks((int)v, (int)nj);
-    if (need <= kNoAllocDoubles) {
-      *x_off = Q * ov;
-      *part_off = Q * ov + ov * v * nj;
-      return (int)nj;
-    }
-  }
-  return 0;
+  for (int64_t nj = std::min<int64_t>(o, std::max<int64_t>(1, (kNoAllocDoubles - Q * ov) / (ov * v))); nj >= 1; --nj)
+    if (Q * ov + ov * v * nj + (o + nj - 1) / nj * std::min<int64_t>(v * nj, 2048) <= kNoAllocDoubles) return true;
+  return false;
 }
 
 // The DF-MP2 energy of mp2_energy() from device-resident eps_o, eps_v, Bov into the device double
-// *E, with every intermediate in the scratch array: the same kernels (permute, FP64 MFMA GEMM with
-// K = naux, pair reduction), blocks of j sized to the scratch.  Nothing in the scratch has to start
-// at zero: the copy, the GEMM (beta = 0) and the pair kernel overwrite what they use.
+// *E, the partial sums in the scratch array.  Nothing in it has to start at zero: the pair kernel
+// writes every partial sum.
 static void mp2_energy_noalloc(Ctx& c, int o, int v, int naux, const double* eo, const double* ev, const double* Bov,
                                double* E) {
-  double* base = noalloc_scratch(c.device);
-  FH_CHECK(base != nullptr, -6, "fh_mp2_energy_noalloc: no scratch address for this device (fh_create sets it)");
-  int64_t xoff = 0, poff = 0;
-  const int nj = noalloc_mp2_block(o, v, naux, &xoff, &poff);
-  FH_CHECK(nj >= 1, -1,
+  double* part = noalloc_scratch(c.device);
+  FH_CHECK(part != nullptr, -6, "fh_mp2_energy_noalloc: no scratch address for this device (fh_create sets it)");
+  FH_CHECK(noalloc_mp2_fits(o, v, naux), -1,
            "fh_mp2_energy_noalloc: naux o v + o v^2 + partial sums exceed the 128 MiB scratch (16777216 doubles)");
-  const int64_t ov = (int64_t)o * v, Q = naux;
-  double* Bvo = base;
-  double* X = base + xoff;
-  double* part = base + poff;
-  permute_to(c, tv(const_cast<double*>(Bov), {Q, (int64_t)o, (int64_t)v}), "Qjb", Bvo, "Qbj", 1.0, 0.0);
-  int64_t np = 0;
-  for (int j0 = 0; j0 < o; j0 += nj) {
-    const int n = std::min(nj, o - j0);
-    // X[(i,a),(b,j)] = sum_Q Bov[Q,(i,a)] Bvo[Q,(b,j)]
-    gemm_f64(c.s, true, false, ov, (int64_t)v * n, Q, 1.0, Bov, Q, 0, Bvo + Q * v * j0, Q, 0, 0.0, nullptr, ov, 0, X,
-             ov, 0, 1, 0);
-    mp2_pairs(c.s, o, v, j0, n, X, eo, ev, part + np);
-    np += mp2_pairs_blocks(v, n);
-  }
-  sum_partials(c.s, np, part, E);
+  mp2_pair_energy(c.s, o, v, naux, Bov, eo, ev, part);
+  sum_partials(c.s, mp2_partials(o, v), part, E);
 }
 
 static void mp2_guess(Ctx& c) {

@@ -198,11 +198,10 @@ void cast_f64_to_f32(hipStream_t s, int64_t n, const double* x, float* y);
 void cc_energy(hipStream_t s, int o, int v, const double* t1, const double* t2, const double* ovov,
                double* partials, double* result);
 
-// DF-MP2 energy of one block of j (RMP2a.jl:112-138): X[(i + o a) + o v (b + v (j - j0))] = (ia|jb)
-// for j in [j0, j0 + nj) -> mp2_pairs_blocks(v, nj) FP64 partial sums
-int64_t mp2_pairs_blocks(int v, int nj);
-void mp2_pairs(hipStream_t s, int o, int v, int j0, int nj, const double* X, const double* eo, const double* ev,
-               double* partials);
+// DF-MP2 energy (RMP2a.jl:91-144, fh_mp2.hip) from Bov[Q, i, a] -> mp2_partials(o, v) FP64 partial sums
+int64_t mp2_partials(int o, int v);
+void mp2_pair_energy(hipStream_t s, int o, int v, int Q, const double* Bov, const double* eo, const double* ev,
+                     double* partials);
 
 // SCF: out = U diag(w)^-1/2 (n x n, column-major); GWH guess Fock matrix (RHFHelper.jl:44-51)
 void scale_cols_rsqrt(hipStream_t s, int n, const double* U, const double* w, double* out);
