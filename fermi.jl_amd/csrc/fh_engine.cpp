@@ -102,9 +102,18 @@ struct Pending {
   hipEvent_t a, b;
 };
 
+struct BlasHandle {
+  rocblas_handle h = nullptr;
+  BlasHandle() = default;
+  BlasHandle(const BlasHandle&) = delete;
+  BlasHandle& operator=(const BlasHandle&) = delete;
+  ~BlasHandle() { if (h) (void)rocblas_destroy_handle(h); }
+};
+
 struct Ctx {
   int device = 0;
   hipStream_t s = nullptr;
+  BlasHandle blas;   // of the eigensolver, made on first use
   // declared before every Buf member, so that it is destroyed after all of them
   std::unique_ptr<Pool> pool;
   int o = 0, v = 0, naux = 0;
@@ -837,31 +846,40 @@ struct DIIS {
   int maxv;
   bool f32;
   std::vector<Buf> vecs, errs;
+  std::vector<std::vector<double>> B;   // B[a][b] = errs[a] . errs[b], b <= a
+  Buf part, row;                        // the newest row on the device until resolve() reads it
+  bool pending = false;
   const char* phase;  // timer name of the vector work (nullptr: untimed)
-  DIIS(Ctx& cc, int64_t nn, int m, bool f, const char* ph = nullptr) : c(cc), n(nn), maxv(m), f32(f), phase(ph) {}
+  DIIS(Ctx& cc, int64_t nn, int m, bool f, const char* ph = nullptr) : c(cc), n(nn), maxv(m), f32(f), phase(ph) {
+    part = dalloc(c, 8 * reduce_blocks_needed(n));
+    row = dalloc(c, 8);
+  }
   double esz() const { return f32 ? 4.0 : 8.0; }
   std::unique_ptr<Timer> timer(double bytes) {
     return std::unique_ptr<Timer>(phase ? new Timer(c, phase, 0.0, bytes) : nullptr);
   }
-  double dot(const Buf& a, const Buf& b) {
-    {
-      auto t = timer(2.0 * esz() * (double)n);
-      if (f32) dot_f32(c.s, n, a.f(), b.f(), c.partials.d(), c.scal.d() + 4);
-      else dot_f64(c.s, n, a.d(), b.d(), c.partials.d(), c.scal.d() + 4);
-    }
-    return read_scalar(c, c.scal.d() + 4);
+  // the products of the newest error vector, one copy for the whole row
+  void resolve() {
+    if (!pending) return;
+    double h[8];
+    d2h(c, h, row.d(), (int64_t)errs.size());
+    B.emplace_back(h, h + errs.size());
+    pending = false;
   }
   // push! takes ownership of the error buffer and copies the vector
   void push(const double* vec, Buf&& err) {
+    resolve();
     if ((int)vecs.size() + 1 > maxv) {
       int idx = 0;
       double best = -1.0;
       for (size_t q = 0; q < errs.size(); ++q) {
-        const double nq = std::sqrt(dot(errs[q], errs[q]));
+        const double nq = std::sqrt(B[q][q]);
         if (nq > best) { best = nq; idx = (int)q; }   // findmax: first maximum
       }
       vecs.erase(vecs.begin() + idx);
       errs.erase(errs.begin() + idx);
+      B.erase(B.begin() + idx);
+      for (size_t q = idx; q < B.size(); ++q) B[q].erase(B[q].begin() + idx);
     }
     Buf vb = dalloc(c, n);
     {
@@ -870,22 +888,23 @@ struct DIIS {
     }
     vecs.push_back(std::move(vb));
     errs.push_back(std::move(err));
+    const void* xs[8];
+    for (size_t q = 0; q < errs.size(); ++q) xs[q] = errs[q].p;
+    auto t = timer(esz() * (double)errs.size() * (double)n);
+    dots(c.s, n, (int)errs.size(), xs, errs.back().p, f32, part.d(), row.d());
+    pending = true;
   }
   void extrapolate(double* out, bool add_res) {
     const int m = (int)vecs.size();
     FH_CHECK(m >= 2, -3, "DIIS cannot extrapolate from one vector");
+    resolve();
     const int N = m + 1;
-    std::vector<double> B(N * N, 1.0), rhs(N, 0.0);
-    B[(N - 1) * N + (N - 1)] = 0.0;
+    std::vector<double> A(N * N, 1.0), x(N, 0.0);
+    A[(N - 1) * N + (N - 1)] = 0.0;
     for (int a = 0; a < m; ++a)
-      for (int b = 0; b <= a; ++b) {
-        const double d = dot(errs[a], errs[b]);
-        B[a * N + b] = d;
-        B[b * N + a] = d;
-      }
-    rhs[N - 1] = 1.0;
+      for (int b = 0; b <= a; ++b) A[a * N + b] = A[b * N + a] = B[a][b];
+    x[N - 1] = 1.0;
     // B \ rhs by LU with partial pivoting (row-major)
-    std::vector<double> A = B, x = rhs;
     for (int k = 0; k < N; ++k) {
       int p = k;
       for (int r = k + 1; r < N; ++r)
@@ -918,18 +937,23 @@ struct DIIS {
 // Symmetric eigensolver on the device (rocSOLVER syevd, the divide-and-conquer LAPACK method):
 // A (n x n, column-major) is overwritten by the eigenvectors, w gets the eigenvalues ascending, as
 // eigen(Symmetric(A), sortby = x -> x) orders them.
+//
+// Up to n = 1024 the context keeps the rocBLAS handle and with it the solver's workspace (a few n^2 doubles), which a
+// handle of one call allocates and frees each time; above, a handle lives as long as the solver.
 struct Eigen {
   Ctx& c;
+  BlasHandle own;
   rocblas_handle h = nullptr;
   Buf work, info;
   int n;
   Eigen(Ctx& cc, int nn) : c(cc), n(nn) {
-    FH_CHECK(rocblas_create_handle(&h) == rocblas_status_success, -2, "rocblas_create_handle failed");
+    BlasHandle& b = n <= 1024 ? c.blas : own;
+    if (!b.h) FH_CHECK(rocblas_create_handle(&b.h) == rocblas_status_success, -2, "rocblas_create_handle failed");
+    h = b.h;
     FH_CHECK(rocblas_set_stream(h, c.s) == rocblas_status_success, -2, "rocblas_set_stream failed");
     work = dalloc(c, n);
     info = dalloc(c, 1);
   }
-  ~Eigen() { if (h) (void)rocblas_destroy_handle(h); }
   void run(double* A, double* w) {
     FH_CHECK(rocsolver_dsyevd(h, rocblas_evect_original, rocblas_fill_upper, n, A, n, w, work.d(),
                               reinterpret_cast<rocblas_int*>(info.p)) == rocblas_status_success, -2,
@@ -1040,7 +1064,14 @@ static void rhf(Ctx& c, const fh_scf_opts& op, int n, int naux, int no, double V
   while (ite <= op.scf_max_iter) {
     orbitals(F.d());                                              // RHFa.jl:137-147
     fock();                                                       // :150
-    const double Enew = dotd(c, nn, D.d(), H, 8) + dotd(c, nn, D.d(), F.d(), 9) + Vnuc;   // :151-154
+    dot_f64(c.s, nn, D.d(), H, c.partials.d(), c.scal.d() + 8);
+    dot_f64(c.s, nn, D.d(), F.d(), c.partials.d(), c.scal.d() + 9);
+    d2d(c, T1.d(), D.d(), nn);                                    // Drms (:189-190)
+    axpby_f64(c.s, nn, -1.0, Dold.d(), 1.0, T1.d());
+    dot_f64(c.s, nn, T1.d(), T1.d(), c.partials.d(), c.scal.d() + 10);
+    double h[3];
+    d2h(c, h, c.scal.d() + 8, 3);
+    const double Enew = h[0] + h[1] + Vnuc;                       // :151-154
     if (dm) {                                                     // err = L^T (F D S - S D F) L  (:157-160)
       mm(c, false, false, n, n, n, 1.0, F.d(), n, D.d(), n, 0.0, T1.d(), n);       // F D
       mm(c, false, false, n, n, n, 1.0, T1.d(), n, S, n, 0.0, T2.d(), n);          // F D S
@@ -1055,8 +1086,8 @@ static void rhf(Ctx& c, const fh_scf_opts& op, int n, int naux, int no, double V
       d2d(c, T1.d(), D.d(), nn);
       axpby_f64(c.s, nn, -1.0, Dtil.d(), 1.0, T1.d());            // dD = D - D~
       transpose_sq(c, n, T1.d(), 1.0, 0.0, T2.d());               // tr(A dD) = sum A .* dD^T
-      const double sv = dotd(c, nn, Ftil.d(), T2.d(), 10);
-      const double cv = dotd(c, nn, F.d(), T2.d(), 11) - sv;
+      const double sv = dotd(c, nn, Ftil.d(), T2.d(), 11);
+      const double cv = dotd(c, nn, F.d(), T2.d(), 12) - sv;
       const double lam = (cv <= -sv / (2.0 * cv)) ? 1.0 : -sv / (2.0 * cv);
       axpby_f64(c.s, nn, lam, F.d(), 1.0 - lam, Ftil.d());
       axpby_f64(c.s, nn, lam, D.d(), 1.0 - lam, Dtil.d());
@@ -1064,9 +1095,7 @@ static void rhf(Ctx& c, const fh_scf_opts& op, int n, int naux, int no, double V
     } else if (dm && ite > op.diis_start) {                       // DIIS (:183-186)
       dm->extrapolate(F.d(), false);
     }
-    d2d(c, T1.d(), D.d(), nn);                                    // Drms (:189-190)
-    axpby_f64(c.s, nn, -1.0, Dold.d(), 1.0, T1.d());
-    Drms = std::sqrt(dotd(c, nn, T1.d(), T1.d(), 12) / (double)nn);
+    Drms = std::sqrt(h[2] / (double)nn);
     dE = Enew - E;
     E = Enew;
     d2d(c, Dold.d(), D.d(), nn);

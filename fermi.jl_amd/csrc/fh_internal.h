@@ -188,7 +188,9 @@ void jacobi_update(hipStream_t s, int o, int v, bool is_t2, const double* eo, co
 int64_t reduce_blocks_needed(int64_t n);
 // deterministic FP64 dot products: partial sums per block, then one final block.
 void dot_f64(hipStream_t s, int64_t n, const double* x, const double* y, double* partials, double* result);
-void dot_f32(hipStream_t s, int64_t n, const float* x, const float* y, double* partials, double* result);
+// result[q] = x_q . y (FP64 sums) for up to 8 FP64 or FP32 vectors; partials: nv reduce_blocks_needed(n)
+void dots(hipStream_t s, int64_t n, int nv, const void* const* xs, const void* y, bool f32, double* partials,
+          double* result);
 void sum_partials(hipStream_t s, int64_t n, const double* partials, double* result);
 // y = sum_i c_i x_i (+ sum_i c_i e_i) for up to 8 FP64 vectors and 8 FP64/FP32 error vectors
 void lincomb(hipStream_t s, int64_t n, int nv, const double* const* xs, const double* cs,

@@ -441,12 +441,10 @@ void jacobi_update(hipStream_t s, int o, int v, bool is_t2, const double* eo, co
 }
 
 // ------------------------------------------------------------------ reductions
-template <typename T>
-__global__ __launch_bounds__(RB) void k_dot(int64_t n, const T* __restrict__ x, const T* __restrict__ y,
+__global__ __launch_bounds__(RB) void k_dot(int64_t n, const double* __restrict__ x, const double* __restrict__ y,
                                             double* __restrict__ partials) {
   double acc = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB)
-    acc += (double)x[i] * (double)y[i];
+  for (int64_t i = (int64_t)blockIdx.x * RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB) acc += x[i] * y[i];
   const double t = block_sum(acc);
   if (threadIdx.x == 0) partials[blockIdx.x] = t;
 }
@@ -462,15 +460,52 @@ void sum_partials(hipStream_t s, int64_t n, const double* partials, double* resu
 }
 void dot_f64(hipStream_t s, int64_t n, const double* x, const double* y, double* partials, double* result) {
   const int64_t g = reduce_blocks_needed(n);
-  hipLaunchKernelGGL((k_dot<double>), dim3(g), dim3(RB), 0, s, n, x, y, partials);
+  hipLaunchKernelGGL(k_dot, dim3(g), dim3(RB), 0, s, n, x, y, partials);
   FH_HIP(hipGetLastError());
   sum_partials(s, g, partials, result);
 }
-void dot_f32(hipStream_t s, int64_t n, const float* x, const float* y, double* partials, double* result) {
+// result[q] = x_q . y for up to 8 vectors, each element of y read once: a row of the DIIS matrix in two launches and one
+// read of the subspace (bound by HBM for large amplitudes, by launches for small ones: a dot and its sum per element of
+// the matrix, each with a copy back, were 132 of them a solve at o = 16, v = 76, 20 us each).
+struct DotsArgs {
+  int nv;
+  const void* x[8];
+};
+template <typename T>
+__global__ __launch_bounds__(RB) void k_dots(int64_t n, DotsArgs a, const T* __restrict__ y, double* __restrict__ partials) {
+  double acc[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  for (int64_t i = (int64_t)blockIdx.x * RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB) {
+    const double v = (double)y[i];
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (q < a.nv) acc[q] += (double)static_cast<const T*>(a.x[q])[i] * v;
+  }
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+    if (q < a.nv) {
+      const double t = block_sum(acc[q]);
+      if (threadIdx.x == 0) partials[(int64_t)q * gridDim.x + blockIdx.x] = t;
+      __syncthreads();
+    }
+}
+__global__ __launch_bounds__(RB) void k_sums(int64_t n, const double* __restrict__ partials, double* __restrict__ result) {
+  double acc = 0.0;
+  for (int64_t i = threadIdx.x; i < n; i += RB) acc += partials[n * blockIdx.x + i];
+  const double t = block_sum(acc);
+  if (threadIdx.x == 0) result[blockIdx.x] = t;
+}
+void dots(hipStream_t s, int64_t n, int nv, const void* const* xs, const void* y, bool f32, double* partials,
+          double* result) {
+  FH_CHECK(nv >= 1 && nv <= 8, -3, "dots: 1..8 vectors");
+  DotsArgs a;
+  a.nv = nv;
+  for (int q = 0; q < 8; ++q) a.x[q] = q < nv ? xs[q] : nullptr;
   const int64_t g = reduce_blocks_needed(n);
-  hipLaunchKernelGGL((k_dot<float>), dim3(g), dim3(RB), 0, s, n, x, y, partials);
+  if (f32) hipLaunchKernelGGL((k_dots<float>), dim3(g), dim3(RB), 0, s, n, a, static_cast<const float*>(y), partials);
+  else hipLaunchKernelGGL((k_dots<double>), dim3(g), dim3(RB), 0, s, n, a, static_cast<const double*>(y), partials);
   FH_HIP(hipGetLastError());
-  sum_partials(s, g, partials, result);
+  hipLaunchKernelGGL(k_sums, dim3(nv), dim3(RB), 0, s, g, partials, result);
+  FH_HIP(hipGetLastError());
 }
 
 // ------------------------------------------------------------------ DIIS extrapolation (DIIS.jl:86-93)
