@@ -134,6 +134,27 @@ __device__ __forceinline__ void read_rows(unsigned a, unsigned b, f32x4& fa, f32
                  : [pa] "v"(a), [pb] "v"(b) : "memory");
 }
 
+// the same for NB = 5 and 6 with the wave's extra blocks: one more A block at a2, and one (three) B blocks at b2
+template <int NB>
+__device__ __forceinline__ void read_rows_extra(unsigned a, unsigned b, unsigned a2, unsigned b2, f32x4& fa, f32x4 (&fb)[NB],
+                                                f32x4& fx, f32x4 (&fy)[NB == 6 ? 3 : 1]) {
+#define FH_X FH_RD(x, px, 0) FH_RD(y0, py, 0)
+#define FH_XO [x] "=&v"(fx), [y0] "=&v"(fy[0])
+#define FH_I [pa] "v"(a), [pb] "v"(b), [px] "v"(a2), [py] "v"(b2)
+  if constexpr (NB == 5)
+    asm volatile(FH_RD(a0, pa, 0) FH_Q(0, 0) FH_Q(1, 1024) FH_Q(2, 2048) FH_Q(3, 3072) FH_Q(4, 4096) FH_X
+                 "s_waitcnt lgkmcnt(0)"
+                 : [a0] "=&v"(fa), FH_QO(0), FH_QO(1), FH_QO(2), FH_QO(3), FH_QO(4), FH_XO : FH_I : "memory");
+  if constexpr (NB == 6)
+    asm volatile(FH_RD(a0, pa, 0) FH_Q(0, 0) FH_Q(1, 1024) FH_Q(2, 2048) FH_Q(3, 3072) FH_Q(4, 4096) FH_Q(5, 5120)
+                 FH_X FH_RD(y1, py, 1024) FH_RD(y2, py, 2048) "s_waitcnt lgkmcnt(0)"
+                 : [a0] "=&v"(fa), FH_QO(0), FH_QO(1), FH_QO(2), FH_QO(3), FH_QO(4), FH_QO(5), FH_XO,
+                   [y1] "=&v"(fy[NB == 6 ? 1 : 0]), [y2] "=&v"(fy[NB == 6 ? 2 : 0]) : FH_I : "memory");
+#undef FH_X
+#undef FH_XO
+#undef FH_I
+}
+
 // two FP32 values -> packed (hi, lo) bf16 pairs, hi = bf16(x), lo = bf16(x - hi)
 __device__ inline void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
   const f32x2 v = {a, b};
@@ -611,15 +632,20 @@ __global__ __launch_bounds__(256, MB == 3 ? 2 : 3) void k_triples_w_bf3(TripW t)
   else tile.template run_n<1>(feed);
 }
 
-// FP64 and FP32: tiles of 16 NB x 16 NB, NB wavefronts of one 16-row block each (NB column blocks).  An MFMA
-// takes 64 (FP64) or 32 (FP32) cycles, so the fragment reads (one per block and k step: a lane's 16 bytes
-// are 2 (4) k, fed to 2 (4) MFMAs in turn -- the k order inside a step is free as long as A and B agree) hide
-// behind them with four or more wavefronts per SIMD, and small tiles cost little: the tile follows v in
-// steps of 16 instead of padding N = v = 76 to 128.
+// FP64 and FP32: tiles of 16 NB x 16 NB, a wavefront per 16-row block (NB column blocks), and at NB = 5 and 6 four
+// wavefronts that share the last rows' blocks: the SIMDs of a CU are dealt a workgroup's wavefronts in order, so a fifth
+// would always land with the first (matrix pipes busy 53 % of the time at NB = 5 with five, 63 % at NB = 6 with six;
+// slices and first launch of o = 16, v = 76 in FP64 7.7 and 3.3 ms so, 5.7 and 2.7 ms with four).  An MFMA takes 64
+// (FP64) or 32 (FP32) cycles, so the fragment reads (one per block and k step: a lane's 16 bytes are 2 (4) k, fed to
+// 2 (4) MFMAs in turn -- the k order inside a step is free as long as A and B agree) hide behind them with four
+// wavefronts per SIMD, and small tiles cost little: the tile follows v in steps of 16 instead of padding N = v = 76
+// to 128.
+constexpr int triples_w_waves(int nb) { return nb < 4 ? nb : 4; }
 template <typename T, int NSEG, int NB>
-__global__ __launch_bounds__(64 * NB) void k_triples_w(TripW t) {
+__global__ __launch_bounds__(64 * triples_w_waves(NB), NB == 6 ? 3 : NB > 3 ? 4 : 1) void k_triples_w(TripW t) {
   constexpr bool F32 = std::is_same<T, float>::value;
   constexpr int NS = 3, ABYTES = NB * 1024, SLOT = 2 * ABYTES, KL = F32 ? 4 : 2;
+  constexpr int NW = triples_w_waves(NB), NX = NB == 5 ? 2 : NB == 6 ? 3 : 0;
   using Acc = typename std::conditional<F32, f32x4, f64x4>::type;
   __shared__ __attribute__((aligned(16))) char ring[NS * SLOT];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -629,69 +655,111 @@ __global__ __launch_bounds__(64 * NB) void k_triples_w(TripW t) {
   const int rows = tl.rows, cols = tl.cols;
   Feed<NSEG, GB> feed(t, tl, lane);
   const int nst = NSEG * (t.nd / 8) * GB / 64;
-  const int r = 16 * wid + copy_row<GB>(lane);
-  const int lofa = 16 * copy_unit<GB>(lane) + GB * min(r, rows - 1);
-  const int lofb = 16 * copy_unit<GB>(lane) + tl.col_off(min(r, cols - 1));
+  // pieces of 16 rows: wid and, of NB = 5 and 6, wid + 4
+  const bool second = NB > 4 && wid + 4 < NB;
+  int lofa[2], lofb[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int r = 16 * (wid + 4 * h) + copy_row<GB>(lane);
+    lofa[h] = 16 * copy_unit<GB>(lane) + GB * min(r, rows - 1);
+    lofb[h] = 16 * copy_unit<GB>(lane) + tl.col_off(min(r, cols - 1));
+  }
   auto dma = [&](int slot) {
     feed.step([&](__amdgpu_buffer_rsrc_t rsa, __amdgpu_buffer_rsrc_t rsb, int dga, int dgb) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_vptr)(ring + slot * SLOT + wid * 1024), 16,
-                                               (unsigned)(lofa + dga), 0, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsb, (lds_vptr)(ring + slot * SLOT + ABYTES + wid * 1024), 16,
-                                               (unsigned)(lofb + dgb), 0, 0, 0);
+      char* d = ring + slot * SLOT + wid * 1024;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_vptr)d, 16, (unsigned)(lofa[0] + dga), 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsb, (lds_vptr)(d + ABYTES), 16, (unsigned)(lofb[0] + dgb), 0, 0, 0);
+      if (second) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_vptr)(d + 4096), 16, (unsigned)(lofa[1] + dga), 0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsb, (lds_vptr)(d + 4096 + ABYTES), 16, (unsigned)(lofb[1] + dgb), 0, 0, 0);
+      }
     });
   };
+  // the extra blocks: NB = 5: (4, wid) and, for one wavefront, in turn over the workgroups, (4, 4); NB = 6: three
+  // of row block 4 or 5
+  const bool last = NB == 5 && wid == ((int)(blockIdx.x >> 8) & 3);
+  const int xr = NB == 6 ? 4 + (wid >> 1) : 4, xc = NB == 6 ? 3 * (wid & 1) : wid;
   // unit l / 16 of the step of row l % 16 (FP32: units of two groups)
   const int fu = lane >> 4;
   const unsigned frag = lds_addr(ring) + unit_at<GB>(lane & 15, F32 ? fu >> 1 : 0, F32 ? fu & 1 : fu);
   const unsigned a_off = frag + wid * 1024, b_off = frag + ABYTES;
-  Acc acc[NB];
+  Acc acc[NB], accx[NX > 0 ? NX : 1];
 #pragma unroll
   for (int j = 0; j < NB; ++j) acc[j] = Acc{0, 0, 0, 0};
+#pragma unroll
+  for (int j = 0; j < NX; ++j) accx[j] = Acc{0, 0, 0, 0};
   dma(0);
   if (nst > 1) dma(1);
   int cur = 0, nxt = 2;
   for (int s = 0; s < nst; ++s) {
-    if (s + 1 < nst) wait_vmcnt<2>();
-    else wait_vmcnt<0>();
+    if (s + 1 >= nst) wait_vmcnt<0>();
+    else if (second) wait_vmcnt<4>();
+    else wait_vmcnt<2>();
     lds_barrier();
     if (s + 2 < nst) dma(nxt);
-    f32x4 fa, fb[NB];
-    read_rows<NB>(a_off + cur * SLOT, b_off + cur * SLOT, fa, fb);
-    T af[KL], bf[NB][KL];
-    __builtin_memcpy(af, &fa, 16);
+    f32x4 fa, fb[NB], fx, fy[NB == 6 ? 3 : 1];
+    if constexpr (NX > 0)
+      read_rows_extra<NB>(a_off + cur * SLOT, b_off + cur * SLOT, frag + xr * 1024 + cur * SLOT,
+                          b_off + xc * 1024 + cur * SLOT, fa, fb, fx, fy);
+    else
+      read_rows<NB>(a_off + cur * SLOT, b_off + cur * SLOT, fa, fb);
+    auto mul = [&](const f32x4& ua, const f32x4& ub, Acc& c, int q) {
+      T ta[KL], tb[KL];
+      __builtin_memcpy(ta, &ua, 16);
+      __builtin_memcpy(tb, &ub, 16);
+      // B as the first operand, so that the accumulator's lanes run along the rows of W
+      if constexpr (F32) c = __builtin_amdgcn_mfma_f32_16x16x4f32(tb[q], ta[q], c, 0, 0, 0);
+      else c = __builtin_amdgcn_mfma_f64_16x16x4f64(tb[q], ta[q], c, 0, 0, 0);
+    };
 #pragma unroll
-    for (int j = 0; j < NB; ++j) __builtin_memcpy(bf[j], &fb[j], 16);
+    for (int q = 0; q < KL; ++q) {
 #pragma unroll
-    for (int q = 0; q < KL; ++q)
+      for (int j = 0; j < NB; ++j) mul(fa, fb[j], acc[j], q);
+      if constexpr (NB == 6) {
 #pragma unroll
-      for (int j = 0; j < NB; ++j) {
-        // B as the first operand, so that the accumulator's lanes run along the rows of W
-        if constexpr (F32) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[j][q], af[q], acc[j], 0, 0, 0);
-        else acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bf[j][q], af[q], acc[j], 0, 0, 0);
+        for (int j = 0; j < 3; ++j) mul(fx, fy[j], accx[j], q);
       }
+      if constexpr (NB == 5) mul(fx, fy[0], accx[0], q);
+    }
+    if constexpr (NB == 5) {
+      if (last) {
+#pragma unroll
+        for (int q = 0; q < KL; ++q) mul(fx, fb[4], accx[1], q);
+      }
+    }
     cur = cur == NS - 1 ? 0 : cur + 1;
     nxt = nxt == NS - 1 ? 0 : nxt + 1;
   }
-  // register e of lane l of block j: row l % 16, column (l / 16) + 4 e (FP64) or 4 (l / 16) + e (FP32)
+  // register e of lane l of a block: row l % 16, column (l / 16) + 4 e (FP64) or 4 (l / 16) + e (FP32)
   T* const W = static_cast<T*>(t.w) + tl.woff;
-  const int ldw = (int)tl.ldw, row = 16 * wid + (lane & 15);
-  auto col = [&](int j, int e) { return 16 * j + (F32 ? 4 * (lane >> 4) + e : (lane >> 4) + 4 * e); };
-  if constexpr (NSEG == 4) {
-    T dv[NB][4];
+  const int ldw = (int)tl.ldw;
+  auto put = [&](auto& blk, auto n, int rb, auto cb) {
+    constexpr int N = decltype(n)::value;
+    const int row = 16 * rb + (lane & 15);
+    auto col = [&](int j, int e) { return 16 * cb(j) + (F32 ? 4 * (lane >> 4) + e : (lane >> 4) + 4 * e); };
+    if constexpr (NSEG == 4) {
+      T dv[N][4];
 #pragma unroll
-    for (int j = 0; j < NB; ++j)
+      for (int j = 0; j < N; ++j)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) dv[j][e] = W[row < rows && col(j, e) < cols ? row + ldw * col(j, e) : 0];
+        for (int e = 0; e < 4; ++e) dv[j][e] = W[row < rows && col(j, e) < cols ? row + ldw * col(j, e) : 0];
 #pragma unroll
-    for (int j = 0; j < NB; ++j)
+      for (int j = 0; j < N; ++j)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc[j][e] += dv[j][e];
+        for (int e = 0; e < 4; ++e) blk[j][e] += dv[j][e];
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (row < rows && col(j, e) < cols) W[row + ldw * col(j, e)] = blk[j][e];
+  };
+  put(acc, std::integral_constant<int, NB>(), wid, [](int j) { return j; });
+  if constexpr (NB == 6) put(accx, std::integral_constant<int, 3>(), xr, [&](int j) { return xc + j; });
+  if constexpr (NB == 5) {
+    if (last) put(accx, std::integral_constant<int, 2>(), 4, [&](int j) { return j ? 4 : wid; });
+    else put(accx, std::integral_constant<int, 1>(), 4, [&](int) { return wid; });
   }
-#pragma unroll
-  for (int j = 0; j < NB; ++j)
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (row < rows && col(j, e) < cols) W[row + ldw * col(j, e)] = acc[j][e];
 }
 
 // ------------------------------------------------------------------ (T) energy epilogue (ijk.jl:116-136)
@@ -1000,11 +1068,15 @@ TriplesTiles triples_tiles(int fmt, int o, int v, double nk) {
   FH_CHECK(vv < ((int64_t)1 << 31), -3, "(T): v^2 exceeds 32 bits");
   auto tiles = [](int64_t n, int g, int per) { return (int)(((n + g - 1) / g + per - 1) / per); };
   if (fmt == 2) {
-    // 128 x 128 tiles (three workgroups per CU) where v fits one, else up to 192 x 192
-    t.nb = v <= 128 ? 2 : 3;
+    // Tiles of up to 6 x 6 blocks of 32, and the 128 x 128 kernel (three workgroups per CU instead of two) where the
+    // slices' tiles come to 4 x 4 at most (the (T) of o = 14, v = 200, two tiles of 4 and 3 blocks: 57.8 ms with the
+    // 192 x 192 kernel, 52.8 so; a 160 x 160 kernel with a fourth ring slot for five blocks: 88.2 ms at o = 27, v = 131
+    // against 87.1).  The first launch has v^2 rows, and tiles of 4 blocks only where v fits one.
+    const int nblk = (v + 31) / 32, nt = tiles(v, 32, 6);
     t.grain = 32;
-    t.per = 2 * t.nb;
-    t.nb_first = t.nb;
+    t.per = 6;
+    t.nb = nblk <= 4 * nt ? 2 : 3;
+    t.nb_first = v <= 128 ? 2 : 3;
   } else {
     // slices: the block count with the least padded area, wider tiles preferred (operand reuse: a tile reads
     // 2 / NB of a block per block product)
@@ -1051,7 +1123,7 @@ int64_t triples_chunk_slots(int v, int elem, const TriplesTiles& tt, int64_t nto
 
 template <int NSEG>
 static void launch_w(hipStream_t s, int fmt, int nb, unsigned grid, const TripW& t) {
-#define FH_W(T, NB) hipLaunchKernelGGL((k_triples_w<T, NSEG, NB>), dim3(grid), dim3(64 * NB), 0, s, t)
+#define FH_W(T, NB) hipLaunchKernelGGL((k_triples_w<T, NSEG, NB>), dim3(grid), dim3(64 * triples_w_waves(NB)), 0, s, t)
 #define FH_WT(T)               \
   switch (nb) {                \
     case 2: FH_W(T, 2); break; \
