@@ -131,6 +131,8 @@ struct Ctx {
   // Vs[cd, ab] over pairs (prepare_ladder) and Pt[c,d,a,k] = (kd|ac); FP32 copies of LX and Vs for the
   // reduced-precision residual (made on first use)
   Buf LX, Vs, Pt, LX32, Vs32;
+  // Lkl[k,l,c,d] = LX[k,c,l,d] and Okl[k,l,i,c] = (ki|lc): the slices of slice_sum
+  Buf Lkl, Okl;
   // GEMM operands made from the integral blocks above (a permuted FP64 copy, or an FP32 copy for
   // split-BF16x3): the same for every CC iteration, so made once and kept, up to opcache_cap
   // bytes; key "<block>|<index order>|<d or f>"
@@ -315,8 +317,9 @@ static void contract(Ctx& c, double alpha, const TView& A, const std::string& ia
   Buf work;
   if (wsz) work = dalloc(c, wsz);
   // split-BF16x3 for the o^3 v^3-class GEMMs of the mixed phase, on FP32 copies of the operands
-  // (half the operand traffic of FP64 loads); smaller GEMMs (and the split-K shapes) stay on FP32 MFMA
-  const bool bf3 = c.lowp == 2 && wsz == 0 && (double)Msz * (double)Nsz * (double)Ksz >= 1e9;
+  // (half the operand traffic of FP64 loads); smaller GEMMs, the split-K shapes and those of fewer than 64 rows or
+  // columns, most of a 128 x 128 tile idle, stay on FP32 MFMA (o x o v^2 x v at o = 28, v = 133: 328 us in split-BF16x3)
+  const bool bf3 = c.lowp == 2 && wsz == 0 && std::min(Msz, Nsz) >= 64 && (double)Msz * (double)Nsz * (double)Ksz >= 1e9;
 
   // The GEMM's copy of an operand: the tensor itself when its index order is GEMM-ready and the
   // GEMM reads FP64, else a permuted and/or FP32 copy.  Copies of the integral blocks go to the
@@ -378,10 +381,12 @@ static void contract(Ctx& c, double alpha, const TView& A, const std::string& ia
   const void* pB = operand(B, ib, readyB, Kord + N, tB, tBf);
   auto gemm = [&](bool ta, bool tb, int64_t m, int64_t n, double al, const void* a, int64_t la, const void* b,
                   int64_t lb, double be, const double* cc, double* d, int64_t ld) {
-    if (bf3)
+    if (bf3) {
+      const int64_t w3 = gemm_bf3_splitk_elems(ta, tb, m, n, Ksz, 1, 0);
+      if (w3) work = dalloc(c, w3);
       gemm_bf3(c.s, ta, tb, m, n, Ksz, al, static_cast<const float*>(a), la, 0, static_cast<const float*>(b), lb, 0, be,
-               cc, ld, d, ld, 0, 1, 0);
-    else
+               cc, ld, d, ld, 0, 1, 0, work.d(), w3);
+    } else
       gemm_f64(c.s, ta, tb, m, n, Ksz, al, static_cast<const double*>(a), la, 0, static_cast<const double*>(b), lb, 0,
                be, cc, ld, 0, d, ld, 0, 1, 0, work.d(), wsz, c.lowp != 0);
   };
@@ -401,6 +406,17 @@ static void contract(Ctx& c, double alpha, const TView& A, const std::string& ia
     for (char ch : N) T.dim[q++] = LB.dim(ch);
     permute_to(c, T, M + N, C.p, ic, alpha, beta);
   }
+}
+
+// out[M, N] (+)= alpha sum_z A_z^T B_z over nz slices, A_z [K, M] and B_z [K, N] with K contiguous: index orders
+// [k.., m, z] of amplitudes, which one GEMM over (k.., z) would need permuted first.  One batched GEMM into slices
+// and their sum.
+static void slice_sum(Ctx& c, int64_t M, int64_t N, int64_t K, int64_t nz, double alpha, const double* A, const double* B,
+                      double beta, double* out) {
+  Buf w = dalloc(c, M * N * nz);
+  gemm_f64(c.s, true, false, M, N, K, 1.0, A, K, K * M, B, K, K * N, 0.0, nullptr, 0, 0, w.d(), M, M * N, nz, 0, nullptr, 0,
+           c.lowp != 0);
+  splitk_reduce_f64(c.s, M, N, nz, w.d(), alpha, beta, out, M, 0, out, M, 0, 1);
 }
 
 // out[outL] = alpha * in[inL] + beta * out
@@ -425,6 +441,10 @@ static void build_lx(Ctx& c) {
   d2d(c, c.LX.d(), c.LX.d() + c.n2(), c.n2());
   axpby_f64(c.s, c.n2(), 2.0, c.OVOV.d(), -1.0, c.LX.d());
   c.LX32.reset();
+  c.Lkl = dalloc(c, c.n2());
+  perm(c, tv(c.LX.d(), {o, v, o, v}), "kcld", tv(c.Lkl.d(), {o, o, v, v}), "klcd", 1.0, 0.0);
+  c.Okl = dalloc(c, o * o * o * v);
+  perm(c, tv(c.OOOV.d(), {o, o, o, v}), "kilc", tv(c.Okl.d(), {o, o, o, v}), "klic", 1.0, 0.0);
 }
 
 static void prepare(Ctx& c) {
@@ -532,7 +552,7 @@ static void residual(Ctx& c, const double* t1p, const double* t2p, double* R1, d
   else
     contract(c, 1.0, ovov, "kcld", u, "ilcd", 0.0, Foo, "ki");
   contract(c, 1.0, Fov, "kc", t1, "ic", 1.0, Foo, "ki");
-  contract(c, -1.0, Lovov, "kcld", t2, "klad", 0.0, Fvv, "ac");
+  slice_sum(c, v, v, o * o, v, -1.0, t2p, c.Lkl.d(), 0.0, Fvv.p);
   contract(c, -1.0, t1, "ka", Fov, "kc", 1.0, Fvv, "ac");
   // Loo = Foo + 2 (ki|lc) t1[l,c] - (li|kc) t1[l,c];  Lvv = Fvv + 2 (kd|ac) t1[k,d] - (kc|ad) t1[k,d]
   Buf bLoo = dalloc(c, o * o), bLvv = dalloc(c, v * v);
@@ -547,13 +567,16 @@ static void residual(Ctx& c, const double* t1p, const double* t2p, double* R1, d
   // ---- T1 numerator
   contract(c, 1.0, Lvv, "ac", t1, "ic", 0.0, r1, "ia");
   contract(c, -1.0, Loo, "ki", t1, "ka", 1.0, r1, "ia");
-  contract(c, 1.0, Fov, "kc", u, "kica", 1.0, r1, "ia");
+  if (!t1_only && !ring32)
+    contract(c, 1.0, Fov, "kc", tv(bring.d(), {o, v, o, v}), "kcia", 1.0, r1, "ia");
+  else
+    contract(c, 1.0, Fov, "kc", u, "kica", 1.0, r1, "ia");
   contract(c, 1.0, Fov, "kc", t1, "ic", 0.0, X, "ik");
   contract(c, 1.0, X, "ik", t1, "ka", 1.0, r1, "ia");
   contract(c, 2.0, ovov, "kcia", t1, "kc", 1.0, r1, "ia");
   contract(c, -1.0, oovv, "kiac", t1, "kc", 1.0, r1, "ia");
   contract(c, 1.0, ovvv, "kdac", u, "ikcd", 1.0, r1, "ia");
-  contract(c, -1.0, ooov, "kilc", u, "klac", 1.0, r1, "ia");
+  slice_sum(c, o, v, o * o, v, -1.0, c.Okl.d(), u.p, 1.0, r1.p);
   if (t1_only) return;
   bu.reset();
 
@@ -562,18 +585,14 @@ static void residual(Ctx& c, const double* t1p, const double* t2p, double* R1, d
   Buf bP = dalloc(c, n2);
   TView P = tv(bP, {o, o, v, v});
   perm(c, ovov, "iajb", P, "ijab", 0.5, 0.0);                       // (ia|jb)  (:134)
-  contract(c, 1.0, ovvv, "iacb", t1, "jc", 1.0, P, "ijab");          // T1 x (ia|cb)
-  {
-    Buf b1 = dalloc(c, o * o * v * o);
-    TView X1 = tv(b1, {o, o, v, o});
-    contract(c, 1.0, oovv, "kibc", t1, "jc", 0.0, X1, "kibj");
-    contract(c, -1.0, X1, "kibj", t1, "ka", 1.0, P, "ijab");
-    Buf b2 = dalloc(c, v * o * o * o);
-    TView X2 = tv(b2, {v, o, o, o});
-    contract(c, 1.0, ovov, "kcia", t1, "jc", 0.0, X2, "akij");
-    perm(c, ooov, "jkia", X2, "akij", 1.0, 1.0);
-    contract(c, -1.0, X2, "akij", t1, "kb", 1.0, P, "ijab");
-  }
+  // (a term may enter as itself or with (i,a) and (j,b) exchanged: each in the form whose GEMM writes P in place)
+  contract(c, 1.0, t1, "ic", ovvv, "jbca", 1.0, P, "ijab");          // T1 x (ia|cb)
+  // Y[i,j,a,k], the part of P that T1 completes as -Y[i,j,a,k] t1[k,b]: (ka|ij) terms here, the ladder's below
+  Buf bY = dalloc(c, o * o * v * o);
+  TView Y = tv(bY, {o, o, v, o});
+  perm(c, ooov, "jkia", Y, "ijak", 1.0, 0.0);
+  contract(c, 1.0, t1, "ic", oovv, "kjac", 1.0, Y, "ijak");
+  contract(c, 1.0, ovov, "kcia", t1, "jc", 1.0, Y, "ijak");
   {
     // Woooo[k,l,i,j] = (ki|lj) + (ki|lc) t1[j,c] + (lj|kc) t1[i,c] + (kc|ld) tau[i,j,c,d]
     Buf bw = dalloc(c, o * o * o * o);
@@ -585,7 +604,7 @@ static void residual(Ctx& c, const double* t1p, const double* t2p, double* R1, d
     contract(c, 0.5, W, "klij", tau, "klab", 1.0, P, "ijab");
   }
   // particle-particle ladder sum_cd tau[i,j,c,d] ((ca|db) - (kd|ac) t1[k,b] - (kc|bd) t1[k,a]): the first part over
-  // packed pairs (prepare_ladder), the others as P -= (tau[i,j,c,d] (kd|ac)) t1[k,b]
+  // packed pairs (prepare_ladder), the others as Y += tau[i,j,c,d] (kd|ac)
   Buf bS = dalloc(c, 2 * mp * np);
   {
     const double fl = 4.0 * (double)mp * (double)np * (double)np;
@@ -593,7 +612,7 @@ static void residual(Ctx& c, const double* t1p, const double* t2p, double* R1, d
       c.Vs32 = Buf(c.pool.get(), (size_t)(2 * ldv * np) * sizeof(float));
       cast_f64_to_f32(c.s, 2 * ldv * np, c.Vs.d(), c.Vs32.f());
     }
-    const int64_t wl = c.lowp == 2 ? 0 : gemm_splitk_elems(mp, np, np, 2);
+    const int64_t wl = c.lowp == 2 ? gemm_bf3_splitk_elems(false, false, mp, np, np, 2, 1) : gemm_splitk_elems(mp, np, np, 2);
     Buf work;
     if (wl) work = dalloc(c, wl);
     Timer tl(c, c.lowp == 2 ? "ladder_bf16x3" : (c.lowp ? "ladder_fp32" : "ladder"), fl);
@@ -602,7 +621,7 @@ static void residual(Ctx& c, const double* t1p, const double* t2p, double* R1, d
                bS.d(), mp, mp * np, 2, /*tag: PP ladder*/ 1, work.d(), wl);
     else if (c.lowp == 2)
       gemm_bf3(c.s, false, false, mp, np, np, 1.0, bpair.f(), mp, mp * np, c.Vs32.f(), ldv, ldv * np, 0.0, nullptr, 0,
-               bS.d(), mp, mp * np, 2, 1);
+               bS.d(), mp, mp * np, 2, 1, work.d(), wl);
     else
       gemm_f32_fd(c.s, mp, np, np, 1.0, bpair.f(), mp, mp * np, c.Vs32.f(), ldv, ldv * np, 0.0, nullptr, 0, bS.d(), mp,
                   mp * np, 2, 1, work.d(), wl);
@@ -610,11 +629,17 @@ static void residual(Ctx& c, const double* t1p, const double* t2p, double* R1, d
   bpair.reset();
   {
     Timer tl(c, "ladder_t1", 2.0 * (double)n2 * (double)ov + 2.0 * (double)n2 * o_);
-    Buf bk = dalloc(c, o * o * v * o);
-    contract(c, 1.0, tau, "ijcd", tv(c.Pt.d(), {v, v, v, o}), "cdak", 0.0, tv(bk, {o, o, v, o}), "ijak");
-    contract(c, -1.0, tv(bk, {o, o, v, o}), "ijak", t1, "kb", 1.0, P, "ijab");
+    contract(c, 1.0, tau, "ijcd", tv(c.Pt.d(), {v, v, v, o}), "cdak", 1.0, Y, "ijak");
+    contract(c, -1.0, Y, "ijak", t1, "kb", 1.0, P, "ijab");
   }
-  contract(c, 1.0, Lvv, "ac", t2, "ijcb", 1.0, P, "ijab");
+  // Lvv[a,c] t2[i,j,c,b]: a product for each b
+  {
+    const int64_t wl = gemm_splitk_elems(o * o, v, v, v);
+    Buf work;
+    if (wl) work = dalloc(c, wl);
+    gemm_f64(c.s, false, true, o * o, v, v, 1.0, t2p, o * o, o * o * v, Lvv.p, v, 0, 1.0, P.p, o * o, o * o * v, P.p, o * o,
+             o * o * v, v, 0, work.d(), wl, c.lowp != 0);
+  }
   contract(c, -1.0, Loo, "ki", t2, "kjab", 1.0, P, "ijab");
   // Rings.  With A = Wvoov[i,a,k,c] and B = Wvovo[i,a,k,c] (operators of the ring and crossed ring) the three
   // applications A u - B t2 - (crossed) B t2 are
@@ -628,18 +653,18 @@ static void residual(Ctx& c, const double* t1p, const double* t2p, double* R1, d
     TView Cw = tv(bW.d(), {o, v, o, v}), Bw = tv(bW.d() + n2, {o, v, o, v});
     perm(c, oovv, "kiac", Bw, "iakc", 1.0, 0.0);
     contract(c, 1.0, t1, "id", ovvv, "kdac", 1.0, Bw, "iakc");
-    TView Y = tv(bXX, {o, o, o, v});
-    // Y[k,i,l,c] = (ki|lc) + (lc|kd) t1[i,d]
-    perm(c, ooov, "kilc", Y, "kilc", 1.0, 0.0);
-    contract(c, 1.0, ovov, "lckd", t1, "id", 1.0, Y, "kilc");
-    contract(c, -1.0, Y, "kilc", t1, "la", 1.0, Bw, "iakc");
+    TView Z = tv(bXX, {o, o, o, v});
+    // Z[k,i,l,c] = (ki|lc) + (lc|kd) t1[i,d]
+    perm(c, ooov, "kilc", Z, "kilc", 1.0, 0.0);
+    contract(c, 1.0, ovov, "lckd", t1, "id", 1.0, Z, "kilc");
+    contract(c, -1.0, Z, "kilc", t1, "la", 1.0, Bw, "iakc");
     // C = 2 A - B: 2 (ia|kc) + 2 (kc|ad) t1[i,d] - 2 ((li|kc) + (ld|kc) t1[i,d]) t1[l,a] - B
     d2d(c, Cw.p, Bw.p, n2);
     axpby_f64(c.s, n2, 2.0, c.OVOV.d(), -1.0, Cw.p);
     contract(c, 2.0, t1, "id", ovvv, "kcad", 1.0, Cw, "iakc");
-    perm(c, ooov, "likc", Y, "likc", 1.0, 0.0);
-    contract(c, 1.0, ovov, "ldkc", t1, "id", 1.0, Y, "likc");
-    contract(c, -2.0, Y, "likc", t1, "la", 1.0, Cw, "iakc");
+    perm(c, ooov, "likc", Z, "likc", 1.0, 0.0);
+    contract(c, 1.0, ovov, "ldkc", t1, "id", 1.0, Z, "likc");
+    contract(c, -2.0, Z, "likc", t1, "la", 1.0, Cw, "iakc");
     // [C | B] += 1/2 [u | -t2[ilda]] [L | (lc|kd)], then [D | F] = [C | B] [u | -t2[kjbc]]
     if (ring32) {
       if (!c.LX32.p) {

@@ -322,6 +322,11 @@ static void splitk_reduce(hipStream_t s, int64_t M, int64_t N, int64_t S, const 
   FH_HIP(hipGetLastError());
 }
 
+void splitk_reduce_f64(hipStream_t s, int64_t M, int64_t N, int64_t S, const double* W, double alpha, double beta,
+                       const double* C, int64_t ldc, int64_t sC, double* D, int64_t ldd, int64_t sD, int64_t batch) {
+  splitk_reduce<double>(s, M, N, S, W, alpha, beta, C, ldc, sC, D, ldd, sD, batch);
+}
+
 static void check_args(int64_t M, int64_t K, int64_t N, bool ta, bool tb, int64_t lda, int64_t ldb, int64_t ldd,
                        double beta, const void* C, int64_t ldc) {
   FH_CHECK(K >= 0, -3, "gemm: negative K");

@@ -9,16 +9,16 @@
 // for higher-precision computations", ARITH 2019).  Three v_mfma_f32_32x32x16_bf16 issue in the
 // time of 3/16 of the FP32 MFMA work of the same tile.
 //
-// Workgroup: 256 threads = 4 wavefronts (2x2), BM x 128 output tile (BM = 128, or 256 for long-K
-// untransposed GEMMs), K staged BK = 32 (two workgroups per CU) or 16 (three per CU, short K; two
-// for BM = 256) at a time through double-buffered LDS (hi and lo planes of both operands).
+// Workgroup: 256 threads = 4 wavefronts (2x2), BM x 128 output tile (BM = 128, three workgroups per
+// CU, or 256 for large untransposed GEMMs, two), K staged BK = 16 at a time through double-buffered
+// LDS (hi and lo planes of both operands).
 // Each wavefront owns BM/2 x 64 as 32x32 accumulator blocks.  The MFMA is issued with the B tile
 // as its first operand, so the accumulator's lane index runs along the rows of D (the output's
 // unit-stride axis).  The (T) W build has kernels of its own (fh_triples.hip).
 //
-// Global loads: k-contiguous operands load four consecutive k per thread (dwordx4 for FP32) when
-// the leading dimensions, batch strides and base addresses allow it (VEC), scalar loads
-// otherwise; row-contiguous operands load one element per (row, k), coalesced across lanes.  The
+// Global loads: k-contiguous operands load four consecutive k per thread (one dwordx4, which needs
+// the alignment of an element only); row-contiguous operands load one element per (row, k), coalesced
+// across lanes.  The
 // loads are branch-free (clamped rows, masks applied at the LDS store).  Tile order: the
 // XCD-aware remap and the L2-grouped raster of the FP64/FP32 kernel.
 #include "fh_internal.h"
@@ -94,24 +94,10 @@ __device__ __forceinline__ void for_blocks(F&& f) {
   else if constexpr (I + 1 < MI) for_blocks<I + 1, 0, MI, NJ>(f);
 }
 
-template <typename TI, bool VEC>
-__device__ inline V4 load4(const TI* p, bool full, int n_ok) {
-  V4 v;
-  if constexpr (VEC) {
-    if (full) {
-      if constexpr (std::is_same<TI, float>::value) {
-        const float4 q = *reinterpret_cast<const float4*>(p);
-        v.x[0] = q.x; v.x[1] = q.y; v.x[2] = q.z; v.x[3] = q.w;
-      } else {
-        const double2 q0 = reinterpret_cast<const double2*>(p)[0], q1 = reinterpret_cast<const double2*>(p)[1];
-        v.x[0] = (float)q0.x; v.x[1] = (float)q0.y; v.x[2] = (float)q1.x; v.x[3] = (float)q1.y;
-      }
-      return v;
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) v.x[i] = i < n_ok ? (float)p[i] : 0.0f;
-  return v;
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ inline V4 load4(const float* p) {
+  const f32x4u q = *reinterpret_cast<const f32x4u*>(p);
+  return V4{{q[0], q[1], q[2], q[3]}};
 }
 
 }  // namespace
@@ -119,14 +105,13 @@ __device__ inline V4 load4(const TI* p, bool full, int n_ok) {
 // Operand tile layout in LDS: plane[row][k] (k fastest, BK + 8 bf16 per row: 16 bytes of padding),
 // row = m for A, n for B.  "row-contiguous" operands (A with TA = false, B with TB = true) are
 // read 4 rows x BK/8 k per thread and transposed in registers; "k-contiguous" operands are read
-// 4 k of one row per load.  BK = 32 (two workgroups per CU) for long K, BK = 16 (three per CU,
-// more overlap of one tile's epilogue with another's loop) for short K.
-template <int BK, bool TA, bool TB, int TAG, typename TI, typename TO, bool VEC, int BM>
-__global__ __launch_bounds__(256, (BK == 16 && BM == 128) ? 3 : 2) void k_gemm_bf3(int64_t M, int64_t N, int64_t K, double alpha,
+// 4 k of one row per load.
+template <int BK, bool TA, bool TB, int TAG, typename TI, typename TO, int BM>
+__global__ __launch_bounds__(256, BM == 128 ? 3 : 2) void k_gemm_bf3(int64_t M, int64_t N, int64_t K, double alpha,
                                                      const TI* __restrict__ A, int64_t lda, int64_t sA,
                                                      const TI* __restrict__ B, int64_t ldb, int64_t sB, double beta,
                                                      const TO* C, int64_t ldc, int64_t sC, TO* D, int64_t ldd,
-                                                     int64_t sD, int tilesM, int tilesN, int gn) {
+                                                     int64_t sD, int tilesM, int tilesN, int64_t kchunk, int gn) {
   constexpr int BN = 128;        // tile width
   constexpr int kRow = BK + 8;   // LDS row (bf16)
   constexpr int KG = BK / 8;      // k per thread (row-contiguous) = loads per thread (both patterns)
@@ -163,11 +148,18 @@ __global__ __launch_bounds__(256, (BK == 16 && BM == 128) ? 3 : 2) void k_gemm_b
     nt = g * gn + rem % wdt;
   }
   const int64_t m0 = mt * BM, n0 = nt * BN;
-  const int64_t bz = blockIdx.y;
+  const int64_t bz = blockIdx.y, kz = blockIdx.z;
   A += bz * sA;
   B += bz * sB;
+  if (kchunk > 0) {
+    // split-K: slice kz covers k in [kz*kchunk, min(K, (kz+1)*kchunk)) and writes its own D slice
+    const int64_t kb = kz * kchunk;
+    K = (K - kb < kchunk) ? K - kb : kchunk;
+    A += TA ? kb : lda * kb;
+    B += TB ? ldb * kb : kb;
+  }
   if (C) C += bz * sC;
-  D += bz * sD;
+  D += (kz * gridDim.y + bz) * sD;
   auto aptr = [&](int64_t gm, int64_t gk) { return TA ? A + gk + lda * gm : A + gm + lda * gk; };
   auto bptr = [&](int64_t gn_, int64_t gk) { return TB ? B + gn_ + ldb * gk : B + gk + ldb * gn_; };
 
@@ -185,18 +177,12 @@ __global__ __launch_bounds__(256, (BK == 16 && BM == 128) ? 3 : 2) void k_gemm_b
   auto keep = [](float x, bool in) { return __uint_as_float(__float_as_uint(x) & (in ? 0xffffffffu : 0u)); };
   auto ld1 = [&](const TI* p, bool in) { return keep((float)*p, in); };
   // 4 consecutive k of row/column r of an operand, k-contiguous (p at k gk; rin: row inside)
-  auto ld4 = [&](auto ptr, int64_t r, bool rin, int64_t gk, bool kfull) {
+  auto ld4 = [&](auto ptr, int64_t r, bool rin, int64_t gk) {
     V4 v;
-    if (VEC && kfull) {
-      const V4 q = load4<TI, VEC>(ptr(rin ? r : 0, gk), true, 4);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v.x[e] = keep(q.x[e], rin);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const bool in = rin && gk + e < K;
-        v.x[e] = ld1(ptr(in ? r : 0, in ? gk + e : 0), in);
-      }
+    for (int e = 0; e < 4; ++e) {
+      const bool in = rin && gk + e < K;
+      v.x[e] = ld1(ptr(in ? r : 0, in ? gk + e : 0), in);
     }
     return v;
   };
@@ -256,7 +242,7 @@ __global__ __launch_bounds__(256, (BK == 16 && BM == 128) ? 3 : 2) void k_gemm_b
     } else {
       const int64_t gk = k0 + 4 * (tid % KQ);
 #pragma unroll
-      for (int j = 0; j < KG; ++j) ra[j] = load4<TI, VEC>(A + aoff[j] + gk, true, 4);
+      for (int j = 0; j < KG; ++j) ra[j] = load4(A + aoff[j] + gk);
     }
     if (TB) {
 #pragma unroll
@@ -269,7 +255,7 @@ __global__ __launch_bounds__(256, (BK == 16 && BM == 128) ? 3 : 2) void k_gemm_b
     } else {
       const int64_t gk = k0 + 4 * (tid % KQ);
 #pragma unroll
-      for (int j = 0; j < LB; ++j) rb[j] = load4<TI, VEC>(B + boff[j] + gk, true, 4);
+      for (int j = 0; j < LB; ++j) rb[j] = load4(B + boff[j] + gk);
     }
   };
   // the last, partial k tile: every element checked
@@ -288,7 +274,7 @@ __global__ __launch_bounds__(256, (BK == 16 && BM == 128) ? 3 : 2) void k_gemm_b
 #pragma unroll
       for (int j = 0; j < KG; ++j) {
         const int64_t gm = m0 + tid / KQ + RS * j;
-        ra[j] = ld4(aptr, gm, gm < M, gk, false);
+        ra[j] = ld4(aptr, gm, gm < M, gk);
       }
     }
     if (TB) {
@@ -305,7 +291,7 @@ __global__ __launch_bounds__(256, (BK == 16 && BM == 128) ? 3 : 2) void k_gemm_b
 #pragma unroll
       for (int j = 0; j < LB; ++j) {
         const int64_t gcol = n0 + tid / KQ + RS * j;
-        rb[j] = ld4(bptr, gcol, gcol < N, gk, false);
+        rb[j] = ld4(bptr, gcol, gcol < N, gk);
       }
     }
   };
@@ -445,51 +431,52 @@ __global__ __launch_bounds__(256, (BK == 16 && BM == 128) ? 3 : 2) void k_gemm_b
 // L2 budget of the B blocks of one raster group (bytes; 1, 4 and 16 MB measured alike)
 static constexpr int64_t kGroupBytesBf3 = 1 << 20;
 
-template <typename TI>
-static bool aligned4(const TI* p, int64_t ld, int64_t stride) {
-  return ((uintptr_t)p % (4 * sizeof(TI))) == 0 && ld % 4 == 0 && stride % 4 == 0;
+// Tile height: 256 (each wavefront 128 rows: fewer LDS fragment reads and operand bytes per MFMA) for the PP ladder
+// (272 vs 241 TFLOP/s at o = 40, v = 190) and for other NN GEMMs with M >= 1024 (the o^3 v^3 ring contractions of the
+// residual, K = o v: 188 against 174 TFLOP/s at o = 40, v = 190), where two workgroups a CU are there to run; 128
+// otherwise (the ladder at o = 28, v = 133, 140 tiles of 256 726 us, 560 of 128 704).  FERMIHIP_BF3_LBM / _CBM = 128 or 256 fix it for
+// tags 1 / 0 (tuning).  Under 384 tiles of 128, K is cut into slices of at least 512 towards three workgroups a CU
+// ((784, 3724, 17689), 210 tiles: 1.04 ms uncut, 0.49 ms in three slices).
+struct Bf3Plan {
+  int bm;
+  int64_t slices;
+};
+static Bf3Plan bf3_plan(bool ta, bool tb, int tag, int64_t M, int64_t N, int64_t K, int64_t batch) {
+  const bool can = !ta && !tb && (tag == 1 || M >= 1024);
+  const int64_t tn = (N + 127) / 128;
+  int bm = can && (M + 255) / 256 * tn * batch >= 512 ? 256 : 128;
+  if (const char* env = std::getenv(tag == 1 ? "FERMIHIP_BF3_LBM" : "FERMIHIP_BF3_CBM"))
+    bm = std::atoi(env) == 256 && can ? 256 : 128;
+  const int64_t tiles = (M + bm - 1) / bm * tn * batch;
+  const int64_t sl = bm == 256 || tiles >= 384 ? 1 : std::min<int64_t>(768 / tiles, K / 512);
+  return {bm, std::max<int64_t>(1, sl)};
+}
+int64_t gemm_bf3_splitk_elems(bool ta, bool tb, int64_t M, int64_t N, int64_t K, int64_t batch, int tag) {
+  if (M <= 0 || N <= 0 || batch <= 0) return 0;
+  const int64_t sl = bf3_plan(ta, tb, tag, M, N, K, batch).slices;
+  return sl > 1 ? sl * M * N * batch : 0;
 }
 
 template <bool TA, bool TB, int TAG, typename TI, typename TO>
-static void launch_bf3(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const TI* A, int64_t lda,
+static void launch_bf3(hipStream_t s, int bm, int64_t M, int64_t N, int64_t K, double alpha, const TI* A, int64_t lda,
                        int64_t sA, const TI* B, int64_t ldb, int64_t sB, double beta, const TO* C, int64_t ldc,
-                       int64_t sC, TO* D, int64_t ldd, int64_t sD, int64_t batch) {
-  // tile height: 128, or 256 (each wavefront 128 rows: fewer LDS fragment reads and operand bytes per
-  // MFMA) for the PP ladder (272 vs 241 TFLOP/s at o = 40, v = 190) and for tag 0 NN GEMMs with
-  // M >= 1024 (the o^3 v^3 ring contractions of the residual, K = o v: 188 against 174 TFLOP/s at
-  // o = 40, v = 190).  FERMIHIP_BF3_LBM / _CBM = 128 or 256 fix it for tags 1 / 0 (tuning)
-  constexpr int bn = 128;
-  const bool nn_big = !TA && !TB && M >= 1024;
-  int bm = (TAG == 1 || (TAG == 0 && nn_big)) ? 256 : 128;
-  if (const char* env = std::getenv(TAG == 1 ? "FERMIHIP_BF3_LBM" : "FERMIHIP_BF3_CBM"))
-    bm = (std::atoi(env) == 256 && (TAG != 0 || nn_big)) ? 256 : 128;
-  const int64_t tm = (M + bm - 1) / bm, tn = (N + bn - 1) / bn;
+                       int64_t sC, TO* D, int64_t ldd, int64_t sD, int64_t batch, int64_t kchunk) {
+  const int64_t tm = (M + bm - 1) / bm, tn = (N + 127) / 128;
   FH_CHECK(tm * tn < (int64_t)1 << 31 && batch < 65536, -3, "gemm grid too large");
   FH_CHECK(M < ((int64_t)1 << 31) && N < ((int64_t)1 << 31), -3, "gemm: M and N must be below 2^31");
-  dim3 grid((unsigned)(tm * tn), (unsigned)batch);
+  dim3 grid((unsigned)(tm * tn), (unsigned)batch, (unsigned)(kchunk > 0 ? (K + kchunk - 1) / kchunk : 1));
   int gn = 0;
   if (M > N) {
-    const int64_t per = std::max<int64_t>(1, K * bn * (int64_t)sizeof(TI));
+    const int64_t per = std::max<int64_t>(1, (kchunk > 0 ? kchunk : K) * 128 * (int64_t)sizeof(TI));
     gn = (int)std::max<int64_t>(1, std::min<int64_t>(tn, kGroupBytesBf3 / per));
   }
-  const bool vec = aligned4(A, lda, batch > 1 ? sA : 0) && aligned4(B, ldb, batch > 1 ? sB : 0);
-#define FH_BF3_GO(BK_, V_, BM_)                                                                                     \
-  hipLaunchKernelGGL((k_gemm_bf3<BK_, TA, TB, TAG, TI, TO, V_, BM_>), grid, dim3(256), 0, s, M, N, K, alpha, A, lda, \
-                     sA, B, ldb, sB, beta, C, ldc, sC, D, ldd, sD, (int)tm, (int)tn, gn)
-  // BK = 16 (three workgroups per CU) for the contractions (tag 0; the o^3 v^3 ring GEMMs, K = o v,
-  // measured 3% faster than BK = 32) and short K; BK = 32 for the long-K PP ladder (tag 1, 5% faster);
-  // 256-row tiles stage BK = 16 (two workgroups per CU)
+#define FH_BF3_GO(BM_)                                                                                              \
+  hipLaunchKernelGGL((k_gemm_bf3<16, TA, TB, TAG, TI, TO, BM_>), grid, dim3(256), 0, s, M, N, K, alpha, A, lda, sA, B, \
+                     ldb, sB, beta, C, ldc, sC, D, ldd, sD, (int)tm, (int)tn, kchunk, gn)
   if constexpr (!TA && !TB) {
-    if (bm == 256) {
-      if (vec) FH_BF3_GO(16, true, 256); else FH_BF3_GO(16, false, 256);
-      FH_HIP(hipGetLastError());
-      return;
-    }
-  }
-  if (TAG == 0 || K <= 512) {
-    if (vec) FH_BF3_GO(16, true, 128); else FH_BF3_GO(16, false, 128);
-  } else if constexpr (TAG != 0) {
-    if (vec) FH_BF3_GO(32, true, 128); else FH_BF3_GO(32, false, 128);
+    if (bm == 256) FH_BF3_GO(256); else FH_BF3_GO(128);
+  } else {
+    FH_BF3_GO(128);
   }
 #undef FH_BF3_GO
   FH_HIP(hipGetLastError());
@@ -497,16 +484,21 @@ static void launch_bf3(hipStream_t s, int64_t M, int64_t N, int64_t K, double al
 
 void gemm_bf3(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, double alpha, const float* A,
               int64_t lda, int64_t sA, const float* B, int64_t ldb, int64_t sB, double beta, const double* C, int64_t ldc,
-              double* D, int64_t ldd, int64_t sD, int64_t batch, int tag) {
+              double* D, int64_t ldd, int64_t sD, int64_t batch, int tag, double* work, int64_t work_elems) {
   if (M <= 0 || N <= 0 || batch <= 0) return;
   FH_CHECK(K >= 0, -3, "gemm: negative K");
   FH_CHECK(lda >= (ta ? (K > 0 ? K : 1) : M) && ldb >= (tb ? N : (K > 0 ? K : 1)) && ldd >= M, -3,
            "gemm: leading dimension too small");
   FH_CHECK(beta == 0.0 || (C != nullptr && ldc >= M), -3, "gemm: C missing");
-#define FH_BF3(TA_, TB_, TAG_) \
-  launch_bf3<TA_, TB_, TAG_, float, double>(s, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sD, D, ldd, sD, batch)
+  FH_CHECK(tag != 1 || (!ta && !tb), -3, "gemm_bf3: the PP ladder (tag 1) takes untransposed operands");
+  const Bf3Plan plan = bf3_plan(ta, tb, tag, M, N, K, batch);
+  const bool split = plan.slices > 1 && work != nullptr && work_elems >= plan.slices * M * N * batch;
+  const int64_t kchunk = split ? (K + plan.slices - 1) / plan.slices : 0;
+#define FH_BF3(TA_, TB_, TAG_)                                                                                       \
+  launch_bf3<TA_, TB_, TAG_, float, double>(s, plan.bm, M, N, K, split ? 1.0 : alpha, A, lda, sA, B, ldb, sB,        \
+                                            split ? 0.0 : beta, split ? nullptr : C, ldc, sD, split ? work : D,      \
+                                            split ? M : ldd, split ? M * N : sD, batch, kchunk)
   if (tag == 1) {
-    FH_CHECK(!ta && !tb, -3, "gemm_bf3: the PP ladder (tag 1) takes untransposed operands");
     FH_BF3(false, false, 1);
   } else if (ta) {
     if (tb) FH_BF3(true, true, 0); else FH_BF3(true, false, 0);
@@ -514,6 +506,8 @@ void gemm_bf3(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, 
     if (tb) FH_BF3(false, true, 0); else FH_BF3(false, false, 0);
   }
 #undef FH_BF3
+  if (split)
+    splitk_reduce_f64(s, M, N, (K + kchunk - 1) / kchunk, work, alpha, beta, C, ldc, sD, D, ldd, sD, batch);
 }
 
 }  // namespace fh

@@ -108,7 +108,13 @@ void gemm_f32(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, 
 // output: tag 0 any transposition, tag 1 (the PP ladder) untransposed; the tags give distinct kernel symbols
 void gemm_bf3(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, double alpha, const float* A,
               int64_t lda, int64_t sA, const float* B, int64_t ldb, int64_t sB, double beta, const double* C, int64_t ldc,
-              double* D, int64_t ldd, int64_t sD, int64_t batch, int tag);  // (C strided as D)
+              double* D, int64_t ldd, int64_t sD, int64_t batch, int tag, double* work = nullptr,
+              int64_t work_elems = 0);
+// its workspace (doubles) to split K for this shape (0: no split)
+int64_t gemm_bf3_splitk_elems(bool ta, bool tb, int64_t M, int64_t N, int64_t K, int64_t batch, int tag);
+// D = alpha sum_s W_s + beta C over the S slices W [M N][batch][S] of a product cut along K
+void splitk_reduce_f64(hipStream_t s, int64_t M, int64_t N, int64_t S, const double* W, double alpha, double beta,
+                       const double* C, int64_t ldc, int64_t sC, double* D, int64_t ldd, int64_t sD, int64_t batch);
 
 // ---------------------------------------------------------------- (T) W build (fh_triples.hip)
 // fmt: 0 FP64, 1 FP32, 2 split-BF16x3 (W in FP32).  Operands hold triples_pitch_elems(o, v) values of k per
