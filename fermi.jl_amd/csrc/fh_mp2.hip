@@ -5,10 +5,9 @@
 // whole o v x o v matrix.  The partner of an off-diagonal tile is computed transposed (B_j rows a, B_i rows b), so that
 // X[a,b] and X[b,a] meet in the same register of the same lane; a diagonal tile is its own partner, through LDS.
 //
-// Bound by the FP64 matrix pipes: o = 40, v = 190, Q = 840 (50 GFLOP) 1.2 ms, 42 TFLOP/s, against 2.7 ms for the GEMM of
+// Bound by the FP64 matrix pipes: o = 40, v = 190, Q = 840 (50 GFLOP) 1.04 ms, 48 TFLOP/s, against 2.7 ms for the GEMM of
 // the whole matrix, its (ia|jb) of 462 MB and a pass that reduced them (2.0 ms with the GEMM's present kernel);
-// o = 5, v = 19 38 us against 50.  With XCDs on contiguous ranges of tiles instead of every eighth block of pairs,
-// half of them had two products a tile and half one: 1.5 ms.
+// o = 5, v = 19 38 us against 50.
 #include "fh_internal.h"
 
 #include <algorithm>
@@ -19,7 +18,6 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef double f64x2 __attribute__((ext_vector_type(2)));
 typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));
 
-constexpr int kPB = 8;                    // orbital pairs run in kPB x kPB blocks: neighbours share both operands' rows
 constexpr int64_t kMaxBlocks = 16384;
 
 // index of the triangle x <= y, y (y + 1) / 2 + x, and back
@@ -35,7 +33,7 @@ __device__ inline void untri(int64_t q, int64_t& x, int64_t& y) {
 template <int BT, int BK>
 __global__ __launch_bounds__(256, BT == 64 ? 3 : 4) void k_mp2(int o, int v, int Q, const double* __restrict__ B,
                                                 const double* __restrict__ eo, const double* __restrict__ ev,
-                                                int64_t nitem, int64_t nbp, double* __restrict__ partials) {
+                                                int64_t nitem, double* __restrict__ partials) {
   constexpr int WB = BT / 32, KS = BK + 2, LD = BT * BK / 512;
   static_assert(4 * BT * KS >= BT * (BT + 1), "the diagonal tile fits the operand buffers");
   __shared__ __attribute__((aligned(16))) double lds[4 * BT * KS];
@@ -120,16 +118,10 @@ __global__ __launch_bounds__(256, BT == 64 ? 3 : 4) void k_mp2(int o, int v, int
   };
 
   double e = 0.0;
-  // XCD-aware order: consecutive workgroups land on different XCDs, and each XCD takes every eighth block of pairs, so
-  // that its L2 holds the rows that the block shares and all of them get as many tiles of two products as of one
-  constexpr int kB2 = kPB * kPB;
   for (int64_t it = blockIdx.x; it < nitem; it += gridDim.x) {
-    const int64_t blk = (it >> 3) / kB2 * 8 + (it & 7), rem = (it >> 3) % kB2, tp = blk / nbp;
-    if (tp >= tri(nt)) continue;
-    int64_t ib, jb, ta, tb;
-    untri(blk % nbp, ib, jb);
-    const int i = (int)(ib * kPB + rem % kPB), j = (int)(jb * kPB + rem / kPB);
-    if (j >= o || i > j) continue;
+    const int64_t tp = it / tri(o);
+    int64_t i, j, ta, tb;
+    untri(it % tri(o), i, j);
     // off-diagonal tiles (two products) first
     if (tp < noff) {
       untri(tp, ta, tb);
@@ -189,23 +181,29 @@ __global__ __launch_bounds__(256, BT == 64 ? 3 : 4) void k_mp2(int o, int v, int
   if (tid == 0) partials[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
 }
 
-// 64 x 64 tiles; 32 x 32 with K steps of 32 where one of them covers X (v <= 32: o = 5, v = 19 is bound by the latency of
-// its 84 / 32 K steps)
-static int mp2_tile(int v) { return v <= 32 ? 32 : 64; }
-static int64_t mp2_items(int o, int v) {
-  const int64_t nt = (v + mp2_tile(v) - 1) / mp2_tile(v);
-  return (tri(nt) * tri((o + kPB - 1) / kPB) + 7) / 8 * 8 * kPB * kPB;
+// 64 x 64 tiles, or 32 x 32 with K steps of 32 where those would be too few to hide their latency, under some six a CU
+// (naux = 4.2 (o + v): o = 12, v = 70 52 us against 71, o = 20, v = 150 205 against 232, o = 40, v = 100 336 against 327).
+// The items go tile by tile over the pairs: in 8 x 8 blocks of pairs an XCD (its L2 to share their rows) o = 40,
+// v = 190 took 1.32 ms, 1.18 so, and few blocks left XCDs idle (o = 20, v = 100: 167 us, 114 so).
+struct Mp2Plan {
+  int tile;
+  int64_t items;
+};
+static Mp2Plan mp2_plan(int o, int v) {
+  const int64_t n64 = tri((v + 63) / 64) * tri(o);
+  if (v <= 32 || n64 < 1400) return {32, tri((v + 31) / 32) * tri(o)};
+  return {64, n64};
 }
-int64_t mp2_partials(int o, int v) { return std::min(mp2_items(o, v), kMaxBlocks); }
+int64_t mp2_partials(int o, int v) { return std::min(mp2_plan(o, v).items, kMaxBlocks); }
 
 void mp2_pair_energy(hipStream_t s, int o, int v, int Q, const double* Bov, const double* eo, const double* ev,
                      double* partials) {
-  const int64_t n = mp2_items(o, v), nbp = tri((o + kPB - 1) / kPB);
-  const dim3 grid((unsigned)mp2_partials(o, v)), block(256);
-  if (mp2_tile(v) == 32)
-    hipLaunchKernelGGL((k_mp2<32, 32>), grid, block, 0, s, o, v, Q, Bov, eo, ev, n, nbp, partials);
+  const Mp2Plan p = mp2_plan(o, v);
+  const dim3 grid((unsigned)std::min(p.items, kMaxBlocks)), block(256);
+  if (p.tile == 32)
+    hipLaunchKernelGGL((k_mp2<32, 32>), grid, block, 0, s, o, v, Q, Bov, eo, ev, p.items, partials);
   else
-    hipLaunchKernelGGL((k_mp2<64, 16>), grid, block, 0, s, o, v, Q, Bov, eo, ev, n, nbp, partials);
+    hipLaunchKernelGGL((k_mp2<64, 16>), grid, block, 0, s, o, v, Q, Bov, eo, ev, p.items, partials);
   FH_HIP(hipGetLastError());
 }
 
