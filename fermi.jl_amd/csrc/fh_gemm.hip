@@ -191,7 +191,18 @@ __global__ __launch_bounds__(256, OCC) void k_gemm(
     col = n0 + wn * WN + j * 16 + (F32 ? 4 * (lane >> 4) + rr : (lane >> 4) + 4 * rr);
     return row < M && col < N;
   };
-  if (beta != 0.0) {
+  if constexpr (TAG == 4) {
+    // a network layer: D = tanh(A B + bias), the bias of a row in C
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) {
+          int64_t row, col;
+          if (at(i, j, rr, row, col)) D[row + ldd * col] = tanhf((float)acc[i][j][rr] + C[row]);
+        }
+  } else if (beta != 0.0) {
     TO cv[MB][NB][4];
 #pragma unroll
     for (int i = 0; i < MB; ++i)
@@ -415,6 +426,14 @@ void gemm_f32(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, 
   }
 #undef FH_F32
   if (split) splitk_reduce<float>(s, M, N, (K + kchunk - 1) / kchunk, work, alpha, beta, C, ldc, 0, C, ldc, 0, 1);
+}
+
+void gemm_f32_tanh(hipStream_t s, int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb,
+                   const float* bias, float* D, int64_t ldd) {
+  if (M <= 0 || N <= 0) return;
+  check_args(M, K, N, false, false, lda, ldb, ldd, 0.0, nullptr, 0);
+  pick<false, false, 4, true, float, float>(s, gemm_plan(M, N, K, 1).small, M, N, K, 1.0, A, lda, 0, B, ldb, 0, 0.0, bias,
+                                            0, 0, D, ldd, 0, 1, 0);
 }
 
 }  // namespace fh

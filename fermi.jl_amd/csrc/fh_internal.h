@@ -104,6 +104,9 @@ void gemm_f32_fd(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, c
 void gemm_f32(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, double alpha, const float* A,
               int64_t lda, const float* B, int64_t ldb, double beta, float* C, int64_t ldc, float* work = nullptr,
               int64_t work_elems = 0);
+// FP32 network layer: D = tanh(A B + bias[row]) (tag 4)
+void gemm_f32_tanh(hipStream_t s, int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb,
+                   const float* bias, float* D, int64_t ldd);
 // split-BF16x3 MFMA GEMM (three bf16 products per FP32 product, FP32 accumulation) on FP32 operands with FP64
 // output: tag 0 any transposition, tag 1 (the PP ladder) untransposed; the tags give distinct kernel symbols
 void gemm_bf3(hipStream_t s, bool ta, bool tb, int64_t M, int64_t N, int64_t K, double alpha, const float* A,

@@ -4,11 +4,11 @@
 // Parameter vector (FP32, flat): W1[h,6] b1[h] W2[h,h] b2[h] W3[h,h] b3[h] w4[h] b4, every W
 // column-major [out, in].  Activations of a batch of B samples are column-major [h, B] (the h
 // values of one sample contiguous), so every layer is one GEMM of the FP32-MFMA kernel
-//     Z_l = W_l A_{l-1}  (M = h, N = B, K = in)
-// followed by a fused bias + tanh pass; the backward pass is the transposed GEMMs
+//     A_l = tanh(W_l A_{l-1} + b_l)  (M = h, N = B, K = in)
+// with bias and tanh in its epilogue; the backward pass is the transposed GEMMs
 //     dW_l = dZ_l A_{l-1}^T,  dA_{l-1} = W_l^T dZ_l
-// plus column reductions for the bias gradients (deterministic two-stage sums) and a fused
-// tanh' pass.  Loss: L = 1/(2B) sum_s (y_s - t_s)^2.  Optimiser: Adam.
+// and one pass a layer that applies tanh' and sums dZ_l over the samples for the bias gradient
+// (deterministic two-stage sums).  Loss: L = 1/(2B) sum_s (y_s - t_s)^2.  Optimiser: Adam.
 //
 // Features of amplitude (i,j,a,b): T2_MP2[i,j,a,b], eps_i, eps_j, eps_a, eps_b, d_ij (occupied pair
 // distance), each standardised with the model's (mean, 1/scale); the network predicts
@@ -40,91 +40,108 @@ static unsigned grid1(int64_t n, int bs = 256) {
   return (unsigned)(b < 1 ? 1 : (b > 65536 ? 65536 : b));
 }
 
-// A[h,B] = tanh(A + b[row])
-__global__ void k_bias_tanh(int h, int64_t n, const float* __restrict__ b, float* __restrict__ A) {
-  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256)
-    A[e] = tanhf(A[e] + b[e % h]);
-}
-
 // y[s] += b4  (after y = w4^T A3 as a GEMM with M = 1)
 __global__ void k_add_scalar(int64_t n, const float* __restrict__ b, float* __restrict__ y) {
   for (int64_t s = (int64_t)blockIdx.x * 256 + threadIdx.x; s < n; s += (int64_t)gridDim.x * 256) y[s] += b[0];
 }
 
-// dZ3[r,s] = w4[r] dy[s] (1 - A3[r,s]^2), element order of [h,B] (coalesced)
-__global__ void k_out_dz(int h, int64_t n, const float* __restrict__ w4, const float* __restrict__ A3,
-                         const float* __restrict__ dy, float* __restrict__ dZ3) {
-  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
-    const float a = A3[e];
-    dZ3[e] = w4[e % h] * dy[e / h] * (1.0f - a * a);
-  }
-}
-
-// dy[s] = (y[s] - t[s]) / B;  per-block partial sums of (y - t)^2 / 2
-__global__ void k_out_back(int64_t B, const float* __restrict__ y, const float* __restrict__ t, float* __restrict__ dy,
-                           double* __restrict__ lpart) {
-  __shared__ double red[256];
-  double l = 0.0;
-  for (int64_t s = (int64_t)blockIdx.x * 256 + threadIdx.x; s < B; s += (int64_t)gridDim.x * 256) {
-    const float r = y[s] - t[s];
-    l += 0.5 * (double)r * (double)r;
-    dy[s] = r / (float)B;
-  }
-  red[threadIdx.x] = l;
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if ((int)threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) lpart[blockIdx.x] = red[0];
-}
-
-// dZ = dA * (1 - A^2)  (in place on dA)
-__global__ void k_tanh_back(int64_t n, const float* __restrict__ A, float* __restrict__ dA) {
-  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256)
-    dA[e] *= 1.0f - A[e] * A[e];
-}
-
-// partial row sums of M[h,B] (h divides 256): block b sums columns [b*cols, (b+1)*cols)
-__global__ void k_rowsum_part(int h, int64_t B, int64_t cols, const float* __restrict__ Mx, float* __restrict__ part) {
+// Row sums of a pass over [h, B] (h divides 256), cols columns a workgroup: a thread's row r = tid % h and its sum t ->
+// part[b h' + r] for the h' >= h rows of a partial
+__device__ inline void put_rowsum(int h, float t, float* __restrict__ part) {
   __shared__ float red[256];
-  const int lanes = 256 / h, r = threadIdx.x % h, c0 = threadIdx.x / h;
-  const int64_t beg = (int64_t)blockIdx.x * cols, end = beg + cols < B ? beg + cols : B;
-  float t = 0.0f;
-  for (int64_t c = beg + c0; c < end; c += lanes) t += Mx[r + (int64_t)h * c];
   red[threadIdx.x] = t;
   __syncthreads();
-  if (threadIdx.x < h) {
+  if ((int)threadIdx.x < h) {
     float u = 0.0f;
-    for (int q = 0; q < lanes; ++q) u += red[threadIdx.x + q * h];
-    part[(int64_t)blockIdx.x * h + threadIdx.x] = u;
+    for (int q = threadIdx.x; q < 256; q += h) u += red[q];
+    part[threadIdx.x] = u;
   }
 }
-// out[r] = sum_b part[b, r]: one workgroup a row
-__global__ __launch_bounds__(256) void k_rowsum_final(int h, int nb, const float* __restrict__ part,
-                                                      float* __restrict__ out) {
+
+// Output layer: dy[s] = (y[s] - t[s]) / B, dZ3[r,s] = w4[r] dy[s] (1 - A3[r,s]^2), the row sums of dZ3 and, as row h, of
+// dy into part[block][h + 1], and the sum of (y - t)^2 / 2 into lpart[block]
+__global__ __launch_bounds__(256) void k_out_back(int h, int64_t B, int64_t cols, const float* __restrict__ y,
+                                                  const float* __restrict__ t, const float* __restrict__ w4,
+                                                  const float* __restrict__ A3, float* __restrict__ dy,
+                                                  float* __restrict__ dZ3, float* __restrict__ part,
+                                                  double* __restrict__ lpart) {
+  __shared__ double red[256];
+  __shared__ float reds[256];
+  const int lanes = 256 / h, r = threadIdx.x % h, c0 = threadIdx.x / h;
+  const int64_t beg = (int64_t)blockIdx.x * cols, end = beg + cols < B ? beg + cols : B;
+  double l = 0.0;
+  float sd = 0.0f, sz = 0.0f;
+  for (int64_t s = beg + threadIdx.x; s < end; s += 256) {
+    const float d = y[s] - t[s];
+    l += 0.5 * (double)d * (double)d;
+    dy[s] = d / (float)B;
+    sd += d / (float)B;
+  }
+  const float w = w4[r];
+  for (int64_t s = beg + c0; s < end; s += lanes) {
+    const float a = A3[r + (int64_t)h * s], z = w * ((y[s] - t[s]) / (float)B) * (1.0f - a * a);
+    dZ3[r + (int64_t)h * s] = z;
+    sz += z;
+  }
+  put_rowsum(h, sz, part + (int64_t)blockIdx.x * (h + 1));
+  red[threadIdx.x] = l;
+  reds[threadIdx.x] = sd;
+  __syncthreads();
+  for (int st = 128; st > 0; st >>= 1) {
+    if ((int)threadIdx.x < st) {
+      red[threadIdx.x] += red[threadIdx.x + st];
+      reds[threadIdx.x] += reds[threadIdx.x + st];
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    lpart[blockIdx.x] = red[0];
+    part[(int64_t)blockIdx.x * (h + 1) + h] = reds[0];
+  }
+}
+
+// dZ = dA (1 - A^2) in place on dA, and its row sums into part[block][h]
+__global__ __launch_bounds__(256) void k_tanh_back(int h, int64_t B, int64_t cols, const float* __restrict__ A,
+                                                   float* __restrict__ dA, float* __restrict__ part) {
+  const int lanes = 256 / h, r = threadIdx.x % h, c0 = threadIdx.x / h;
+  const int64_t beg = (int64_t)blockIdx.x * cols, end = beg + cols < B ? beg + cols : B;
+  float sz = 0.0f;
+  for (int64_t s = beg + c0; s < end; s += lanes) {
+    const int64_t e = r + (int64_t)h * s;
+    const float z = dA[e] * (1.0f - A[e] * A[e]);
+    dA[e] = z;
+    sz += z;
+  }
+  put_rowsum(h, sz, part + (int64_t)blockIdx.x * h);
+}
+
+// out[r] = sum_b part[b, r], the last of rows h + 1 into out2: one workgroup a row
+__global__ __launch_bounds__(256) void k_rowsum_final(int rows, int nb, const float* __restrict__ part,
+                                                      float* __restrict__ out, float* __restrict__ out2) {
   __shared__ float red[256];
   const int r = blockIdx.x;
   float u = 0.0f;
-  for (int b = threadIdx.x; b < nb; b += 256) u += part[(int64_t)b * h + r];
+  for (int b = threadIdx.x; b < nb; b += 256) u += part[(int64_t)b * rows + r];
   red[threadIdx.x] = u;
   __syncthreads();
   for (int st = 128; st > 0; st >>= 1) {
     if ((int)threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[r] = red[0];
+  if (threadIdx.x == 0) {
+    if (out2 && r == rows - 1) *out2 = red[0];
+    else out[r] = red[0];
+  }
 }
 
-// Columns of one k_rowsum_part workgroup: 64 keep its chain of dependent adds at 32 for h = 128, and with up to 1024
-// workgroups the chip is full from B = 16 k on (h = 128, B = 8192: 345 us with 4096 columns a workgroup, 9 us so).
-static int64_t rowsum_cols(int64_t B) { return std::max<int64_t>(64, (B + 1023) / 1024); }
+// Columns of a workgroup of these passes: 16 keep its chain of dependent adds at 8 for h = 128, and with up to 1024
+// workgroups the chip is full from B = 16 k on (h = 128, B = 8192: a separate row sum took 345 us with 4096 columns a
+// workgroup and 9 us with 64, tanh' 4 us; 5 us together so).
+static int64_t rowsum_cols(int64_t B) { return std::max<int64_t>(16, (B + 1023) / 1024); }
 static int64_t rowsum_blocks(int64_t B) { return (B + rowsum_cols(B) - 1) / rowsum_cols(B); }
 
-static void rowsum(hipStream_t s, int h, int64_t B, const float* Mx, float* part, float* out) {
-  const int nb = (int)rowsum_blocks(B);
-  hipLaunchKernelGGL(k_rowsum_part, dim3(nb), dim3(256), 0, s, h, B, rowsum_cols(B), Mx, part);
-  hipLaunchKernelGGL(k_rowsum_final, dim3(h), dim3(256), 0, s, h, nb, part, out);
+static void rowsum_final(hipStream_t s, int rows, int64_t B, const float* part, float* out, float* out2 = nullptr) {
+  hipLaunchKernelGGL(k_rowsum_final, dim3(rows), dim3(256), 0, s, rows, (int)rowsum_blocks(B), part, out, out2);
   FH_HIP(hipGetLastError());
 }
 
@@ -137,20 +154,17 @@ static int64_t wgrad_elems(int h, int64_t B) {
 }
 
 int64_t mlp_partial_elems(int h, int64_t B) {
-  const int64_t blocks = std::min<int64_t>((B + 63) / 64, 1024);   // >= rowsum_blocks of every batch up to B
-  return std::max(blocks * std::max(h, 1) + 1024, wgrad_elems(h, B));
+  const int64_t blocks = std::min<int64_t>((B + 15) / 16, 1024);   // >= rowsum_blocks of every batch up to B
+  return blocks * (h + 1) + wgrad_elems(h, B);
 }
 
 void mlp_forward(hipStream_t s, int h, const float* P, int64_t B, const float* X, float* A1, float* A2, float* A3,
                  float* y) {
   FH_CHECK(h > 0 && 256 % h == 0, -1, "mlp: width must divide 256");
   const MlpOffsets o = mlp_offsets(h);
-  gemm_f32(s, false, false, h, B, 6, 1.0, P + o.W1, h, X, 6, 0.0, A1, h);
-  hipLaunchKernelGGL(k_bias_tanh, dim3(grid1(h * B)), dim3(256), 0, s, h, (int64_t)h * B, P + o.b1, A1);
-  gemm_f32(s, false, false, h, B, h, 1.0, P + o.W2, h, A1, h, 0.0, A2, h);
-  hipLaunchKernelGGL(k_bias_tanh, dim3(grid1(h * B)), dim3(256), 0, s, h, (int64_t)h * B, P + o.b2, A2);
-  gemm_f32(s, false, false, h, B, h, 1.0, P + o.W3, h, A2, h, 0.0, A3, h);
-  hipLaunchKernelGGL(k_bias_tanh, dim3(grid1(h * B)), dim3(256), 0, s, h, (int64_t)h * B, P + o.b3, A3);
+  gemm_f32_tanh(s, h, B, 6, P + o.W1, h, X, 6, P + o.b1, A1, h);
+  gemm_f32_tanh(s, h, B, h, P + o.W2, h, A1, h, P + o.b2, A2, h);
+  gemm_f32_tanh(s, h, B, h, P + o.W3, h, A2, h, P + o.b3, A3, h);
   gemm_f32(s, false, false, 1, B, h, 1.0, P + o.w4, 1, A3, h, 0.0, y, 1);
   hipLaunchKernelGGL(k_add_scalar, dim3(grid1(B)), dim3(256), 0, s, B, P + o.b4, y);
   FH_HIP(hipGetLastError());
@@ -160,28 +174,26 @@ void mlp_backward(hipStream_t s, int h, const float* P, int64_t B, const float* 
                   const float* A2, const float* A3, const float* y, float* dy, float* dA, float* dZ, float* G,
                   float* part, double* lpart, int64_t* nlpart) {
   const MlpOffsets o = mlp_offsets(h);
-  const unsigned gb = grid1(B);
-  const int64_t wl = wgrad_elems(h, B);
-  hipLaunchKernelGGL(k_out_back, dim3(gb), dim3(256), 0, s, B, y, T, dy, lpart);
-  *nlpart = gb;
-  hipLaunchKernelGGL(k_out_dz, dim3(grid1(h * B)), dim3(256), 0, s, h, (int64_t)h * B, P + o.w4, A3, dy, dZ);
-  // output layer: g w4 = A3 dy, g b4 = sum dy
-  gemm_f32(s, false, false, h, 1, B, 1.0, A3, h, dy, B, 0.0, G + o.w4, h, part, wl);
-  rowsum(s, 1, B, dy, part, G + o.b4);
+  const int64_t cols = rowsum_cols(B), wl = wgrad_elems(h, B);
+  const unsigned nb = (unsigned)rowsum_blocks(B);
+  float* work = part + std::min<int64_t>((B + 15) / 16, 1024) * (h + 1);   // behind the row sums
+  // output layer: dy, dZ3, g b3 and g b4 = sum dy; g w4 = A3 dy
+  hipLaunchKernelGGL(k_out_back, dim3(nb), dim3(256), 0, s, h, B, cols, y, T, P + o.w4, A3, dy, dZ, part, lpart);
+  *nlpart = nb;
+  rowsum_final(s, h + 1, B, part, G + o.b3, G + o.b4);
+  gemm_f32(s, false, false, h, 1, B, 1.0, A3, h, dy, B, 0.0, G + o.w4, h, work, wl);
   // layer 3
-  gemm_f32(s, false, true, h, h, B, 1.0, dZ, h, A2, h, 0.0, G + o.W3, h, part, wl);
-  rowsum(s, h, B, dZ, part, G + o.b3);
+  gemm_f32(s, false, true, h, h, B, 1.0, dZ, h, A2, h, 0.0, G + o.W3, h, work, wl);
   gemm_f32(s, true, false, h, B, h, 1.0, P + o.W3, h, dZ, h, 0.0, dA, h);
-  hipLaunchKernelGGL(k_tanh_back, dim3(grid1(h * B)), dim3(256), 0, s, (int64_t)h * B, A2, dA);
+  hipLaunchKernelGGL(k_tanh_back, dim3(nb), dim3(256), 0, s, h, B, cols, A2, dA, part);
+  rowsum_final(s, h, B, part, G + o.b2);
   // layer 2 (dA now holds dZ2)
-  gemm_f32(s, false, true, h, h, B, 1.0, dA, h, A1, h, 0.0, G + o.W2, h, part, wl);
-  rowsum(s, h, B, dA, part, G + o.b2);
+  gemm_f32(s, false, true, h, h, B, 1.0, dA, h, A1, h, 0.0, G + o.W2, h, work, wl);
   gemm_f32(s, true, false, h, B, h, 1.0, P + o.W2, h, dA, h, 0.0, dZ, h);
-  hipLaunchKernelGGL(k_tanh_back, dim3(grid1(h * B)), dim3(256), 0, s, (int64_t)h * B, A1, dZ);
+  hipLaunchKernelGGL(k_tanh_back, dim3(nb), dim3(256), 0, s, h, B, cols, A1, dZ, part);
+  rowsum_final(s, h, B, part, G + o.b1);
   // layer 1 (dZ holds dZ1)
-  gemm_f32(s, false, true, h, 6, B, 1.0, dZ, h, X, 6, 0.0, G + o.W1, h, part, wl);
-  rowsum(s, h, B, dZ, part, G + o.b1);
-  FH_HIP(hipGetLastError());
+  gemm_f32(s, false, true, h, 6, B, 1.0, dZ, h, X, 6, 0.0, G + o.W1, h, work, wl);
 }
 
 __global__ void k_adam(int64_t n, float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
