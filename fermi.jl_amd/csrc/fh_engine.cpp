@@ -133,6 +133,8 @@ struct Ctx {
   Buf LX, Vs, Pt, LX32, Vs32;
   // Lkl[k,l,c,d] = LX[k,c,l,d] and Okl[k,l,i,c] = (ki|lc): the slices of slice_sum
   Buf Lkl, Okl;
+  // what T1 multiplies: Lo1[l,c,k,i] = 2 (ki|lc) - (li|kc), L1[k,c,i,a] = 2 (kc|ia) - (ki|ac)
+  Buf Lo1, L1;
   // GEMM operands made from the integral blocks above (a permuted FP64 copy, or an FP32 copy for
   // split-BF16x3): the same for every CC iteration, so made once and kept, up to opcache_cap
   // bytes; key "<block>|<index order>|<d or f>"
@@ -259,6 +261,13 @@ static bool is_concat(const std::string& full, const std::string& first, const s
   return full == first + second;
 }
 
+// the integral blocks, whose copies contract() keeps
+static const char* block_name(const Ctx& c, const TView& X) {
+  return X.p == c.OVOV.d() ? "ovov" : X.p == c.OVVV.d() ? "ovvv" : X.p == c.OOOV.d() ? "ooov"
+         : X.p == c.OOVV.d() ? "oovv" : X.p == c.OOOO.d() ? "oooo" : X.p == c.LX.d() ? "Lovov"
+         : X.p == c.Pt.d() ? "Pt" : nullptr;
+}
+
 static void contract(Ctx& c, double alpha, const TView& A, const std::string& ia, const TView& B,
                      const std::string& ib, double beta, const TView& C, const std::string& ic) {
   FH_CHECK((int)ia.size() == A.nd && (int)ib.size() == B.nd && (int)ic.size() == C.nd, -3,
@@ -304,9 +313,11 @@ static void contract(Ctx& c, double alpha, const TView& A, const std::string& ia
   for (char ch : ib) if (K.find(ch) != std::string::npos) KB += ch;
   auto fitsA = [&](const std::string& k) { return is_concat(ia, M, k) || is_concat(ia, k, M); };
   auto fitsB = [&](const std::string& k) { return is_concat(ib, k, N) || is_concat(ib, N, k); };
+  // (a copy of an integral block is cached below, one of an amplitude made each time)
   std::string Kord = KA;
   if (!(fitsA(KA) && fitsB(KA)) && fitsA(KB) && fitsB(KB)) Kord = KB;
   else if (!fitsA(KA) && fitsB(KB)) Kord = KB;
+  else if (!fitsB(KA) && fitsB(KB) && block_name(c, A) && !block_name(c, B)) Kord = KB;
 
   int64_t Msz = 1, Nsz = 1, Ksz = 1;
   for (char ch : M) Msz *= LA.dim(ch);
@@ -327,9 +338,7 @@ static void contract(Ctx& c, double alpha, const TView& A, const std::string& ia
   auto operand = [&](const TView& X, const std::string& ix, bool ready, const std::string& layout, Buf& tmp,
                      Buf& tmpf) -> const void* {
     if (ready && !bf3) return X.p;
-    const char* blk = X.p == c.OVOV.d() ? "ovov" : X.p == c.OVVV.d() ? "ovvv" : X.p == c.OOOV.d() ? "ooov"
-                      : X.p == c.OOVV.d() ? "oovv" : X.p == c.OOOO.d() ? "oooo" : X.p == c.LX.d() ? "Lovov"
-                      : X.p == c.Pt.d() ? "Pt" : nullptr;
+    const char* blk = block_name(c, X);
     std::string key;
     if (blk) {
       // the source index string is part of the key: two contractions that bind the letters to the
@@ -445,6 +454,12 @@ static void build_lx(Ctx& c) {
   perm(c, tv(c.LX.d(), {o, v, o, v}), "kcld", tv(c.Lkl.d(), {o, o, v, v}), "klcd", 1.0, 0.0);
   c.Okl = dalloc(c, o * o * o * v);
   perm(c, tv(c.OOOV.d(), {o, o, o, v}), "kilc", tv(c.Okl.d(), {o, o, o, v}), "klic", 1.0, 0.0);
+  c.Lo1 = dalloc(c, o * o * o * v);
+  perm(c, tv(c.OOOV.d(), {o, o, o, v}), "kilc", tv(c.Lo1.d(), {o, v, o, o}), "lcki", 2.0, 0.0);
+  perm(c, tv(c.OOOV.d(), {o, o, o, v}), "likc", tv(c.Lo1.d(), {o, v, o, o}), "lcki", -1.0, 1.0);
+  c.L1 = dalloc(c, c.n2());
+  d2d(c, c.L1.d(), c.OVOV.d(), c.n2());
+  perm(c, tv(c.OOVV.d(), {o, o, v, v}), "kiac", tv(c.L1.d(), {o, v, o, v}), "kcia", -1.0, 2.0);
 }
 
 static void prepare(Ctx& c) {
@@ -525,8 +540,8 @@ static void residual(Ctx& c, const double* t1p, const double* t2p, double* R1, d
   TView r1 = tv(R1, {o, v});
   const int64_t n2 = c.n2(), ov = o * v, np = v * (v + 1) / 2, mp = o * (o + 1) / 2, ldv = vv_pairs_ld(v);
 
-  Buf bFov = dalloc(c, o * v), bFoo = dalloc(c, o * o), bFvv = dalloc(c, v * v), bX = dalloc(c, o * o);
-  TView Fov = tv(bFov, {o, v}), Foo = tv(bFoo, {o, o}), Fvv = tv(bFvv, {v, v}), X = tv(bX, {o, o});
+  Buf bFov = dalloc(c, o * v), bLoo = dalloc(c, o * o), bLvv = dalloc(c, v * v);
+  TView Fov = tv(bFov, {o, v}), Loo = tv(bLoo, {o, o}), Lvv = tv(bLvv, {v, v});
   // forms of the amplitudes (k_amp_forms).  Split-BF16x3 takes the ring operands in FP32 where its GEMM is used
   // (the o^3 v^3 products of at least 1e9 elements, as in contract); the ladder's pairs are FP32 in both
   // reduced precisions
@@ -544,41 +559,33 @@ static void residual(Ctx& c, const double* t1p, const double* t2p, double* R1, d
   }
   TView u = tv(bu, {o, o, v, v});
 
-  // Fov[k,c] = L[k,c,l,d] t1[l,d];  Foo[k,i] = L[k,c,l,d] t2[i,l,c,d] + Fov[k,c] t1[i,c] with L t2 = (kc|ld) u[i,l,c,d];
-  // Fvv[a,c] = -L[k,c,l,d] t2[k,l,a,d] - t1[k,a] Fov[k,c]
+  // Fov[k,c] = L[k,c,l,d] t1[l,d]
+  // Loo[k,i] = L[k,c,l,d] t2[i,l,c,d] + (2 (ki|lc) - (li|kc)) t1[l,c] + Fov[k,c] t1[i,c] with L t2 = (kc|ld) u[i,l,c,d]
+  // Lvv[a,c] = -L[k,c,l,d] t2[k,l,a,d] - t1[k,a] Fov[k,c] + 2 (kd|ac) t1[k,d] - (kc|ad) t1[k,d]
   contract(c, 1.0, Lovov, "kcld", t1, "ld", 0.0, Fov, "kc");
   if (!t1_only && !ring32)
-    contract(c, 1.0, ovov, "kcld", tv(bring.d(), {o, v, o, v}), "icld", 0.0, Foo, "ki");
+    contract(c, 1.0, ovov, "kcld", tv(bring.d(), {o, v, o, v}), "icld", 0.0, Loo, "ki");
   else
-    contract(c, 1.0, ovov, "kcld", u, "ilcd", 0.0, Foo, "ki");
-  contract(c, 1.0, Fov, "kc", t1, "ic", 1.0, Foo, "ki");
-  slice_sum(c, v, v, o * o, v, -1.0, t2p, c.Lkl.d(), 0.0, Fvv.p);
-  contract(c, -1.0, t1, "ka", Fov, "kc", 1.0, Fvv, "ac");
-  // Loo = Foo + 2 (ki|lc) t1[l,c] - (li|kc) t1[l,c];  Lvv = Fvv + 2 (kd|ac) t1[k,d] - (kc|ad) t1[k,d]
-  Buf bLoo = dalloc(c, o * o), bLvv = dalloc(c, v * v);
-  TView Loo = tv(bLoo, {o, o}), Lvv = tv(bLvv, {v, v});
-  d2d(c, Loo.p, Foo.p, o * o);
-  d2d(c, Lvv.p, Fvv.p, v * v);
-  contract(c, 2.0, ooov, "kilc", t1, "lc", 1.0, Loo, "ki");
-  contract(c, -1.0, ooov, "likc", t1, "lc", 1.0, Loo, "ki");
+    contract(c, 1.0, ovov, "kcld", u, "ilcd", 0.0, Loo, "ki");
+  contract(c, 1.0, tv(c.Lo1.d(), {o, v, o, o}), "lcki", t1, "lc", 1.0, Loo, "ki");
+  slice_sum(c, v, v, o * o, v, -1.0, t2p, c.Lkl.d(), 0.0, Lvv.p);
+  contract(c, -1.0, t1, "ka", Fov, "kc", 1.0, Lvv, "ac");
   contract(c, 2.0, ovvv, "kdac", t1, "kd", 1.0, Lvv, "ac");
   contract(c, -1.0, ovvv, "kcad", t1, "kd", 1.0, Lvv, "ac");
 
-  // ---- T1 numerator
+  // ---- T1 numerator (Fov[k,c] t1[i,c] t1[k,a] appears with both signs: Loo takes it after its product here)
   contract(c, 1.0, Lvv, "ac", t1, "ic", 0.0, r1, "ia");
   contract(c, -1.0, Loo, "ki", t1, "ka", 1.0, r1, "ia");
+  contract(c, 1.0, tv(c.L1.d(), {o, v, o, v}), "kcia", t1, "kc", 1.0, r1, "ia");
   if (!t1_only && !ring32)
     contract(c, 1.0, Fov, "kc", tv(bring.d(), {o, v, o, v}), "kcia", 1.0, r1, "ia");
   else
     contract(c, 1.0, Fov, "kc", u, "kica", 1.0, r1, "ia");
-  contract(c, 1.0, Fov, "kc", t1, "ic", 0.0, X, "ik");
-  contract(c, 1.0, X, "ik", t1, "ka", 1.0, r1, "ia");
-  contract(c, 2.0, ovov, "kcia", t1, "kc", 1.0, r1, "ia");
-  contract(c, -1.0, oovv, "kiac", t1, "kc", 1.0, r1, "ia");
   contract(c, 1.0, ovvv, "kdac", u, "ikcd", 1.0, r1, "ia");
   slice_sum(c, o, v, o * o, v, -1.0, c.Okl.d(), u.p, 1.0, r1.p);
   if (t1_only) return;
   bu.reset();
+  contract(c, 1.0, Fov, "kc", t1, "ic", 1.0, Loo, "ki");
 
   // ---- T2 numerator: P, the ring products and the ladder, then R2 = P + P[j,i,b,a] + ... (k_t2_numerator)
   TView tau = tv(btau, {o, o, v, v});
