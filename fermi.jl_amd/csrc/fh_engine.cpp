@@ -14,6 +14,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -23,6 +24,7 @@
 #include <mutex>
 #include <random>
 #include <sstream>
+#include <thread>
 #include <type_traits>
 
 namespace fh {
@@ -110,9 +112,42 @@ struct BlasHandle {
   ~BlasHandle() { if (h) (void)rocblas_destroy_handle(h); }
 };
 
+// Pinned chunks for large copies between the device and pageable host memory (copy_staged): 16 MiB a context, made by
+// its first such copy and freed with it.
+struct HostStage {
+  static constexpr int kThreads = 4;
+  static constexpr size_t kChunk = (size_t)2 << 20;
+  char* buf[kThreads][2] = {};
+  hipEvent_t ev[kThreads][2] = {};
+  HostStage() = default;
+  bool init() {
+    for (auto& t : buf)
+      for (char*& b : t) {
+        void* p = nullptr;
+        if (hipHostMalloc(&p, kChunk, hipHostMallocDefault) != hipSuccess) return false;
+        b = static_cast<char*>(p);
+      }
+    for (auto& t : ev)
+      for (hipEvent_t& e : t)
+        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
+    return true;
+  }
+  HostStage(const HostStage&) = delete;
+  HostStage& operator=(const HostStage&) = delete;
+  ~HostStage() {
+    for (auto& t : ev)
+      for (hipEvent_t e : t)
+        if (e) (void)hipEventDestroy(e);
+    for (auto& t : buf)
+      for (char* b : t)
+        if (b) (void)hipHostFree(b);
+  }
+};
+
 struct Ctx {
   int device = 0;
   hipStream_t s = nullptr;
+  std::unique_ptr<HostStage> stage;
   BlasHandle blas;   // of the eigensolver, made on first use
   // declared before every Buf member, so that it is destroyed after all of them
   std::unique_ptr<Pool> pool;
@@ -200,10 +235,78 @@ static void flush_timers(Ctx& c) {
 }
 
 static Buf dalloc(Ctx& c, int64_t n) { return Buf(c.pool.get(), (size_t)std::max<int64_t>(n, 1) * sizeof(double)); }
+// Copy of n bytes between the device and pageable host memory in pinned chunks, chunk i by thread i mod 4: the DMA of a
+// chunk runs while the chunks before it are moved between the pinned buffers and the host memory (whose pages, when it
+// is new, are made by four threads at once instead of one).  For copies of 4 MiB and more; false: not taken (memory that
+// the runtime knows, which it copies directly, or no pinned memory).  Returns with the host memory free for other use.
+// (mu nu|la si) of two water molecules, 42 MB into new memory: 4.7 ms with one pageable copy, 2.2 ms so, 0.6 of them
+// kernels.
+static bool copy_staged(Ctx& c, char* dev, char* host, size_t n, bool to_host) {
+  if (n < ((size_t)4 << 20)) return false;
+  hipPointerAttribute_t at{};
+  if (hipPointerGetAttributes(&at, host) == hipSuccess) {
+    if (at.type != hipMemoryTypeUnregistered) return false;
+  } else {
+    (void)hipGetLastError();
+  }
+  if (!c.stage) {
+    auto made = std::make_unique<HostStage>();
+    if (!made->init()) {
+      (void)hipGetLastError();
+      return false;
+    }
+    c.stage = std::move(made);
+  }
+  HostStage& st = *c.stage;
+  constexpr size_t CH = HostStage::kChunk;
+  const size_t nch = (n + CH - 1) / CH;
+  std::atomic<int> err{(int)hipSuccess};
+  auto work = [&](int t) {
+    auto ok = [&](hipError_t e) {
+      if (e != hipSuccess) err = (int)e;
+      return e == hipSuccess;
+    };
+    if (!ok(hipSetDevice(c.device))) return;
+    auto len = [&](size_t i) { return std::min(CH, n - i * CH); };
+    size_t in[2] = {nch, nch};   // chunk in flight in each buffer
+    auto finish = [&](int k) {
+      if (in[k] == nch) return true;
+      if (!ok(hipEventSynchronize(st.ev[t][k]))) return false;
+      if (to_host) std::memcpy(host + in[k] * CH, st.buf[t][k], len(in[k]));
+      in[k] = nch;
+      return true;
+    };
+    int k = 0;
+    for (size_t i = t; i < nch; i += HostStage::kThreads, k ^= 1) {
+      if (!finish(k)) return;
+      if (!to_host) std::memcpy(st.buf[t][k], host + i * CH, len(i));
+      const hipError_t e = to_host ? hipMemcpyAsync(st.buf[t][k], dev + i * CH, len(i), hipMemcpyDeviceToHost, c.s)
+                                   : hipMemcpyAsync(dev + i * CH, st.buf[t][k], len(i), hipMemcpyHostToDevice, c.s);
+      if (!ok(e) || !ok(hipEventRecord(st.ev[t][k], c.s))) return;
+      in[k] = i;
+    }
+    if (finish(k)) finish(k ^ 1);
+  };
+  std::vector<std::thread> th;
+  int started = 1;
+  try {
+    th.reserve(HostStage::kThreads - 1);
+    for (; started < HostStage::kThreads; ++started) th.emplace_back(work, started);
+  } catch (const std::exception&) {
+    // no more threads: this one takes their chunks
+  }
+  work(0);
+  for (int t = started; t < HostStage::kThreads; ++t) work(t);
+  for (auto& x : th) x.join();
+  FH_HIP((hipError_t)err.load());
+  return true;
+}
 static void h2d(Ctx& c, double* d, const double* h, int64_t n) {
+  if (copy_staged(c, reinterpret_cast<char*>(d), reinterpret_cast<char*>(const_cast<double*>(h)), n * sizeof(double), false)) return;
   FH_HIP(hipMemcpyAsync(d, h, n * sizeof(double), hipMemcpyHostToDevice, c.s));
 }
 static void d2h(Ctx& c, double* h, const double* d, int64_t n) {
+  if (copy_staged(c, reinterpret_cast<char*>(const_cast<double*>(d)), reinterpret_cast<char*>(h), n * sizeof(double), true)) return;
   FH_HIP(hipMemcpyAsync(h, d, n * sizeof(double), hipMemcpyDeviceToHost, c.s));
   FH_HIP(hipStreamSynchronize(c.s));
 }

@@ -481,6 +481,9 @@ class Context:
         return n1, n2
 
     def solve(self, opts=None, T1=None, T2=None, copy_out=True):
+        return self._solve(opts, T1, T2, copy_out)
+
+    def _solve(self, opts, T1, T2, copy_out=True, in_place=False):
         opts = Options() if opts is None else opts
         c = _Opts()
         self.L.fh_default_opts(ctypes.byref(c))
@@ -505,7 +508,7 @@ class Context:
             if copy_out:
                 raise FermiException("copy_out requires starting amplitudes; use T1/T2 arrays")
         else:
-            out1, out2 = _colmajor(T1).copy(order="F"), _colmajor(T2).copy(order="F")
+            out1, out2 = (T1, T2) if in_place else (_colmajor(T1).copy(order="F"), _colmajor(T2).copy(order="F"))
             self._check(self.L.fh_ccsd_solve(self.h, ctypes.byref(c), _ptr(out1), _ptr(out2), ctypes.byref(r)))
         return r, out1, out2
 
@@ -663,7 +666,8 @@ def RCCSD(moints, *args, alg=None, options=None, device=0):
         raise FermiException(f"invalid algorithm {type(alg).__name__} for the MI355X RCCSD backend")
     ctx = _ctx_for(moints, device)
     opts = Options() if options is None else options
-    if len(args) == 0:
+    own = len(args) == 0
+    if own:
         T1, T2 = ctx.guess(0)
     elif len(args) == 2:
         T1, T2 = args
@@ -671,8 +675,9 @@ def RCCSD(moints, *args, alg=None, options=None, device=0):
             raise FermiException("amplitude shapes do not match the orbital spaces")
     else:
         raise FermiException("invalid arguments for RCCSD method")
-    Eguess = ctx.energy(T1, T2)
-    r, nT1, nT2 = ctx.solve(opts, T1, T2)
+    # the guess is on the device, and its arrays are free to take the result
+    Eguess = ctx.energy() if own else ctx.energy(T1, T2)
+    r, nT1, nT2 = ctx._solve(opts, T1, T2, in_place=own)
     Eref = float(moints.sd_energy)
     return RCCSDResult(Eguess + Eref, r.correlation, r.correlation + Eref, nT1, nT2, r.e_conv, r.t_conv, r.niter,
                        bool(r.converged))
