@@ -819,8 +819,8 @@ static double energy(Ctx& c, const double* t1, const double* t2) {
 }
 
 // newT = residual(T) ./ D; returns rms of (newT1 - T1), (newT2 - T2); errors optionally kept
-static void update_amp(Ctx& c, const double* t1, const double* t2, double* n1, double* n2, void* e1, void* e2,
-                       bool f32, double* r1, double* r2) {
+// New amplitudes; the sums of their squared changes (T1, T2) go to c.scal[0], [1]
+static void update_amp(Ctx& c, const double* t1, const double* t2, double* n1, double* n2, void* e1, void* e2, bool f32) {
   residual(c, t1, t2, n1, n2);
   if (!c.partials.p) c.partials = dalloc(c, 4096);
   if (!c.scal.p) c.scal = dalloc(c, 64);
@@ -833,11 +833,6 @@ static void update_amp(Ctx& c, const double* t1, const double* t2, double* n1, d
     jacobi_update(c.s, c.o, c.v, true, c.eo.d(), c.ev.d(), n2, t2, e2, f32, c.partials.d() + 2048, &nb);
     sum_partials(c.s, nb, c.partials.d() + 2048, c.scal.d() + 1);
   }
-  double h[2];
-  FH_HIP(hipMemcpyAsync(h, c.scal.d(), 2 * sizeof(double), hipMemcpyDeviceToHost, c.s));
-  FH_HIP(hipStreamSynchronize(c.s));
-  *r1 = std::sqrt(h[0] / (double)c.nov());
-  *r2 = std::sqrt(h[1] / (double)c.n2());
 }
 
 // DF-MP2 correlation energy RMP2_energy (RMP2a.jl:91-144) from Bov and the orbital energies alone:
@@ -982,28 +977,27 @@ struct DIIS {
   bool f32;
   std::vector<Buf> vecs, errs;
   std::vector<std::vector<double>> B;   // B[a][b] = errs[a] . errs[b], b <= a
-  Buf part, row;                        // the newest row on the device until resolve() reads it
+  Buf part;
+  int slot;                             // the newest row's place in c.scal, until resolve() takes it from a host copy
   bool pending = false;
   const char* phase;  // timer name of the vector work (nullptr: untimed)
-  DIIS(Ctx& cc, int64_t nn, int m, bool f, const char* ph = nullptr) : c(cc), n(nn), maxv(m), f32(f), phase(ph) {
+  DIIS(Ctx& cc, int64_t nn, int m, bool f, int sl, const char* ph = nullptr)
+      : c(cc), n(nn), maxv(m), f32(f), slot(sl), phase(ph) {
     part = dalloc(c, 8 * reduce_blocks_needed(n));
-    row = dalloc(c, 8);
+    if (!c.scal.p) c.scal = dalloc(c, 64);
   }
   double esz() const { return f32 ? 4.0 : 8.0; }
   std::unique_ptr<Timer> timer(double bytes) {
     return std::unique_ptr<Timer>(phase ? new Timer(c, phase, 0.0, bytes) : nullptr);
   }
-  // the products of the newest error vector, one copy for the whole row
-  void resolve() {
+  // the products of the newest error vector, from a host copy of c.scal made after push()
+  void resolve(const double* scal) {
     if (!pending) return;
-    double h[8];
-    d2h(c, h, row.d(), (int64_t)errs.size());
-    B.emplace_back(h, h + errs.size());
+    B.emplace_back(scal + slot, scal + slot + errs.size());
     pending = false;
   }
   // push! takes ownership of the error buffer and copies the vector
   void push(const double* vec, Buf&& err) {
-    resolve();
     if ((int)vecs.size() + 1 > maxv) {
       int idx = 0;
       double best = -1.0;
@@ -1026,13 +1020,12 @@ struct DIIS {
     const void* xs[8];
     for (size_t q = 0; q < errs.size(); ++q) xs[q] = errs[q].p;
     auto t = timer(esz() * (double)errs.size() * (double)n);
-    dots(c.s, n, (int)errs.size(), xs, errs.back().p, f32, part.d(), row.d());
+    dots(c.s, n, (int)errs.size(), xs, errs.back().p, f32, part.d(), c.scal.d() + slot);
     pending = true;
   }
   void extrapolate(double* out, bool add_res) {
     const int m = (int)vecs.size();
     FH_CHECK(m >= 2, -3, "DIIS cannot extrapolate from one vector");
-    resolve();
     const int N = m + 1;
     std::vector<double> A(N * N, 1.0), x(N, 0.0);
     A[(N - 1) * N + (N - 1)] = 0.0;
@@ -1192,7 +1185,7 @@ static void rhf(Ctx& c, const fh_scf_opts& op, int n, int naux, int no, double V
   d2d(c, Dtil.d(), D.d(), nn);
   d2d(c, Dold.d(), D.d(), nn);
   std::unique_ptr<DIIS> dm;
-  if (op.diis) dm.reset(new DIIS(c, nn, op.ndiis, false));
+  if (op.diis) dm.reset(new DIIS(c, nn, op.ndiis, false, 16));
   int ite = 1;
   double E = 0.0, dE = 1.0, Drms = 1.0;
   bool converged = false;
@@ -1204,9 +1197,6 @@ static void rhf(Ctx& c, const fh_scf_opts& op, int n, int naux, int no, double V
     d2d(c, T1.d(), D.d(), nn);                                    // Drms (:189-190)
     axpby_f64(c.s, nn, -1.0, Dold.d(), 1.0, T1.d());
     dot_f64(c.s, nn, T1.d(), T1.d(), c.partials.d(), c.scal.d() + 10);
-    double h[3];
-    d2h(c, h, c.scal.d() + 8, 3);
-    const double Enew = h[0] + h[1] + Vnuc;                       // :151-154
     if (dm) {                                                     // err = L^T (F D S - S D F) L  (:157-160)
       mm(c, false, false, n, n, n, 1.0, F.d(), n, D.d(), n, 0.0, T1.d(), n);       // F D
       mm(c, false, false, n, n, n, 1.0, T1.d(), n, S, n, 0.0, T2.d(), n);          // F D S
@@ -1217,6 +1207,10 @@ static void rhf(Ctx& c, const fh_scf_opts& op, int n, int naux, int no, double V
       mm(c, true, false, n, n, n, 1.0, L.d(), n, T1.d(), n, 0.0, err.d(), n);
       dm->push(F.d(), std::move(err));
     }
+    double h[24];                                                 // both energies, Drms and the DIIS row in one copy
+    d2h(c, h, c.scal.d(), 24);
+    const double Enew = h[8] + h[9] + Vnuc;                       // :151-154
+    if (dm) dm->resolve(h);
     if (op.oda && Drms > op.oda_cutoff && ite < op.oda_shutoff) {   // ODA (:163-180)
       d2d(c, T1.d(), D.d(), nn);
       axpby_f64(c.s, nn, -1.0, Dtil.d(), 1.0, T1.d());            // dD = D - D~
@@ -1230,7 +1224,7 @@ static void rhf(Ctx& c, const fh_scf_opts& op, int n, int naux, int no, double V
     } else if (dm && ite > op.diis_start) {                       // DIIS (:183-186)
       dm->extrapolate(F.d(), false);
     }
-    Drms = std::sqrt(h[2] / (double)nn);
+    Drms = std::sqrt(h[10] / (double)nn);
     dE = Enew - E;
     E = Enew;
     d2d(c, Dold.d(), D.d(), nn);
@@ -1265,7 +1259,7 @@ static void solve(Ctx& c, const fh_cc_opts& op, fh_cc_result& res) {
   const bool do_diis = op.cc_diis != 0;
   const bool f32 = op.diis_prec != 0;
   const double dp = op.cc_damp_ratio;
-  std::unique_ptr<DIIS> dm1(new DIIS(c, n1, op.cc_ndiis, f32)), dm2(new DIIS(c, n2, op.cc_ndiis, f32, "diis"));
+  std::unique_ptr<DIIS> dm1(new DIIS(c, n1, op.cc_ndiis, f32, 16)), dm2(new DIIS(c, n2, op.cc_ndiis, f32, 24, "diis"));
   c.iters.clear();
   // mixed precision: the residual's contractions run at `level` (2 split-BF16x3 or 1 FP32, then
   // 0 FP64).  A reduced-precision phase ends when |dE| and rms fall below its switch thresholds,
@@ -1300,8 +1294,8 @@ static void solve(Ctx& c, const fh_cc_opts& op, fh_cc_result& res) {
     while (level > 0 && ((std::fabs(dE) < (level == 2 ? sw_e2 : sw_e) && rms < (level == 2 ? sw_rms2 : sw_rms)) ||
                          stall >= kStall)) {
       level = 0;                                           // FP64 polish
-      dm1.reset(new DIIS(c, n1, op.cc_ndiis, f32));
-      dm2.reset(new DIIS(c, n2, op.cc_ndiis, f32, "diis"));
+      dm1.reset(new DIIS(c, n1, op.cc_ndiis, f32, 16));
+      dm2.reset(new DIIS(c, n2, op.cc_ndiis, f32, 24, "diis"));
       dE = 1.0;
       rms = 1.0;
       stall = 0;
@@ -1324,8 +1318,7 @@ static void solve(Ctx& c, const fh_cc_opts& op, fh_cc_result& res) {
       e1 = Buf(c.pool.get(), (size_t)n1 * (f32 ? 4 : 8));
       e2 = Buf(c.pool.get(), (size_t)n2 * (f32 ? 4 : 8));
     }
-    double r1 = 0.0, r2 = 0.0;
-    update_amp(c, oT1.d(), oT2.d(), nT1.d(), nT2.d(), e1.p, e2.p, f32, &r1, &r2);               // :190-194
+    update_amp(c, oT1.d(), oT2.d(), nT1.d(), nT2.d(), e1.p, e2.p, f32);                         // :190-194
     c.lowp = 0;
     if (op.fault_inject > 0 && ite == op.fault_inject && !injected) {      // test hook: one NaN in the new T2
       const double nan = std::nan("");
@@ -1337,6 +1330,14 @@ static void solve(Ctx& c, const fh_cc_opts& op, fh_cc_result& res) {
     if (do_diis) {
       dm1->push(nT1.d(), std::move(e1));                                                        // :199-202
       dm2->push(nT2.d(), std::move(e2));
+    }
+    // the changes and both rows of products in one copy
+    double h[32];
+    d2h(c, h, c.scal.d(), 32);
+    const double r1 = std::sqrt(h[0] / (double)n1), r2 = std::sqrt(h[1] / (double)n2);
+    if (do_diis) {
+      dm1->resolve(h);
+      dm2->resolve(h);
       if (ite >= op.diis_start && ite % op.cc_diis_relax == 0 &&                             // :204
           (op.precision_mode == 0 || dm2->vecs.size() >= 2)) {
         dm2->extrapolate(nT2.d(), true);                                                        // :206
@@ -1358,8 +1359,8 @@ static void solve(Ctx& c, const fh_cc_opts& op, fh_cc_result& res) {
       d2d(c, nT2.d(), oT2.d(), n2);
       Ecc = oldE;
       level = 0;
-      dm1.reset(new DIIS(c, n1, op.cc_ndiis, f32));
-      dm2.reset(new DIIS(c, n2, op.cc_ndiis, f32, "diis"));
+      dm1.reset(new DIIS(c, n1, op.cc_ndiis, f32, 16));
+      dm2.reset(new DIIS(c, n2, op.cc_ndiis, f32, 24, "diis"));
       dE = 1.0;
       rms = 1.0;
       stall = 0;
@@ -2071,8 +2072,7 @@ int fh_ccsd_residual(fh_ctx* x, const double* T1, const double* T2, double* n1, 
     Buf a = dalloc(c, c.nov()), b = dalloc(c, c.n2()), ra = dalloc(c, c.nov()), rb = dalloc(c, c.n2());
     h2d(c, a.d(), T1, c.nov());
     h2d(c, b.d(), T2, c.n2());
-    double r1, r2;
-    update_amp(c, a.d(), b.d(), ra.d(), rb.d(), nullptr, nullptr, false, &r1, &r2);
+    update_amp(c, a.d(), b.d(), ra.d(), rb.d(), nullptr, nullptr, false);
     d2h(c, n1, ra.d(), c.nov());
     d2h(c, n2, rb.d(), c.n2());
     flush_timers(c);

@@ -276,6 +276,7 @@ struct GemmPlan {
 static GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t batch) {
   const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64) * batch;
   if (tiles >= 384) return {false, 1};
+  if (K > 32 && K <= 256) return {true, 1};
   const int64_t most = K < 384 ? 1 : K / 128;
   if (tiles * most >= 256) return {false, std::min<int64_t>(std::max<int64_t>(1, 1024 / tiles), most)};
   const int64_t tiles32 = ((M + 31) / 32) * ((N + 31) / 32) * batch;
