@@ -1525,8 +1525,8 @@ static double triples_t(Ctx& c, bool bf3, int64_t t0 = 0, int64_t nt = -1) {
     perm(c, tv(c.OVOV.d(), {o, v, o, v}), "iajb", tv(vvoo.d(), {v, v, o, o}), "abij", 1.0, 0.0);
     triples_block_vv(c.s, (int)o, (int)v, vvoo.d(), vvb.d());
   }
-  // the energy kernel reads whole 8 x 8 blocks of a plane: up to 8 rows past the end of the last slot
-  Buf Wbuf(c.pool.get(), (size_t)(v3 * std::min(KC, ntot) + 8 * v + 64) * sizeof(T));
+  // the energy kernel reads whole 8 x 8 blocks of a panel: up to 56 elements past the end of the last slot
+  Buf Wbuf(c.pool.get(), (size_t)(triples_plane((int)v) * v * std::min(KC, ntot) + 64) * sizeof(T));
   T* W = static_cast<T*>(Wbuf.p);
   Buf part = dalloc(c, norb * max_erun + 16);
   Buf acc = dalloc(c, 1);

@@ -120,6 +120,8 @@ void splitk_reduce_f64(hipStream_t s, int64_t M, int64_t N, int64_t S, const dou
                        const double* C, int64_t ldc, int64_t sC, double* D, int64_t ldd, int64_t sD, int64_t batch);
 
 // ---------------------------------------------------------------- (T) W build (fh_triples.hip)
+// elements of an (a, b) plane of W, in panels of 8 a: [a / 8][b][a % 8]
+__host__ __device__ inline int64_t triples_plane(int v) { return (int64_t)8 * ((v + 7) / 8) * v; }
 // fmt: 0 FP64, 1 FP32, 2 split-BF16x3 (W in FP32).  Operands hold triples_pitch_elems(o, v) values of k per
 // row (8 bytes each for fmt 0, else 4): av, avs v^2 o rows each, bvp, bvq v o^2 rows each.
 struct TriplesOperands {
@@ -137,7 +139,7 @@ TriplesTiles triples_tiles(int fmt, int o, int v, double nk);  // nk: mean k per
 int64_t triples_chunk_slots(int v, int elem, const TriplesTiles& tt, int64_t ntot);
 // appends the column tiles of the run k0 .. k0 + nk - 1 of (i, j), its W slots from `slot`: 8 ints each
 void triples_col_tiles(const TriplesTiles& t, int v, int i, int j, int k0, int nk, int slot, std::vector<int>& out);
-// W[a + v b + v^2 c + v^3 slot] = classes abc + bac; then += the other four (slots: 4 ints (i, j, k, 0) each)
+// W[plane(a, b) of c of a slot, v planes a slot] = classes abc + bac; then += the other four (slots: 4 ints (i, j, k, 0) each)
 void triples_w_first(hipStream_t s, int fmt, int o, int v, const TriplesTiles& tt, const TriplesOperands& op, void* W,
                      const int* cols, int ncol);
 void triples_w_slices(hipStream_t s, int fmt, int o, int v, const TriplesTiles& tt, const TriplesOperands& op, void* W,
@@ -218,7 +220,7 @@ void mp2_pair_energy(hipStream_t s, int o, int v, int Q, const double* Bov, cons
 void scale_cols_rsqrt(hipStream_t s, int n, const double* U, const double* w, double* out);
 void gwh_fock(hipStream_t s, int n, const double* S, const double* H, double* F);
 
-// (T) energy of nrun runs of k (8 ints each: i, j, k0, nk, W slot of k0): W[a + v*b + v^2*c + v^3*slot]
+// (T) energy of nrun runs of k (8 ints each: i, j, k0, nk, W slot of k0): W
 // holds the W intermediate of ijk.jl:108-115; one FP64 partial per orbit and run.
 // orbits: device list of cube-block triples (A>=B>=C), 3 ints each (triples_orbits)
 int triples_orbit_count(int v);

@@ -8,7 +8,13 @@
 //   slice launch   with c fixed the other four are GEMMs with rows a and columns b (K = 4 nd):
 //                  cab: AVs_i[(a,c)] Bcat_{k,j}[b] + cba: Bcat_{k,i}[a] AVs_j[(b,c)]
 //                  acb: AV_k[(a,c)] Bcat_{i,j}[b]  + bca: Bcat_{j,i}[a] AV_k[(b,c)].
-// So W is written once and read and written once more per chunk of triples.  Bcat is kept as BVp (blocks
+// So W is written once and read and written once more per chunk of triples.  An (a, b) plane of W lies in panels of 8
+// a, [a / 8][b][a % 8] with a up to a multiple of 8 (triples_plane elements, the rows beyond v unused).  The rows
+// (x, y) of AV and AVs lie likewise, their last panel v % 8 wide, so that the first launch's rows are the plane's
+// elements in order and v^2 in number (rows up to the multiple of 8 cost v = 76 in FP64 1.2 % of the (T)).  The energy
+// kernel
+// then copies the 8 x 8 elements of a cube's plane as one run of whole cache lines (rows of 8 a, a quarter of a line
+// each, with a fastest over all of v), and the slice launch adds to 4 a of a column at a time.  Bcat is kept as BVp (blocks
 // (p, q) with p fastest) and BVq (q fastest), AV as rows (x, y) and AVs as rows (y, x).
 //
 // Operand layout: the k of a row are cut into groups of 8 (32 bytes, 64 for FP64), stored group-major, [group]
@@ -184,6 +190,17 @@ __device__ __forceinline__ unsigned unit_at(int r, int g, int u) {
                   : (unsigned)((r >> 4) * 1024 + (r & 15) * 64 + (u ^ ((r >> 2) & 3)) * 16);
 }
 
+// row (x, y) of AV, and the element of a plane of W that row r is
+__device__ __forceinline__ int64_t av_row(int v, int x, int y) {
+  return (int64_t)8 * v * (x >> 3) + min(8, v - (x & ~7)) * y + (x & 7);
+}
+__device__ __forceinline__ int plane_at(int v, int r) {
+  const int last = (v & ~7) * v;  // rows of the whole panels
+  if (r < last) return r;
+  const int w = v & 7, y = (r - last) / w;
+  return last + 8 * y + (r - last - w * y);
+}
+
 // n elements in blocks of g, dealt to nt tiles of nearly equal block counts: first element of tile t
 __host__ __device__ inline int tile_begin(int n, int g, int nt, int t) {
   const int nb = (n + g - 1) / g;
@@ -242,9 +259,9 @@ __global__ __launch_bounds__(256) void k_triples_av(int o, int v, int nd, const 
       const int lo = e & 3, hi = e >> 2 & 3, n = e >> 4;
       if (n0 + n >= o) continue;
       if (x0 + lo < v && y0 + hi < v)
-        put_k8<FMT>(av + (n0 + n) * an + (vv * g + x0 + lo + (int64_t)v * (y0 + hi)) * GB, &tile[0][lo + 4 * hi][n], 16 * 33);
+        put_k8<FMT>(av + (n0 + n) * an + (vv * g + av_row(v, x0 + lo, y0 + hi)) * GB, &tile[0][lo + 4 * hi][n], 16 * 33);
       if (y0 + lo < v && x0 + hi < v)
-        put_k8<FMT>(avs + (n0 + n) * an + (vv * g + y0 + lo + (int64_t)v * (x0 + hi)) * GB, &tile[0][hi + 4 * lo][n], 16 * 33);
+        put_k8<FMT>(avs + (n0 + n) * an + (vv * g + av_row(v, y0 + lo, x0 + hi)) * GB, &tile[0][hi + 4 * lo][n], 16 * 33);
     }
   }
 }
@@ -298,8 +315,13 @@ template <int NSEG, int GB>
 struct TripTile {
   const char *A[NSEG], *B[NSEG];  // per K segment: the operands' first group at the tile's first row / column
   int rows, cols;
-  int64_t ldw, woff;  // leading dimension of the output tile and its first element's offset in W
+  // first launch: leading dimension of the output tile; slices: of its panels.  Offset of its first element in W, and
+  // elements from there to the end of its last column (first launch) or of its plane
+  int64_t ldw, woff, wleft;
   int bcol, v;        // first launch: the tile's first column within its k
+  int m0;             // first row
+  // slices: offset of column c in a whole and in the last panel of AV, and that of the last panel's first row in Bcat
+  int c8, cw, thra, thrb;
   int64_t bs;
 
   // whether segment s takes its A operand from AV / AVs (group stride v^2 rows) and B from Bcat (v rows), or
@@ -314,13 +336,13 @@ struct TripTile {
     const int64_t L = x8 * q8 + (x8 < r8 ? x8 : r8) + (w >> 3);
     v = t.v;
     const int o = t.o;
-    const int64_t vv = (int64_t)v * v, an = vv * (t.nd / 8) * GB;
+    const int64_t pl = triples_plane(v), vv = (int64_t)v * v, an = vv * (t.nd / 8) * GB;
     bs = (int64_t)v * (t.nd / 8) * GB;
     bcol = 0;
     if constexpr (NSEG == 2) {
       const int ct = (int)(L % t.ncol), mt = (int)(L / t.ncol);
       const int4 p = t.cols[2 * ct], q = t.cols[2 * ct + 1];
-      const int m0 = tile_begin((int)vv, grain, t.nt, mt);
+      m0 = tile_begin((int)vv, grain, t.nt, mt);
       rows = min(tile_begin((int)vv, grain, t.nt, mt + 1), (int)vv) - m0;
       cols = q.y;
       const int kk = q.x / v;
@@ -329,8 +351,10 @@ struct TripTile {
       A[1] = t.avs + an * p.x + (int64_t)GB * m0;
       B[0] = t.bvq + bs * (p.z + kk + (int64_t)o * p.x);
       B[1] = t.bvq + bs * (p.z + kk + (int64_t)o * p.y);
-      ldw = vv;
-      woff = vv * v * p.w + m0 + vv * q.x;
+      ldw = pl;
+      woff = pl * v * p.w + pl * q.x;
+      wleft = ldw * cols;
+      c8 = cw = thra = thrb = 0;
     } else {
       // groups of kSlotGroup slots, then c, then the slots of the group, then the tiles of a slice: the 64
       // workgroups of an XCD in flight share AV_i, AV_j (same c) and the Bcat blocks (same slots)
@@ -339,20 +363,29 @@ struct TripTile {
       const int gr = (int)(L / per), s0 = gr * t.group, ns = min(t.group, t.ncol - s0);
       const int rem = (int)(L - gr * per), c = rem / (ns * tt), r2 = rem - c * ns * tt, s = s0 + r2 / tt, tl = r2 % tt;
       const int4 p = t.slots[s];
-      const int m0 = tile_begin(v, grain, t.nt, tl % t.nt), n0 = tile_begin(v, grain, t.nt, tl / t.nt);
+      const int n0 = tile_begin(v, grain, t.nt, tl / t.nt);
+      m0 = tile_begin(v, grain, t.nt, tl % t.nt);
       rows = min(tile_begin(v, grain, t.nt, tl % t.nt + 1), v) - m0;
       cols = min(tile_begin(v, grain, t.nt, tl / t.nt + 1), v) - n0;
-      const int64_t co = (int64_t)GB * v * c, ao = (int64_t)GB * m0, bo = (int64_t)GB * n0;
-      A[0] = t.avs + an * p.x + co + ao;                       // cab: AV_i[(c,a)]
+      // the panels of rows m0 .. and n0 .. (multiples of 8) of AV, in which column c starts at c8, cw in the last, and
+      // rows m0 .. and n0 .. of Bcat
+      c8 = GB * 8 * c;
+      cw = GB * (v & 7) * c;
+      thra = GB * ((v & ~7) - m0);
+      thrb = GB * ((v & ~7) - n0);
+      const int64_t ca = (int64_t)GB * v * m0, cb = (int64_t)GB * v * n0;
+      const int64_t ao = (int64_t)GB * m0, bo = (int64_t)GB * n0;
+      A[0] = t.avs + an * p.x + ca;                            // cab: AV_i[(c,a)]
       B[0] = t.bvp + bs * (p.z + (int64_t)o * p.y) + bo;       //      Bcat_{k,j}[., b]
       A[1] = t.bvp + bs * (p.z + (int64_t)o * p.x) + ao;       // cba: Bcat_{k,i}[., a]
-      B[1] = t.avs + an * p.y + co + bo;                       //      AV_j[(c,b)]
-      A[2] = t.av + an * p.z + co + ao;                        // acb: AV_k[(a,c)]
+      B[1] = t.avs + an * p.y + cb;                            //      AV_j[(c,b)]
+      A[2] = t.av + an * p.z + ca;                             // acb: AV_k[(a,c)]
       B[2] = t.bvp + bs * (p.x + (int64_t)o * p.y) + bo;       //      Bcat_{i,j}[., b]
       A[3] = t.bvp + bs * (p.y + (int64_t)o * p.x) + ao;       // bca: Bcat_{j,i}[., a]
-      B[3] = t.av + an * p.z + co + bo;                        //      AV_k[(b,c)], in L2 from the previous segment
-      ldw = v;
-      woff = vv * v * s + vv * c + m0 + (int64_t)v * n0;
+      B[3] = t.av + an * p.z + cb;                             //      AV_k[(b,c)], in L2 from the previous segment
+      ldw = 8 * v;
+      woff = pl * v * s + pl * c + (int64_t)v * m0 + 8 * n0;
+      wleft = pl - (int64_t)v * m0 - 8 * n0;
     }
   }
   // byte offset of column n of the tile within a k group of B
@@ -366,9 +399,9 @@ struct TripTile {
   }
 };
 
-// The k steps of a tile in order: step() calls copy(A, B, dga, dgb) with resources at the step's first group
-// and the lane's byte offset from there to its own group.  With 32-byte groups a step is two groups, which may
-// lie in two segments (an odd number of groups per segment): the lanes of the second group then copy in a
+// The k steps of a tile in order: step() calls copy(A, B, dga, dgb, odd) with resources at the step's first group,
+// the lane's byte offset from there to its own group and whether the segment is an odd one (row_at).  With 32-byte
+// groups a step is two groups, which may lie in two segments (an odd number of groups per segment): the lanes of the second group then copy in a
 // second, masked pass, which only makes the waits that count copies stricter.  The passes end in different
 // (empty) asm markers: merged into one copy with a choice of resource, they would run as a loop over the
 // wave's distinct resources.
@@ -379,6 +412,26 @@ struct Feed {
   const char *pa, *pb;
   int64_t sav, sbv;  // group strides of AV and Bcat
   int ng, seg, g, second;
+  int panel, c8, cw, thra, thrb;
+  // Offset of a row of A (or B) in AV from that in Bcat (16 times the unit + GB times the row): a panel of 8 rows is
+  // 8 v rows after the panel before it
+  template <bool OF_A>
+  __device__ __forceinline__ unsigned av_at(int lof) const {
+    if constexpr (NSEG == 2) return (unsigned)lof;
+    else return (unsigned)lof + __umul24((unsigned)lof >> (GB == 32 ? 8 : 9), (unsigned)panel) +
+                (unsigned)(lof >= (OF_A ? thra : thrb) ? cw : c8);
+  }
+  // the same in the operand that the segment has there: A is AV in the even segments, B in the odd ones
+  template <bool OF_A>
+  __device__ __forceinline__ unsigned row_at(int lof, bool odd) const {
+    if constexpr (NSEG == 2) {
+      return (unsigned)lof;
+    } else {
+      const bool is_av = odd != OF_A;
+      const int col = lof >= (OF_A ? thra : thrb) ? (is_av ? cw : 0) : (is_av ? c8 : 0);
+      return (unsigned)lof + __umul24((unsigned)lof >> (GB == 32 ? 8 : 9), (unsigned)(is_av ? panel : 0)) + (unsigned)col;
+    }
+  }
   __device__ __forceinline__ Feed(const TripW& t, const Tile& tl, int lane) {
 #pragma unroll
     for (int s = 0; s + 1 < NSEG; ++s) {
@@ -387,6 +440,11 @@ struct Feed {
     }
     sbv = (int64_t)GB * t.v;
     sav = sbv * t.v;
+    panel = GB * 8 * (t.v - 1);
+    c8 = tl.c8;
+    cw = tl.cw;
+    thra = tl.thra;
+    thrb = tl.thrb;
     ng = t.nd / 8;
     seg = g = 0;
     pa = tl.A[0];
@@ -409,19 +467,19 @@ struct Feed {
   __device__ __forceinline__ void step(Copy&& copy) {
     constexpr int G = 64 / GB;
     if (G == 1 || g + 1 < ng) {
-      copy(uniform_rsrc(pa), uniform_rsrc(pb), second ? (int)sa() : 0, second ? (int)sb() : 0);
+      copy(uniform_rsrc(pa), uniform_rsrc(pb), second ? (int)sa() : 0, second ? (int)sb() : 0, seg & 1);
       asm volatile("; step");
       g += G;
       pa += G * sa();
       pb += G * sb();
     } else {
       if (!second) {
-        copy(uniform_rsrc(pa), uniform_rsrc(pb), 0, 0);
+        copy(uniform_rsrc(pa), uniform_rsrc(pb), 0, 0, seg & 1);
         asm volatile("; step, last group of a segment");
       }
       next_segment();
       if (second) {
-        copy(uniform_rsrc(pa), uniform_rsrc(pb), 0, 0);
+        copy(uniform_rsrc(pa), uniform_rsrc(pb), 0, 0, seg & 1);
         asm volatile("; step, first group of a segment");
       }
       g = 1;
@@ -435,57 +493,67 @@ struct Feed {
   }
 };
 
-// Epilogue of a wave's MI x NJ blocks at (r0, c0) of its tile: element e of lane l of block (i, j) at row l % 32
-// and column 8 (e / 4) + 4 (l / 32) + e % 4 of the block.  W goes through a buffer resource that ends with the
-// tile's last column, at one running lane offset: an element outside the tile (a row beyond it starts out of
-// range) reads 0 and is not written, with no masks and no 48 addresses.  Per 32-row block row of the wave the
-// values of W are loaded before any is stored, and the sums replace them before the first store: a store's
-// data register is then not reused, which would make the next instruction wait for that store to complete.
-template <bool ADD, int MI, int NJ>
+// First launch: a wave's MI x NJ blocks at (r0, c0) of its tile, element e of lane l of block (i, j) at row l % 32 and
+// column 8 (e / 4) + 4 (l / 32) + e % 4 of the block.  W goes through a buffer resource that ends with the tile's last
+// column, at one running lane offset: an element outside the tile (a row beyond it starts out of range) is not
+// written, with no masks and no 48 addresses.
+template <int MI, int NJ>
 __device__ __forceinline__ void store_blocks(const f32x16 (&acc)[MI][NJ], __amdgpu_buffer_rsrc_t rw, int r0, int c0,
-                                             int rows, int ldw4) {
+                                             int rows, int ldw4, int m0, int v) {
   const int lane = threadIdx.x & 63, cl = c0 + 4 * (lane >> 5);
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
     const int row = r0 + i * 32 + (lane & 31);
-    const unsigned vo = row < rows ? (unsigned)(4 * row + ldw4 * cl) : 0x80000000u;
-    auto step = [&](unsigned& o, int e) {
-      o += (e & 3) == 3 ? 5 * ldw4 : ldw4;
-      asm volatile("" : "+v"(o));  // a running sum: not folded into 48 live offsets
-    };
-    float dv[NJ][16];
-    unsigned o = vo;
+    unsigned o = row < rows ? (unsigned)(4 * plane_at(v, m0 + row) + ldw4 * cl) : 0x80000000u;
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        if constexpr (ADD) {
-          dv[j][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rw, o, 0, 0));
-          step(o, e);
-        } else {
-          dv[j][e] = acc[i][j][e];
-        }
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i][j][e]), rw, o, 0, 0);
+        o += (e & 3) == 3 ? 5 * ldw4 : ldw4;
+        asm volatile("" : "+v"(o));  // a running sum: not folded into 48 live offsets
       }
     }
-    if constexpr (ADD) {
+  }
+}
+// Slices: adds a wave's blocks to a plane of W, element e of lane l of block (i, j) at row 8 (e / 4) + 4 (l / 32) + e % 4
+// and column l % 32: four consecutive elements of a panel a time, 64 lanes a run of 1 KB.  The resource ends with the
+// plane, a panel beyond v starts behind it and a column beyond the tile out of range.  Per 32-row block row of the wave
+// the values of W are loaded before any is stored, and the sums replace them before the first store: a store's
+// data register is then not reused, which would make the next instruction wait for that store to complete.
+template <int MI, int NJ>
+__device__ __forceinline__ void store_slice(const f32x16 (&acc)[MI][NJ], __amdgpu_buffer_rsrc_t rw, int r0, int c0,
+                                            int cols, int panel4) {
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  const int lane = threadIdx.x & 63;
+  unsigned vo[NJ];
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) {
+  for (int j = 0; j < NJ; ++j) {
+    const int col = c0 + 32 * j + (lane & 31);
+    vo[j] = col < cols ? (unsigned)(32 * col + 16 * (lane >> 5)) : 0x80000000u;
+  }
 #pragma unroll
-        for (int e = 0; e < 16; ++e) dv[j][e] += acc[i][j][e];
-        asm volatile("" : "+v"(dv[j][0]), "+v"(dv[j][1]), "+v"(dv[j][2]), "+v"(dv[j][3]), "+v"(dv[j][4]),
-                     "+v"(dv[j][5]), "+v"(dv[j][6]), "+v"(dv[j][7]), "+v"(dv[j][8]), "+v"(dv[j][9]), "+v"(dv[j][10]),
-                     "+v"(dv[j][11]), "+v"(dv[j][12]), "+v"(dv[j][13]), "+v"(dv[j][14]), "+v"(dv[j][15]));
-      }
-    }
-    o = vo;
+  for (int i = 0; i < MI; ++i) {
+    const unsigned po = (unsigned)(panel4 * ((r0 >> 3) + 4 * i));
+    f32x4 dv[NJ][4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        dv[j][q] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, vo[j] + (po + panel4 * q), 0, 0));
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dv[j][e]), rw, o, 0, 0);
-        step(o, e);
-      }
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dv[j][q][e] += acc[i][j][4 * q + e];
+      asm volatile("" : "+v"(dv[j][0]), "+v"(dv[j][1]), "+v"(dv[j][2]), "+v"(dv[j][3]));
     }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, dv[j][q]), rw, vo[j] + (po + panel4 * q), 0, 0);
   }
 }
 
@@ -497,15 +565,16 @@ __device__ __forceinline__ void store_blocks(const f32x16 (&acc)[MI][NJ], __amdg
 // blocks are dealt to the two wave rows, so v = 131 costs 5 x 5 blocks, not 6 x 6; blocks, copies and
 // fragment reads beyond the edge are not issued.
 // Bound by the matrix cores at the rate the card sustains (a plain bf16 product of 8192^3 reaches 1122 TFLOP/s,
-// 374 for three products): o = 40, v = 190: first launch 345 TFLOP/s (per-pair launches with row-major operands
-// split in the kernel: 224), slices 336 (224); o = 27, v = 131: slices 202 (two batched launches of 128 x 192
+// 374 for three products): o = 40, v = 190: first launch 363 TFLOP/s (345 with a fastest over all of v in W, whose
+// stores then begin inside a cache line; per-pair launches with row-major operands split in the kernel: 224), slices 359
+// (336 with one W element a load and store, 224); o = 27, v = 131: slices 202 (two batched launches of 128 x 192
 // tiles: 98).
 template <int NSEG, int MB>
 struct Bf3Tile {
   static constexpr int NS = 3, ABYTES = 64 * MB * 64, SLOT = 2 * ABYTES;
   __amdgpu_buffer_rsrc_t rw;
   char* ring;
-  int lane, wid, rows, cols, nst, npa, npb, cps, ldw4;
+  int lane, wid, rows, cols, nst, npa, npb, cps, ldw4, m0, v;
   int rb0, mi, cb0, nj;  // the wave's first row / column block of the tile and its block counts
   int lofa[MB], lofb[MB];
 
@@ -524,7 +593,9 @@ struct Bf3Tile {
     cb0 = wn ? (ncb + 1) / 2 : 0;
     nj = wn ? ncb - cb0 : (ncb + 1) / 2;
     ldw4 = 4 * (int)tl.ldw;
-    rw = uniform_rsrc(reinterpret_cast<const char*>(static_cast<float*>(t.w) + tl.woff), ldw4 * cols);
+    m0 = __builtin_amdgcn_readfirstlane(tl.m0);
+    v = t.v;
+    rw = uniform_rsrc(reinterpret_cast<const char*>(static_cast<float*>(t.w) + tl.woff), 4 * (int)tl.wleft);
     nst = NSEG * t.nd / 16;
     npa = (rows + 15) / 16;
     npb = (cols + 15) / 16;
@@ -538,17 +609,17 @@ struct Bf3Tile {
     }
   }
   __device__ __forceinline__ void dma(Feed<NSEG, 32>& feed, int slot) const {
-    feed.step([&](__amdgpu_buffer_rsrc_t rsa, __amdgpu_buffer_rsrc_t rsb, int dga, int dgb) {
+    feed.step([&](__amdgpu_buffer_rsrc_t rsa, __amdgpu_buffer_rsrc_t rsb, int dga, int dgb, bool odd) {
 #pragma unroll
       for (int q = 0; q < MB; ++q)
         if (wid + 4 * q < npa)
           __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_vptr)(ring + slot * SLOT + (wid + 4 * q) * 1024), 16,
-                                                   (unsigned)(lofa[q] + dga), 0, 0, 0);
+                                                   feed.template row_at<true>(lofa[q], odd) + dga, 0, 0, 0);
 #pragma unroll
       for (int q = 0; q < MB; ++q)
         if (wid + 4 * q < npb)
           __builtin_amdgcn_raw_ptr_buffer_load_lds(rsb, (lds_vptr)(ring + slot * SLOT + ABYTES + (wid + 4 * q) * 1024), 16,
-                                                   (unsigned)(lofb[q] + dgb), 0, 0, 0);
+                                                   feed.template row_at<false>(lofb[q], odd) + dgb, 0, 0, 0);
     });
   }
   // MI x NJ blocks of this wave (0 x 0: a wave without a block, which still copies and meets the barriers).
@@ -582,23 +653,28 @@ struct Bf3Tile {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
           const bf16x8 bh = __builtin_bit_cast(bf16x8, fb[j][0]), bl = __builtin_bit_cast(bf16x8, fb[j][1]);
-          // B as the first operand, so that the accumulator's lanes run along the rows of W
+          // first launch: B as the first operand, so that the accumulator's lanes run along the rows of W; slices: A, so
+          // that they run along its columns and four registers are four rows (store_slice)
+          auto mul = [&](int i, const bf16x8& a, const bf16x8& b) {
+            if constexpr (NSEG == 2) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, a, acc[i][j], 0, 0, 0);
+            else acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[i][j], 0, 0, 0);
+          };
 #pragma unroll
-          for (int i = 0; i < MI; ++i)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bl, __builtin_bit_cast(bf16x8, fa[i][0]), acc[i][j], 0, 0, 0);
+          for (int i = 0; i < MI; ++i) mul(i, __builtin_bit_cast(bf16x8, fa[i][0]), bl);
 #pragma unroll
-          for (int i = 0; i < MI; ++i)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bh, __builtin_bit_cast(bf16x8, fa[i][1]), acc[i][j], 0, 0, 0);
+          for (int i = 0; i < MI; ++i) mul(i, __builtin_bit_cast(bf16x8, fa[i][1]), bh);
 #pragma unroll
-          for (int i = 0; i < MI; ++i)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bh, __builtin_bit_cast(bf16x8, fa[i][0]), acc[i][j], 0, 0, 0);
+          for (int i = 0; i < MI; ++i) mul(i, __builtin_bit_cast(bf16x8, fa[i][0]), bh);
         }
         __builtin_amdgcn_s_setprio(0);
       }
       cur = cur == NS - 1 ? 0 : cur + 1;
       nxt = nxt == NS - 1 ? 0 : nxt + 1;
     }
-    if constexpr (MI > 0 && NJ > 0) store_blocks<NSEG == 4, MI, NJ>(acc, rw, rb0 * 32, cb0 * 32, rows, ldw4);
+    if constexpr (MI > 0 && NJ > 0) {
+      if constexpr (NSEG == 2) store_blocks<MI, NJ>(acc, rw, rb0 * 32, cb0 * 32, rows, ldw4, m0, v);
+      else store_slice<MI, NJ>(acc, rw, rb0 * 32, cb0 * 32, cols, ldw4);
+    }
   }
   template <int MI>
   __device__ __forceinline__ void run_n(const Feed<NSEG, 32>& feed) const {
@@ -632,6 +708,22 @@ __global__ __launch_bounds__(256, MB == 3 ? 2 : 3) void k_triples_w_bf3(TripW t)
   else tile.template run_n<1>(feed);
 }
 
+// adds N blocks of a wave of the FP32 slices to W (the tile's first element; panels of ldw elements): row block rb, column
+// blocks cb, cb + 1, ...; element e of lane l at row 4 (l / 16) + e, column l % 16: a panel holds all four rows
+template <int N>
+__device__ __forceinline__ void add_rows4(float* W, const f32x4* blk, int rb, int cb, int rows, int cols, int ldw) {
+  const int lane = threadIdx.x & 63, row = 16 * rb + 4 * (lane >> 4), col = 16 * cb + (lane & 15);
+  float* const Wr = W + ldw * (row >> 3) + (row & 7) + 8 * col;
+  f32x4 dv[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j)
+    dv[j] = *reinterpret_cast<const f32x4*>(row < rows && col + 16 * j < cols ? Wr + 128 * j : W);
+#pragma unroll
+  for (int j = 0; j < N; ++j) dv[j] += blk[j];
+#pragma unroll
+  for (int j = 0; j < N; ++j)
+    if (row < rows && col + 16 * j < cols) *reinterpret_cast<f32x4*>(Wr + 128 * j) = dv[j];
+}
 // FP64 and FP32: tiles of 16 NB x 16 NB, a wavefront per 16-row block (NB column blocks), and at NB = 5 and 6 four
 // wavefronts that share the last rows' blocks: the SIMDs of a CU are dealt a workgroup's wavefronts in order, so a fifth
 // would always land with the first (matrix pipes busy 53 % of the time at NB = 5 with five, 63 % at NB = 6 with six;
@@ -657,21 +749,25 @@ __global__ __launch_bounds__(64 * triples_w_waves(NB), NB == 6 ? 3 : NB > 3 ? 4 
   const int nst = NSEG * (t.nd / 8) * GB / 64;
   // pieces of 16 rows: wid and, of NB = 5 and 6, wid + 4
   const bool second = NB > 4 && wid + 4 < NB;
-  int lofa[2], lofb[2];
+  int lofa[2], lofb[2], ava[2], avb[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int r = 16 * (wid + 4 * h) + copy_row<GB>(lane);
     lofa[h] = 16 * copy_unit<GB>(lane) + GB * min(r, rows - 1);
     lofb[h] = 16 * copy_unit<GB>(lane) + tl.col_off(min(r, cols - 1));
+    ava[h] = (int)feed.template av_at<true>(lofa[h]);
+    avb[h] = (int)feed.template av_at<false>(lofb[h]);
   }
   auto dma = [&](int slot) {
-    feed.step([&](__amdgpu_buffer_rsrc_t rsa, __amdgpu_buffer_rsrc_t rsb, int dga, int dgb) {
+    feed.step([&](__amdgpu_buffer_rsrc_t rsa, __amdgpu_buffer_rsrc_t rsb, int dga, int dgb, bool odd) {
       char* d = ring + slot * SLOT + wid * 1024;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_vptr)d, 16, (unsigned)(lofa[0] + dga), 0, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsb, (lds_vptr)(d + ABYTES), 16, (unsigned)(lofb[0] + dgb), 0, 0, 0);
-      if (second) {
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_vptr)(d + 4096), 16, (unsigned)(lofa[1] + dga), 0, 0, 0);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsb, (lds_vptr)(d + 4096 + ABYTES), 16, (unsigned)(lofb[1] + dgb), 0, 0, 0);
+#pragma unroll
+      for (int h = 0; h < (NB > 4 ? 2 : 1); ++h) {
+        if (h == 1 && !second) break;
+        const unsigned oa = (unsigned)((NSEG == 4 && !odd ? ava[h] : lofa[h]) + dga);
+        const unsigned ob = (unsigned)((NSEG == 4 && odd ? avb[h] : lofb[h]) + dgb);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_vptr)(d + 4096 * h), 16, oa, 0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsb, (lds_vptr)(d + 4096 * h + ABYTES), 16, ob, 0, 0, 0);
       }
     });
   };
@@ -707,8 +803,10 @@ __global__ __launch_bounds__(64 * triples_w_waves(NB), NB == 6 ? 3 : NB > 3 ? 4 
       T ta[KL], tb[KL];
       __builtin_memcpy(ta, &ua, 16);
       __builtin_memcpy(tb, &ub, 16);
-      // B as the first operand, so that the accumulator's lanes run along the rows of W
-      if constexpr (F32) c = __builtin_amdgcn_mfma_f32_16x16x4f32(tb[q], ta[q], c, 0, 0, 0);
+      // B as the first operand, so that the accumulator's lanes run along the rows of W; the FP32 slices A, so that
+      // they run along its columns and a lane's four registers are four rows of a panel
+      if constexpr (F32 && NSEG == 4) c = __builtin_amdgcn_mfma_f32_16x16x4f32(ta[q], tb[q], c, 0, 0, 0);
+      else if constexpr (F32) c = __builtin_amdgcn_mfma_f32_16x16x4f32(tb[q], ta[q], c, 0, 0, 0);
       else c = __builtin_amdgcn_mfma_f64_16x16x4f64(tb[q], ta[q], c, 0, 0, 0);
     };
 #pragma unroll
@@ -730,19 +828,22 @@ __global__ __launch_bounds__(64 * triples_w_waves(NB), NB == 6 ? 3 : NB > 3 ? 4 
     cur = cur == NS - 1 ? 0 : cur + 1;
     nxt = nxt == NS - 1 ? 0 : nxt + 1;
   }
-  // register e of lane l of a block: row l % 16, column (l / 16) + 4 e (FP64) or 4 (l / 16) + e (FP32)
+  // register e of lane l of a block: row l % 16, column (l / 16) + 4 e (FP64) or 4 (l / 16) + e (FP32); FP32 slices:
+  // row 4 (l / 16) + e, column l % 16
   T* const W = static_cast<T*>(t.w) + tl.woff;
   const int ldw = (int)tl.ldw;
   auto put = [&](auto& blk, auto n, int rb, auto cb) {
     constexpr int N = decltype(n)::value;
     const int row = 16 * rb + (lane & 15);
     auto col = [&](int j, int e) { return 16 * cb(j) + (F32 ? 4 * (lane >> 4) + e : (lane >> 4) + 4 * e); };
+    const int r0 = NSEG == 4 ? ldw * (row >> 3) + (row & 7) : row < rows ? plane_at(tl.v, tl.m0 + row) : 0;
+    auto at = [&](int j, int e) { return r0 + (NSEG == 4 ? 8 : ldw) * col(j, e); };
     if constexpr (NSEG == 4) {
       T dv[N][4];
 #pragma unroll
       for (int j = 0; j < N; ++j)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) dv[j][e] = W[row < rows && col(j, e) < cols ? row + ldw * col(j, e) : 0];
+        for (int e = 0; e < 4; ++e) dv[j][e] = W[row < rows && col(j, e) < cols ? at(j, e) : 0];
 #pragma unroll
       for (int j = 0; j < N; ++j)
 #pragma unroll
@@ -752,13 +853,22 @@ __global__ __launch_bounds__(64 * triples_w_waves(NB), NB == 6 ? 3 : NB > 3 ? 4 
     for (int j = 0; j < N; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if (row < rows && col(j, e) < cols) W[row + ldw * col(j, e)] = blk[j][e];
+        if (row < rows && col(j, e) < cols) W[at(j, e)] = blk[j][e];
   };
-  put(acc, std::integral_constant<int, NB>(), wid, [](int j) { return j; });
-  if constexpr (NB == 6) put(accx, std::integral_constant<int, 3>(), xr, [&](int j) { return xc + j; });
-  if constexpr (NB == 5) {
-    if (last) put(accx, std::integral_constant<int, 2>(), 4, [&](int j) { return j ? 4 : wid; });
-    else put(accx, std::integral_constant<int, 1>(), 4, [&](int) { return wid; });
+  if constexpr (F32 && NSEG == 4) {
+    add_rows4<NB>(W, acc, wid, 0, rows, cols, ldw);
+    if constexpr (NB == 6) add_rows4<3>(W, accx, xr, xc, rows, cols, ldw);
+    if constexpr (NB == 5) {
+      add_rows4<1>(W, accx, 4, wid, rows, cols, ldw);
+      if (last) add_rows4<1>(W, accx + 1, 4, 4, rows, cols, ldw);
+    }
+  } else {
+    put(acc, std::integral_constant<int, NB>(), wid, [](int j) { return j; });
+    if constexpr (NB == 6) put(accx, std::integral_constant<int, 3>(), xr, [&](int j) { return xc + j; });
+    if constexpr (NB == 5) {
+      if (last) put(accx, std::integral_constant<int, 2>(), 4, [&](int j) { return j ? 4 : wid; });
+      else put(accx, std::integral_constant<int, 1>(), 4, [&](int) { return wid; });
+    }
   }
 }
 
@@ -767,17 +877,19 @@ __global__ __launch_bounds__(64 * triples_w_waves(NB), NB == 6 ? 3 : NB > 3 ? 4 
 // V = W + T1p[a,i] (jb|kc) + (ia|kc) T1p[b,j] + (ia|jb) T1p[c,k] (ijk.jl:116) and the sums S+ of V and W+ of W
 // over the even orderings (abc, bca, cab) and S-, W- over the odd ones (acb, bac, cba),
 //     Ef = 3 sum_p W_p V_p + W+ (S+ - 2 S-) + W- (S- - 2 S+)                    (ijk.jl:129-132)
-// over D_abc, times (2 - d_ij - d_jk); a=b=c terms vanish.  W[a,b,c] of a W slot has a fastest
-// (W + a + v*b + v^2*c + v^3*slot).  The virtual space is cut into 8x8x8 cubes; one workgroup takes an orbit
+// over D_abc, times (2 - d_ij - d_jk); a=b=c terms vanish.  W slots are v planes (a, b), c
+// slowest, each in panels of 8 a.  The virtual space is cut into 8x8x8 cubes; one workgroup takes an orbit
 // {A,B,C} (A>=B>=C) of cube blocks for a run of consecutive k: the six permuted cubes and the (jb|kc) and (ia|kc)
 // blocks are copied straight into LDS, and a thread owns two elements (a,b,c) with all six orderings, so the
 // denominator, its reciprocal and the sums are formed once per six elements of W and V never leaves the
 // registers.  What does not depend on k ((ia|jb) and T1 of i and j) stays in registers.  Per k a thread reads all it
 // needs from LDS, and the copies of the next k run while it computes (an LDS read behind a copy in flight
 // would be made to wait for it).
-// o = 40, v = 190, FP32 W: 169 ms per (T) against 260 with one ordering per thread, V cubes in LDS and a
-// reciprocal per element (o = 27, v = 131 17.7 against 27.8; FP64 o = 16, v = 76 1.0 against 1.5).  Bound by the
-// fetch: 314 GB of W and as much again of (ia|jb) blocks that miss the L2, about 4 TB/s together.
+// o = 40, v = 190, FP32 W: 114 ms per (T), 2.8 TB/s of W (162 with a fastest over all of v in W, rows of 8 a being
+// a quarter of a cache line, and all nine (ia|jb) blocks of a pair copied; 260 with one ordering per thread, V cubes in
+// LDS and a reciprocal per element); o = 27, v = 131 13.1 (17.7, 27.8); FP64 o = 16, v = 76 0.83 (0.96, 1.5).  Bound by
+// latency: three workgroups per CU (153 registers; four, 128, spill: 220 ms) wait for their copies a third of the
+// time; the vector units are busy for another third, LDS for as much.
 static constexpr int CT = 8, CT3 = CT * CT * CT;
 
 // LDS position of element (x, y, z) of a W cube: a Latin-square swizzle under which every x-, y- and z-plane of
@@ -803,7 +915,7 @@ __global__ __launch_bounds__(256, 3) void k_triples_energy(int o, int v, const i
                                                            double* __restrict__ partials) {
   constexpr int ED = (int)sizeof(TW) / 4;  // dwords of a W element
   __shared__ __attribute__((aligned(16))) TW Wl[6 * CT3];
-  __shared__ __attribute__((aligned(16))) double s_vv[2][10][CT * CT];  // [(jk) (ik)][3 x + y (9: unused)][x + 8 y]
+  __shared__ __attribute__((aligned(16))) double s_vv[2][6][CT * CT];  // [(jk) (ik)][ab ba ac ca bc cb][x + 8 y]
   __shared__ double red[4];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -813,9 +925,10 @@ __global__ __launch_bounds__(256, 3) void k_triples_energy(int o, int v, const i
   const int ob = (w & 7) * (nwg >> 3) + min(w & 7, nwg & 7) + (w >> 3);
   const int4 run = runs[2 * blockIdx.y];
   const int i = run.x, j = run.y, k0 = run.z, nk = run.w;
-  const int64_t vv = (int64_t)v * v;
-  const TW* W = Wc + vv * v * runs[2 * blockIdx.y + 1].x;
+  const int64_t pl = triples_plane(v);
+  const TW* W = Wc + pl * v * runs[2 * blockIdx.y + 1].x;
   const int blk[3] = {orbits[3 * ob], orbits[3 * ob + 1], orbits[3 * ob + 2]};
+  auto blk_of = [&](unsigned q) { return q == 0 ? blk[0] : q == 1 ? blk[1] : blk[2]; };
   // the six orderings of the orbit's blocks: (abc) (acb) (bac) (bca) (cab) (cba)
   constexpr int pb[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
   // (ia|jb) of occupied pair (p, q) in 8x8 blocks: vvb + PS (p + o q) + 64 (A + nb B) + x + 8 y
@@ -835,24 +948,26 @@ __global__ __launch_bounds__(256, 3) void k_triples_energy(int o, int v, const i
 #pragma unroll
     for (int q = 0; q < ED; ++q) {
       const int z = wid + 4 * h, pos = (lane + 64 * q) / ED;
-      clo[h][q] = (((pos - z) & 7) + v * (((pos >> 3) - z) & 7)) * (int)sizeof(TW) + 4 * ((lane + 64 * q) % ED);
+      clo[h][q] = (((pos - z) & 7) + 8 * (((pos >> 3) - z) & 7)) * (int)sizeof(TW) + 4 * ((lane + 64 * q) % ED);
     }
-  int vlo[3];
+  int vlo[2];
 #pragma unroll
-  for (int l = 0; l < 3; ++l) {
-    const int q = (wid + 4 * l) % 5, e = min(2 * q + (lane >> 5), 8);
-    vlo[l] = (blk[e / 3] + nb * blk[e % 3]) * 512 + (lane & 31) * 16;
+  for (int l = 0; l < 2; ++l) {
+    constexpr unsigned vx = 0x212010u, vy = 0x120201u;  // blocks of ab, ba, ac, ca, bc, cb, 4 bits each
+    const int e = 4 * (2 * ((wid + 4 * l) % 3) + (lane >> 5));
+    vlo[l] = (blk_of((vx >> e) & 3) + nb * blk_of((vy >> e) & 3)) * 512 + (lane & 31) * 16;
   }
   auto copy = [&](int kk) {
-    const TW* Wk = W + vv * v * kk;
+    const TW* Wk = W + pl * v * kk;
 #pragma unroll
     for (int p = 0; p < 6; ++p) {
-      const int X0 = blk[pb[p][0]] * CT, Y0 = blk[pb[p][1]] * CT, Z0 = blk[pb[p][2]] * CT;
+      const int X = blk[pb[p][0]], Y = blk[pb[p][1]], Z0 = blk[pb[p][2]] * CT;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const int z = wid + 4 * h;
         if (Z0 + z >= v) continue;
-        const __amdgpu_buffer_rsrc_t r = uniform_rsrc(reinterpret_cast<const char*>(Wk + X0 + (int64_t)v * Y0 + vv * (Z0 + z)));
+        const TW* cube = Wk + (int64_t)8 * v * X + 64 * Y + pl * (Z0 + z);
+        const __amdgpu_buffer_rsrc_t r = uniform_rsrc(reinterpret_cast<const char*>(cube));
 #pragma unroll
         for (int q = 0; q < ED; ++q)
           __builtin_amdgcn_raw_ptr_buffer_load_lds(
@@ -862,13 +977,13 @@ __global__ __launch_bounds__(256, 3) void k_triples_energy(int o, int v, const i
     const __amdgpu_buffer_rsrc_t rj = uniform_rsrc(reinterpret_cast<const char*>(vv_jk + PS * o * kk));
     const __amdgpu_buffer_rsrc_t ri = uniform_rsrc(reinterpret_cast<const char*>(vv_ik + PS * o * kk));
 #pragma unroll
-    for (int l = 0; l < 3; ++l) {
+    for (int l = 0; l < 2; ++l) {
       const int q = wid + 4 * l;
-      if (q < 5) {
+      if (q < 3) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rj, (lds_vptr)(&s_vv[0][2 * q][0]), 16, (unsigned)vlo[l], 0, 0, 0);
         asm volatile("; (jk)");
-      } else if (q < 10) {
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(ri, (lds_vptr)(&s_vv[1][2 * (q - 5)][0]), 16, (unsigned)vlo[l], 0, 0, 0);
+      } else if (q < 6) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(ri, (lds_vptr)(&s_vv[1][2 * (q - 3)][0]), 16, (unsigned)vlo[l], 0, 0, 0);
         asm volatile("; (ik)");
       }
     }
@@ -916,16 +1031,16 @@ __global__ __launch_bounds__(256, 3) void k_triples_energy(int o, int v, const i
       wv[h][5] = Wl[5 * CT3 + cube_off(z, y, x)];
     }
     // u = V - W of the six orderings
-    const double jk_ab = s_vv[0][1][x + 8 * y], jk_ba = s_vv[0][3][y + 8 * x];
-    const double ik_ab = s_vv[1][1][x + 8 * y], ik_ba = s_vv[1][3][y + 8 * x];
+    const double jk_ab = s_vv[0][0][x + 8 * y], jk_ba = s_vv[0][1][y + 8 * x];
+    const double ik_ab = s_vv[1][0][x + 8 * y], ik_ba = s_vv[1][1][y + 8 * x];
     double u[2][6];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int z = wid + 4 * h;
-      const double jk_ac = s_vv[0][2][x + 8 * z], jk_ca = s_vv[0][6][z + 8 * x];
-      const double jk_bc = s_vv[0][5][y + 8 * z], jk_cb = s_vv[0][7][z + 8 * y];
-      const double ik_ac = s_vv[1][2][x + 8 * z], ik_ca = s_vv[1][6][z + 8 * x];
-      const double ik_bc = s_vv[1][5][y + 8 * z], ik_cb = s_vv[1][7][z + 8 * y];
+      const double jk_ac = s_vv[0][2][x + 8 * z], jk_ca = s_vv[0][3][z + 8 * x];
+      const double jk_bc = s_vv[0][4][y + 8 * z], jk_cb = s_vv[0][5][z + 8 * y];
+      const double ik_ac = s_vv[1][2][x + 8 * z], ik_ca = s_vv[1][3][z + 8 * x];
+      const double ik_bc = s_vv[1][4][y + 8 * z], ik_cb = s_vv[1][5][z + 8 * y];
       u[h][0] = fma(ia, jk_bc, fma(ik_ac, jb, ij_ab * kc[h]));
       u[h][1] = fma(ia, jk_cb, fma(ik_ab, jc[h], ij_ac[h] * kb));
       u[h][2] = fma(ib, jk_ac, fma(ik_bc, ja, ij_ba * kc[h]));
@@ -1114,7 +1229,7 @@ void triples_col_tiles(const TriplesTiles& t, int v, int i, int j, int k0, int n
 // 114, 108, 106 and 108 ms (at 4096 the W written by the first launch no longer meets the second in the
 // memory-side cache).  FERMIHIP_TRIPLES_CHUNK_MB fixes it, for tests.
 int64_t triples_chunk_slots(int v, int elem, const TriplesTiles& tt, int64_t ntot) {
-  const int64_t slot = (int64_t)v * v * v * elem, tiles = (int64_t)tt.nt * tt.nt * v;
+  const int64_t slot = triples_plane(v) * v * elem, tiles = (int64_t)tt.nt * tt.nt * v;
   int64_t n = std::max(((int64_t)1 << 30) / slot, (2048 + tiles - 1) / tiles);
   if (const char* env = std::getenv("FERMIHIP_TRIPLES_CHUNK_MB")) n = (std::max<int64_t>(1, std::atoll(env)) << 20) / slot;
   n = std::min(n, std::min<int64_t>((int64_t)8e9 / slot, 60000));  // 60000: the energy launch's grid
@@ -1158,7 +1273,7 @@ static TripW trip_args(int fmt, int o, int v, const TriplesOperands& op, void* W
   t.v = v;
   t.nd = (int)triples_pitch_elems(o, v);
   // offsets inside a k step of an operand tile and inside an output tile are 32-bit byte offsets
-  FH_CHECK((int64_t)v * v * 192 * (fmt == 2 ? 4 : 1) < ((int64_t)1 << 31) &&
+  FH_CHECK(triples_plane(v) * 192 * (fmt == 2 ? 4 : 1) < ((int64_t)1 << 31) &&
                (192 + 2 * (int64_t)v) * t.nd * 8 < ((int64_t)1 << 31),
            -3, "(T) W build: a tile exceeds 32-bit offsets");
   return t;

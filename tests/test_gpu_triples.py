@@ -45,3 +45,9 @@ def test_triples_chunks(mb, monkeypatch):
     """Chunks of 1 or 3 MiB of W: at v = 30 4 and 14 slots (FP64), 9 and 29 (FP32), cutting the runs of k (up to 8)."""
     monkeypatch.setenv("FERMIHIP_TRIPLES_CHUNK_MB", mb)
     run(8, 30, 5)
+
+
+@pytest.mark.parametrize("o,v", [(3, 4), (2, 5), (3, 20), (3, 29), (2, 46), (3, 78), (2, 100), (2, 196), (2, 203)])
+def test_triples_last_panel(o, v):
+    """W's planes lie in panels of 8 a: every v % 8, with the last panel alone, in a tile of its own and behind others."""
+    run(o, v, 5 * o + v)
