@@ -216,6 +216,11 @@ int64_t mp2_partials(int o, int v);
 void mp2_pair_energy(hipStream_t s, int o, int v, int Q, const double* Bov, const double* eo, const double* ev,
                      double* partials);
 
+// Symmetric A (n x n, its upper triangle) -> T (d, e) = Q^T A Q, the reflectors of Q in the columns of V [n, n] and
+// tau (fh_eigen.hip); out = Q Z
+inline bool tridiag_fits(int n) { return n >= 3 && n <= 160; }
+void tridiag(hipStream_t s, int n, const double* A, double* V, double* d, double* e, double* tau);
+void tridiag_apply(hipStream_t s, int n, const double* V, const double* tau, const double* Z, double* out);
 // SCF: out = U diag(w)^-1/2 (n x n, column-major); GWH guess Fock matrix (RHFHelper.jl:44-51)
 void scale_cols_rsqrt(hipStream_t s, int n, const double* U, const double* w, double* out);
 void gwh_fock(hipStream_t s, int n, const double* S, const double* H, double* F);

@@ -9,7 +9,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), "csrc")
 LIB = os.path.join(HERE, "libfermihip.so")
-SOURCES = ["fh_gemm.hip", "fh_gemm_bf3.hip", "fh_kernels.hip", "fh_triples.hip", "fh_mp2.hip", "fh_mlp.hip", "fh_integrals.hip", "fh_engine.cpp"]
+SOURCES = ["fh_gemm.hip", "fh_gemm_bf3.hip", "fh_kernels.hip", "fh_triples.hip", "fh_mp2.hip", "fh_mlp.hip", "fh_eigen.hip", "fh_integrals.hip", "fh_engine.cpp"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     # keep hipcc from emitting packed-FP32 instructions in device code
