@@ -1417,14 +1417,14 @@ static void solve(Ctx& c, const fh_cc_opts& op, fh_cc_result& res) {
 }
 
 // ------------------------------------------------------------------ (T), ijk.jl:20-150
-__global__ void k_accumulate(int64_t n, const double* __restrict__ partials, double* __restrict__ acc) {
+__global__ __launch_bounds__(1024) void k_accumulate(int64_t n, const double* __restrict__ partials, double* __restrict__ acc) {
   // single block; fixed order -> deterministic
-  __shared__ double red[256];
+  __shared__ double red[1024];
   double t = 0.0;
-  for (int64_t i = threadIdx.x; i < n; i += 256) t += partials[i];
+  for (int64_t i = threadIdx.x; i < n; i += 1024) t += partials[i];
   red[threadIdx.x] = t;
   __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
+  for (int st = 512; st > 0; st >>= 1) {
     if ((int)threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
     __syncthreads();
   }
@@ -1563,7 +1563,7 @@ static double triples_t(Ctx& c, bool bf3, int64_t t0 = 0, int64_t nt = -1) {
     Timer te(c, "triples_energy" + sfx, 0.0, (double)sizeof(T) * (double)v3 * (double)ch.nslot);
     triples_energy(c.s, (int)o, (int)v, ch.nerun, dtab + ch.eruns, W, (int)norb, static_cast<const int*>(orbits.p),
                    T1p.d(), vvb.d(), c.eo.d(), c.ev.d(), part.d());
-    hipLaunchKernelGGL(k_accumulate, dim3(1), dim3(256), 0, c.s, norb * ch.nerun, part.d(), acc.d());
+    hipLaunchKernelGGL(k_accumulate, dim3(1), dim3(1024), 0, c.s, norb * ch.nerun, part.d(), acc.d());
     FH_HIP(hipGetLastError());
   }
   const double Et = read_scalar(c, acc.d());

@@ -882,20 +882,25 @@ __global__ __launch_bounds__(64 * triples_w_waves(NB), NB == 6 ? 3 : NB > 3 ? 4 
 // {A,B,C} (A>=B>=C) of cube blocks for a run of consecutive k: the six permuted cubes and the (jb|kc) and (ia|kc)
 // blocks are copied straight into LDS, and a thread owns two elements (a,b,c) with all six orderings, so the
 // denominator, its reciprocal and the sums are formed once per six elements of W and V never leaves the
-// registers.  What does not depend on k ((ia|jb) and T1 of i and j) stays in registers.  Per k a thread reads all it
-// needs from LDS, and the copies of the next k run while it computes (an LDS read behind a copy in flight
-// would be made to wait for it).
-// o = 40, v = 190, FP32 W: 114 ms per (T), 2.8 TB/s of W (162 with a fastest over all of v in W, rows of 8 a being
-// a quarter of a cache line, and all nine (ia|jb) blocks of a pair copied; 260 with one ordering per thread, V cubes in
-// LDS and a reciprocal per element); o = 27, v = 131 13.1 (17.7, 27.8); FP64 o = 16, v = 76 0.83 (0.96, 1.5).  Bound by
-// latency: three workgroups per CU (153 registers; four, 128, spill: 220 ms) wait for their copies a third of the
-// time; the vector units are busy for another third, LDS for as much.
+// registers.  What does not depend on k ((ia|jb) and T1 of i and j) stays in registers.  A turn is two k (FP64 W: one): a
+// thread reads all it needs of a k from LDS, and the copies of the next turn run while it computes the last k (an LDS
+// read behind a copy in flight would be made to wait for it).
+// o = 40, v = 190, FP32 W: 95 ms per (T), 3.3 TB/s of W (114 with a k a turn and copies of a dword per lane, 162 with a
+// fastest over all of v in W, rows of 8 a being a quarter of a cache line, and all nine (ia|jb) blocks of a pair copied,
+// 260 with one ordering per thread, V cubes in LDS and a reciprocal per element); o = 27, v = 131 10.7 (13.1, 17.7, 27.8);
+// FP64 o = 16, v = 76 0.72 (0.83, 0.96, 1.5).  Bound by the copies' latency: three workgroups per CU (144 registers; at
+// 128, for four, the compiler's schedule takes 160 ms); the vector units are busy for a third of the time, LDS for a quarter.
 static constexpr int CT = 8, CT3 = CT * CT * CT;
 
-// LDS position of element (x, y, z) of a W cube: a Latin-square swizzle under which every x-, y- and z-plane of
-// the cube covers 64 distinct positions modulo 64, so that the six permuted reads (each a plane with one
-// index fixed) have no bank conflicts.
-__device__ __forceinline__ int cube_off(int x, int y, int z) { return 64 * z + ((x + z) & 7) + 8 * ((y + z) & 7); }
+// LDS position of element (x, y, z) of a W cube, in units of 16 bytes (4 or 2 elements along x, a lane's share of a
+// copy): planes of z, in which the rows turn with z and the units of a row with y.  The reads of a plane with z or y
+// fixed are free of bank conflicts, those with x fixed take four passes for FP32 (a unit's four elements fall on
+// different banks) and none more for FP64.
+template <typename TW>
+__device__ __forceinline__ int cube_off(int x, int y, int z) {
+  constexpr int EU = 16 / (int)sizeof(TW), HN = 8 / EU;
+  return 64 * z + 8 * ((y + z) & 7) + EU * ((x / EU) ^ (y & (HN - 1))) + x % EU;
+}
 
 // 1/d by the hardware reciprocal and two Newton steps (relative error ~1 ulp; d is a negative
 // orbital-energy denominator, never zero, denormal or infinite)
@@ -913,14 +918,18 @@ __global__ __launch_bounds__(256, 3) void k_triples_energy(int o, int v, const i
                                                            const double* __restrict__ t1p, const double* __restrict__ vvb,
                                                            const double* __restrict__ eo, const double* __restrict__ ev,
                                                            double* __restrict__ partials) {
-  constexpr int ED = (int)sizeof(TW) / 4;  // dwords of a W element
-  __shared__ __attribute__((aligned(16))) TW Wl[6 * CT3];
-  __shared__ __attribute__((aligned(16))) double s_vv[2][6][CT * CT];  // [(jk) (ik)][ab ba ac ca bc cb][x + 8 y]
+  // units of 16 bytes: elements, units of a row, planes of a copy instruction, instructions of a cube
+  constexpr int EU = 16 / (int)sizeof(TW), HN = 8 / EU, PZ = 8 / HN, NI = 8 / PZ;
+  // values of k a turn: FP32 W has room for two in LDS with three workgroups per CU
+  constexpr int KD = sizeof(TW) == 4 ? 2 : 1;
+  __shared__ __attribute__((aligned(16))) TW Wl[KD][6 * CT3];
+  __shared__ __attribute__((aligned(16))) double s_t1[KD][32];  // T1 of k: 8 a, b, c (and 8 unused)
+  __shared__ __attribute__((aligned(16))) double s_vv[KD][2][6][CT * CT];  // [(jk) (ik)][ab ba ac ca bc cb][x + 8 y]
   __shared__ double red[4];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // consecutive workgroups go to different XCDs: give each XCD a contiguous range of orbits, so
-  // the neighbouring cubes of concurrently resident orbits share the W lines in its L2
+  // consecutive workgroups go to different XCDs: give each XCD a contiguous range of orbits, so that concurrently
+  // resident orbits share their (ia|jb) blocks in its L2
   const int nwg = gridDim.x, w = blockIdx.x;
   const int ob = (w & 7) * (nwg >> 3) + min(w & 7, nwg & 7) + (w >> 3);
   const int4 run = runs[2 * blockIdx.y];
@@ -929,8 +938,8 @@ __global__ __launch_bounds__(256, 3) void k_triples_energy(int o, int v, const i
   const TW* W = Wc + pl * v * runs[2 * blockIdx.y + 1].x;
   const int blk[3] = {orbits[3 * ob], orbits[3 * ob + 1], orbits[3 * ob + 2]};
   auto blk_of = [&](unsigned q) { return q == 0 ? blk[0] : q == 1 ? blk[1] : blk[2]; };
-  // the six orderings of the orbit's blocks: (abc) (acb) (bac) (bca) (cab) (cba)
-  constexpr int pb[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
+  // the six orderings of the orbit's blocks, (abc) (acb) (bac) (bca) (cab) (cba): 2 bits an index, 6 an ordering
+  constexpr uint64_t pb = 0x192261624ull;
   // (ia|jb) of occupied pair (p, q) in 8x8 blocks: vvb + PS (p + o q) + 64 (A + nb B) + x + 8 y
   const int nb = (v + CT - 1) / CT;
   const int64_t PS = (int64_t)nb * nb * CT * CT;
@@ -938,18 +947,14 @@ __global__ __launch_bounds__(256, 3) void k_triples_energy(int o, int v, const i
   const double* vv_ik = vvb + PS * (i + (int64_t)o * k0);
   const double* vv_ij = vvb + PS * (i + (int64_t)o * j);
 
-  // Copies of a k.  W: planes z = wid, wid + 4 of the six cubes, a dword per lane and instruction (ED per plane and
-  // element), lane -> LDS position -> (x, y).  vv: two 512-byte blocks per instruction.
-  // Rows and columns beyond v are copied as they lie (the caller pads the end of W): the elements that would
-  // use them are dropped.
-  int clo[2][ED];
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int q = 0; q < ED; ++q) {
-      const int z = wid + 4 * h, pos = (lane + 64 * q) / ED;
-      clo[h][q] = (((pos - z) & 7) + 8 * (((pos >> 3) - z) & 7)) * (int)sizeof(TW) + 4 * ((lane + 64 * q) % ED);
-    }
+  // Copies of a k.  W: PZ planes of a cube per instruction, lane -> LDS position -> (y, z) and unit of the row; planes
+  // beyond v lie behind the slot's end, where the resource ends, rows and columns beyond v are copied as they lie: the
+  // elements that would use them are dropped.  vv: two 512-byte blocks per instruction.
+  int clo;
+  {
+    const int z = PZ * (wid % NI) + lane / (8 * HN), t = lane % (8 * HN), y = (t / HN - z) & 7, h = (t % HN) ^ (y & (HN - 1));
+    clo = (int)((pl * z + 8 * y + EU * h) * (int64_t)sizeof(TW));
+  }
   int vlo[2];
 #pragma unroll
   for (int l = 0; l < 2; ++l) {
@@ -957,22 +962,18 @@ __global__ __launch_bounds__(256, 3) void k_triples_energy(int o, int v, const i
     const int e = 4 * (2 * ((wid + 4 * l) % 3) + (lane >> 5));
     vlo[l] = (blk_of((vx >> e) & 3) + nb * blk_of((vy >> e) & 3)) * 512 + (lane & 31) * 16;
   }
-  auto copy = [&](int kk) {
+  const int tlo = min(lane, 47), t1lo = (int)(blk_of(tlo >> 4) * 8 + ((tlo >> 1) & 7)) * 8 + 4 * (tlo & 1);
+  auto copy = [&](int kk, int u) {
     const TW* Wk = W + pl * v * kk;
 #pragma unroll
-    for (int p = 0; p < 6; ++p) {
-      const int X = blk[pb[p][0]], Y = blk[pb[p][1]], Z0 = blk[pb[p][2]] * CT;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int z = wid + 4 * h;
-        if (Z0 + z >= v) continue;
-        const TW* cube = Wk + (int64_t)8 * v * X + 64 * Y + pl * (Z0 + z);
-        const __amdgpu_buffer_rsrc_t r = uniform_rsrc(reinterpret_cast<const char*>(cube));
-#pragma unroll
-        for (int q = 0; q < ED; ++q)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(
-              r, (lds_vptr)(reinterpret_cast<char*>(Wl) + ((p * CT + z) * ED + q) * 256), 4, (unsigned)clo[h][q], 0, 0, 0);
-      }
+    for (int m = 0; m < 6 * NI / 4; ++m) {
+      const int p = wid / NI + 4 / NI * m;
+      const int64_t at = (int64_t)8 * v * blk_of(pb >> (6 * p) & 3) + 64 * blk_of(pb >> (6 * p + 2) & 3) +
+                         pl * CT * blk_of(pb >> (6 * p + 4) & 3);
+      const int64_t left = (pl * v - at) * (int64_t)sizeof(TW);
+      const __amdgpu_buffer_rsrc_t r = uniform_rsrc(reinterpret_cast<const char*>(Wk + at), (int)min(left, (int64_t)0x7fffffff));
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          r, (lds_vptr)(reinterpret_cast<char*>(Wl[u]) + (p * NI + wid % NI) * 1024), 16, (unsigned)clo, 0, 0, 0);
     }
     const __amdgpu_buffer_rsrc_t rj = uniform_rsrc(reinterpret_cast<const char*>(vv_jk + PS * o * kk));
     const __amdgpu_buffer_rsrc_t ri = uniform_rsrc(reinterpret_cast<const char*>(vv_ik + PS * o * kk));
@@ -980,23 +981,31 @@ __global__ __launch_bounds__(256, 3) void k_triples_energy(int o, int v, const i
     for (int l = 0; l < 2; ++l) {
       const int q = wid + 4 * l;
       if (q < 3) {
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rj, (lds_vptr)(&s_vv[0][2 * q][0]), 16, (unsigned)vlo[l], 0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rj, (lds_vptr)(&s_vv[u][0][2 * q][0]), 16, (unsigned)vlo[l], 0, 0, 0);
         asm volatile("; (jk)");
       } else if (q < 6) {
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(ri, (lds_vptr)(&s_vv[1][2 * (q - 3)][0]), 16, (unsigned)vlo[l], 0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(ri, (lds_vptr)(&s_vv[u][1][2 * (q - 3)][0]), 16, (unsigned)vlo[l], 0, 0, 0);
         asm volatile("; (ik)");
       }
+    }
+    if (wid == 3) {
+      // T1 of k, up to the end of T1
+      const int k = k0 + kk;
+      const __amdgpu_buffer_rsrc_t rt = uniform_rsrc(reinterpret_cast<const char*>(t1p + (int64_t)v * k), 8 * v * (o - k));
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rt, (lds_vptr)(&s_t1[u][0]), 4, (unsigned)t1lo, 0, 0, 0);
     }
   };
   // the thread's two elements: a and b from the lane, c from the wave and h
   const int x = lane & 7, y = lane >> 3;
   const int a = blk[0] * CT + x, b = blk[1] * CT + y;
-  copy(0);
+#pragma unroll
+  for (int u = 0; u < KD; ++u)
+    if (u < nk) copy(u, u);
   auto t1 = [&](int e, int q) { return e < v ? t1p[e + (int64_t)v * q] : 0.0; };
   auto ij = [&](int P, int Q, int r, int q) { return vv_ij[((int64_t)(blk[P] + nb * blk[Q]) << 6) + r + 8 * q]; };
   const double ia = t1(a, i), ib = t1(b, i), ja = t1(a, j), jb = t1(b, j);
   const double ij_ab = ij(0, 1, x, y), ij_ba = ij(1, 0, y, x);
-  double ic[2], jc[2], ij_ac[2], ij_ca[2], ij_bc[2], ij_cb[2], es[2], kc[2];
+  double ic[2], jc[2], ij_ac[2], ij_ca[2], ij_bc[2], ij_cb[2], es[2];
   float wt[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -1011,65 +1020,68 @@ __global__ __launch_bounds__(256, 3) void k_triples_energy(int o, int v, const i
     wt[h] = in ? (a == b || b == c ? 0.5f : 1.0f) : 0.0f;
     es[h] = in ? ev[a] + ev[b] + ev[c] : 0.0;
   }
-  double ka = t1(a, k0), kb = t1(b, k0), acc = 0.0;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) kc[h] = t1(blk[2] * CT + wid + 4 * h, k0);
+  double acc = 0.0;
   const double eij = eo[i] + eo[j];
-  for (int kk = 0; kk < nk; ++kk) {
+  auto one = [&](int kk, int u) {
     const int k = k0 + kk;
-    wait_vmcnt<0>();
-    __syncthreads();
+    const TW* Wu = Wl[u];
+    const double ka = s_t1[u][x], kb = s_t1[u][8 + y], kc[2] = {s_t1[u][16 + wid], s_t1[u][20 + wid]};
     TW wv[2][6];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int z = wid + 4 * h;
-      wv[h][0] = Wl[0 * CT3 + cube_off(x, y, z)];
-      wv[h][1] = Wl[1 * CT3 + cube_off(x, z, y)];
-      wv[h][2] = Wl[2 * CT3 + cube_off(y, x, z)];
-      wv[h][3] = Wl[3 * CT3 + cube_off(y, z, x)];
-      wv[h][4] = Wl[4 * CT3 + cube_off(z, x, y)];
-      wv[h][5] = Wl[5 * CT3 + cube_off(z, y, x)];
+      wv[h][0] = Wu[0 * CT3 + cube_off<TW>(x, y, z)];
+      wv[h][1] = Wu[1 * CT3 + cube_off<TW>(x, z, y)];
+      wv[h][2] = Wu[2 * CT3 + cube_off<TW>(y, x, z)];
+      wv[h][3] = Wu[3 * CT3 + cube_off<TW>(y, z, x)];
+      wv[h][4] = Wu[4 * CT3 + cube_off<TW>(z, x, y)];
+      wv[h][5] = Wu[5 * CT3 + cube_off<TW>(z, y, x)];
     }
-    // u = V - W of the six orderings
-    const double jk_ab = s_vv[0][0][x + 8 * y], jk_ba = s_vv[0][1][y + 8 * x];
-    const double ik_ab = s_vv[1][0][x + 8 * y], ik_ba = s_vv[1][1][y + 8 * x];
-    double u[2][6];
+    // V - W of the six orderings
+    const double jk_ab = s_vv[u][0][0][x + 8 * y], jk_ba = s_vv[u][0][1][y + 8 * x];
+    const double ik_ab = s_vv[u][1][0][x + 8 * y], ik_ba = s_vv[u][1][1][y + 8 * x];
+    double uv[2][6];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int z = wid + 4 * h;
-      const double jk_ac = s_vv[0][2][x + 8 * z], jk_ca = s_vv[0][3][z + 8 * x];
-      const double jk_bc = s_vv[0][4][y + 8 * z], jk_cb = s_vv[0][5][z + 8 * y];
-      const double ik_ac = s_vv[1][2][x + 8 * z], ik_ca = s_vv[1][3][z + 8 * x];
-      const double ik_bc = s_vv[1][4][y + 8 * z], ik_cb = s_vv[1][5][z + 8 * y];
-      u[h][0] = fma(ia, jk_bc, fma(ik_ac, jb, ij_ab * kc[h]));
-      u[h][1] = fma(ia, jk_cb, fma(ik_ab, jc[h], ij_ac[h] * kb));
-      u[h][2] = fma(ib, jk_ac, fma(ik_bc, ja, ij_ba * kc[h]));
-      u[h][3] = fma(ib, jk_ca, fma(ik_ba, jc[h], ij_bc[h] * ka));
-      u[h][4] = fma(ic[h], jk_ab, fma(ik_cb, ja, ij_ca[h] * kb));
-      u[h][5] = fma(ic[h], jk_ba, fma(ik_ca, jb, ij_cb[h] * ka));
+      const double jk_ac = s_vv[u][0][2][x + 8 * z], jk_ca = s_vv[u][0][3][z + 8 * x];
+      const double jk_bc = s_vv[u][0][4][y + 8 * z], jk_cb = s_vv[u][0][5][z + 8 * y];
+      const double ik_ac = s_vv[u][1][2][x + 8 * z], ik_ca = s_vv[u][1][3][z + 8 * x];
+      const double ik_bc = s_vv[u][1][4][y + 8 * z], ik_cb = s_vv[u][1][5][z + 8 * y];
+      uv[h][0] = fma(ia, jk_bc, fma(ik_ac, jb, ij_ab * kc[h]));
+      uv[h][1] = fma(ia, jk_cb, fma(ik_ab, jc[h], ij_ac[h] * kb));
+      uv[h][2] = fma(ib, jk_ac, fma(ik_bc, ja, ij_ba * kc[h]));
+      uv[h][3] = fma(ib, jk_ca, fma(ik_ba, jc[h], ij_bc[h] * ka));
+      uv[h][4] = fma(ic[h], jk_ab, fma(ik_cb, ja, ij_ca[h] * kb));
+      uv[h][5] = fma(ic[h], jk_ba, fma(ik_ca, jb, ij_cb[h] * ka));
     }
-    lds_barrier();  // every wave has read this k
-    const double D0 = eij + eo[k];
-    if (kk + 1 < nk) {
-      copy(kk + 1);
-      ka = t1(a, k + 1);
-      kb = t1(b, k + 1);
+    if (u == KD - 1) {
+      lds_barrier();  // every wave has read these k
 #pragma unroll
-      for (int h = 0; h < 2; ++h) kc[h] = t1(blk[2] * CT + wid + 4 * h, k + 1);
+      for (int q = 0; q < KD; ++q)
+        if (kk + 1 + q < nk) copy(kk + 1 + q, q);
     }
+    const double D0 = eij + eo[k];
     double ak = 0.0;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const double w0 = (double)wv[h][0], w1 = (double)wv[h][1], w2 = (double)wv[h][2], w3 = (double)wv[h][3],
                    w4 = (double)wv[h][4], w5 = (double)wv[h][5];
-      const double v0 = w0 + u[h][0], v1 = w1 + u[h][1], v2 = w2 + u[h][2], v3 = w3 + u[h][3], v4 = w4 + u[h][4],
-                   v5 = w5 + u[h][5];
+      const double v0 = w0 + uv[h][0], v1 = w1 + uv[h][1], v2 = w2 + uv[h][2], v3 = w3 + uv[h][3], v4 = w4 + uv[h][4],
+                   v5 = w5 + uv[h][5];
       const double sp = v0 + v3 + v4, sm = v1 + v2 + v5, wp = w0 + w3 + w4, wm = w1 + w2 + w5;
       const double xx = fma(w0, v0, fma(w1, v1, fma(w2, v2, fma(w3, v3, fma(w4, v4, w5 * v5)))));
       const double ef = fma(3.0, xx, fma(wp, fma(-2.0, sm, sp), wm * fma(-2.0, sp, sm)));
       ak += wt[h] != 0.0f ? (double)wt[h] * ef * rcp_nr(D0 - es[h]) : 0.0;
     }
     acc += (2.0 - (i == j ? 1.0 : 0.0) - (j == k ? 1.0 : 0.0)) * ak;
+  };
+  for (int kk = 0; kk < nk; kk += KD) {
+    wait_vmcnt<0>();
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < KD; ++u)
+      if (kk + u < nk) one(kk + u, u);
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
@@ -1083,10 +1095,9 @@ int triples_orbit_count(int v) {
   return nb * (nb + 1) * (nb + 2) / 6;
 }
 
-// The orbits a >= b >= c of 8-wide cubes, in blocks of 4 x 4 x 4 cube indices: a 128-byte line of W holds
-// the rows of four x-adjacent cubes, so a line read for one cube of an orbit is read again by the orbits
-// whose corresponding cube differs in x within the same group of four; with the (at most 64) orbits of
-// a block consecutive, and consecutive orbits on one XCD (k_triples_energy), those reads meet in its L2.
+// The orbits a >= b >= c of 8-wide cubes, in blocks of 4 x 4 x 4 cube indices: the orbits of a block share their
+// (jb|kc) and (ia|kc) blocks, 96 of them for up to 64 orbits of 12 each; with the orbits of a block consecutive, and
+// consecutive orbits on one XCD (k_triples_energy), those reads meet in its L2.
 void triples_orbits(int v, std::vector<int>& out) {
   const int nb = (v + CT - 1) / CT;
   const int ng = (nb + 3) / 4;
@@ -1132,11 +1143,11 @@ void triples_block_vv(hipStream_t s, int o, int v, const double* vvoo, double* v
 }
 
 // k values per workgroup: enough workgroups to fill the chip several times over, and a run of k long enough
-// to amortise the k-independent loads (runs of 1, 2, 4, 8, 16 at o = 40, v = 190: 298, 221, 184, 173, 169 ms;
+// to amortise the k-independent loads (runs of 8, 16, 24, 32 at o = 40, v = 190: 102, 97, 95, 95 ms;
 // FERMIHIP_TRIPLES_KPW = n fixes it, for tuning and for the tests that compare runs of k)
 int triples_energy_kpw(int norb, int nslot) {
   int kpw = 1;
-  while (kpw < 16 && (int64_t)norb * ((nslot + 2 * kpw - 1) / (2 * kpw)) >= 4096) kpw *= 2;
+  while (kpw < 32 && (int64_t)norb * ((nslot + 2 * kpw - 1) / (2 * kpw)) >= 4096) kpw *= 2;
   if (const char* env = std::getenv("FERMIHIP_TRIPLES_KPW")) kpw = std::max(1, std::min(64, std::atoi(env)));
   return kpw;
 }
