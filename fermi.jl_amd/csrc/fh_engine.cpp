@@ -1682,6 +1682,7 @@ static void new_molecule(Ctx& c, int o, int v, int naux, const double* eps_o, co
   c.have_amp = false;
   c.OOOO.reset(); c.OOOV.reset(); c.OOVV.reset(); c.OVOV.reset(); c.OVVV.reset();
   c.LX.reset(); c.LX32.reset(); c.Vs.reset(); c.Vs32.reset(); c.Pt.reset(); c.T1.reset(); c.T2.reset();
+  c.Lkl.reset(); c.Okl.reset(); c.Lo1.reset(); c.L1.reset();
   c.Boo.reset(); c.Bov.reset(); c.Bvv.reset();
   c.opcache.clear(); c.opcache_bytes = 0;
   c.have_model = false; c.pair_d.reset();
