@@ -28,8 +28,8 @@ PREC_NAMES = {"double": "FP64", "mixed": "FP32 MFMA + FP64 polish",
 # HBM bytes per launch of the roofline kernels ((T) W build, PP ladder), from rocprofv3 --pmc
 # FETCH_SIZE / WRITE_SIZE runs scaled by a plain 1 GiB copy (FETCH x 2.0, WRITE x 1.0):
 # profiles/triples_bf16x3_water10_hbm_counters.md
-MEASURED_TRAFFIC = {("water10", "triples_w_slices_bf16x3"): 3.270e9, ("water10", "triples_w_first_bf16x3"): 1.521e9,
-                    ("water10", "ladder_bf16x3"): 17.79e9}
+MEASURED_TRAFFIC = {("water10", "triples_w_slices_bf16x3"): 5.853e9, ("water10", "triples_w_first_bf16x3"): 3.298e9,
+                    ("water10", "ladder_bf16x3"): 5.060e9}
 
 
 def log(*a):
@@ -388,7 +388,7 @@ def main():
     # a span of its own
     launches_per_call = {"ladder": 1, "triples_gemm": 2, "triples_w_first": 1, "triples_w_slices": 1}
     # FP64/FP32 kernel template arguments: BM, BN, BK, TA, TB, waves-per-EU hint, tag, FP32 MFMA,
-    # operand type, output type; bf16x3 kernel: BK, TA, TB, tag, operand type, output type, vector loads, BM;
+    # operand type, output type; bf16x3 kernel: BK, TA, TB, tag, operand type, output type, BM;
     # W build: element type, K segments, 16-wide blocks / K segments, 32-wide blocks of a wavefront
     variants = {
         "": ({"ladder": "k_gemm<64, 64, 16, false, false, 4, 1, false, double, double> (PP ladder, FP64 MFMA)",
@@ -397,7 +397,7 @@ def main():
         "_fp32": ({"ladder": "k_gemm<64, 64, 16, false, false, 4, 1, true, float, double> (PP ladder, FP32 MFMA)",
                    "triples_gemm": "k_triples_w<float, {2|4}, NB> ((T) W build, FP32 MFMA)"},
                   FP32_MFMA_PEAK_TFLOPS, "FP32 MFMA dense"),
-        "_bf16x3": ({"ladder": "k_gemm_bf3<16, false, false, 1, float, double, true, 256> (PP ladder, "
+        "_bf16x3": ({"ladder": "k_gemm_bf3<16, false, false, 1, float, double, 256> (PP ladder, "
                                "split-BF16x3 MFMA, 256 x 128 tiles)",
                      "triples_w_first": "k_triples_w_bf3<2, {2|3}> ((T) W build, first launch: classes abc + bac as "
                                         "one GEMM per run of k with two K segments, split-BF16x3 MFMA)",

@@ -889,7 +889,7 @@ __global__ __launch_bounds__(64 * triples_w_waves(NB), NB == 6 ? 3 : NB > 3 ? 4 
 // fastest over all of v in W, rows of 8 a being a quarter of a cache line, and all nine (ia|jb) blocks of a pair copied,
 // 260 with one ordering per thread, V cubes in LDS and a reciprocal per element); o = 27, v = 131 10.7 (13.1, 17.7, 27.8);
 // FP64 o = 16, v = 76 0.72 (0.83, 0.96, 1.5).  Bound by the copies' latency: three workgroups per CU (144 registers; at
-// 128, for four, the compiler's schedule takes 160 ms); the vector units are busy for a third of the time, LDS for a quarter.
+// 128, for four, the compiler's schedule takes 160 ms); the vector units are busy for a third of the time, LDS for half.
 static constexpr int CT = 8, CT3 = CT * CT * CT;
 
 // LDS position of element (x, y, z) of a W cube, in units of 16 bytes (4 or 2 elements along x, a lane's share of a
