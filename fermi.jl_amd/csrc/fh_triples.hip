@@ -1222,6 +1222,9 @@ TriplesTiles triples_tiles(int fmt, int o, int v, double nk) {
     t.per = t.nb;
   }
   t.per_first = fmt == 2 ? 2 * t.nb_first : t.nb_first;
+  // the columns of a first-launch tile are planes apart and have to fit a buffer resource: tiles of fewer blocks from
+  // v = 1673 on
+  while (fmt == 2 && t.per_first > 1 && triples_plane(v) * t.grain * t.per_first * 4 >= ((int64_t)1 << 31)) --t.per_first;
   t.nt = tiles(v, t.grain, t.per);
   t.nt_first = tiles(vv, t.grain, t.per_first);
   (void)o;
@@ -1271,7 +1274,8 @@ static void launch_w(hipStream_t s, int fmt, int nb, unsigned grid, const TripW&
   FH_HIP(hipGetLastError());
 }
 
-static TripW trip_args(int fmt, int o, int v, const TriplesOperands& op, void* W, const int* slots, const int* cols) {
+static TripW trip_args(int fmt, int o, int v, const TriplesTiles& tt, const TriplesOperands& op, void* W, const int* slots,
+                       const int* cols) {
   TripW t;
   t.av = static_cast<const char*>(op.av);
   t.avs = static_cast<const char*>(op.avs);
@@ -1284,14 +1288,14 @@ static TripW trip_args(int fmt, int o, int v, const TriplesOperands& op, void* W
   t.v = v;
   t.nd = (int)triples_pitch_elems(o, v);
   // offsets inside a k step of an operand tile and inside an output tile are 32-bit byte offsets
-  FH_CHECK(triples_plane(v) * 192 * (fmt == 2 ? 4 : 1) < ((int64_t)1 << 31) &&
+  FH_CHECK(triples_plane(v) * tt.grain * tt.per_first * (fmt == 2 ? 4 : 1) < ((int64_t)1 << 31) &&
                (192 + 2 * (int64_t)v) * t.nd * 8 < ((int64_t)1 << 31),
            -3, "(T) W build: a tile exceeds 32-bit offsets");
   return t;
 }
 void triples_w_first(hipStream_t s, int fmt, int o, int v, const TriplesTiles& tt, const TriplesOperands& op, void* W,
                      const int* cols, int ncol) {
-  TripW t = trip_args(fmt, o, v, op, W, nullptr, cols);
+  TripW t = trip_args(fmt, o, v, tt, op, W, nullptr, cols);
   t.nt = tt.nt_first;
   t.ncol = ncol;
   t.group = 1;
@@ -1301,7 +1305,7 @@ void triples_w_first(hipStream_t s, int fmt, int o, int v, const TriplesTiles& t
 }
 void triples_w_slices(hipStream_t s, int fmt, int o, int v, const TriplesTiles& tt, const TriplesOperands& op, void* W,
                       const int* slots, int nslot) {
-  TripW t = trip_args(fmt, o, v, op, W, slots, nullptr);
+  TripW t = trip_args(fmt, o, v, tt, op, W, slots, nullptr);
   t.nt = tt.nt;
   t.ncol = nslot;
   t.group = kSlotGroup;
