@@ -12,6 +12,7 @@
 // missing partner; spherical components are the normalised real solid harmonics (m = -l .. l) of the
 // table the host passes (fh_integrals_tables).  The Coulomb integrals run in two steps (k_pair_e,
 // k_eri): the E^{ab} of every pair of shells once, then a kernel for each pair of Hermite orders.
+#include "fh_host.h"
 #include "fh_internal.h"
 
 #include <algorithm>
@@ -639,15 +640,13 @@ void eri_launch(hipStream_t s, const EriBuild& b, const int* order, const PairHe
   int lsub = 0;
   while (lsub < 5 && (nb * nk << lsub) < 64 * 1024 && (2 << lsub) <= b.kets[LK][0].np) ++lsub;
   const int64_t nch = (nk + (64 >> lsub) - 1) / (64 >> lsub);
-  FH_CHECK(nk < ((int64_t)1 << 31), -3, "integrals: grid too large");
-  // at most 2^30 workgroups a launch
-  const int64_t per = std::max<int64_t>(1, ((int64_t)1 << 30) / nch);
-  for (int64_t b0 = 0; b0 < nb; b0 += per) {
-    const int64_t m = std::min(per, nb - b0);
-    hipLaunchKernelGGL((k_eri<LAB, LK>), dim3((unsigned)(m * nch)), dim3(64 * eri_waves<LAB>()), 0, s, order + b0, heads,
-                       kets, (int)nk, (int)nch, lsub, E, prim, boys, mode, LAB > LK ? 1 : 0, n, out);
+  constexpr int NT = 64 * eri_waves<LAB>();
+  FH_CHECK(nk < ((int64_t)1 << 31) && nch <= max_workgroups(NT), -3, "integrals: grid too large");
+  for_launches(nb, nch, NT, [&](int64_t b0, int64_t m) {
+    hipLaunchKernelGGL((k_eri<LAB, LK>), dim3((unsigned)(m * nch)), dim3(NT), 0, s, order + b0, heads, kets, (int)nk, (int)nch,
+                       lsub, E, prim, boys, mode, LAB > LK ? 1 : 0, n, out);
     FH_HIP(hipGetLastError());
-  }
+  });
 }
 
 void eri_run(hipStream_t s, Pool* pool, IntScratch& sc, EriBuild& b, const SphTab& tab, int mode, int64_t n, double* out) {
@@ -674,9 +673,11 @@ void eri_run(hipStream_t s, Pool* pool, IntScratch& sc, EriBuild& b, const SphTa
   const char* d = static_cast<const char*>(sc.lists.p);
   const PairHead* heads = reinterpret_cast<const PairHead*>(d + oH);
   double *E = sc.tables.d(), *prim = E + b.ne;
-  hipLaunchKernelGGL(k_pair_e, dim3((unsigned)b.heads.size()), dim3(256), 0, s, heads, reinterpret_cast<const IntShell*>(d + oS),
-                     reinterpret_cast<const double*>(d + oX), reinterpret_cast<const double*>(d + oC), tab, E, prim);
-  FH_HIP(hipGetLastError());
+  for_launches((int64_t)b.heads.size(), 1, 256, [&](int64_t h0, int64_t m) {
+    hipLaunchKernelGGL(k_pair_e, dim3((unsigned)m), dim3(256), 0, s, heads + h0, reinterpret_cast<const IntShell*>(d + oS),
+                       reinterpret_cast<const double*>(d + oX), reinterpret_cast<const double*>(d + oC), tab, E, prim);
+    FH_HIP(hipGetLastError());
+  });
   const double* bt = reinterpret_cast<const double*>(d + oB);
 #define FH_ERI(A_, K_)                                                                                              \
   eri_launch<A_, K_>(s, b, reinterpret_cast<const int*>(d + oO[A_]), heads, reinterpret_cast<const Ket*>(d + oK[K_]), \
