@@ -22,6 +22,7 @@
 // B are neighbours), or -- when A is the larger operand -- in groups of gn N-tiles whose B
 // blocks fit in L2: each group sweeps all M-tiles, so B stays in L2 and A is streamed once
 // per group instead of once per N-tile.
+#include "fh_host.h"
 #include "fh_internal.h"
 
 #include <algorithm>
@@ -245,7 +246,7 @@ static void launch(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha,
                    const TI* B, int64_t ldb, int64_t sB, double beta, const TO* C, int64_t ldc, int64_t sC, TO* D,
                    int64_t ldd, int64_t sD, int64_t batch, int64_t kchunk) {
   const int64_t tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
-  FH_CHECK(tm * tn < (int64_t)1 << 31 && batch < 65536, -3, "gemm grid too large");
+  FH_CHECK(tm * tn <= max_workgroups(256) && batch < 65536, -3, "gemm grid too large");
   dim3 grid((unsigned)(tm * tn), (unsigned)batch, (unsigned)(kchunk > 0 ? (K + kchunk - 1) / kchunk : 1));
   // A larger than B: group N-tiles so that a group's B blocks stay in L2
   int gn = 0;

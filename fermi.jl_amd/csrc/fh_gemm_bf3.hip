@@ -21,6 +21,7 @@
 // across lanes.  The
 // loads are branch-free (clamped rows, masks applied at the LDS store).  Tile order: the
 // XCD-aware remap and the L2-grouped raster of the FP64/FP32 kernel.
+#include "fh_host.h"
 #include "fh_internal.h"
 
 #include <algorithm>
@@ -462,7 +463,7 @@ static void launch_bf3(hipStream_t s, int bm, int64_t M, int64_t N, int64_t K, d
                        int64_t sA, const TI* B, int64_t ldb, int64_t sB, double beta, const TO* C, int64_t ldc,
                        int64_t sC, TO* D, int64_t ldd, int64_t sD, int64_t batch, int64_t kchunk) {
   const int64_t tm = (M + bm - 1) / bm, tn = (N + 127) / 128;
-  FH_CHECK(tm * tn < (int64_t)1 << 31 && batch < 65536, -3, "gemm grid too large");
+  FH_CHECK(tm * tn <= max_workgroups(256) && batch < 65536, -3, "gemm grid too large");
   FH_CHECK(M < ((int64_t)1 << 31) && N < ((int64_t)1 << 31), -3, "gemm: M and N must be below 2^31");
   dim3 grid((unsigned)(tm * tn), (unsigned)batch, (unsigned)(kchunk > 0 ? (K + kchunk - 1) / kchunk : 1));
   int gn = 0;

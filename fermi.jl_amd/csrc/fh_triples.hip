@@ -30,6 +30,7 @@
 // writing 16 l bytes past the wave-uniform LDS address), which costs no registers; a copy instruction carries
 // a piece of 16 rows x 64 bytes.  The ring keeps two k steps in flight behind an explicit vector-memory wait
 // and one barrier per step.
+#include "fh_host.h"
 #include "fh_internal.h"
 
 #include <algorithm>
@@ -240,8 +241,7 @@ __global__ __launch_bounds__(256) void k_triples_av(int o, int v, int nd, const 
                                                     char* __restrict__ avs) {
   constexpr int GB = FMT == 0 ? 64 : 32;
   __shared__ double tile[8][16][33];  // [d'][x + 4 y][n]
-  const int nb = (v + 3) / 4;
-  const int y0 = 4 * (blockIdx.x % nb), x0 = 4 * (blockIdx.x / nb % nb), g = blockIdx.x / (nb * nb);
+  const int y0 = 4 * blockIdx.x, x0 = 4 * blockIdx.y, g = blockIdx.z;
   const int64_t vv = (int64_t)v * v, an = vv * (nd / 8) * GB;
   for (int n0 = 0; n0 < o; n0 += 32) {
     __syncthreads();
@@ -275,8 +275,7 @@ __global__ __launch_bounds__(256) void k_triples_bv(int o, int v, int nd, const 
   constexpr int GB = FMT == 0 ? 64 : 32;
   __shared__ double tile[8][4][33];  // [d'][z][pair]
   const int64_t bs = (int64_t)v * (nd / 8) * GB;
-  const int nz = (v + 3) / 4, ng = nd / 8, oo = o * o;
-  const int z0 = 4 * (blockIdx.x % nz), g = blockIdx.x / nz % ng, s0 = 32 * (int)(blockIdx.x / ((int64_t)nz * ng));
+  const int oo = o * o, z0 = 4 * blockIdx.x, g = blockIdx.y, s0 = 32 * blockIdx.z;
   for (int e = threadIdx.x; e < 8 * 4 * 32; e += 256) {
     const int s = s0 + (e & 31), z = z0 + (e >> 5 & 3), d = 8 * g + (e >> 7);
     double val = 0.0;
@@ -1155,7 +1154,7 @@ int triples_energy_kpw(int norb, int nslot) {
 template <typename TW>
 void triples_energy(hipStream_t s, int o, int v, int nrun, const int* runs, const TW* W, int norb, const int* orbits,
                     const double* t1p, const double* vvb, const double* eo, const double* ev, double* partials) {
-  FH_CHECK(nrun > 0 && nrun < 65536, -3, "(T) energy: too many runs in a launch");
+  FH_CHECK(nrun > 0 && nrun < 65536 && norb <= max_workgroups(256), -3, "(T) energy: too many runs in a launch");
   hipLaunchKernelGGL(k_triples_energy<TW>, dim3((unsigned)norb, (unsigned)nrun), dim3(256), 0, s, o, v,
                      reinterpret_cast<const int4*>(runs), W, orbits, t1p, vvb, eo, ev, partials);
   FH_HIP(hipGetLastError());
@@ -1172,9 +1171,10 @@ int64_t triples_pitch_elems(int o, int v) { return ((int64_t)(v + o) + 7) / 8 * 
 void triples_operands(hipStream_t s, int fmt, int o, int v, const double* ovvv, const double* t2, const double* ooov,
                       void* av, void* avs, void* bvp, void* bvq) {
   const int nd = (int)triples_pitch_elems(o, v);
-  const int64_t n4 = (v + 3) / 4, na = n4 * n4 * (nd / 8), nb = n4 * (nd / 8) * (((int64_t)o * o + 31) / 32);
-  FH_CHECK(na < ((int64_t)1 << 31) && nb < ((int64_t)1 << 31), -3, "(T) operand grid too large");
-  const dim3 ga((unsigned)na), gb((unsigned)nb);
+  // along three axes: as one, v = 1300 has 17 million workgroups, more than an axis takes (max_workgroups)
+  const int64_t n4 = (v + 3) / 4, ng = nd / 8, np = ((int64_t)o * o + 31) / 32;
+  FH_CHECK(n4 < 65536 && ng < 65536 && np < 65536, -3, "(T) operand grid too large");
+  const dim3 ga((unsigned)n4, (unsigned)n4, (unsigned)ng), gb((unsigned)n4, (unsigned)ng, (unsigned)np);
 #define FH_OPS(F)                                                                                                     \
   do {                                                                                                                \
     hipLaunchKernelGGL(k_triples_av<F>, ga, dim3(256), 0, s, o, v, nd, ovvv, t2, (char*)av, (char*)avs);              \
@@ -1251,7 +1251,9 @@ int64_t triples_chunk_slots(int v, int elem, const TriplesTiles& tt, int64_t nto
 }
 
 template <int NSEG>
-static void launch_w(hipStream_t s, int fmt, int nb, unsigned grid, const TripW& t) {
+static void launch_w(hipStream_t s, int fmt, int nb, int64_t g, const TripW& t) {
+  FH_CHECK(g > 0 && g <= max_workgroups(fmt == 2 ? 256 : 64 * triples_w_waves(nb)), -3, "(T) W build: grid too large");
+  const unsigned grid = (unsigned)g;
 #define FH_W(T, NB) hipLaunchKernelGGL((k_triples_w<T, NSEG, NB>), dim3(grid), dim3(64 * triples_w_waves(NB)), 0, s, t)
 #define FH_WT(T)               \
   switch (nb) {                \
@@ -1300,8 +1302,7 @@ void triples_w_first(hipStream_t s, int fmt, int o, int v, const TriplesTiles& t
   t.ncol = ncol;
   t.group = 1;
   const int64_t g = (int64_t)tt.nt_first * ncol;
-  FH_CHECK(g > 0 && g < ((int64_t)1 << 31), -3, "gemm grid too large");
-  launch_w<2>(s, fmt, tt.nb_first, (unsigned)g, t);
+  launch_w<2>(s, fmt, tt.nb_first, g, t);
 }
 void triples_w_slices(hipStream_t s, int fmt, int o, int v, const TriplesTiles& tt, const TriplesOperands& op, void* W,
                       const int* slots, int nslot) {
@@ -1310,8 +1311,7 @@ void triples_w_slices(hipStream_t s, int fmt, int o, int v, const TriplesTiles& 
   t.ncol = nslot;
   t.group = kSlotGroup;
   const int64_t g = (int64_t)tt.nt * tt.nt * v * nslot;
-  FH_CHECK(g > 0 && g < ((int64_t)1 << 31), -3, "gemm grid too large");
-  launch_w<4>(s, fmt, tt.nb, (unsigned)g, t);
+  launch_w<4>(s, fmt, tt.nb, g, t);
 }
 
 }  // namespace fh
