@@ -60,14 +60,26 @@ __global__ __launch_bounds__(512) void k_tridiag(int n, const double* __restrict
   for (int k = n - 1; k >= 1; --k) {
     __syncthreads();
     const double* x = xb[k & 1];
-    const double alpha = x[k - 1];
-    double v[NS], vc[NC], ss = 0.0;
+    double alpha = x[k - 1], v[NS], vc[NC], ss, up = 1.0;
+    auto squares = [&] {
+      ss = 0.0;
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      v[s] = rl + 16 * s < k - 1 ? x[rl + 16 * s] : 0.0;
-      ss = fma(v[s], v[s], ss);
+      for (int s = 0; s < NS; ++s) ss = fma(v[s], v[s], ss);
+      ss = sum16(ss);
+    };
+#pragma unroll
+    for (int s = 0; s < NS; ++s) v[s] = rl + 16 * s < k - 1 ? x[rl + 16 * s] : 0.0;
+    squares();
+    // A column whose squares come near the ends of the exponent's range is taken times a power of two: the coupling of
+    // two molecules far apart, 1e-160 of the rest, has squares of a few bits, with which H is not orthogonal.
+    const double norm2 = fma(alpha, alpha, ss);
+    if (norm2 < 0x1p-900 || norm2 > 0x1p900) {
+      up = norm2 < 1.0 ? 0x1p600 : 0x1p-600;
+      alpha *= up;
+#pragma unroll
+      for (int s = 0; s < NS; ++s) v[s] *= up;
+      squares();
     }
-    ss = sum16(ss);
     double beta = alpha, t = 0.0, sc = 0.0;  // x = 0: H = 1
     if (ss != 0.0) {
       beta = -copysign(sqrt(fma(alpha, alpha, ss)), alpha);
@@ -81,7 +93,7 @@ __global__ __launch_bounds__(512) void k_tridiag(int n, const double* __restrict
       const int c = cl + 32 * j;
       vc[j] = 0.0;
       if (32 * j >= k) continue;
-      vc[j] = c < k - 1 ? x[c] * sc : c == k - 1 ? 1.0 : 0.0;
+      vc[j] = c < k - 1 ? x[c] * up * sc : c == k - 1 ? 1.0 : 0.0;
       double q0 = 0.0, q1 = 0.0;
 #pragma unroll
       for (int s = 0; s < NS; s += 2) {
@@ -98,7 +110,7 @@ __global__ __launch_bounds__(512) void k_tridiag(int n, const double* __restrict
     }
     if (tid == 0) {
       d[k] = x[k];
-      e[k - 1] = beta;
+      e[k - 1] = beta / up;
       tau[k - 1] = t;
     }
     __syncthreads();
