@@ -6,6 +6,7 @@
 // the same function of (T1, T2) and is checked against a term-by-term restatement of that
 // file.  The T2 numerator is accumulated as P and symmetrised at the end,
 // newT2 = P + P[j,i,b,a] (RCCSDHelper.jl:190).
+#include "fh_host.h"
 #include "fh_internal.h"
 #include "../../include/fermihip.h"
 
@@ -96,12 +97,16 @@ struct IterRow {
   bool diis;
 };
 
-// A timed span recorded on the context stream (hipEvent pair), read back at the next
-// synchronisation point by flush_timers so that timing adds no host syncs.
-struct Pending {
-  std::string name;
-  double flops, bytes;
-  hipEvent_t a, b;
+// Timed spans on the context stream, read back at the next synchronisation point by flush_timers; between
+// those, timing waits only for work that many spans have been queued behind.
+struct EventRt {
+  using Event = hipEvent_t;
+  using Stream = hipStream_t;
+  static bool create(Event& e) { return hipEventCreate(&e) == hipSuccess; }
+  static void destroy(Event e) { (void)hipEventDestroy(e); }
+  static bool record(Event e, Stream s) { return hipEventRecord(e, s) == hipSuccess; }
+  static bool wait(Event e) { return hipEventSynchronize(e) == hipSuccess; }
+  static bool elapsed(float& ms, Event a, Event b) { return hipEventElapsedTime(&ms, a, b) == hipSuccess; }
 };
 
 struct BlasHandle {
@@ -187,7 +192,7 @@ struct Ctx {
   double mlp_ys = 0.0;
   bool have_model = false;
   std::map<std::string, Phase> phases;
-  std::vector<Pending> pending;
+  Spans<EventRt> spans;
   std::vector<IterRow> iters;
   double last_energy = 0.0, last_et = 0.0;
 
@@ -195,44 +200,34 @@ struct Ctx {
   int64_t n2() const { return (int64_t)o * o * v * v; }
 };
 
-// RAII span timer (see Pending)
+static auto add_span(Ctx& c) {
+  return [&c](const Spans<EventRt>::Span& p, float ms) {
+    Phase& ph = c.phases[p.name];
+    ph.ms += ms;
+    ph.flops += p.flops;
+    ph.bytes += p.bytes;
+    ph.calls += 1;
+  };
+}
+// RAII span timer
 struct Timer {
   Ctx& c;
-  Pending p;
+  Spans<EventRt>::Span p;
   hipStream_t st;
   Timer(Ctx& cc, const std::string& n, double f = 0.0, double bytes = 0.0, hipStream_t on = nullptr)
       : c(cc), st(on ? on : cc.s) {
     p.name = n;
     p.flops = f;
     p.bytes = bytes;
-    FH_HIP(hipEventCreate(&p.a));
-    FH_HIP(hipEventCreate(&p.b));
-    FH_HIP(hipEventRecord(p.a, st));
+    if (!c.spans.begin(p, st)) throw Error{-2, std::string("HIP event: ") + hipGetErrorString(hipGetLastError())};
   }
-  ~Timer();
+  Timer(const Timer&) = delete;
+  Timer& operator=(const Timer&) = delete;
+  ~Timer() { c.spans.end(p, st, add_span(c)); }
 };
 
-Timer::~Timer() {
-  if (hipEventRecord(p.b, st) == hipSuccess) c.pending.push_back(p);
-  else { (void)hipEventDestroy(p.a); (void)hipEventDestroy(p.b); }
-}
-
 // resolve recorded spans (call after the stream has been synchronised)
-static void flush_timers(Ctx& c) {
-  for (auto& p : c.pending) {
-    float ms = 0.f;
-    if (hipEventSynchronize(p.b) == hipSuccess && hipEventElapsedTime(&ms, p.a, p.b) == hipSuccess) {
-      Phase& ph = c.phases[p.name];
-      ph.ms += ms;
-      ph.flops += p.flops;
-      ph.bytes += p.bytes;
-      ph.calls += 1;
-    }
-    (void)hipEventDestroy(p.a);
-    (void)hipEventDestroy(p.b);
-  }
-  c.pending.clear();
-}
+static void flush_timers(Ctx& c) { c.spans.resolve(SIZE_MAX, add_span(c)); }
 
 static Buf dalloc(Ctx& c, int64_t n) { return Buf(c.pool.get(), (size_t)std::max<int64_t>(n, 1) * sizeof(double)); }
 // Copy of n bytes between the device and pageable host memory in pinned chunks, chunk i by thread i mod 4: the DMA of a

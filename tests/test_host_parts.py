@@ -40,3 +40,83 @@ int main() {
   check(0, 1, 64, 0);
 }
 """)
+
+
+def test_spans_hold_few_events(tmp_path):
+    """A call of 5700 chunks with four spans each inside one: every span is read back once, with its own time, in the
+    order of their ends; the events at hand stay below two for each of 256 spans and the open ones, and none is
+    left. An event that cannot be made or recorded loses no other."""
+    run_cpp(tmp_path, """
+#include <map>
+#include <set>
+static std::set<int> live;
+static size_t most = 0;
+static int made = 0, clock_ = 0, fail_create = -1, fail_record = -1, records = 0, waits = 0;
+static std::map<int, int> at;
+struct Rt {
+  using Event = int;
+  using Stream = int;
+  static bool create(int& e) {
+    if (made == fail_create) return false;
+    e = made++;
+    live.insert(e);
+    most = std::max(most, live.size());
+    return true;
+  }
+  static void destroy(int e) { CHECK(live.erase(e) == 1); }
+  static bool record(int e, int) {
+    CHECK(live.count(e));
+    if (records++ == fail_record) return false;
+    at[e] = ++clock_;
+    return true;
+  }
+  static bool wait(int e) { ++waits; return live.count(e) == 1; }
+  static bool elapsed(float& ms, int a, int b) { ms = (float)(at[b] - at[a]); return true; }
+};
+using S = fh::Spans<Rt>;
+int main() {
+  {
+    S spans;
+    int seen = 0, inner = 0;
+    auto sink = [&](const S::Span& p, float ms) {
+      ++seen;
+      if (p.name == "outer") CHECK(ms == 2 * 4 * 5700 + 1);
+      else { CHECK(p.flops == inner++); CHECK(ms == 1); }
+    };
+    S::Span outer;
+    outer.name = "outer";
+    CHECK(spans.begin(outer, 0));
+    for (int k = 0; k < 4 * 5700; ++k) {
+      S::Span p;
+      p.flops = k;
+      CHECK(spans.begin(p, 0));
+      spans.end(p, 0, sink);
+      CHECK(k - inner <= (int)S::kMax);
+      if (k < (int)S::kMax) CHECK(waits == 0);
+    }
+    spans.end(outer, 0, sink);
+    CHECK(seen < 4 * 5700);
+    spans.resolve(SIZE_MAX, sink);
+    CHECK(seen == 4 * 5700 + 1);
+    CHECK(most <= 2 * (S::kMax + 3));
+  }
+  CHECK(live.empty());
+  for (int f = 0; f < 6; ++f) {
+    S spans;
+    made = records = 0;
+    fail_create = f < 2 ? f : -1;
+    fail_record = f < 2 ? -1 : f - 2;
+    int ok = 0, seen = 0;
+    for (int k = 0; k < 3; ++k) {
+      S::Span p;
+      if (!spans.begin(p, 0)) { fail_create = fail_record = -1; continue; }
+      ++ok;
+      spans.end(p, 0, [](const S::Span&, float) {});
+    }
+    spans.resolve(SIZE_MAX, [&](const S::Span&, float) { ++seen; });
+    CHECK(ok == (f == 3 || f == 5 ? 3 : 2) && seen == 2);
+  }
+  CHECK(live.empty());
+  return 0;
+}
+""")
