@@ -230,9 +230,29 @@ struct Timer {
 static void flush_timers(Ctx& c) { c.spans.resolve(SIZE_MAX, add_span(c)); }
 
 static Buf dalloc(Ctx& c, int64_t n) { return Buf(c.pool.get(), (size_t)std::max<int64_t>(n, 1) * sizeof(double)); }
-// Copy of n bytes between the device and pageable host memory in pinned chunks, chunk i by thread i mod 4: the DMA of a
-// chunk runs while the chunks before it are moved between the pinned buffers and the host memory (whose pages, when it
-// is new, are made by four threads at once instead of one).  For copies of 4 MiB and more; false: not taken (memory that
+struct StagedCopy {
+  static constexpr int kThreads = HostStage::kThreads;
+  static constexpr size_t kChunk = HostStage::kChunk;
+  Ctx& c;
+  char* dev;
+  bool to_host;
+  std::atomic<int> err{(int)hipSuccess};
+  bool ok(hipError_t e) {
+    if (e != hipSuccess) err = (int)e;
+    return e == hipSuccess;
+  }
+  char* buf(int t, int k) { return c.stage->buf[t][k]; }
+  bool enter() { return ok(hipSetDevice(c.device)); }
+  bool start(int t, int k, size_t at, size_t n) {
+    return ok(to_host ? hipMemcpyAsync(buf(t, k), dev + at, n, hipMemcpyDeviceToHost, c.s)
+                      : hipMemcpyAsync(dev + at, buf(t, k), n, hipMemcpyHostToDevice, c.s));
+  }
+  bool mark(int t, int k) { return ok(hipEventRecord(c.stage->ev[t][k], c.s)); }
+  bool wait(int t, int k) { return ok(hipEventSynchronize(c.stage->ev[t][k])); }
+  void drain() { (void)hipStreamSynchronize(c.s); }
+};
+// Copy of n bytes between the device and pageable host memory in pinned chunks (copy_chunked; pages of new host memory
+// are made by four threads at once instead of one).  For copies of 4 MiB and more; false: not taken (memory that
 // the runtime knows, which it copies directly, or no pinned memory).  Returns with the host memory free for other use.
 // (mu nu|la si) of two water molecules, 42 MB into new memory: 4.7 ms with one pageable copy, 2.2 ms so, 0.6 of them
 // kernels.
@@ -252,48 +272,11 @@ static bool copy_staged(Ctx& c, char* dev, char* host, size_t n, bool to_host) {
     }
     c.stage = std::move(made);
   }
-  HostStage& st = *c.stage;
-  constexpr size_t CH = HostStage::kChunk;
-  const size_t nch = (n + CH - 1) / CH;
-  std::atomic<int> err{(int)hipSuccess};
-  auto work = [&](int t) {
-    auto ok = [&](hipError_t e) {
-      if (e != hipSuccess) err = (int)e;
-      return e == hipSuccess;
-    };
-    if (!ok(hipSetDevice(c.device))) return;
-    auto len = [&](size_t i) { return std::min(CH, n - i * CH); };
-    size_t in[2] = {nch, nch};   // chunk in flight in each buffer
-    auto finish = [&](int k) {
-      if (in[k] == nch) return true;
-      if (!ok(hipEventSynchronize(st.ev[t][k]))) return false;
-      if (to_host) std::memcpy(host + in[k] * CH, st.buf[t][k], len(in[k]));
-      in[k] = nch;
-      return true;
-    };
-    int k = 0;
-    for (size_t i = t; i < nch; i += HostStage::kThreads, k ^= 1) {
-      if (!finish(k)) return;
-      if (!to_host) std::memcpy(st.buf[t][k], host + i * CH, len(i));
-      const hipError_t e = to_host ? hipMemcpyAsync(st.buf[t][k], dev + i * CH, len(i), hipMemcpyDeviceToHost, c.s)
-                                   : hipMemcpyAsync(dev + i * CH, st.buf[t][k], len(i), hipMemcpyHostToDevice, c.s);
-      if (!ok(e) || !ok(hipEventRecord(st.ev[t][k], c.s))) return;
-      in[k] = i;
-    }
-    if (finish(k)) finish(k ^ 1);
-  };
-  std::vector<std::thread> th;
-  int started = 1;
-  try {
-    th.reserve(HostStage::kThreads - 1);
-    for (; started < HostStage::kThreads; ++started) th.emplace_back(work, started);
-  } catch (const std::exception&) {
-    // no more threads: this one takes their chunks
+  StagedCopy rt{c, dev, to_host};
+  if (!copy_chunked(rt, host, n, to_host)) {
+    c.stage.reset();
+    FH_HIP((hipError_t)rt.err.load());
   }
-  work(0);
-  for (int t = started; t < HostStage::kThreads; ++t) work(t);
-  for (auto& x : th) x.join();
-  FH_HIP((hipError_t)err.load());
   return true;
 }
 static void h2d(Ctx& c, double* d, const double* h, int64_t n) {

@@ -3,8 +3,11 @@
 #include <algorithm>
 #include <cstddef>
 #include <cstdint>
+#include <cstring>
 #include <deque>
+#include <exception>
 #include <string>
+#include <thread>
 #include <vector>
 
 namespace fh {
@@ -87,5 +90,51 @@ class Spans {
   std::deque<Span> ended_;
   std::vector<typename Rt::Event> free_;
 };
+
+// Copy of n bytes between the device and host memory in chunks of Rt::kChunk through pinned buffers, two a thread, chunk i
+// by thread i mod Rt::kThreads: the DMA of a chunk runs while those before it are moved between the buffers and
+// the host memory. false: a step failed; then too nothing is in flight any more.
+// Rt: char* buf(t, k); bool enter() on a thread's first step, start(t, k, offset, bytes) and mark(t, k) a DMA, wait(t, k) for
+// its mark; void drain() waits for everything started.
+template <typename Rt>
+bool copy_chunked(Rt& rt, char* host, size_t n, bool to_host) {
+  constexpr size_t CH = Rt::kChunk;
+  const size_t nch = (n + CH - 1) / CH;
+  bool good[Rt::kThreads] = {};
+  auto work = [&](int t) {
+    if (!rt.enter()) return;
+    auto len = [&](size_t i) { return std::min(CH, n - i * CH); };
+    size_t in[2] = {nch, nch};   // chunk in flight in each buffer
+    auto finish = [&](int k) {
+      if (in[k] == nch) return true;
+      if (!rt.wait(t, k)) return false;
+      if (to_host) std::memcpy(host + in[k] * CH, rt.buf(t, k), len(in[k]));
+      in[k] = nch;
+      return true;
+    };
+    int k = 0;
+    for (size_t i = t; i < nch; i += Rt::kThreads, k ^= 1) {
+      if (!finish(k)) return;
+      if (!to_host) std::memcpy(rt.buf(t, k), host + i * CH, len(i));
+      if (!rt.start(t, k, i * CH, len(i)) || !rt.mark(t, k)) return;
+      in[k] = i;
+    }
+    good[t] = finish(k) && finish(k ^ 1);
+  };
+  std::vector<std::thread> th;
+  int started = 1;
+  try {
+    th.reserve(Rt::kThreads - 1);
+    for (; started < Rt::kThreads; ++started) th.emplace_back(work, started);
+  } catch (const std::exception&) {
+    // no more threads: this one takes their chunks
+  }
+  work(0);
+  for (int t = started; t < Rt::kThreads; ++t) work(t);
+  for (auto& x : th) x.join();
+  if (std::all_of(good, good + Rt::kThreads, [](bool g) { return g; })) return true;
+  rt.drain();
+  return false;
+}
 
 }  // namespace fh

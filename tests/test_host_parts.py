@@ -120,3 +120,65 @@ int main() {
   return 0;
 }
 """)
+
+
+def test_chunked_copy(tmp_path):
+    """copy_chunked with DMAs that move their bytes as late as they may (at the wait for their mark, or at the drain): both
+    directions, sizes around a chunk and a round of buffers; and with each step failing in turn, no chunk is in flight
+    when it returns."""
+    run_cpp(tmp_path, """
+#include <mutex>
+struct Rt {
+  static constexpr int kThreads = 3;
+  static constexpr size_t kChunk = 16;
+  std::mutex m;
+  char* dev;
+  bool to_host;
+  int fail, step = 0;
+  struct Dma { size_t at = 0, n = 0; bool flying = false; } dma[kThreads][2];
+  char pinned[kThreads][2][kChunk];
+  Rt(char* d, bool h, int f) : dev(d), to_host(h), fail(f) {}
+  bool good() { std::lock_guard<std::mutex> g(m); return step++ != fail; }
+  void land(int t, int k) {
+    Dma& d = dma[t][k];
+    if (d.flying) {
+      if (to_host) std::memcpy(pinned[t][k], dev + d.at, d.n);
+      else std::memcpy(dev + d.at, pinned[t][k], d.n);
+    }
+    d.flying = false;
+  }
+  char* buf(int t, int k) { CHECK(!dma[t][k].flying); return pinned[t][k]; }
+  bool enter() { return good(); }
+  bool start(int t, int k, size_t at, size_t n) {
+    CHECK(!dma[t][k].flying && n > 0 && n <= kChunk);
+    if (!good()) return false;
+    dma[t][k].at = at;
+    dma[t][k].n = n;
+    dma[t][k].flying = true;
+    return true;
+  }
+  bool mark(int, int) { return good(); }
+  bool wait(int t, int k) {
+    if (!good()) return false;
+    land(t, k);
+    return true;
+  }
+  void drain() { for (int t = 0; t < kThreads; ++t) for (int k = 0; k < 2; ++k) land(t, k); }
+};
+int main() {
+  for (bool to_host : {false, true})
+    for (size_t n : {1, 15, 16, 17, 48, 95, 96, 97, 500})
+      for (int fail = -1; ; ++fail) {
+        std::vector<char> dev(n), host(n), want(n);
+        for (size_t i = 0; i < n; ++i) want[i] = (char)(i * 7 + 1);
+        (to_host ? dev : host) = want;
+        Rt rt(dev.data(), to_host, fail);
+        const bool ok = fh::copy_chunked(rt, host.data(), n, to_host);
+        for (auto& t : rt.dma) for (auto& d : t) CHECK(!d.flying);
+        if (ok) CHECK(host == want && dev == want);
+        if (fail < 0) CHECK(ok);
+        else if (rt.step > fail) CHECK(!ok);
+        else break;
+      }
+}
+""")
