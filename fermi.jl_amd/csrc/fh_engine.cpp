@@ -252,12 +252,12 @@ struct StagedCopy {
   void drain() { (void)hipStreamSynchronize(c.s); }
 };
 // Copy of n bytes between the device and pageable host memory in pinned chunks (copy_chunked; pages of new host memory
-// are made by four threads at once instead of one).  For copies of 4 MiB and more; false: not taken (memory that
+// are made by four threads at once instead of one).  false: not taken (chunks_pay, memory that
 // the runtime knows, which it copies directly, or no pinned memory).  Returns with the host memory free for other use.
 // (mu nu|la si) of two water molecules, 42 MB into new memory: 4.7 ms with one pageable copy, 2.2 ms so, 0.6 of them
 // kernels.
 static bool copy_staged(Ctx& c, char* dev, char* host, size_t n, bool to_host) {
-  if (n < ((size_t)4 << 20)) return false;
+  if (!chunks_pay(n, to_host)) return false;
   hipPointerAttribute_t at{};
   if (hipPointerGetAttributes(&at, host) == hipSuccess) {
     if (at.type != hipMemoryTypeUnregistered) return false;

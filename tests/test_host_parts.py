@@ -182,3 +182,15 @@ int main() {
       }
 }
 """)
+
+
+def test_chunked_copy_sizes(tmp_path):
+    """Copies in chunks from 4 MiB to the host and from 32 MiB to the device on."""
+    run_cpp(tmp_path, """
+int main() {
+  for (bool to_host : {false, true}) {
+    const size_t from = (size_t)(to_host ? 4 : 32) << 20;
+    CHECK(!fh::chunks_pay(from - 8, to_host) && fh::chunks_pay(from, to_host));
+  }
+}
+""")
