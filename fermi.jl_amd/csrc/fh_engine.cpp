@@ -61,6 +61,11 @@ void* Pool::get(size_t bytes) {
     (void)hipGetLastError();
     release_free();
     e = hipMalloc(&p, bytes);
+    if (e != hipSuccess && give_back) {
+      (void)hipGetLastError();
+      give_back();
+      e = hipMalloc(&p, bytes);
+    }
     if (e != hipSuccess) {
       (void)hipGetLastError();
       throw Error{-4, "out of device memory allocating " + std::to_string(bytes) + " bytes"};
@@ -114,7 +119,11 @@ struct BlasHandle {
   BlasHandle() = default;
   BlasHandle(const BlasHandle&) = delete;
   BlasHandle& operator=(const BlasHandle&) = delete;
-  ~BlasHandle() { if (h) (void)rocblas_destroy_handle(h); }
+  ~BlasHandle() { reset(); }
+  void reset() {
+    if (h) (void)rocblas_destroy_handle(h);
+    h = nullptr;
+  }
 };
 
 // Pinned chunks for large copies between the device and pageable host memory (copy_staged): 16 MiB a context, made by
@@ -153,7 +162,8 @@ struct Ctx {
   int device = 0;
   hipStream_t s = nullptr;
   std::unique_ptr<HostStage> stage;
-  BlasHandle blas;   // of the eigensolver, made on first use
+  BlasHandle blas;   // of the eigensolver, made on first use; given back when an allocation would fail and no solver lives
+  int solvers = 0;
   // declared before every Buf member, so that it is destroyed after all of them
   std::unique_ptr<Pool> pool;
   int o = 0, v = 0, naux = 0;
@@ -1044,19 +1054,25 @@ struct DIIS {
 // A (n x n, column-major) is overwritten by the eigenvectors, w gets the eigenvalues ascending, as
 // eigen(Symmetric(A), sortby = x -> x) orders them.
 //
-// Up to n = 1024 the context keeps the rocBLAS handle and with it the solver's workspace (a few n^2 doubles), which a
-// handle of one call allocates and frees each time; above, a handle lives as long as the solver.
+// Up to n = 1024 the context keeps the rocBLAS handle and with it the solver's workspace (some 170 MiB), which a
+// handle of one call allocates and frees each time, until an allocation would fail (Pool::give_back); above, a handle
+// lives as long as the solver.
 //
 // From n = 3 to 160, what a workgroup's registers hold, the matrix is made tridiagonal and the eigenvectors of T turned
 // back by fh_eigen.hip, rocSOLVER does what lies between: n = 96 0.15 + 0.03 ms for the two against 0.62 + 0.2 in dsyevd,
 // the whole SCF of 24, 64, 96, 128, 160 functions 7.0, 10.5, 13.6, 16.9, 21.0 ms against 10.7, 21.8, 20.5, 26.9, 36.9.
 struct Eigen {
   Ctx& c;
+  struct Alive {
+    int& n;
+    explicit Alive(int& m) : n(m) { ++n; }
+    ~Alive() { --n; }
+  } alive;
   BlasHandle own;
   rocblas_handle h = nullptr;
   Buf work, info, tau, Z;
   int n;
-  Eigen(Ctx& cc, int nn) : c(cc), n(nn) {
+  Eigen(Ctx& cc, int nn) : c(cc), alive(cc.solvers), n(nn) {
     BlasHandle& b = n <= 1024 ? c.blas : own;
     if (!b.h) FH_CHECK(rocblas_create_handle(&b.h) == rocblas_status_success, -2, "rocblas_create_handle failed");
     h = b.h;
@@ -1626,6 +1642,11 @@ int fh_create(fh_ctx** out, int device) {
     auto* x = new fh_ctx();
     x->c.device = device;
     x->c.pool.reset(new Pool(device));
+    x->c.pool->give_back = [c = &x->c] {
+      if (c->solvers || !c->blas.h) return;
+      (void)hipStreamSynchronize(c->s);
+      c->blas.reset();
+    };
     hipError_t e = hipStreamCreateWithFlags(&x->c.s, hipStreamNonBlocking);
     if (e != hipSuccess) { delete x; throw Error{-2, std::string("hipStreamCreate: ") + hipGetErrorString(e)}; }
     try {

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <cstdint>
 #include <cstddef>
+#include <functional>
 #include <string>
 #include <vector>
 #include <map>
@@ -30,7 +31,7 @@ void set_error(const std::string& m);
 
 // ---------------------------------------------------------------- device memory pool
 // Size-bucketed caching allocator: buffers are returned to a free list and reused;
-// nothing is released to HIP until the pool is destroyed.
+// nothing is released to HIP until the pool is destroyed or an allocation would fail.
 class Pool {
  public:
   explicit Pool(int device) : device_(device) {}
@@ -40,6 +41,8 @@ class Pool {
   size_t in_use() const { return in_use_; }
   size_t peak() const { return peak_; }
   void release_free();
+  // what else can be freed when an allocation still fails without the free list
+  std::function<void()> give_back;
  private:
   int device_;
   std::multimap<size_t, void*> free_;
