@@ -602,14 +602,14 @@ static void prepare_ladder(Ctx& c) {
     // (ca|db) for a block of a and every b up to its last, at most 1 GiB at a time
     const int64_t na = std::max<int64_t>(1, std::min<int64_t>(((int64_t)1 << 27) / (v * v * v), std::max<int64_t>(8, v / 8)));
     Timer t(c, "integrals_vvvv", 1.0 * Q * (double)(v * v * v * v));
-    c.Vs = dalloc(c, 2 * ldv * np);
-    Buf T = dalloc(c, std::min(na, v) * v * v * v);
+    Buf Vs = dalloc(c, 2 * ldv * np), T = dalloc(c, std::min(na, v) * v * v * v);
     for (int64_t a0 = 0; a0 < v; a0 += na) {
       const int64_t m = std::min(na, v - a0);
       gemm_f64(c.s, true, false, v * m, v * (a0 + m), Q, 1.0, c.Bvv.d() + Q * v * a0, Q, 0, c.Bvv.d(), Q, 0, 0.0, nullptr, 0,
                0, T.d(), v * m, 0);
-      vv_pairs(c.s, (int)v, (int)a0, (int)m, T.d(), v, v * m, v * v * m, false, c.Vs.d());
+      vv_pairs(c.s, (int)v, (int)a0, (int)m, T.d(), v, v * m, v * v * m, false, Vs.d());
     }
+    c.Vs = std::move(Vs);   // only whole: T may have failed to be allocated
   }
   c.Pt = dalloc(c, v * v * v * o);
   perm(c, tv(c.OVVV.d(), {o, v, v, v}), "kdac", tv(c.Pt.d(), {v, v, v, o}), "cdak", 1.0, 0.0);
