@@ -1,6 +1,7 @@
 """A residual whose first call runs out of device memory while it makes its constants: the next call makes them, and is
 held to the oracle at 1e-12 as in the other residual tests."""
 import ctypes
+import gc
 
 import pytest
 
@@ -20,21 +21,35 @@ def test_ladder_operand_after_a_failed_call():
     T1, T2 = random_amplitudes(o, v, 2)
     n1, n2 = R.update_amp(T1, T2, R.build_moints(Boo, Bov, Bvv), eo, ev)
     hip = _hip()
+    gc.collect()   # contexts of other tests
     c = fermihip.Context(0)
     c.set_df(eo, ev, Boo, Bov, Bvv)
     c.energy(T1, T2)   # the integral blocks
     ballast = []
+
+    def take(n):
+        p = ctypes.c_void_p()
+        if hip.hipMalloc(ctypes.byref(p), n) != 0:
+            hip.hipGetLastError()
+            return None
+        return p
+
     try:
-        while True:
-            a, b = ctypes.c_size_t(), ctypes.c_size_t()
-            assert hip.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
-            n = min(a.value - left, 16 << 30)
-            if n < 4 << 20:
-                break
-            p = ctypes.c_void_p()
-            assert hip.hipMalloc(ctypes.byref(p), n) == 0
-            ballast.append(p)
-        print(f"  free: {a.value >> 20} MiB", flush=True)
+        # all but 6 GB, then ever smaller pieces, each only where `left` is still to be had with it
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        ballast.append(take(a.value - (6 << 30)))
+        n = 2 << 30
+        while n >= 16 << 20:
+            p = take(n + left)
+            if p is None:
+                n //= 2
+                continue
+            hip.hipFree(p)
+            ballast.append(take(n))
+        p = take(left)
+        assert p is not None
+        hip.hipFree(p)
         with pytest.raises(fermihip.FermiException, match="out of device memory"):
             c.update_amp(T1, T2)
     finally:
