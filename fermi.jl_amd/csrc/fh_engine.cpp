@@ -532,32 +532,10 @@ static void require_df(Ctx& c, bool full = true) {
   FH_CHECK(!full || !c.ov_only, -6, "only Bov was given to fh_set_df: this entry point needs Boo and Bvv too");
 }
 
-// L[k,c,l,d] = 2 (kc|ld) - (kd|lc) and the exchange block (kd|lc), the ring products' constants
-static void build_lx(Ctx& c) {
-  const int64_t o = c.o, v = c.v;
-  c.LX = dalloc(c, 2 * c.n2());
-  TView ovov = tv(c.OVOV.d(), {o, v, o, v});
-  perm(c, ovov, "kdlc", tv(c.LX.d() + c.n2(), {o, v, o, v}), "kcld", 1.0, 0.0);
-  d2d(c, c.LX.d(), c.LX.d() + c.n2(), c.n2());
-  axpby_f64(c.s, c.n2(), 2.0, c.OVOV.d(), -1.0, c.LX.d());
-  c.LX32.reset();
-  c.Lkl = dalloc(c, c.n2());
-  perm(c, tv(c.LX.d(), {o, v, o, v}), "kcld", tv(c.Lkl.d(), {o, o, v, v}), "klcd", 1.0, 0.0);
-  c.Okl = dalloc(c, o * o * o * v);
-  perm(c, tv(c.OOOV.d(), {o, o, o, v}), "kilc", tv(c.Okl.d(), {o, o, o, v}), "klic", 1.0, 0.0);
-  c.Lo1 = dalloc(c, o * o * o * v);
-  perm(c, tv(c.OOOV.d(), {o, o, o, v}), "kilc", tv(c.Lo1.d(), {o, v, o, o}), "lcki", 2.0, 0.0);
-  perm(c, tv(c.OOOV.d(), {o, o, o, v}), "likc", tv(c.Lo1.d(), {o, v, o, o}), "lcki", -1.0, 1.0);
-  c.L1 = dalloc(c, c.n2());
-  d2d(c, c.L1.d(), c.OVOV.d(), c.n2());
-  perm(c, tv(c.OOVV.d(), {o, o, v, v}), "kiac", tv(c.L1.d(), {o, v, o, v}), "kcia", -1.0, 2.0);
-}
-
 static void prepare(Ctx& c) {
   require_df(c);
   if (c.prepared) return;
   if (c.conventional) {  // the blocks came with fh_set_mo
-    build_lx(c);
     c.prepared = true;
     return;
   }
@@ -578,14 +556,38 @@ static void prepare(Ctx& c) {
   contract(c, 1.0, Boo, "Qij", Bvv, "Qab", 0.0, tv(c.OOVV.d(), {o, o, v, v}), "ijab");
   contract(c, 1.0, Bov, "Qia", Bov, "Qjb", 0.0, tv(c.OVOV.d(), {o, v, o, v}), "iajb");
   contract(c, 1.0, Bov, "Qia", Bvv, "Qbc", 0.0, tv(c.OVVV.d(), {o, v, v, v}), "iabc");
-  build_lx(c);
-  c.Vs.reset();   // the ladder operands follow on first use (prepare_ladder)
+  c.L1.reset();   // the residual's constants follow on first use (prepare_rings, prepare_ladder)
+  c.Vs.reset();
   c.Vs32.reset();
   c.Pt.reset();
   c.opcache.clear();  // copies of the previous blocks
   c.opcache_bytes = 0;
   c.prepared = true;
   c.lowp = keep;
+}
+
+// The residual's constants of the blocks without VVVV (built on the first residual; (T) does not need them, 4 o^2 v^2 of
+// memory): L[k,c,l,d] = 2 (kc|ld) - (kd|lc) and the exchange block (kd|lc) of the ring products, and the forms below them.
+static void prepare_rings(Ctx& c) {
+  prepare(c);
+  if (c.L1.p) return;   // the last one
+  const int64_t o = c.o, v = c.v;
+  c.LX = dalloc(c, 2 * c.n2());
+  TView ovov = tv(c.OVOV.d(), {o, v, o, v});
+  perm(c, ovov, "kdlc", tv(c.LX.d() + c.n2(), {o, v, o, v}), "kcld", 1.0, 0.0);
+  d2d(c, c.LX.d(), c.LX.d() + c.n2(), c.n2());
+  axpby_f64(c.s, c.n2(), 2.0, c.OVOV.d(), -1.0, c.LX.d());
+  c.LX32.reset();
+  c.Lkl = dalloc(c, c.n2());
+  perm(c, tv(c.LX.d(), {o, v, o, v}), "kcld", tv(c.Lkl.d(), {o, o, v, v}), "klcd", 1.0, 0.0);
+  c.Okl = dalloc(c, o * o * o * v);
+  perm(c, tv(c.OOOV.d(), {o, o, o, v}), "kilc", tv(c.Okl.d(), {o, o, o, v}), "klic", 1.0, 0.0);
+  c.Lo1 = dalloc(c, o * o * o * v);
+  perm(c, tv(c.OOOV.d(), {o, o, o, v}), "kilc", tv(c.Lo1.d(), {o, v, o, o}), "lcki", 2.0, 0.0);
+  perm(c, tv(c.OOOV.d(), {o, o, o, v}), "likc", tv(c.Lo1.d(), {o, v, o, o}), "lcki", -1.0, 1.0);
+  c.L1 = dalloc(c, c.n2());
+  d2d(c, c.L1.d(), c.OVOV.d(), c.n2());
+  perm(c, tv(c.OOVV.d(), {o, o, v, v}), "kiac", tv(c.L1.d(), {o, v, o, v}), "kcia", -1.0, 2.0);
 }
 
 // The PP ladder's operands (built on the first residual; (T) does not need them): Vs[cd, ab] = (ca|db) +- (da|cb)
@@ -621,6 +623,7 @@ static void prepare_ladder(Ctx& c) {
 // (RCCSDHelper.jl:123-220), both without the diagonal Fock term.
 // t1_only: the T1 numerator alone (R2 is not touched)
 static void residual(Ctx& c, const double* t1p, const double* t2p, double* R1, double* R2, bool t1_only = false) {
+  prepare_rings(c);
   if (!t1_only) prepare_ladder(c);
   const int64_t o = c.o, v = c.v;
   const double o_ = (double)o, v_ = (double)v;

@@ -1,13 +1,34 @@
-"""What a context holds on the device: the eigensolver's rocBLAS workspace is given back when an allocation would fail."""
+"""What a context holds on the device: the (T) without the constants of the CCSD residual, and the eigensolver's rocBLAS
+workspace given back when an allocation would fail."""
 import ctypes
 
 import numpy as np
 import pytest
 
-from helpers import random_scf
+from helpers import random_amplitudes, random_df, random_scf
 from test_zz_no_alloc import _hip
 
 pytestmark = pytest.mark.gpu
+
+
+def test_triples_holds_no_residual_constants(monkeypatch):
+    """The peak of a (T) on new integrals, in doubles: B, the five blocks, T1 and T2, AV and Bcat twice each, (ia|jb) of
+    which a second copy is made by blocks, a chunk of W of 1 MiB, tables under 2 MiB; no other o^2 v^2 tensor."""
+    import fermihip
+    o, v, Q = 40, 24, 30
+    print(f"memory triples o={o} v={v}", flush=True)
+    monkeypatch.setenv("FERMIHIP_TRIPLES_CHUNK_MB", "1")
+    eo, ev, Boo, Bov, Bvv = random_df(o, v, Q, 3)
+    T1, T2 = random_amplitudes(o, v, 3)
+    c = fermihip.Context(0)
+    c.set_df(eo, ev, Boo, Bov, Bvv)
+    c.triples(T1, T2)
+    n2, nd = (o * v) ** 2, (o + v + 7) // 8 * 8
+    need = Q * (o + v) ** 2 + o**4 + o**3 * v + 2 * n2 + o * v**3 + n2 + 2 * v * v * o * nd + 2 * nd * v * o * o + 2 * n2
+    peak = c.stats()["pool_peak_bytes"]
+    c.close()
+    print(f"  peak {peak / 8 / n2:.2f} o^2 v^2, needed {need / n2:.2f}", flush=True)
+    assert peak < 8 * need + (3 << 20) + 0.3 * 8 * n2
 
 
 def test_failed_allocation_gives_the_eigensolver_workspace_back():
