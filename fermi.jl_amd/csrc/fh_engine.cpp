@@ -1539,8 +1539,7 @@ static double triples_t(Ctx& c, bool bf3, int64_t t0 = 0, int64_t nt = -1) {
     perm(c, tv(c.OVOV.d(), {o, v, o, v}), "iajb", tv(vvoo.d(), {v, v, o, o}), "abij", 1.0, 0.0);
     triples_block_vv(c.s, (int)o, (int)v, vvoo.d(), vvb.d());
   }
-  // the energy kernel reads whole 8 x 8 blocks of a panel: up to 56 elements past the end of the last slot
-  Buf Wbuf(c.pool.get(), (size_t)(triples_plane((int)v) * v * std::min(KC, ntot) + 64) * sizeof(T));
+  Buf Wbuf(c.pool.get(), (size_t)(triples_plane((int)v) * v * std::min(KC, ntot)) * sizeof(T));
   T* W = static_cast<T*>(Wbuf.p);
   Buf part = dalloc(c, norb * max_erun + 16);
   Buf acc = dalloc(c, 1);
@@ -2567,7 +2566,7 @@ struct MlpWork {
         dy(n->pool.get(), (size_t)B * sizeof(float)),
         dAZ(n->pool.get(), (size_t)(2 * n->h * B) * sizeof(float)),
         part(n->pool.get(), (size_t)mlp_partial_elems(n->h, B) * sizeof(float)),
-        lpart(n->pool.get(), (size_t)65536 * sizeof(double)) {}
+        lpart(n->pool.get(), (size_t)kMlpLossPartials * sizeof(double)) {}
 };
 
 int fh_mlp_loss_grad(fh_mlp* n, long long ns, const float* X, const float* T, double* loss, float* grad) {

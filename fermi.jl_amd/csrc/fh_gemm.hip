@@ -269,7 +269,10 @@ static void launch(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha,
 // add them; one tile with K = 1805 110 us uncut, 6 + 4 us cut.
 // A shape that leaves the chip under 256 workgroups even so is bound by the latency of a K step, about 1 us
 // whatever its depth: 32x32 tiles in K steps of 32 spread it over more CUs in a quarter of the steps (the products
-// of the residual at o = 5, v = 19: 10 us each with 64x64 tiles in steps of 8, 5 us so).
+// of the residual at o = 5, v = 19: 10 us each with 64x64 tiles in steps of 8, 5 us so).  So does every shape under
+// 1.5 tiles a CU with 32 < K <= 256, which has no K to cut and few steps to hide the latency of the first ones in: eight
+// CC iterations at o = 16, v = 76 11.2 ms against 11.5 with 64x64 tiles, the network's gradient of 8192 samples (layers
+// of K = 128) 219 us against 243; o = 5, v = 19, o = 10, v = 40 and o = 28, v = 133 the same either way.
 struct GemmPlan {
   bool small;
   int64_t slices;

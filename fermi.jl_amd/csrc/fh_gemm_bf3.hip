@@ -170,7 +170,7 @@ __global__ __launch_bounds__(256, BM == 128 ? 3 : 2) void k_gemm_bf3(int64_t M, 
   //   consecutive rows (a row stride of 4 rows would put every lane on the same few banks)
   // k-contiguous pattern:  k 4*(tid%KQ)..+3, rows tid/KQ + RS j, j < LB
   // The loads are branch-free: an element outside the operand is read at a clamped, valid
-  // address and replaced by zero, and the K segment is a pointer select, so that the loads of a
+  // address and replaced by zero, so that the loads of a
   // tile issue back to back.  A k tile entirely inside K (all but the last) skips the k tests.
   // operand values of the next k tile, loaded while the current one is multiplied
   V4 ra_s[KGA], rb_s[KL];
@@ -192,8 +192,7 @@ __global__ __launch_bounds__(256, BM == 128 ? 3 : 2) void k_gemm_bf3(int64_t M, 
   // (row-contiguous) or as column offsets (k-contiguous).  A full k tile then costs one pointer
   // per k column (row-contiguous) or per row (k-contiguous) and an add per element.
   constexpr int NA = TA ? KG : 1, NB = TB ? 1 : LB;
-  // row-contiguous: the thread's row (M, N < 2^31, checked at launch); k-contiguous: ld * row,
-  // per segment
+  // row-contiguous: the thread's row (M, N < 2^31, checked at launch); k-contiguous: ld * row
   int arow = 0, brow = 0;
   int64_t aoff[TA ? KG : 1], boff[TB ? 1 : LB];
   bool ain[NA], bin[NB];
@@ -222,7 +221,7 @@ __global__ __launch_bounds__(256, BM == 128 ? 3 : 2) void k_gemm_bf3(int64_t M, 
     }
   }
   // row-contiguous pattern: row tid & 127 of the tile, 8-wide k chunks kc0 + 2 q (q < BK / 16):
-  // kc0 = tid >> 7 is the same for a whole wavefront, so a chunk's column pointer, segment and
+  // kc0 = tid >> 7 is the same for a whole wavefront, so a chunk's column pointer and
   // stride are uniform, the loads of one k are coalesced across the lanes' consecutive rows, and
   // each lane stores 16 contiguous bytes per plane to LDS
   const int kc0 = tid >> 7;

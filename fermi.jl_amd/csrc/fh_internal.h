@@ -158,7 +158,8 @@ int64_t mlp_partial_elems(int h, int64_t B);  // floats of the bias-gradient scr
 void mlp_forward(hipStream_t s, int h, const float* P, int64_t B, const float* X, float* A1, float* A2, float* A3,
                  float* y);
 // gradient G of L = 1/(2B) sum (y - T)^2 after mlp_forward; dy[B], dA/dZ [h,B] scratch; lpart gets
-// *nlpart partial sums of B*L (grid-sized, at most 65536 doubles)
+// *nlpart partial sums of B*L (at most kMlpLossPartials doubles, one a workgroup of the output layer's pass)
+constexpr int kMlpLossPartials = 1024;
 void mlp_backward(hipStream_t s, int h, const float* P, int64_t B, const float* X, const float* T, const float* A1,
                   const float* A2, const float* A3, const float* y, float* dy, float* dA, float* dZ, float* G,
                   float* part, double* lpart, int64_t* nlpart);

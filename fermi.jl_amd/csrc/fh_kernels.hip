@@ -1,6 +1,6 @@
 // Bandwidth-bound kernels of the DF-RCCSD(T) engine: tensor permutes, amplitude
 // updates with on-the-fly denominators, deterministic FP64 reductions, DIIS linear
-// combinations, the CC energy and the (T) energy epilogue.
+// combinations and the CC energy.
 //
 // Reductions are deterministic: every kernel writes one FP64 partial per workgroup
 // (fixed grid for a given length) and a single workgroup adds the partials in a fixed

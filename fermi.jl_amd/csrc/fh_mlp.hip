@@ -137,7 +137,7 @@ __global__ __launch_bounds__(256) void k_rowsum_final(int rows, int nb, const fl
 // Columns of a workgroup of these passes: 16 keep its chain of dependent adds at 8 for h = 128, and with up to 1024
 // workgroups the chip is full from B = 16 k on (h = 128, B = 8192: a separate row sum took 345 us with 4096 columns a
 // workgroup and 9 us with 64, tanh' 4 us; 5 us together so).
-static int64_t rowsum_cols(int64_t B) { return std::max<int64_t>(16, (B + 1023) / 1024); }
+static int64_t rowsum_cols(int64_t B) { return std::max<int64_t>(16, (B + kMlpLossPartials - 1) / kMlpLossPartials); }
 static int64_t rowsum_blocks(int64_t B) { return (B + rowsum_cols(B) - 1) / rowsum_cols(B); }
 
 static void rowsum_final(hipStream_t s, int rows, int64_t B, const float* part, float* out, float* out2 = nullptr) {
@@ -154,7 +154,7 @@ static int64_t wgrad_elems(int h, int64_t B) {
 }
 
 int64_t mlp_partial_elems(int h, int64_t B) {
-  const int64_t blocks = std::min<int64_t>((B + 15) / 16, 1024);   // >= rowsum_blocks of every batch up to B
+  const int64_t blocks = std::min<int64_t>((B + 15) / 16, kMlpLossPartials);   // >= rowsum_blocks of every batch up to B
   return blocks * (h + 1) + wgrad_elems(h, B);
 }
 
@@ -176,7 +176,7 @@ void mlp_backward(hipStream_t s, int h, const float* P, int64_t B, const float* 
   const MlpOffsets o = mlp_offsets(h);
   const int64_t cols = rowsum_cols(B), wl = wgrad_elems(h, B);
   const unsigned nb = (unsigned)rowsum_blocks(B);
-  float* work = part + std::min<int64_t>((B + 15) / 16, 1024) * (h + 1);   // behind the row sums
+  float* work = part + std::min<int64_t>((B + 15) / 16, kMlpLossPartials) * (h + 1);   // behind the row sums
   // output layer: dy, dZ3, g b3 and g b4 = sum dy; g w4 = A3 dy
   hipLaunchKernelGGL(k_out_back, dim3(nb), dim3(256), 0, s, h, B, cols, y, T, P + o.w4, A3, dy, dZ, part, lpart);
   *nlpart = nb;

@@ -294,7 +294,7 @@ __global__ __launch_bounds__(256) void k_triples_bv(int o, int v, int nd, const 
 }
 
 // ------------------------------------------------------------------ W build
-// slices: W slots that share a c before the next c (1, 4, 8 and 16 measured alike: 430 ms of slice launches at
+// slices: W slots that share a c before the next c (1, 4, 8 and 16: 441, 436, 434 and 437 ms of slice launches at
 // o = 40, v = 190)
 constexpr int kSlotGroup = 8;
 
@@ -1195,17 +1195,19 @@ TriplesTiles triples_tiles(int fmt, int o, int v, double nk) {
   auto tiles = [](int64_t n, int g, int per) { return (int)(((n + g - 1) / g + per - 1) / per); };
   if (fmt == 2) {
     // Tiles of up to 6 x 6 blocks of 32, and the 128 x 128 kernel (three workgroups per CU instead of two) where the
-    // slices' tiles come to 4 x 4 at most (the (T) of o = 14, v = 200, two tiles of 4 and 3 blocks: 57.8 ms with the
-    // 192 x 192 kernel, 52.8 so; a 160 x 160 kernel with a fourth ring slot for five blocks: 88.2 ms at o = 27, v = 131
-    // against 87.1).  The first launch has v^2 rows, and tiles of 4 blocks only where v fits one.
+    // slices' tiles come to 4 x 4 at most: slices at o = 14, v = 60, 97, 120, 200 0.61, 2.35, 3.84, 32.3 ms, with the
+    // 192 x 192 kernel 0.84, 2.95, 4.63, 41.6.  (A 160 x 160 kernel with a fourth ring slot for five blocks was 1 %
+    // slower at o = 27, v = 131.)  The first launch has v^2 rows, and tiles of 4 blocks only where v fits one.
     const int nblk = (v + 31) / 32, nt = tiles(v, 32, 6);
     t.grain = 32;
     t.per = 6;
     t.nb = nblk <= 4 * nt ? 2 : 3;
     t.nb_first = v <= 128 ? 2 : 3;
   } else {
-    // slices: the block count with the least padded area, wider tiles preferred (operand reuse: a tile reads
-    // 2 / NB of a block per block product)
+    // slices: the block count with the least padded area, wider tiles preferred (operand reuse: a tile reads 2 / NB of a
+    // block per block product, at 0.3 of a product's cost).  Of NB = 2 .. 6 at v = 19, 40, 62, 76, 100, 131 and 190
+    // it takes the fastest, FP64 and FP32, but for v = 131 in FP64 (3: 15.9 ms, 5: 14.2); others cost up to 2.3 times
+    // as much (v = 76 in FP64 5.5 ms with 5, 13.0 with 4)
     auto best = [&](int64_t m, int64_t n) {
       int nb = 2;
       double c0 = 1e300;
@@ -1238,10 +1240,9 @@ void triples_col_tiles(const TriplesTiles& t, int v, int i, int j, int k0, int n
   }
 }
 
-// 1 GiB of W a chunk (and 2048 slice tiles, four rounds of 512): the (T) of o = 40, v = 190 takes 1147, 1134,
-// 1100, 1061 and 1045 ms at 128, 256, 512, 1024 and 4096 MiB (fewer partial rounds), o = 27, v = 131 takes 126,
-// 114, 108, 106 and 108 ms (at 4096 the W written by the first launch no longer meets the second in the
-// memory-side cache).  FERMIHIP_TRIPLES_CHUNK_MB fixes it, for tests.
+// 1 GiB of W a chunk (and 2048 slice tiles, four rounds of 512): the (T) of o = 40, v = 190 takes 960, 830,
+// 782, 763 and 757 ms at 128, 256, 512, 1024 and 4096 MiB (fewer partial rounds), o = 27, v = 131 100,
+// 92.0, 86.4, 84.3 and 84.5 ms.  FERMIHIP_TRIPLES_CHUNK_MB fixes it, for tests.
 int64_t triples_chunk_slots(int v, int elem, const TriplesTiles& tt, int64_t ntot) {
   const int64_t slot = triples_plane(v) * v * elem, tiles = (int64_t)tt.nt * tt.nt * v;
   int64_t n = std::max(((int64_t)1 << 30) / slot, (2048 + tiles - 1) / tiles);
