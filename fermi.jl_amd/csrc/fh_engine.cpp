@@ -2015,6 +2015,7 @@ int fh_prepare(fh_ctx* x) {
   return guarded([&] {
     FH_CHECK(x != nullptr, -1, "null context");
     DeviceGuard g(x->c.device);
+    prepare_rings(x->c);
     prepare_ladder(x->c);
     FH_HIP(hipStreamSynchronize(x->c.s));
     flush_timers(x->c);

@@ -31,6 +31,21 @@ def test_triples_holds_no_residual_constants(monkeypatch):
     assert peak < 8 * need + (3 << 20) + 0.3 * 8 * n2
 
 
+def test_prepare_leaves_no_constants_to_the_first_residual():
+    """fh_prepare makes what the residual keeps. At o = v the tensors are o^4: five blocks, the ladder's two operands (one
+    (1 + 1/v)^2 / 2), the residual's six others and B, 3 x 30 o^2; tables and rounding under a tenth."""
+    import fermihip
+    o = v = 24
+    print(f"memory prepare o={o} v={v}", flush=True)
+    c = fermihip.Context(0)
+    c.set_df(*random_df(o, v, 30, 4))
+    c.prepare()
+    peak = c.stats()["pool_peak_bytes"] / (8 * o**4)
+    c.close()
+    print(f"  peak {peak:.1f} o^4", flush=True)
+    assert 0 <= peak - (12 + (1 + 1 / v) ** 2 / 2 + 90 / v**2) < 0.1
+
+
 def test_failed_allocation_gives_the_eigensolver_workspace_back():
     """(ij|kl) of 1000 occupied orbitals (8 TB) is refused (-4); what the device has free is then again what it had before
     the SCF, but for the small buffers of the two problems."""
