@@ -237,7 +237,7 @@ struct Timer {
 };
 
 // resolve recorded spans (call after the stream has been synchronised)
-static void flush_timers(Ctx& c) { c.spans.resolve(SIZE_MAX, add_span(c)); }
+static void flush_timers(Ctx& c) { c.spans.flush(add_span(c)); }
 
 static Buf dalloc(Ctx& c, int64_t n) { return Buf(c.pool.get(), (size_t)std::max<int64_t>(n, 1) * sizeof(double)); }
 struct StagedCopy {

@@ -24,8 +24,8 @@ void for_launches(int64_t items, int64_t each, int threads, F&& f) {
 
 // Timed spans on a stream: an event pair each, read back in the order in which the spans ended.  No more than kMax ended
 // spans wait for that: the next one takes the older half first, which waits for their work, behind which that of the
-// other half is queued, so that the device does not idle.  The events are used again, at most two for each
-// waiting and each open span: the (T) of o = 64, v = 320 has 23 000 spans in a call.
+// other half is queued, so that the device does not idle.  Within a call the events are used again, at most two for each
+// waiting and each open span (the (T) of o = 64, v = 320 has 23 000 spans); flush() leaves none.
 // Rt: Event, Stream and bool create(Event&), record(Event, Stream), wait(Event), elapsed(float& ms, Event, Event),
 // void destroy(Event).
 template <typename Rt>
@@ -36,13 +36,13 @@ class Spans {
     double flops = 0.0, bytes = 0.0;
     typename Rt::Event a{}, b{};
   };
-  static constexpr size_t kMax = 256;
+  static constexpr size_t kMax = 32;
   Spans() = default;
   Spans(const Spans&) = delete;
   Spans& operator=(const Spans&) = delete;
   ~Spans() {
     for (Span& p : ended_) give(p);
-    for (auto e : free_) Rt::destroy(e);
+    clear();
   }
   // false: no event could be had or recorded
   bool begin(Span& p, typename Rt::Stream s) {
@@ -64,7 +64,15 @@ class Spans {
     ended_.push_back(p);
     if (ended_.size() > kMax) resolve(kMax / 2, sink);
   }
-  // sink(span, ms) for the n spans that ended first (all: SIZE_MAX)
+  // sink(span, ms) for all ended spans
+  template <typename F>
+  void flush(F&& sink) {
+    resolve(ended_.size(), sink);
+    clear();
+  }
+
+ private:
+  // the n spans that ended first
   template <typename F>
   void resolve(size_t n, F&& sink) {
     for (; n > 0 && !ended_.empty(); --n) {
@@ -75,8 +83,10 @@ class Spans {
       give(p);
     }
   }
-
- private:
+  void clear() {
+    for (auto e : free_) Rt::destroy(e);
+    free_.clear();
+  }
   bool take(typename Rt::Event& e) {
     if (free_.empty()) return Rt::create(e);
     e = free_.back();
