@@ -126,42 +126,50 @@ struct BlasHandle {
   }
 };
 
-// Pinned chunks for large copies between the device and pageable host memory (copy_staged): 16 MiB a context, made by
-// its first such copy and freed with it.
+// Pinned chunks for large copies between the device and pageable host memory (copy_staged): 16 MiB, lent by the contexts
+// of the process to one another.  (One in each context cost its first such copy 2 ms.)
 struct HostStage {
   static constexpr int kThreads = 4;
   static constexpr size_t kChunk = (size_t)2 << 20;
-  char* buf[kThreads][2] = {};
+  const int device;
+  char* mem = nullptr;
   hipEvent_t ev[kThreads][2] = {};
-  HostStage() = default;
+  explicit HostStage(int d) : device(d) {}
   bool init() {
-    for (auto& t : buf)
-      for (char*& b : t) {
-        void* p = nullptr;
-        if (hipHostMalloc(&p, kChunk, hipHostMallocDefault) != hipSuccess) return false;
-        b = static_cast<char*>(p);
-      }
+    void* p = nullptr;
+    if (hipHostMalloc(&p, 2 * kThreads * kChunk, hipHostMallocDefault) != hipSuccess) return false;
+    mem = static_cast<char*>(p);
     for (auto& t : ev)
       for (hipEvent_t& e : t)
         if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
     return true;
   }
+  char* buf(int t, int k) { return mem + (2 * t + k) * kChunk; }
   HostStage(const HostStage&) = delete;
   HostStage& operator=(const HostStage&) = delete;
   ~HostStage() {
     for (auto& t : ev)
       for (hipEvent_t e : t)
         if (e) (void)hipEventDestroy(e);
-    for (auto& t : buf)
-      for (char* b : t)
-        if (b) (void)hipHostFree(b);
+    if (mem) (void)hipHostFree(mem);
   }
+};
+static IdlePool<HostStage>& stages() {
+  static auto* const p = new IdlePool<HostStage>;   // not torn down at exit, after the HIP runtime
+  return *p;
+}
+struct StageUser {
+  StageUser() { stages().enter(); }
+  ~StageUser() { stages().leave(); }
+  StageUser(const StageUser&) = delete;
+  StageUser& operator=(const StageUser&) = delete;
 };
 
 struct Ctx {
   int device = 0;
   hipStream_t s = nullptr;
-  std::unique_ptr<HostStage> stage;
+  StageUser stage_user;
+  size_t unstaged = 0;   // chunks_worth_making
   BlasHandle blas;   // of the eigensolver, made on first use; given back when an allocation would fail and no solver lives
   int solvers = 0;
   // declared before every Buf member, so that it is destroyed after all of them
@@ -244,6 +252,7 @@ struct StagedCopy {
   static constexpr int kThreads = HostStage::kThreads;
   static constexpr size_t kChunk = HostStage::kChunk;
   Ctx& c;
+  HostStage& st;
   char* dev;
   bool to_host;
   std::atomic<int> err{(int)hipSuccess};
@@ -251,18 +260,18 @@ struct StagedCopy {
     if (e != hipSuccess) err = (int)e;
     return e == hipSuccess;
   }
-  char* buf(int t, int k) { return c.stage->buf[t][k]; }
+  char* buf(int t, int k) { return st.buf(t, k); }
   bool enter() { return ok(hipSetDevice(c.device)); }
   bool start(int t, int k, size_t at, size_t n) {
     return ok(to_host ? hipMemcpyAsync(buf(t, k), dev + at, n, hipMemcpyDeviceToHost, c.s)
                       : hipMemcpyAsync(dev + at, buf(t, k), n, hipMemcpyHostToDevice, c.s));
   }
-  bool mark(int t, int k) { return ok(hipEventRecord(c.stage->ev[t][k], c.s)); }
-  bool wait(int t, int k) { return ok(hipEventSynchronize(c.stage->ev[t][k])); }
+  bool mark(int t, int k) { return ok(hipEventRecord(st.ev[t][k], c.s)); }
+  bool wait(int t, int k) { return ok(hipEventSynchronize(st.ev[t][k])); }
   void drain() { (void)hipStreamSynchronize(c.s); }
 };
 // Copy of n bytes between the device and pageable host memory in pinned chunks (copy_chunked; pages of new host memory
-// are made by four threads at once instead of one).  false: not taken (chunks_pay, memory that
+// are made by four threads at once instead of one).  false: not taken (chunks_pay, chunks_worth_making, memory that
 // the runtime knows, which it copies directly, or no pinned memory).  Returns with the host memory free for other use.
 // (mu nu|la si) of two water molecules, 42 MB into new memory: 4.7 ms with one pageable copy, 2.2 ms so, 0.6 of them
 // kernels.
@@ -274,19 +283,18 @@ static bool copy_staged(Ctx& c, char* dev, char* host, size_t n, bool to_host) {
   } else {
     (void)hipGetLastError();
   }
-  if (!c.stage) {
-    auto made = std::make_unique<HostStage>();
-    if (!made->init()) {
+  std::unique_ptr<HostStage> st = stages().take(c.device);
+  if (!st) {
+    if (!chunks_worth_making(c.unstaged, n, to_host)) return false;
+    st = std::make_unique<HostStage>(c.device);
+    if (!st->init()) {
       (void)hipGetLastError();
       return false;
     }
-    c.stage = std::move(made);
   }
-  StagedCopy rt{c, dev, to_host};
-  if (!copy_chunked(rt, host, n, to_host)) {
-    c.stage.reset();
-    FH_HIP((hipError_t)rt.err.load());
-  }
+  StagedCopy rt{c, *st, dev, to_host};
+  if (!copy_chunked(rt, host, n, to_host)) FH_HIP((hipError_t)rt.err.load());
+  stages().give(std::move(st));
   return true;
 }
 static void h2d(Ctx& c, double* d, const double* h, int64_t n) {

@@ -6,6 +6,8 @@
 #include <cstring>
 #include <deque>
 #include <exception>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <thread>
 #include <vector>
@@ -101,11 +103,54 @@ class Spans {
   std::vector<typename Rt::Event> free_;
 };
 
-// Sizes from which a copy in chunks is the faster one. To the host 4 MiB: 4.5, 12, 24 MiB into one array 232, 460, 750 us
-// against 277, 705, 1410, into new memory each time 310, 870, 1270 against 370, 1450, 2610. To the device 32 MiB: 6, 16,
-// 24, 40 MiB from one array 273, 537, 745, 1150 us against 204, 481, 697, 1420, from new memory 318, 590, 800, 1250
-// against 245, 600, 895, 1480.
-inline bool chunks_pay(size_t n, bool to_host) { return n >= ((size_t)(to_host ? 4 : 32) << 20); }
+// What several users of a process lend one another: take() gives an idle one (of a device) or none, give() keeps at most
+// kKeep of them idle, and the last user to leave frees those.
+template <typename T>
+class IdlePool {
+ public:
+  static constexpr size_t kKeep = 2;
+  void enter() {
+    std::lock_guard<std::mutex> g(m_);
+    ++users_;
+  }
+  void leave() {
+    std::vector<std::unique_ptr<T>> gone;
+    std::lock_guard<std::mutex> g(m_);
+    if (--users_ == 0) gone.swap(idle_);
+  }
+  std::unique_ptr<T> take(int device) {
+    std::lock_guard<std::mutex> g(m_);
+    for (auto& p : idle_)
+      if (p->device == device) {
+        std::swap(p, idle_.back());
+        std::unique_ptr<T> r = std::move(idle_.back());
+        idle_.pop_back();
+        return r;
+      }
+    return nullptr;
+  }
+  void give(std::unique_ptr<T> p) {
+    std::lock_guard<std::mutex> g(m_);
+    if (users_ > 0 && idle_.size() < kKeep) idle_.push_back(std::move(p));
+  }
+
+ private:
+  std::mutex m_;
+  int users_ = 0;
+  std::vector<std::unique_ptr<T>> idle_;
+};
+
+// Sizes from which a copy in chunks is the faster one, with the pinned buffers at hand. To the host 4 MiB: 4.5, 12, 24 MiB
+// into one array 232, 460, 750 us against 277, 705, 1410, into new memory each time 310, 870, 1270 against 370, 1450,
+// 2610. To the device 32 MiB: 6, 16, 24, 40 MiB from one array 273, 537, 745, 1150 us against 204, 481, 697, 1420,
+// from new memory 318, 590, 800, 1250 against 245, 600, 895, 1480.
+inline bool chunks_pay(size_t n, bool to_host) { return n >= (size_t)(to_host ? 4 : 32) << 20; }
+// Whether to make the buffers, which takes a millisecond: when the copies that missed them, this one among them, would
+// have gained as much (24 MiB to the host, five times that to the device).
+inline bool chunks_worth_making(size_t& missed, size_t n, bool to_host) {
+  missed += to_host ? n : n / 5;
+  return missed >= (size_t)24 << 20;
+}
 
 // Copy of n bytes between the device and host memory in chunks of Rt::kChunk through pinned buffers, two a thread, chunk i
 // by thread i mod Rt::kThreads: the DMA of a chunk runs while those before it are moved between the buffers and

@@ -191,12 +191,69 @@ int main() {
 
 
 def test_chunked_copy_sizes(tmp_path):
-    """Copies in chunks from 4 MiB to the host and from 32 MiB to the device on."""
+    """Copies in chunks from 4 MiB to the host and from 32 MiB to the device on; the buffers are made for one copy of 24 or
+    120 MiB or for several that come to as much."""
     run_cpp(tmp_path, """
 int main() {
+  const size_t M = (size_t)1 << 20;
   for (bool to_host : {false, true}) {
-    const size_t from = (size_t)(to_host ? 4 : 32) << 20;
+    const size_t from = (to_host ? 4 : 32) * M, once = (to_host ? 24 : 120) * M;
     CHECK(!fh::chunks_pay(from - 8, to_host) && fh::chunks_pay(from, to_host));
+    size_t missed = 0;
+    CHECK(!fh::chunks_worth_making(missed, once - 8, to_host));
+    missed = 0;
+    CHECK(fh::chunks_worth_making(missed, once, to_host) && fh::chunks_worth_making(missed, from, to_host));
   }
+  size_t missed = 0;
+  CHECK(!fh::chunks_worth_making(missed, 11 * M, true) && !fh::chunks_worth_making(missed, 40 * M, false));
+  CHECK(fh::chunks_worth_making(missed, 5 * M, true));
+}
+""")
+
+
+def test_idle_pool(tmp_path):
+    """Lent objects: one user at a time, of the device asked for, no more than two idle, none after the last user left; from
+    eight threads as from one."""
+    run_cpp(tmp_path, """
+#include <atomic>
+static std::atomic<int> alive{0};
+struct Thing {
+  const int device;
+  std::atomic<int> held{0};
+  explicit Thing(int d) : device(d) { ++alive; }
+  ~Thing() { --alive; }
+};
+int main() {
+  fh::IdlePool<Thing> pool;
+  pool.enter();
+  CHECK(!pool.take(0));
+  for (int d : {0, 1, 1}) pool.give(std::make_unique<Thing>(d));
+  CHECK(alive == 2 && !pool.take(2));
+  auto a = pool.take(1);
+  CHECK(a && a->device == 1 && !pool.take(1));
+  pool.give(std::move(a));
+  pool.enter();
+  pool.leave();
+  CHECK(alive == 2);
+  a = pool.take(0);
+  pool.leave();
+  CHECK(alive == 1);
+  pool.give(std::move(a));   // nobody is left to lend it to
+  CHECK(alive == 0 && !pool.take(0));
+  std::vector<std::thread> th;
+  for (int t = 0; t < 8; ++t)
+    th.emplace_back([&, t] {
+      for (int r = 0; r < 2000; ++r) {
+        pool.enter();
+        auto p = pool.take(t % 2);
+        if (!p) p = std::make_unique<Thing>(t % 2);
+        CHECK(p->device == t % 2 && p->held++ == 0);
+        p->held--;
+        pool.give(std::move(p));
+        pool.leave();
+      }
+    });
+  for (auto& x : th) x.join();
+  CHECK(alive == 0);
 }
 """)
