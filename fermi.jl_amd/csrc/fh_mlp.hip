@@ -13,6 +13,7 @@
 // Features of amplitude (i,j,a,b): T2_MP2[i,j,a,b], eps_i, eps_j, eps_a, eps_b, d_ij (occupied pair
 // distance), each standardised with the model's (mean, 1/scale); the network predicts
 // (T2_CCSD - T2_MP2) / y_scale, and the guess is symmetrised in (ij)(ab).
+#include "fh_host.h"
 #include "fh_internal.h"
 
 #include <algorithm>
@@ -336,7 +337,8 @@ __global__ __launch_bounds__(256, 2) void k_t2_mlp_fused(int o, int v, int64_t n
   __shared__ float Xs[kFN][6];
   __shared__ float red[2][kFN];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, wm = wid & 1, wn = wid >> 1;
-  const int64_t e0 = (int64_t)blockIdx.x * kFN;
+  const int64_t e0 = (blockIdx.x + (int64_t)gridDim.x * blockIdx.y) * kFN;
+  if (e0 >= n) return;
   if (tid < kFN) {
     const int64_t e = e0 + tid;
     float f[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -465,8 +467,10 @@ void t2_mlp_fused(hipStream_t s, int o, int v, const double* t2, const double* e
   hipLaunchKernelGGL(k_mlp_split_w, dim3(64), dim3(256), 0, s, P, off.W2, off.W3, static_cast<uint32_t*>(wsplit));
   const int64_t n = (int64_t)o * o * v * v;
   const int64_t nb = (n + kFN - 1) / kFN;
-  FH_CHECK(nb < ((int64_t)1 << 31), -3, "t2_mlp_fused: too many amplitudes");
-  hipLaunchKernelGGL(k_t2_mlp_fused, dim3((unsigned)nb), dim3(256), 0, s, o, v, n, t2, eo, ev, dij, xm, xs, P, off,
+  // along two axes: one takes the workgroups of 2^31 amplitudes (max_workgroups)
+  const int64_t nx = std::min(nb, max_workgroups(256)), ny = (nb + nx - 1) / nx;
+  FH_CHECK(ny < 65536, -3, "t2_mlp_fused: too many amplitudes");
+  hipLaunchKernelGGL(k_t2_mlp_fused, dim3((unsigned)nx, (unsigned)ny), dim3(256), 0, s, o, v, n, t2, eo, ev, dij, xm, xs, P, off,
                      static_cast<const uint16_t*>(wsplit), Y);
   FH_HIP(hipGetLastError());
 }
