@@ -564,7 +564,7 @@ __device__ __forceinline__ void store_slice(const f32x16 (&acc)[MI][NJ], __amdgp
 // blocks are dealt to the two wave rows, so v = 131 costs 5 x 5 blocks, not 6 x 6; blocks, copies and
 // fragment reads beyond the edge are not issued.
 // Bound by the matrix cores at the rate the card sustains (a plain bf16 product of 8192^3 reaches 1122 TFLOP/s,
-// 374 for three products): o = 40, v = 190: first launch 344 to 359 TFLOP/s over boxes (on one 363 so and 345 with a
+// 374 for three products): o = 40, v = 190: first launch 344 to 359 TFLOP/s on several cards (on one 363 so and 345 with a
 // fastest over all of v in W, whose stores then begin inside a cache line; per-pair launches with row-major operands split
 // in the kernel: 224), slices 335 to 352 (on one 359 so and 336 with one W element a load and store; 224);
 // o = 27, v = 131: slices 202 (two batched launches of 128 x 192 tiles: 98).
@@ -884,9 +884,10 @@ __global__ __launch_bounds__(64 * triples_w_waves(NB), NB == 6 ? 3 : NB > 3 ? 4 
 // registers.  What does not depend on k ((ia|jb) and T1 of i and j) stays in registers.  A turn is two k (FP64 W: one): a
 // thread reads all it needs of a k from LDS, and the copies of the next turn run while it computes the last k (an LDS
 // read behind a copy in flight would be made to wait for it).
-// o = 40, v = 190, FP32 W: 95 ms per (T), 3.3 TB/s of W (103 on a slower box; 114 with a k a turn and copies of a dword per lane, 162 with a
-// fastest over all of v in W, rows of 8 a being a quarter of a cache line, and all nine (ia|jb) blocks of a pair copied,
-// 260 with one ordering per thread, V cubes in LDS and a reciprocal per element); o = 27, v = 131 10.7 (13.1, 17.7, 27.8);
+// o = 40, v = 190, FP32 W: 95 ms per (T), 3.3 TB/s of W (103 on a slower card; 114 with a k a turn and copies of a dword
+// per lane, 162 with a fastest over all of v in W, rows of 8 a being a quarter of a cache line, and all nine (ia|jb) blocks
+// of a pair copied, 260 with one ordering per thread, V cubes in LDS and a reciprocal per element); o = 27, v = 131 10.7
+// (13.1, 17.7, 27.8);
 // FP64 o = 16, v = 76 0.72 (0.83, 0.96, 1.5).  Bound by the copies' latency: three workgroups per CU (144 registers; at
 // 128, for four, the compiler's schedule takes 160 ms); the vector units are busy for a third of the time, LDS for half.
 static constexpr int CT = 8, CT3 = CT * CT * CT;
